@@ -881,6 +881,10 @@ struct TileLane {
     c0 = threadIdx.x / LANES_PER_ROW;
     valid = j < width ? min(4u, width - j) : 0u;
   }
+  // KEEP: leave the lines in the Infinity Cache (Softmax, [16,150,72,72] 28.9 -> 25.9 us);
+  // Normalize streams past it, which leaves it to the score maps of a detection head
+  // (the head's five operators 64.0 us, 66.9 us with the feature map kept).
+  template <bool KEEP>
   SHDW_DEVICE void load(const float* xs, v4f (&r)[kTilePerLane]) const {
     if (valid == 0) return;
 #pragma unroll
@@ -889,7 +893,7 @@ struct TileLane {
       if (c >= dim) continue;
       const float* src = xs + static_cast<uint64_t>(c) * inner + j;
       if (!TAIL || valid == 4) {
-        r[u] = __builtin_nontemporal_load(reinterpret_cast<const v4f_unaligned*>(src));
+        r[u] = KEEP ? load4_stream_any(src) : __builtin_nontemporal_load(reinterpret_cast<const v4f_unaligned*>(src));
       } else {
         r[u] = v4f{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -970,7 +974,7 @@ __global__ __launch_bounds__(kBlock) void normalize_tile_kernel(const float* x, 
   const uint64_t base = static_cast<uint64_t>(n) * dim * inner + p0;
   const TileLane<TS_SHIFT, ROWS> lane(width, dim, inner);
   v4f r[kTilePerLane];
-  lane.load(x + base, r);
+  lane.template load<false>(x + base, r);
   // the tile holds the terms of the sums, fp32 values that widen exactly: the folding wave's chain sets the
   // pace of a tall, narrow tile, and every instruction taken off it is time off the tile
   lane.park(lds, r, [p](const v4f& v) {
@@ -1087,7 +1091,7 @@ __global__ __launch_bounds__(kBlock) void softmax_tile_kernel(const float* x, fl
   const uint64_t base = static_cast<uint64_t>(n) * dim * inner + p0;
   const Lane lane(width, dim, inner);
   v4f r[kTilePerLane];
-  lane.load(x + base, r);
+  lane.template load<true>(x + base, r);
   if (lane.valid != 0) {
     v4f m = {-FLT_MAX, -FLT_MAX, -FLT_MAX, -FLT_MAX};
     bool nan[4] = {false, false, false, false};
