@@ -141,9 +141,9 @@ static int launch_rowparam(int n, int num, int inner, const float* x, const floa
 // stride walk of the general kernel: [8,64,112,112] + [1,64,1,1] 10.2 -> 9.1 us).
 // Any float pointers, any inner >= 1; the operand order f(a, b) is kept.
 template <class F, bool ROWVEC>
-__global__ __launch_bounds__(kStream) void rowbinary_vec_kernel(F f, const float* a, const float* b,
-                                                                float* y, uint32_t n4, uint32_t n,
-                                                                FastDiv inner, FastDiv num) {
+__global__ __launch_bounds__(kStream) void rowbinary_vec_kernel(const float* a, const float* b, float* y,
+                                                                uint32_t n4, uint32_t n, FastDiv inner,
+                                                                FastDiv num, F f) {
   const uint64_t* tab = uses_exp_table<F>::value ? libm::kExp2fTab : nullptr;
   auto param = [&](uint32_t e) {
     const uint32_t row = fd_div(e, inner);
@@ -188,10 +188,10 @@ struct BcastArgs {
 // extent is a multiple of 4.  AVEC/BVEC: the operand's innermost stride is 1
 // (128-bit load) rather than 0 (one scalar, replicated).
 template <class F, int NDIM, bool AVEC, bool BVEC>
-__global__ __launch_bounds__(kBlock) void bcast_vec_kernel(F f, BcastArgs p, const float* a,
-                                                            const float* b, float* y,
-                                                            uint32_t n4) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;  // 64 or 256 lanes, see the launch
+__global__ __launch_bounds__(kBlock) void bcast_vec_kernel(const float* a, const float* b, float* y,
+                                                            uint32_t n4, uint32_t lanes, BcastArgs p,
+                                                            F f) {
+  const uint32_t i = blockIdx.x * lanes + threadIdx.x;  // 64 or 256 lanes, see the launch
   // Pow reads the 2^(i/32) table; broadcast Pow is not a throughput case, the
   // table stays in global memory here.
   const uint64_t* tab = uses_exp_table<F>::value ? libm::kExp2fTab : nullptr;
@@ -251,10 +251,10 @@ SHDW_DEVICE void bcast_offsets(const BcastArgs& p, uint32_t e, uint32_t& oa, uin
 }
 
 template <class F, int NDIM>
-__global__ __launch_bounds__(kBlock) void bcast_flat_kernel(F f, BcastArgs p, const float* a,
-                                                             const float* b, float* y, uint32_t n4,
-                                                             uint32_t n) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;  // 64 or 256 lanes, see the launch
+__global__ __launch_bounds__(kBlock) void bcast_flat_kernel(const float* a, const float* b, float* y,
+                                                             uint32_t n4, uint32_t n, uint32_t lanes,
+                                                             BcastArgs p, F f) {
+  const uint32_t i = blockIdx.x * lanes + threadIdx.x;  // 64 or 256 lanes, see the launch
   const uint64_t* tab = uses_exp_table<F>::value ? libm::kExp2fTab : nullptr;
   const uint32_t last = p.fd[NDIM - 1].d;
   const int sa = p.sa[NDIM - 1], sb = p.sb[NDIM - 1];  // 0 or 1
@@ -306,13 +306,13 @@ static void launch_bcast_vec(F f, const BcastArgs& p, bool avec, bool bvec, cons
   const uint32_t lanes = (p.a_full || p.b_full) ? kStream : kBlock;
   const uint32_t grid = (n4 + lanes - 1) / lanes;
   if (avec && bvec)
-    bcast_vec_kernel<F, NDIM, true, true><<<grid, lanes, 0, st>>>(f, p, a, b, y, n4);
+    bcast_vec_kernel<F, NDIM, true, true><<<grid, lanes, 0, st>>>(a, b, y, n4, lanes, p, f);
   else if (avec)
-    bcast_vec_kernel<F, NDIM, true, false><<<grid, lanes, 0, st>>>(f, p, a, b, y, n4);
+    bcast_vec_kernel<F, NDIM, true, false><<<grid, lanes, 0, st>>>(a, b, y, n4, lanes, p, f);
   else if (bvec)
-    bcast_vec_kernel<F, NDIM, false, true><<<grid, lanes, 0, st>>>(f, p, a, b, y, n4);
+    bcast_vec_kernel<F, NDIM, false, true><<<grid, lanes, 0, st>>>(a, b, y, n4, lanes, p, f);
   else
-    bcast_vec_kernel<F, NDIM, false, false><<<grid, lanes, 0, st>>>(f, p, a, b, y, n4);
+    bcast_vec_kernel<F, NDIM, false, false><<<grid, lanes, 0, st>>>(a, b, y, n4, lanes, p, f);
 }
 
 template <class F>
@@ -338,9 +338,9 @@ static int launch_bcast(F f, const BroadcastPlan& plan, const float* a, const fl
     const FastDiv fi = make_fastdiv(static_cast<uint32_t>(inner)), fn = make_fastdiv(static_cast<uint32_t>(num));
     const uint32_t n4 = n / 4, grid = stream_grid(n4 + 1);
     if (inner % 4 == 0)
-      rowbinary_vec_kernel<F, true><<<grid, kStream, 0, st>>>(f, a, b, y, n4, n, fi, fn);
+      rowbinary_vec_kernel<F, true><<<grid, kStream, 0, st>>>(a, b, y, n4, n, fi, fn, f);
     else
-      rowbinary_vec_kernel<F, false><<<grid, kStream, 0, st>>>(f, a, b, y, n4, n, fi, fn);
+      rowbinary_vec_kernel<F, false><<<grid, kStream, 0, st>>>(a, b, y, n4, n, fi, fn, f);
     return launch_status();
   }
   const bool vec_ok = nd <= 4 && pl.dims[last] % 4 == 0 && aligned16(y) &&
@@ -379,14 +379,14 @@ static int launch_bcast(F f, const BroadcastPlan& plan, const float* a, const fl
     const uint32_t lanes = (p.a_full || p.b_full) ? kStream : kBlock;  // as in launch_bcast_vec
     const uint32_t grid = (n4 + 1 + lanes - 1) / lanes;
     switch (nd) {
-      case 1: bcast_flat_kernel<F, 1><<<grid, lanes, 0, st>>>(f, p, a, b, y, n4, n); break;
-      case 2: bcast_flat_kernel<F, 2><<<grid, lanes, 0, st>>>(f, p, a, b, y, n4, n); break;
-      case 3: bcast_flat_kernel<F, 3><<<grid, lanes, 0, st>>>(f, p, a, b, y, n4, n); break;
-      case 4: bcast_flat_kernel<F, 4><<<grid, lanes, 0, st>>>(f, p, a, b, y, n4, n); break;
-      case 5: bcast_flat_kernel<F, 5><<<grid, lanes, 0, st>>>(f, p, a, b, y, n4, n); break;
-      case 6: bcast_flat_kernel<F, 6><<<grid, lanes, 0, st>>>(f, p, a, b, y, n4, n); break;
-      case 7: bcast_flat_kernel<F, 7><<<grid, lanes, 0, st>>>(f, p, a, b, y, n4, n); break;
-      default: bcast_flat_kernel<F, 8><<<grid, lanes, 0, st>>>(f, p, a, b, y, n4, n); break;
+      case 1: bcast_flat_kernel<F, 1><<<grid, lanes, 0, st>>>(a, b, y, n4, n, lanes, p, f); break;
+      case 2: bcast_flat_kernel<F, 2><<<grid, lanes, 0, st>>>(a, b, y, n4, n, lanes, p, f); break;
+      case 3: bcast_flat_kernel<F, 3><<<grid, lanes, 0, st>>>(a, b, y, n4, n, lanes, p, f); break;
+      case 4: bcast_flat_kernel<F, 4><<<grid, lanes, 0, st>>>(a, b, y, n4, n, lanes, p, f); break;
+      case 5: bcast_flat_kernel<F, 5><<<grid, lanes, 0, st>>>(a, b, y, n4, n, lanes, p, f); break;
+      case 6: bcast_flat_kernel<F, 6><<<grid, lanes, 0, st>>>(a, b, y, n4, n, lanes, p, f); break;
+      case 7: bcast_flat_kernel<F, 7><<<grid, lanes, 0, st>>>(a, b, y, n4, n, lanes, p, f); break;
+      default: bcast_flat_kernel<F, 8><<<grid, lanes, 0, st>>>(a, b, y, n4, n, lanes, p, f); break;
     }
   }
   return launch_status();

@@ -97,8 +97,8 @@ struct ShuffleRows {
 
 // inner % 4 == 0 and 16-byte aligned pointers: lane i moves vector i.
 template <class MAP>
-__global__ __launch_bounds__(kStream) void rows_pick_kernel(MAP map, const float* x, float* y,
-                                                            uint32_t work, FastDiv f_inner) {
+__global__ __launch_bounds__(kStream) void rows_pick_kernel(const float* x, float* y, uint32_t work,
+                                                            FastDiv f_inner, MAP map) {
   const uint32_t i = blockIdx.x * kStream + threadIdx.x;
   if (i >= work) return;
   uint32_t r, p;
@@ -115,9 +115,8 @@ __global__ __launch_bounds__(kStream) void rows_pick_kernel(MAP map, const float
 // that looks up a row per element (below) waits for one dependent load after the
 // other (rows of 1: 17 us against 30 us per 17 MB gathered).
 template <class MAP>
-__global__ __launch_bounds__(kStream) void rows_pick_any_kernel(MAP map, const float* x, float* y,
-                                                                uint32_t work, uint32_t inner,
-                                                                FastDiv f_units) {
+__global__ __launch_bounds__(kStream) void rows_pick_any_kernel(const float* x, float* y, uint32_t work,
+                                                                uint32_t inner, FastDiv f_units, MAP map) {
   const uint32_t i = blockIdx.x * kStream + threadIdx.x;
   if (i >= work) return;
   uint32_t r, p;
@@ -142,8 +141,8 @@ __global__ __launch_bounds__(kStream) void rows_pick_any_kernel(MAP map, const f
 // (ShuffleChannel; with four floats of a row per lane, above, rows of 49 ran at 1.8 x,
 // rows of 7 at 3.1 x and rows of 1 at 2.7 x the time of a copy; here 1.4, 2.0, 1.1).
 template <class MAP>
-__global__ __launch_bounds__(kStream) void rows_pick_flat_kernel(MAP map, const float* x, float* y,
-                                                                 uint32_t n4, uint32_t n, FastDiv f_inner) {
+__global__ __launch_bounds__(kStream) void rows_pick_flat_kernel(const float* x, float* y, uint32_t n4, uint32_t n,
+                                                                 FastDiv f_inner, MAP map) {
   const uint32_t i = blockIdx.x * kStream + threadIdx.x;
   const uint32_t inner = f_inner.d;
   if (i < n4) {
@@ -176,16 +175,16 @@ static int launch_rows_pick(const MAP& map, int64_t rows, int inner, const float
                             hipStream_t st) {
   if (inner % 4 == 0 && aligned16(x) && aligned16(y)) {
     const uint32_t work = static_cast<uint32_t>(rows * (inner / 4));
-    rows_pick_kernel<MAP><<<stream_grid(work), kStream, 0, st>>>(map, x, y, work, make_fastdiv(inner / 4));
+    rows_pick_kernel<MAP><<<stream_grid(work), kStream, 0, st>>>(x, y, work, make_fastdiv(inner / 4), map);
   } else if (MAP::kFlat) {
     const uint32_t n = static_cast<uint32_t>(rows * inner), n4 = n / 4;
-    rows_pick_flat_kernel<MAP><<<stream_grid(n4 + 1), kStream, 0, st>>>(map, x, y, n4, n,
-                                                                       make_fastdiv(static_cast<uint32_t>(inner)));
+    rows_pick_flat_kernel<MAP><<<stream_grid(n4 + 1), kStream, 0, st>>>(x, y, n4, n,
+                                                                       make_fastdiv(static_cast<uint32_t>(inner)), map);
   } else {
     const uint32_t units = (static_cast<uint32_t>(inner) + 3) / 4;
     const uint32_t work = static_cast<uint32_t>(rows * units);
-    rows_pick_any_kernel<MAP><<<stream_grid(work), kStream, 0, st>>>(map, x, y, work, static_cast<uint32_t>(inner),
-                                                                  make_fastdiv(units));
+    rows_pick_any_kernel<MAP><<<stream_grid(work), kStream, 0, st>>>(x, y, work, static_cast<uint32_t>(inner),
+                                                                  make_fastdiv(units), map);
   }
   return launch_status();
 }

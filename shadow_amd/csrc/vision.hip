@@ -92,8 +92,8 @@ struct BatchNormScaleRows {
 
 // ROWVEC: inner % 4 == 0, the four elements of a vector share a row.
 template <class P, bool ROWVEC>
-__global__ __launch_bounds__(kStream) void rows_vec_kernel(P p, const float* x, float* out,
-                                                           uint32_t n4, uint32_t n, FastDiv inner) {
+__global__ __launch_bounds__(kStream) void rows_vec_kernel(const float* x, float* out, uint32_t n4,
+                                                           uint32_t n, FastDiv inner, P p) {
   const uint32_t i = blockIdx.x * kStream + threadIdx.x;
   if (i < n4) {
     const v4f vx = load4_stream_any(x + 4ull * i);
@@ -138,9 +138,9 @@ static int launch_rows(const P& p, uint32_t n, uint32_t inner, const float* x, c
   const uint32_t n4 = n / 4;  // any float pointers: the 128-bit accesses need dword alignment only
   const uint32_t grid = stream_grid(n4 + 1);
   if (inner % 4 == 0)
-    rows_vec_kernel<P, true><<<grid, kStream, 0, st>>>(p, x, out, n4, n, fi);
+    rows_vec_kernel<P, true><<<grid, kStream, 0, st>>>(x, out, n4, n, fi, p);
   else
-    rows_vec_kernel<P, false><<<grid, kStream, 0, st>>>(p, x, out, n4, n, fi);
+    rows_vec_kernel<P, false><<<grid, kStream, 0, st>>>(x, out, n4, n, fi, p);
   return launch_status();
 }
 
