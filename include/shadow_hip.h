@@ -292,6 +292,31 @@ int shdw_hip_batch_norm_scale_residual_relu(int n, int channel, int inner_num, c
                                             int residual_first, float* y, float* mean,
                                             void* stream);
 
+/* A gated block in one launch: an optional BatchNorm (stat_mean and stat_variance,
+ * global statistics), Scale (`scale` or `bias` or both) and ReLU (`relu` != 0) give
+ *   f = relu(((x - stat_mean[c]*scale_factor) / sqrt(|stat_variance[c]*scale_factor| + eps)) * scale[c] + bias[c]);
+ * the average of every (n, c) plane, the sigmoid of it and the product with f give
+ *   t = f * sigmoid(average(f));
+ * and, when `residual` is given, the residual tail of shdw_hip_scale_residual_relu
+ * with tail_scale and tail_bias (one of them at least) gives
+ *   y = relu((0 + 1*s) + 1*residual), s = t*tail_scale[c] + tail_bias[c];  mean[row] = average(y)
+ * (residual_first as there; `mean` may be NULL).  Without a residual y = t, and
+ * tail_scale, tail_bias and mean must be NULL.  Rows are the n / inner_num planes,
+ * c = row % channel; every per-channel array holds `channel` values, and NULL
+ * leaves its step out.  Every step is rounded as in the operators; the average of f
+ * is the fp32 sum in order of Pooling, the mean the fp64 sum of Reduce.  y may alias
+ * x or the residual.  inner_num > SHDW_SQUEEZE_GATE_MAX_INNER returns
+ * SHDW_E_UNSUPPORTED (a workgroup holds whole planes in LDS).
+ * ref: shadow/operators/kernels/{batch_norm,scale,activate,pooling,binary,reduce}.cpp,
+ *      eltwise.hpp:37-44 */
+#define SHDW_SQUEEZE_GATE_MAX_INNER 15360
+int shdw_hip_squeeze_gate(int n, int channel, int inner_num, const float* x,
+                          const float* stat_mean, const float* stat_variance,
+                          float scale_factor, float eps, const float* scale, const float* bias,
+                          int relu, const float* tail_scale, const float* tail_bias,
+                          const float* residual, int residual_first, float* y, float* mean,
+                          void* stream);
+
 /* ==================== neighbouring operators of the path ==================== */
 
 /* Axpy: out[r*inner_num + i] = y[..] + alpha[r] * x[..] for r < outer_num

@@ -40,7 +40,7 @@ HIP_FLAGS = [
     "-mllvm", "-amdgpu-kernarg-preload-count=16",
     "-Wno-unused-command-line-argument",
 ]
-HIP_SOURCES = ["elementwise.hip", "broadcast.hip", "reduce.hip", "fused.hip", "vision.hip", "softmax.hip", "norm.hip", "movers.hip",
+HIP_SOURCES = ["elementwise.hip", "broadcast.hip", "reduce.hip", "fused.hip", "gate.hip", "vision.hip", "softmax.hip", "norm.hip", "movers.hip",
                "lrn.hip", "grid_sample.hip", "runtime.hip"]
 
 def _run(cmd):

@@ -11,6 +11,11 @@
 //                          -> Activate(relu) [-> Reduce(AVG over the trailing axes)]
 //   BatchNorm(global statistics) -> Scale(blob parameters, one per channel) [-> Activate(relu)]
 //   Eltwise(any operation, any number of inputs) -> Activate(relu)
+//   [Scale or BatchNorm -> Scale, [-> Activate(relu)] ->] f, Pooling(global average of f)
+//                          -> Activate(sigmoid) -> Binary(MUL with f) [-> a residual tail]
+//
+// The last form takes groups of the other forms in as its front and its tail; where
+// the shapes of a run do not fit it, those still run as one launch each.
 //
 // A blob that a group no longer writes (the Scale output, the Eltwise output when
 // the Activate is not in place) must have the next member as its only reader and
@@ -40,12 +45,16 @@ class FusedGroup {
   // by one, which also reports whatever is wrong with them.
   virtual bool Run(Workspace* ws) = 0;
 
+  // Groups of some of the members, for a run whose shapes do not allow the whole.
+  const std::vector<std::unique_ptr<FusedGroup>>& parts() const { return parts_; }
+
   // "bn(Scale) + add(Eltwise) + relu(Activate) + gap(Reduce) -> e, pool"
   const std::string& describe() const { return description_; }
   void set_description(const std::string& text) { description_ = text; }
 
  protected:
   std::vector<int> members_;
+  std::vector<std::unique_ptr<FusedGroup>> parts_;
 
  private:
   std::string description_;
@@ -55,9 +64,13 @@ class FusedGroup {
 // the group does not have.  Found from the operators' parameters alone, so that the
 // matching can be checked without a device.
 struct FusedPlan {
-  enum Kind { kScaleRelu, kResidualTail, kBatchNormScale, kEltwiseRelu };
+  enum Kind { kScaleRelu, kResidualTail, kBatchNormScale, kEltwiseRelu, kSqueezeGate };
   Kind kind;
   int bn, scale, eltwise, relu, mean;
+  int pool = -1, gate = -1, mul = -1;  // kSqueezeGate
+  std::vector<FusedPlan> front, tail;  // kSqueezeGate: one group or none each
+  FusedPlan(Kind kind, int bn, int scale, int eltwise, int relu, int mean)
+      : kind(kind), bn(bn), scale(scale), eltwise(eltwise), relu(relu), mean(mean) {}
   std::vector<int> members() const;  // ascending
 };
 

@@ -30,6 +30,15 @@ class PoolingKernel : public Kernel {
                    int pad_h, int pad_w, bool full_pooling) = 0;
 };
 
+// What a Pooling operator tells a launch that stands for it (fusion.cpp).
+class GlobalPooling {
+ public:
+  virtual ~GlobalPooling() = default;
+  // The window of a global pooling over `input`, captured on the first run as
+  // Operator::Run captures it; the window is that of the first input ever after.
+  virtual const VecInt& global_window(const Blob& input) = 0;
+};
+
 }  // namespace Shadow
 
 #endif  // SHADOW_AMD_HOST_KERNELS_POOLING_HPP_

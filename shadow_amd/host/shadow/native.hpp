@@ -38,6 +38,7 @@ class Native : public Backend {
 
  private:
   void RunOperator(Operator* op);
+  void RunGroup(FusedGroup* group);
   void Initial(const shadow::NetParam& net_param);
   void SetInputData(const std::string& blob_name, const std::vector<int>& blob_shape,
                     const void* blob_data);

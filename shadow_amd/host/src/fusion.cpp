@@ -3,6 +3,7 @@
 #include <algorithm>
 #include <set>
 
+#include "shadow/kernels/pooling.hpp"
 #include "shadow_hip.h"
 
 namespace Shadow {
@@ -10,6 +11,9 @@ namespace Shadow {
 namespace {
 
 constexpr int kActivateRelu = 1;  // shadow/operators/kernels/activate.hpp:12
+constexpr int kActivateSigmoid = 3;
+constexpr int kBinaryMul = 2;     // shadow/operators/kernels/binary.hpp
+constexpr int kPoolingAverage = 1;
 constexpr int kEltwiseSum = 1;    // shadow/operators/kernels/eltwise.hpp:10
 constexpr int kReduceAvg = 4;     // shadow/operators/kernels/reduce.hpp:18
 
@@ -23,6 +27,7 @@ class Node {
   const shadow::OpParam& op_param() const { return op_param_; }
   const std::string& name() const { return op_param_.name(); }
   const std::string& type() const { return op_param_.type(); }
+  bool has_argument(const std::string& name) const { return arg_helper_.HasArgument(name); }
   template <typename T>
   T get_single_argument(const std::string& name, const T& default_value) const {
     return arg_helper_.GetSingleArgument<T>(name, default_value);
@@ -203,13 +208,37 @@ bool view_batch_norm(const Operator& op, Workspace* ws, NormView* v) {
   return true;
 }
 
-// The Scale behind a BatchNorm must work on the same channels: axis 1, one
-// parameter per channel.
-bool view_scale_per_channel(const Operator& scale, Workspace* ws, const NormView& n, ScaleView* v) {
-  if (!view_scale(scale, ws, v, n.x)) return false;
+// A Scale on the channels of x: axis 1, one parameter per channel, as the BatchNorm in
+// front of it has them.
+bool view_scale_per_channel(const Operator& scale, Workspace* ws, const std::shared_ptr<Blob>& x, ScaleView* v) {
+  if (!view_scale(scale, ws, v, x)) return false;
   int axis = scale.get_single_argument<int>("axis", 1);
-  if (axis < 0) axis += n.x->num_axes();
-  return axis == 1 && v->num == n.channel && v->inner == n.x->count(2);
+  if (axis < 0) axis += x->num_axes();
+  return axis == 1 && v->num == x->shape(1) && v->inner == x->count(2);
+}
+
+// The Reduce member's axes must be exactly the trailing run of `inner` elements one
+// Scale parameter applies to; the shape it gives its output, and that without the
+// reduced axes (keep_dims).
+bool view_mean(const Operator& op, const Blob& x, int inner, VecInt* shape, VecInt* squeezed) {
+  const int rank = x.num_axes();
+  VecInt axes = op.get_repeated_argument<int>("axes");
+  if (axes.empty())
+    for (int n = 0; n < rank; ++n) axes.push_back(n);
+  std::vector<bool> listed(rank, false);
+  for (int a : axes) {
+    if (a < -rank || a >= rank) return false;
+    listed[a < 0 ? a + rank : a] = true;
+  }
+  int first = rank;
+  while (first > 0 && listed[first - 1]) --first;
+  for (int n = 0; n < first; ++n)
+    if (listed[n]) return false;
+  if (first == rank || x.count(first) != inner) return false;
+  *shape = x.shape();
+  for (int n = first; n < rank; ++n) (*shape)[n] = 1;
+  squeezed->assign(shape->begin(), shape->begin() + first);
+  return true;
 }
 
 std::string label(const Node& op) { return op.name() + "(" + op.type() + ")"; }
@@ -261,7 +290,7 @@ class ResidualTail : public FusedGroup {
     ScaleView v;
     NormView n;
     if (bn_ != nullptr) {
-      if (!view_batch_norm(*bn_, ws, &n) || !view_scale_per_channel(*scale_, ws, n, &v)) return false;
+      if (!view_batch_norm(*bn_, ws, &n) || !view_scale_per_channel(*scale_, ws, n.x, &v)) return false;
     } else if (!view_scale(*scale_, ws, &v)) {
       return false;
     }
@@ -275,24 +304,7 @@ class ResidualTail : public FusedGroup {
       mean = float_blob(ws, mean_->op_param().top(0));
       if (mean == nullptr || mean == y || mean == v.x || mean == r) return false;
       if (mean == v.scale || mean == v.bias || mean == n.mean || mean == n.variance) return false;
-      // the reduced axes must be exactly the run one parameter applies to
-      const int rank = v.x->num_axes();
-      VecInt axes = mean_->get_repeated_argument<int>("axes");
-      if (axes.empty())
-        for (int n = 0; n < rank; ++n) axes.push_back(n);
-      std::vector<bool> listed(rank, false);
-      for (int a : axes) {
-        if (a < -rank || a >= rank) return false;
-        listed[a < 0 ? a + rank : a] = true;
-      }
-      int first = rank;
-      while (first > 0 && listed[first - 1]) --first;
-      for (int n = 0; n < first; ++n)
-        if (listed[n]) return false;
-      if (first == rank || v.x->count(first) != v.inner) return false;
-      mean_shape = v.x->shape();
-      for (int n = first; n < rank; ++n) mean_shape[n] = 1;
-      squeezed.assign(mean_shape.begin(), mean_shape.begin() + first);
+      if (!view_mean(*mean_, *v.x, v.inner, &mean_shape, &squeezed)) return false;
     }
     y->reshape(v.x->shape());
     if (mean != nullptr) mean->reshape(mean_shape);
@@ -333,7 +345,7 @@ class BatchNormScale : public FusedGroup {
   bool Run(Workspace* ws) override {
     NormView n;
     ScaleView v;
-    if (!view_batch_norm(*bn_, ws, &n) || !view_scale_per_channel(*scale_, ws, n, &v)) return false;
+    if (!view_batch_norm(*bn_, ws, &n) || !view_scale_per_channel(*scale_, ws, n.x, &v)) return false;
     const auto& last = relu_ != nullptr ? relu_ : scale_;
     auto y = float_blob(ws, last->op_param().top(0));
     if (y == nullptr || y == n.mean || y == n.variance || y == v.scale || y == v.bias) return false;
@@ -402,12 +414,158 @@ class EltwiseRelu : public FusedGroup {
   std::shared_ptr<Operator> eltwise_, relu_;
 };
 
+// ---- [Scale or BatchNorm -> Scale, [ReLU],] global average -> sigmoid -> product
+//      [-> Scale -> Eltwise(SUM) -> ReLU [-> Reduce(AVG)]]: shdw_hip_squeeze_gate ----
+// Pooling over the whole plane, average.
+bool is_plane_average(const Node& op) {
+  return op.type() == "Pooling" && op.get_single_argument<int>("pool", 0) == kPoolingAverage &&
+         op.get_single_argument<bool>("global_pooling", false) && op.op_param().bottom_size() == 1 &&
+         op.op_param().top_size() == 1 && op.op_param().top(0) != op.op_param().bottom(0);
+}
+
+bool is_sigmoid(const Node& op) {
+  return op.type() == "Activate" && op.get_single_argument<int>("type", 1) == kActivateSigmoid &&
+         op.op_param().bottom_size() == 1 && op.op_param().top_size() == 1;
+}
+
+// The product of the two blobs, in either order.
+bool is_product_of(const Node& op, const std::string& f, const std::string& g) {
+  if (op.type() != "Binary" || op.get_single_argument<int>("operation", -1) != kBinaryMul) return false;
+  const auto& p = op.op_param();
+  if (op.has_argument("scalar") || p.bottom_size() != 2 || p.top_size() != 1) return false;
+  return f != g && p.top(0) != g &&
+         ((p.bottom(0) == f && p.bottom(1) == g) || (p.bottom(0) == g && p.bottom(1) == f));
+}
+
+class SqueezeGate : public FusedGroup {
+ public:
+  SqueezeGate(const OpList& ops, const FusedPlan& plan, std::vector<std::unique_ptr<FusedGroup>> parts)
+      : pool_(ops[plan.pool]), mul_(ops[plan.mul]) {
+    members_ = plan.members();
+    parts_ = std::move(parts);
+    if (!plan.front.empty()) {
+      const FusedPlan& front = plan.front[0];
+      if (front.bn >= 0) bn_ = ops[front.bn];
+      scale_ = ops[front.scale];
+      front_relu_ = front.relu >= 0;
+    }
+    if (!plan.tail.empty()) {
+      const FusedPlan& tail = plan.tail[0];
+      tail_scale_ = ops[tail.scale], sum_ = ops[tail.eltwise], relu_ = ops[tail.relu];
+      if (tail.mean >= 0) mean_ = ops[tail.mean];
+      residual_first_ = sum_->op_param().bottom(1) == tail_scale_->op_param().top(0);
+    }
+  }
+
+  bool Run(Workspace* ws) override {
+    NormView n;
+    ScaleView v, t;
+    std::shared_ptr<Blob> x;
+    if (bn_ != nullptr) {
+      if (!view_batch_norm(*bn_, ws, &n)) return false;
+      x = n.x;
+    } else {
+      x = float_blob(ws, (scale_ != nullptr ? scale_ : pool_)->op_param().bottom(0));
+    }
+    if (x == nullptr || (x->num_axes() != 4 && x->num_axes() != 5) || x->count() == 0) return false;
+    const int inner = x->count(2);
+    if (inner > SHDW_SQUEEZE_GATE_MAX_INNER) return false;
+    if (scale_ != nullptr && !view_scale_per_channel(*scale_, ws, x, &v)) return false;
+    auto* pool = dynamic_cast<GlobalPooling*>(pool_.get());
+    if (pool == nullptr || pool->global_window(*x) != VecInt(x->shape().begin() + 2, x->shape().end())) return false;
+    auto y = float_blob(ws, (relu_ != nullptr ? relu_ : mul_)->op_param().top(0));
+    std::shared_ptr<Blob> r, mean;
+    VecInt mean_shape, squeezed;
+    if (sum_ != nullptr) {
+      if (!view_scale_per_channel(*tail_scale_, ws, x, &t)) return false;
+      r = float_blob(ws, sum_->op_param().bottom(residual_first_ ? 0 : 1));
+      if (r == nullptr || r->shape() != x->shape()) return false;
+    }
+    const auto parameter = [&](const std::shared_ptr<Blob>& b) {
+      return b == n.mean || b == n.variance || b == v.scale || b == v.bias || b == t.scale || b == t.bias;
+    };
+    if (y == nullptr || parameter(y)) return false;
+    if (mean_ != nullptr) {
+      mean = float_blob(ws, mean_->op_param().top(0));
+      if (mean == nullptr || mean == y || mean == x || mean == r || parameter(mean)) return false;
+      if (!view_mean(*mean_, *x, inner, &mean_shape, &squeezed)) return false;
+    }
+    y->reshape(x->shape());
+    if (mean != nullptr) mean->reshape(mean_shape);
+    const auto data = [](const std::shared_ptr<Blob>& b) { return b != nullptr ? b->data<float>() : nullptr; };
+    SHADOW_HIP_CHECK(shdw_hip_squeeze_gate(
+        x->count(), x->shape(1), inner, data(x), data(n.mean), data(n.variance), n.scale_factor, n.eps, data(v.scale),
+        data(v.bias), front_relu_ ? 1 : 0, data(t.scale), data(t.bias), data(r), residual_first_ ? 1 : 0,
+        y->mutable_data<float>(), mean != nullptr ? mean->mutable_data<float>() : nullptr, ws->Ctx()->stream()));
+    if (mean != nullptr && !mean_->get_single_argument<bool>("keep_dims", true)) mean->set_shape(squeezed);
+    return true;
+  }
+
+ private:
+  std::shared_ptr<Operator> bn_, scale_, pool_, mul_, tail_scale_, sum_, relu_, mean_;
+  bool front_relu_ = false, residual_first_ = false;
+};
+
+// The gate around the plane average at `pool`, or false.  A front and a tail found as
+// groups before are taken in where the blobs between them and the gate have no other use.
+bool plan_squeeze_gate(const NodeList& ops, const std::vector<std::string>& out_blob, int pool,
+                       const std::vector<FusedPlan>& groups, FusedPlan* plan, int* front_group, int* tail_group) {
+  const std::string &f = ops[pool].op_param().bottom(0), &squeezed = ops[pool].op_param().top(0);
+  const int act = next_reader(ops, squeezed, pool);
+  if (act < 0 || !is_sigmoid(ops[act]) || !sole_reader(ops, out_blob, squeezed, pool, act)) return false;
+  const std::string& g = ops[act].op_param().top(0);
+  const int mul = next_reader(ops, g, act);
+  if (mul < 0 || !is_product_of(ops[mul], f, g) || !sole_reader(ops, out_blob, g, act, mul)) return false;
+  if (last_writer(ops, f, mul) != last_writer(ops, f, pool)) return false;
+  const std::string& t = ops[mul].op_param().top(0);
+
+  // a front whose result only the average and the product read
+  int front = -1, tail = -1;
+  for (size_t k = 0; k < groups.size(); ++k) {
+    if (groups[k].kind != FusedPlan::kScaleRelu && groups[k].kind != FusedPlan::kBatchNormScale) continue;
+    const int last = groups[k].members().back();
+    if (last != last_writer(ops, f, pool)) continue;
+    bool alone = std::find(out_blob.begin(), out_blob.end(), f) == out_blob.end();
+    for (int j = last + 1; alone && j < static_cast<int>(ops.size()); ++j) {
+      alone = !reads(ops[j], f) || j == pool || j == mul;
+      if (writes(ops[j], f)) break;
+    }
+    if (alone) front = static_cast<int>(k);
+  }
+  // a residual tail that starts from the product alone
+  for (size_t k = 0; k < groups.size(); ++k) {
+    if (groups[k].kind != FusedPlan::kResidualTail || groups[k].bn >= 0) continue;
+    const int scale = groups[k].scale;
+    const auto& p = ops[scale].op_param();
+    if (p.bottom(0) != t || last_writer(ops, t, scale) != mul || !sole_reader(ops, out_blob, t, mul, scale)) continue;
+    bool as_parameter = false;
+    for (int j = 1; j < p.bottom_size(); ++j) as_parameter = as_parameter || p.bottom(j) == t;
+    if (!as_parameter) tail = static_cast<int>(k);
+  }
+  for (int choice = 0; choice < 4; ++choice) {  // both, the tail, the front, neither
+    const bool with_front = choice % 2 == 0, with_tail = choice < 2;
+    if ((with_front && front < 0) || (with_tail && tail < 0)) continue;
+    *plan = FusedPlan(FusedPlan::kSqueezeGate, -1, -1, -1, -1, -1);
+    plan->pool = pool, plan->gate = act, plan->mul = mul;
+    if (with_front) plan->front.push_back(groups[front]);
+    if (with_tail) plan->tail.push_back(groups[tail]);
+    if (!movable(ops, plan->members())) continue;
+    *front_group = with_front ? front : -1;
+    *tail_group = with_tail ? tail : -1;
+    return true;
+  }
+  return false;
+}
+
 }  // namespace
 
 std::vector<int> FusedPlan::members() const {
   std::vector<int> all;
-  for (int m : {bn, scale, eltwise, relu, mean})
+  for (int m : {bn, scale, eltwise, relu, mean, pool, gate, mul})
     if (m >= 0) all.push_back(m);
+  for (const auto* part : {&front, &tail})
+    for (const FusedPlan& plan : *part)
+      for (int m : plan.members()) all.push_back(m);
   std::sort(all.begin(), all.end());
   return all;
 }
@@ -512,6 +670,16 @@ std::vector<FusedPlan> PlanFusedGroups(const std::vector<shadow::OpParam>& op_pa
     groups.push_back(FusedPlan{FusedPlan::kEltwiseRelu, -1, -1, i, relu, -1});
     taken[i] = taken[relu] = true;
   }
+  // Gates last, around the groups found so far.
+  for (int i = 0; i < count; ++i) {
+    if (!is_plane_average(ops[i])) continue;
+    FusedPlan gate(FusedPlan::kSqueezeGate, -1, -1, -1, -1, -1);
+    int front = -1, tail = -1;
+    if (!plan_squeeze_gate(ops, out_blob, i, groups, &gate, &front, &tail)) continue;
+    for (int k : {std::max(front, tail), std::min(front, tail)})
+      if (k >= 0) groups.erase(groups.begin() + k);
+    groups.push_back(gate);
+  }
   std::sort(groups.begin(), groups.end(), [](const FusedPlan& a, const FusedPlan& b) {
     return a.members().back() < b.members().back();
   });
@@ -539,8 +707,47 @@ std::string DescribeFusedPlan(const FusedPlan& plan, const std::vector<shadow::O
       if (plan.mean >= 0) text += ", " + top(plan.mean);
       return text;
     }
+    case FusedPlan::kSqueezeGate: {
+      std::string text = name(plan.pool) + " + " + name(plan.gate) + " + " + name(plan.mul);
+      if (!plan.front.empty()) {
+        const FusedPlan& f = plan.front[0];
+        std::string front = (f.bn >= 0 ? name(f.bn) + " + " : "") + name(f.scale);
+        if (f.relu >= 0) front += " + " + name(f.relu);
+        text = front + " + " + text;
+      }
+      if (plan.tail.empty()) return text + " -> " + top(plan.mul);
+      return text + " + " + DescribeFusedPlan(plan.tail[0], op_params);
+    }
   }
   return "";
+}
+
+static std::unique_ptr<FusedGroup> MakeFusedGroup(const OpList& ops, const FusedPlan& plan,
+                                                  const std::vector<shadow::OpParam>& op_params) {
+  std::unique_ptr<FusedGroup> group;
+  switch (plan.kind) {
+    case FusedPlan::kScaleRelu:
+      group.reset(new ScaleRelu(ops, plan.scale, plan.relu));
+      break;
+    case FusedPlan::kEltwiseRelu:
+      group.reset(new EltwiseRelu(ops, plan.eltwise, plan.relu));
+      break;
+    case FusedPlan::kBatchNormScale:
+      group.reset(new BatchNormScale(ops, plan.bn, plan.scale, plan.relu));
+      break;
+    case FusedPlan::kResidualTail:
+      group.reset(new ResidualTail(ops, plan.bn, plan.scale, plan.eltwise, plan.relu, plan.mean));
+      break;
+    case FusedPlan::kSqueezeGate: {
+      std::vector<std::unique_ptr<FusedGroup>> parts;
+      for (const auto* part : {&plan.front, &plan.tail})
+        for (const FusedPlan& p : *part) parts.push_back(MakeFusedGroup(ops, p, op_params));
+      group.reset(new SqueezeGate(ops, plan, std::move(parts)));
+      break;
+    }
+  }
+  group->set_description(DescribeFusedPlan(plan, op_params));
+  return group;
 }
 
 std::vector<std::unique_ptr<FusedGroup>> FindFusedGroups(const OpList& ops,
@@ -548,25 +755,8 @@ std::vector<std::unique_ptr<FusedGroup>> FindFusedGroups(const OpList& ops,
   std::vector<shadow::OpParam> op_params;
   for (const auto& op : ops) op_params.push_back(op->op_param());
   std::vector<std::unique_ptr<FusedGroup>> groups;
-  for (const FusedPlan& plan : PlanFusedGroups(op_params, out_blob)) {
-    std::unique_ptr<FusedGroup> group;
-    switch (plan.kind) {
-      case FusedPlan::kScaleRelu:
-        group.reset(new ScaleRelu(ops, plan.scale, plan.relu));
-        break;
-      case FusedPlan::kEltwiseRelu:
-        group.reset(new EltwiseRelu(ops, plan.eltwise, plan.relu));
-        break;
-      case FusedPlan::kBatchNormScale:
-        group.reset(new BatchNormScale(ops, plan.bn, plan.scale, plan.relu));
-        break;
-      case FusedPlan::kResidualTail:
-        group.reset(new ResidualTail(ops, plan.bn, plan.scale, plan.eltwise, plan.relu, plan.mean));
-        break;
-    }
-    group->set_description(DescribeFusedPlan(plan, op_params));
-    groups.push_back(std::move(group));
-  }
+  for (const FusedPlan& plan : PlanFusedGroups(op_params, out_blob))
+    groups.push_back(MakeFusedGroup(ops, plan, op_params));
   return groups;
 }
 

@@ -1,5 +1,7 @@
 #include "shadow/native.hpp"
 
+#include <algorithm>
+
 #include "shadow/io.hpp"
 #include "shadow/parser.hpp"
 
@@ -119,6 +121,20 @@ void Native::RunOperator(Operator* op) {
   if (debug_) LOG(INFO) << op->debug_log(inputs, outputs);
 }
 
+void Native::RunGroup(FusedGroup* group) {
+  if (group->Run(ws_.get())) {
+    if (debug_) LOG(INFO) << "Fused: " << group->describe();
+    return;
+  }
+  for (int member : group->members()) {
+    FusedGroup* part = nullptr;
+    for (const auto& p : group->parts())
+      if (std::find(p->members().begin(), p->members().end(), member) != p->members().end()) part = p.get();
+    if (part == nullptr) RunOperator(ops_[member].get());
+    else if (part->members().back() == member) RunGroup(part);
+  }
+}
+
 void Native::Run(const std::map<std::string, void*>& data_map,
                  const std::map<std::string, std::vector<int>>& shape_map) {
   if (ops_.empty()) return;
@@ -138,14 +154,9 @@ void Native::Run(const std::map<std::string, void*>& data_map,
       continue;
     }
     // a group runs where its last member stands, as one launch; when the shapes of
-    // this run do not fit it, as its members one by one
+    // this run do not fit it, as its parts and its other members one by one
     auto& group = *groups_[g];
-    if (static_cast<int>(i) != group.members().back()) continue;
-    if (group.Run(ws_.get())) {
-      if (debug_) LOG(INFO) << "Fused: " << group.describe();
-    } else {
-      for (int member : group.members()) RunOperator(ops_[member].get());
-    }
+    if (static_cast<int>(i) == group.members().back()) RunGroup(&group);
   }
   if (debug_) LOG(INFO) << "Forward Network!";
 }

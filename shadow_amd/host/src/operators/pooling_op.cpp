@@ -21,7 +21,7 @@ inline VecInt expand_param(const VecInt& param, int num) {
   return param;
 }
 
-class PoolingOp : public Operator {
+class PoolingOp : public Operator, public GlobalPooling {
  public:
   PoolingOp(const shadow::OpParam& op_param, Workspace* ws) : Operator(op_param, ws) {
     pool_type_ = get_single_argument<int>("pool", 0);
@@ -50,10 +50,7 @@ class PoolingOp : public Operator {
     const int num_spatial_axes = input->num_axes() - 2;
     CHECK(num_spatial_axes == 2 || num_spatial_axes == 3) << "Only support 2D or 3D Pooling";
 
-    // The plane extents are captured on the first run only, as in the reference.
-    if (global_pooling_ && static_cast<int>(kernel_size_.size()) != num_spatial_axes) {
-      for (int n = 0; n < num_spatial_axes; ++n) kernel_size_.push_back(input->shape(n + 2));
-    }
+    if (global_pooling_) global_window(*input);
     const auto kernel_size = expand_param(kernel_size_, num_spatial_axes);
     const auto stride = expand_param(stride_, num_spatial_axes);
     const auto pad = expand_param(pad_, num_spatial_axes);
@@ -72,6 +69,15 @@ class PoolingOp : public Operator {
       kernel_->Run(input, output, ws_, pool_type_, kernel_size[0], kernel_size[1], kernel_size[2],
                    stride[0], stride[1], stride[2], pad[0], pad[1], pad[2], full_pooling_);
     }
+  }
+
+  // The plane extents are captured on the first run only, as in the reference.
+  const VecInt& global_window(const Blob& input) override {
+    const int num_spatial_axes = input.num_axes() - 2;
+    if (static_cast<int>(kernel_size_.size()) != num_spatial_axes) {
+      for (int n = 0; n < num_spatial_axes; ++n) kernel_size_.push_back(input.shape(n + 2));
+    }
+    return kernel_size_;
   }
 
  private:

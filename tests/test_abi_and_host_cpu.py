@@ -176,6 +176,15 @@ def test_entry_points_validate_before_touching_the_device():
     assert lib.shdw_hip_batch_norm_scale_residual_relu(16, 2, 8, p, p, p, 1.0, 0.0, p, p, None, 0, p, p, None) == E
     assert lib.shdw_hip_batch_norm_scale_residual_relu(15, 2, 8, p, p, p, 1.0, 0.0, p, p, p, 0, p, p, None) == E
     assert lib.shdw_hip_batch_norm_scale_residual_relu(0, 2, 8, p, p, p, 1.0, 0.0, p, p, p, 0, p, p, None) == 0
+    gate = lib.shdw_hip_squeeze_gate
+    assert gate(16, 2, 8, p, p, None, 1.0, 0.0, p, p, 1, p, p, p, 0, p, p, None) == E       # half of the statistics
+    assert gate(16, 2, 8, p, p, p, 1.0, 0.0, p, p, 1, None, None, p, 0, p, p, None) == E    # a residual without a scale
+    assert gate(16, 2, 8, p, p, p, 1.0, 0.0, p, p, 1, p, p, None, 0, p, None, None) == E    # a tail without a residual
+    assert gate(16, 2, 8, p, p, p, 1.0, 0.0, p, p, 1, None, None, None, 0, p, p, None) == E # a mean without a tail
+    assert gate(15, 2, 8, p, p, p, 1.0, 0.0, p, p, 1, p, p, p, 0, p, p, None) == E
+    assert gate(16, 2, 8, p, p, p, 1.0, 0.0, p, p, 1, p, p, p, 0, None, p, None) == E
+    assert gate(15361, 1, 15361, p, p, p, 1.0, 0.0, p, p, 1, p, p, p, 0, p, p, None) == U
+    assert gate(0, 2, 8, p, p, p, 1.0, 0.0, p, p, 1, p, p, p, 0, p, p, None) == 0
     gs = ints([1, 2, 2, 2])
     assert lib.shdw_hip_grid_sample(gs, gs, 2, 0, p, p, ctypes.c_void_p(8192), None) == E
     assert lib.shdw_hip_grid_sample(gs, gs, 1, 2, p, p, ctypes.c_void_p(8192), None) == E

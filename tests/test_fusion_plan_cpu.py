@@ -186,3 +186,41 @@ def test_a_model_without_out_blob_is_refused():
     with pytest.raises(shadow_amd.ShadowError, match="out_blob"):
         plan(net)
     assert plan(make([neg("x", "y")], ["y"], params=())) == []
+
+
+# ---- [front ->] plane average -> sigmoid -> product [-> tail] ----
+def test_squeeze_gate_takes_its_front_and_tail():
+    from tests.test_gpu_fusion import GATE, GATE_TAIL, SHAPE, gate_net
+    assert plan(gate_net(SHAPE, ["e", "pool"])) == [GATE + GATE_TAIL + " + gap(Reduce) -> e, pool"]
+    assert plan(gate_net(SHAPE, ["e"], mean=False, swap=True, residual="r", residual_first=True)) == [GATE + GATE_TAIL + " -> e"]
+    assert plan(gate_net(SHAPE, ["t"], tail=False)) == [GATE + " -> t"]
+    assert plan(gate_net(SHAPE, ["t"], tail=False, front="none")) == ["squeeze(Pooling) + gate(Activate) + mul(Binary) -> t"]
+    # the Scale alone is no group: the gate reads what it writes
+    assert plan(gate_net(SHAPE, ["t"], tail=False, front="scale")) == ["squeeze(Pooling) + gate(Activate) + mul(Binary) -> t"]
+
+
+def test_squeeze_gate_leaves_what_is_read_elsewhere():
+    from tests.test_gpu_fusion import GATE, GATE_TAIL, SHAPE, gate_net
+    front = "bn(BatchNorm) + sc(Scale) + act(Activate) -> f"
+    gate = "squeeze(Pooling) + gate(Activate) + mul(Binary)"
+    # the gated map is handed out, or the residual: its front writes it
+    assert plan(gate_net(SHAPE, ["e", "f"], mean=False)) == [front, gate + GATE_TAIL + " -> e"]
+    assert plan(gate_net(SHAPE, ["e"], mean=False, residual="f")) == [front, gate + GATE_TAIL + " -> e"]
+    # the product is handed out: the tail reads it
+    assert plan(gate_net(SHAPE, ["e", "t"], mean=False)) == [GATE + " -> t", (GATE_TAIL + " -> e")[3:]]
+    # the average or the gate is: no group
+    parts = [front, (GATE_TAIL + " -> e")[3:]]
+    assert plan(gate_net(SHAPE, ["e", "q"], mean=False)) == parts
+    assert plan(gate_net(SHAPE, ["e", "g"], mean=False)) == parts
+    # another activation, another product, another window
+    for name, arg in (("gate", ("type", "s_i", 1)), ("mul", ("operation", "s_i", 0)), ("squeeze", ("pool", "s_i", 0))):
+        net = gate_net(SHAPE, ["e"], mean=False)
+        for o in net["op"]:
+            if o["name"] == name:
+                o["arg"] = [arg] + [a for a in o["arg"] if a[0] != arg[0]]
+        assert plan(net) == parts, name
+    # the map is rewritten between the average and the product
+    net = gate_net(SHAPE, ["e"], mean=False)
+    at = [o["name"] for o in net["op"]].index("gate")
+    net["op"].insert(at, neg("f", "f"))
+    assert plan(net) == parts

@@ -394,3 +394,87 @@ def test_batch_norm_scale_in_front_of_a_sum_without_relu(gpu):
     net = bn_net(ops, ["e"])
     weights, feed = bn_data()
     run_all(net, weights, feed, ["s", "e"], expect_fused=["bn(BatchNorm) + sc(Scale) -> s"])
+
+
+def gate_ops(front="bn+scale+relu", tail=True, swap=False, residual="x", residual_first=False, mean=True):
+    """front -> f; f * sigmoid(plane average of f) -> t [-> scale, + residual, relu [, mean]]."""
+    ops, f = [], "x"
+    if front != "none":
+        if front.startswith("bn"):
+            ops.append(bn_op("x", "n"))
+        ops.append(scale_op("n" if front.startswith("bn") else "x", "f", name="sc"))
+        if front.endswith("relu"):
+            ops.append(op("Activate", "act", ["f"], ["f"], arg_i("type", 1)))
+        f = "f"
+    ops += [op("Pooling", "squeeze", [f], ["q"], arg_i("pool", 1), arg_i("global_pooling", 1)),
+            op("Activate", "gate", ["q"], ["g"], arg_i("type", 3)),
+            op("Binary", "mul", ["g", f] if swap else [f, "g"], ["t"], arg_i("operation", 2))]
+    if tail:
+        ops += [scale_op("t", "u", name="sc2"),
+                op("Eltwise", "add", [residual, "u"] if residual_first else ["u", residual], ["e"], arg_i("operation", 1)),
+                op("Activate", "relu", ["e"], ["e"], arg_i("type", 1))]
+        if mean:
+            ops.append(op("Reduce", "gap", ["e"], ["pool"], arg_i("operation", 4), ("axes", "v_i", [2, 3])))
+    return ops
+
+
+def gate_net(shape, out, **form):
+    net = bn_net(gate_ops(**form), out, shape=shape)
+    net["op"][0] = op("Input", "in", [], ["x", "r"], ("x", "v_i", list(shape)), ("r", "v_i", list(shape)))
+    return net
+
+
+GATE = "bn(BatchNorm) + sc(Scale) + act(Activate) + squeeze(Pooling) + gate(Activate) + mul(Binary)"
+GATE_TAIL = " + sc2(Scale) + add(Eltwise) + relu(Activate)"
+
+
+# rows that are whole vectors and not, a quarter of a wave to a workgroup per row, several rows and
+# one per workgroup, the last workgroup cut, one vector and sixteen per lane, the longest row and past it
+@pytest.mark.parametrize("shape", [SHAPE, (2, 8, 4, 8), (5, 3, 1, 1), (1, 16, 14, 14), (1040, 2, 5, 6), (1031, 1, 8, 8),
+                                   (530, 2, 9, 9), (515, 2, 28, 28), (1030, 1, 27, 29), (513, 2, 45, 45),
+                                   (2, 3, 60, 61), (1100, 1, 60, 60), (1, 2, 100, 101), (1, 2, 120, 128), (1, 2, 124, 124)])
+def test_squeeze_gate(gpu, shape):
+    weights, feed = bn_data(shape)
+    feed["r"] = normal(77, shape)
+    run_all(gate_net(shape, ["e", "pool"]), weights, feed, ["e", "pool"], fp64=("pool",),
+            expect_fused=[GATE + GATE_TAIL + " + gap(Reduce) -> e, pool"])
+
+
+@pytest.mark.parametrize("shape", [SHAPE, (2, 8, 4, 8)])
+@pytest.mark.parametrize("front", ["none", "scale", "scale+relu", "bn+scale", "bn+scale+relu"])
+@pytest.mark.parametrize("tail", ["none", "other", "first"])
+def test_squeeze_gate_forms(gpu, shape, front, tail):
+    """With and without each part; the residual another blob, on either side of the sum; special values."""
+    out = ["t"] if tail == "none" else ["e"]
+    net = gate_net(shape, out, front=front, tail=tail != "none", swap=tail == "first", residual="r",
+                   residual_first=tail == "first", mean=False)
+    weights, feed = bn_data(shape)
+    feed = {"x": with_specials(normal(78, shape, 2.0), 1).reshape(shape), "r": with_specials(normal(79, shape), 2).reshape(shape)}
+    fused = run_all(net, weights, feed, out)
+    assert any("mul(Binary)" in line for line in fused)
+
+
+def test_squeeze_gate_window_of_the_first_run(gpu):
+    """A global pooling keeps the window of its first input: a plane of another size is no gate any more."""
+    shape = (2, 4, 6, 8)
+    net, (weights, feed) = gate_net(shape, ["e"], mean=False), bn_data(shape)
+    feed["r"] = normal(80, shape)
+    small = {k: np.ascontiguousarray(v[:1, :, :6, :8]) for k, v in feed.items()}
+    wide = {k: np.ascontiguousarray(v.reshape(2, 4, 12, 4)[:, :, :, :]) for k, v in feed.items()}
+    text = onet.write_text(net)
+    with shadow_amd.Network(text, weights) as fused, shadow_amd.Network(text, weights, fuse=False) as plain:
+        for given in (feed, small):
+            for nw in (fused, plain):
+                nw.forward(given, reshape=True)
+            assert_bit_exact(fused.blob("e"), plain.blob("e"), "same window")
+        errors = []
+        for nw in (fused, plain):  # a 12x4 plane under a 6x8 window
+            try:
+                nw.forward(wide, reshape=True)
+                errors.append(nw.blob("e"))
+            except shadow_amd.ShadowError as e:
+                errors.append(str(e))
+        if isinstance(errors[0], str):
+            assert isinstance(errors[1], str)
+        else:
+            assert_bit_exact(errors[0], errors[1], "another window")
