@@ -12,12 +12,13 @@
 // adds; the mean at the end is fp64, rounded once after the divide.
 //
 // What bounds it: 25 KB of LDS a workgroup leave six on a CU, whose loads, ordered
-// sums (784 dependent additions: 3 us) and stores overlap each other's.  A block on
-// [32,512,28,28] takes 31 us (103 MB) where its five launches took 78; two such
-// blocks behind a text model 239 -> 135 us a call, four on [1,256,14,14] 170 -> 108;
-// four on [16,64,56,56] 241 -> 120, on [64,1024,7,7] 155 -> 77.  Long planes keep one
-// row per workgroup and few workgroups per CU: four blocks on [16,64,112,112] 711 ->
-// 501, on [64,64,112,112] level (1376, 1386).
+// sums (784 dependent additions: 3 us) and stores overlap each other's, and 30 vector
+// instructions an element.  One block with its tail takes, per call: [32,512,28,28]
+// (103 MB) 27 us, where its five launches took 78; [64,64,56,56] 43; [64,512,14,14]
+// 11.9; [64,1024,7,7] 8.5; [16,64,112,112] 80 (its sums are 12 544 long).  With loads in
+// branches of their own, a division per element, LDS reads next to the additions that
+// use them and rows whole in LDS whatever their length: 29, 43, 13.9, 11.3 and 112; with the residual
+// another tensor than x 35 -> 27.5, 49 -> 44, 15.1 -> 12.0, 12.3 -> 8.2, 116 -> 80.
 #include <hip/hip_runtime.h>
 
 #include "../../include/shadow_hip.h"
@@ -30,9 +31,34 @@
 namespace shdw {
 
 // Per-row parameters, as the rows' lanes leave them in LDS.
-struct GateRow {
-  float m, d, s, b, tail_s, tail_b;
+struct alignas(16) GateRow {
+  float m, d, rd, s, b, tail_s, tail_b, gate;  // rd = 1 / d, or 0 where d is out of range for quotients4
 };
+
+// t / d, correctly rounded, by the reciprocal rd of d rounded to nearest: an estimate
+// and two corrections from the exact remainder (Markstein, "Computation of elementary
+// functions on the IBM RISC System/6000 processor", 1990; the second is needed because
+// the estimate may be two last places off).  Nothing may overflow or lose bits on the
+// way: |d| in [2^-30, 2^30], |t| in [2^-60, 2^60] (NaN passes); a wave with any other
+// element divides.  5 instructions an element instead of the 11 of a division.
+SHDW_DEVICE v4f quotients4(v4f t, float d, float rd) {
+  const float a0 = __builtin_fabsf(t[0]), a1 = __builtin_fabsf(t[1]), a2 = __builtin_fabsf(t[2]), a3 = __builtin_fabsf(t[3]);
+  const float lo = __builtin_fminf(__builtin_fminf(a0, a1), __builtin_fminf(a2, a3));
+  const float hi = __builtin_fmaxf(__builtin_fmaxf(a0, a1), __builtin_fmaxf(a2, a3));
+  if (__builtin_amdgcn_ballot_w64(!(lo >= 0x1p-60f && hi <= 0x1p60f && rd != 0.f)) == 0) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      float q = t[j] * rd;
+      q = __builtin_fmaf(__builtin_fmaf(-d, q, t[j]), rd, q);
+      t[j] = __builtin_fmaf(__builtin_fmaf(-d, q, t[j]), rd, q);
+    }
+  } else {
+    asm volatile("");  // keeps the compiler from evaluating both sides
+#pragma unroll
+    for (int j = 0; j < 4; ++j) t[j] = t[j] / d;
+  }
+  return t;
+}
 
 struct GateParams {
   const float *stat_mean, *stat_variance, *scale, *bias, *tail_scale, *tail_bias;
@@ -45,130 +71,211 @@ enum { kNoResidual = 0, kOtherResidual = 1, kSameResidual = 2 };
 
 constexpr uint32_t kGateMaxRows = 64;  // per workgroup: a lane of one wave each in the ordered sum
 
+// Waves per SIMD that the registers are held to: what a lane's vectors leave room for.
+constexpr int gate_waves(int slots) { return slots == 16 ? 4 : slots == 8 ? 5 : 6; }
+
+// sum + row[0] + row[1] + ..., in that order.  Two sets of six vectors take turns: one is
+// read while the other is added.  A last part of a vector reads the whole of it.
+SHDW_DEVICE float add_in_order(float sum, const v4f* row, uint32_t cols) {
+  constexpr uint32_t kSet = 6;
+  const uint32_t n = cols / 4;
+  uint32_t v = 0;
+  const auto read = [&](v4f* q) {
+#pragma unroll
+    for (uint32_t k = 0; k < kSet; ++k) q[k] = row[v + k];
+    v += kSet;
+    __builtin_amdgcn_sched_barrier(0);  // requested here, not where they are first used
+  };
+  const auto add = [&](const v4f* q) {
+#pragma unroll
+    for (uint32_t k = 0; k < 4 * kSet; ++k) sum += q[k / 4][k % 4];
+  };
+  v4f a[kSet], b[kSet];
+  if (n >= kSet) {
+    read(a);
+    while (v + 2 * kSet <= n) {
+      read(b);
+      add(a);
+      read(a);
+      add(b);
+    }
+    if (v + kSet <= n) {
+      read(b);
+      add(a);
+      add(b);
+    } else {
+      add(a);
+    }
+  }
+  const uint32_t left = cols - 4 * v, last = (cols - 1) / 4;
+  if (left) {
+#pragma unroll
+    for (uint32_t k = 0; k < kSet; ++k) a[k] = row[min(v + k, last)];
+#pragma unroll
+    for (uint32_t k = 0; k < 4 * kSet; ++k) {
+      if (k >= left) break;
+      sum += a[k / 4][k % 4];
+    }
+  }
+  return sum;
+}
+
 // L = 2^log2_lanes lanes share a row, so a workgroup takes 256 / L rows per turn and
-// `pieces` steps of 4 L columns per row; SLOTS >= turns * pieces vectors per lane, all
-// requested before anything else happens.
-template <int SLOTS, bool VEC, int RESIDUAL>
-__global__ __launch_bounds__(kBlock) void squeeze_gate_kernel(const float* x, const float* res, float* y, float* mean,
+// `pieces` steps of 4 L columns per row; slot i of a lane's SLOTS vectors is a piece of
+// a turn, the same for all lanes.  Every vector is requested before anything else
+// happens, and without a branch (a branch around a load has the compiler copy the
+// registers of the loads before it, and wait for them): lanes with nothing to load take
+// the row's or the group's last vector again.  WHOLE: the front's result stays in LDS;
+// otherwise LDS holds `chunk` pieces of the rows at a time and the front is taken again
+// on the way out.
+template <int SLOTS, bool VEC, bool WHOLE, int RESIDUAL>
+__global__ __launch_bounds__(kBlock, gate_waves(SLOTS)) void squeeze_gate_kernel(const float* x, const float* res, float* y, float* mean,
                                                               uint32_t rows, uint32_t len, uint32_t group,
-                                                              uint32_t log2_lanes, uint32_t pieces, uint32_t pitch,
-                                                              GateParams p) {
-  extern __shared__ __align__(16) float tile[];  // group rows of pitch floats
+                                                              uint32_t log2_lanes, uint32_t pieces, uint32_t chunk,
+                                                              uint32_t pitch, GateParams p) {
+  extern __shared__ v4f tile[];  // a chunk of the group's rows, pitch vectors apart
   __shared__ uint64_t tab[32];
   __shared__ GateRow row_params[kGateMaxRows];
-  __shared__ float gate[kGateMaxRows];
   __shared__ double part[kGateMaxRows / 8][kBlock / kWave];  // rows split over the waves: at most 8
   const uint32_t lanes = 1u << log2_lanes, turn_rows = kBlock >> log2_lanes;
-  const uint32_t sub = threadIdx.x & (lanes - 1), lead = threadIdx.x >> log2_lanes;
+  uint32_t sub = threadIdx.x & (lanes - 1), lead = threadIdx.x >> log2_lanes;
   const uint32_t row0 = xcd_runs(blockIdx.x, gridDim.x, 2) * group;
   const uint32_t nrows = min(group, rows - row0);
+  const uint32_t last = len < 4 ? 0 : len - 4;  // of a row's columns that a vector can start at
 
-  v4f reg[SLOTS], other[RESIDUAL == kOtherResidual ? SLOTS : 1];
-  auto request = [&](const float* src, v4f* to) {
-    uint32_t r = lead, c = 4 * sub, k = 0;
+  const auto step = [&](uint32_t& k, uint32_t& turn_row) {
+    if (++k == pieces) k = 0, turn_row += turn_rows;
+  };
+  const auto vector = [&](const float* src, uint32_t k, uint32_t turn_row) {
+    const float* at = src + static_cast<uint64_t>(row0) * len + min(lead + turn_row, nrows - 1) * len +
+                      min(4 * (sub + k * lanes), last);
+    if (VEC) return load4_stream(at);
+    if (len >= 4) return load4_stream_any(at);
+    return v4f{at[0], at[len > 1 ? 1 : 0], at[len > 2 ? 2 : 0], 0.f};
+  };
+  const auto request = [&](const float* src, v4f* to) {
+    uint32_t k = 0, turn_row = 0;
 #pragma unroll
     for (int i = 0; i < SLOTS; ++i) {
-      if (r < nrows && c < len) {
-        const float* at = src + static_cast<uint64_t>(row0 + r) * len + c;
-        if (VEC) {
-          to[i] = load4_stream(at);
-        } else if (c + 4 <= len) {
-          to[i] = load4_stream_any(at);
-        } else {
-          to[i] = v4f{at[0], c + 1 < len ? at[1] : 0.f, c + 2 < len ? at[2] : 0.f, 0.f};
-        }
-      }
-      if (++k == pieces) k = 0, c = 4 * sub, r += turn_rows;
-      else c += 4 * lanes;
+      to[i] = vector(src, k, turn_row);
+      step(k, turn_row);
     }
   };
+  // A row's last vector was requested from where it ends inside the row: its elements to the front.
+  const auto arrange = [&](v4f& v, uint32_t c) {
+    if (VEC || len < 4) return;
+    const uint32_t by = c - min(c, last);
+    if (by & 1u) v = v4f{v[1], v[2], v[3], v[3]};
+    if (by & 2u) v = v4f{v[2], v[3], v[3], v[3]};
+  };
+  // The rows' parameters are requested ahead of the rows (a wait for them is then no wait
+  // for the rows), an absent one from an address that is there.
+  const uint32_t own = row0 + min(threadIdx.x, nrows - 1), ch = own - fd_div(own, p.channel) * p.channel.d;
+  const auto param = [&](const float* from) { return (from ? from : x)[ch]; };
+  const float stat_mean = param(p.stat_mean), stat_variance = param(p.stat_variance), scale = param(p.scale);
+  const float bias = param(p.bias), tail_scale = param(p.tail_scale), tail_bias = param(p.tail_bias);
+  const uint64_t entry = libm::kExp2fTab[threadIdx.x & 31u];
+  constexpr int kTurn = 4;  // vectors of the residual in flight where x keeps its registers
+  v4f reg[SLOTS], other[kTurn];
   request(x, reg);
-  if (RESIDUAL == kOtherResidual) request(res, other);
-
   if (threadIdx.x < nrows) {
-    const uint32_t row = row0 + threadIdx.x, c = row - fd_div(row, p.channel) * p.channel.d;
-    GateRow g{0.f, 1.f, 1.f, -0.f, 1.f, -0.f};
+    GateRow g{0.f, 1.f, 1.f, 1.f, -0.f, 1.f, -0.f, 0.f};
     if (p.stat_mean) {
-      g.m = p.stat_mean[c] * p.scale_factor;
-      g.d = __builtin_sqrtf(__builtin_fabsf(p.stat_variance[c] * p.scale_factor) + p.eps);
+      g.m = stat_mean * p.scale_factor;
+      g.d = __builtin_sqrtf(__builtin_fabsf(stat_variance * p.scale_factor) + p.eps);
+      g.rd = g.d >= 0x1p-30f && g.d <= 0x1p30f ? 1.f / g.d : 0.f;
     }
-    if (p.scale) g.s = p.scale[c];
-    if (p.bias) g.b = p.bias[c];
-    if (p.tail_scale) g.tail_s = p.tail_scale[c];
-    if (p.tail_bias) g.tail_b = p.tail_bias[c];
+    if (p.scale) g.s = scale;
+    if (p.bias) g.b = bias;
+    if (p.tail_scale) g.tail_s = tail_scale;
+    if (p.tail_bias) g.tail_b = tail_bias;
     row_params[threadIdx.x] = g;
   }
-  if (threadIdx.x >= kBlock - 32) tab[threadIdx.x - (kBlock - 32)] = libm::kExp2fTab[threadIdx.x - (kBlock - 32)];
+  if (threadIdx.x < 32) tab[threadIdx.x] = entry;
   __syncthreads();
 
-  {
-    uint32_t r = lead, c = 4 * sub, k = 0;
+  const auto front = [&](v4f t, const GateRow& g) {
+    if (p.stat_mean) {
 #pragma unroll
-    for (int i = 0; i < SLOTS; ++i) {
-      if (r < nrows && c < len) {
-        const GateRow g = row_params[r];
-        v4f t = reg[i];
-        if (p.stat_mean) {
-#pragma unroll
-          for (int j = 0; j < 4; ++j) t[j] = (t[j] - g.m) / g.d;
-        }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          t[j] = t[j] * g.s;
-          t[j] = t[j] + g.b;
-          if (p.relu) t[j] = t[j] > 0 ? t[j] : 0;
-        }
-        *reinterpret_cast<v4f*>(tile + r * pitch + c) = t;
-      }
-      if (++k == pieces) k = 0, c = 4 * sub, r += turn_rows;
-      else c += 4 * lanes;
+      for (int j = 0; j < 4; ++j) t[j] = t[j] - g.m;
+      t = quotients4(t, g.d, g.rd);
     }
-  }
-  __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      t[j] = t[j] * g.s;
+      t[j] = t[j] + g.b;
+      if (p.relu) t[j] = t[j] > 0 ? t[j] : 0;
+    }
+    return t;
+  };
 
   // The ordered sums, a lane per row: all in one wave, which issues one addition for
   // all rows; a different wave in neighbouring workgroups, so that the walks of a CU
   // do not meet on one SIMD.
-  if (threadIdx.x / kWave == ((blockIdx.x / kXcds) & 3u) && (threadIdx.x & (kWave - 1)) < nrows) {
-    const uint32_t r = threadIdx.x & (kWave - 1);
-    const float* mine = tile + r * pitch;
-    constexpr int kAhead = 16, kStep = 4 * kAhead;
-    float sum = 0.f;
-    uint32_t c = 0;
-    for (; c + kStep <= len; c += kStep) {
-      v4f q[kAhead];
+  const uint32_t walked = threadIdx.x & (kWave - 1);
+  const bool walks = threadIdx.x / kWave == ((blockIdx.x / kXcds) & 3u) && walked < nrows;
+  float sum = 0.f;
+  for (uint32_t k0 = 0; k0 < pieces; k0 += chunk) {
+    if (!WHOLE && k0) __syncthreads();
+    asm("" : "+v"(sub), "+v"(lead));
+    uint32_t k = 0, turn_row = 0;
 #pragma unroll
-      for (int k = 0; k < kAhead; ++k) q[k] = *reinterpret_cast<const v4f*>(mine + c + 4 * k);
-#pragma unroll
-      for (int k = 0; k < kStep; ++k) sum += q[k / 4][k % 4];
+    for (int i = 0; i < SLOTS; ++i) {
+      const uint32_t r = lead + turn_row, v = sub + k * lanes;
+      if (WHOLE || k - k0 < chunk) {
+        arrange(reg[i], 4 * v);
+        const v4f t = front(reg[i], row_params[min(r, nrows - 1)]);
+        if (r < nrows && 4 * v < len) tile[r * pitch + v - k0 * lanes] = t;
+      }
+      step(k, turn_row);
     }
-    for (; c < len; ++c) sum += mine[c];
-    gate[r] = libm::exact_sigmoidf(sum / p.plane, tab);
+    // the residual travels while the rows are summed
+    if (RESIDUAL == kOtherResidual && WHOLE) request(res, reg);
+    __syncthreads();
+    if (walks) {
+      const v4f* mine = tile + walked * pitch;
+      const uint32_t cols = WHOLE ? len : min(len - 4 * k0 * lanes, 4 * chunk * lanes);
+      sum = add_in_order(sum, mine, cols);
+    }
+    if (WHOLE) break;
   }
+  if (walks) row_params[walked].gate = libm::exact_sigmoidf(sum / p.plane, tab);
   __syncthreads();
 
+  asm("" : "+v"(sub), "+v"(lead));  // the slots' offsets are taken again instead of kept
   double total = 0.0;
-  uint32_t r = lead, c = 4 * sub, k = 0;
+  uint32_t k = 0, turn_row = 0;
 #pragma unroll
   for (int i = 0; i < SLOTS; ++i) {
-    if (r < nrows && c < len) {
-      const float g = gate[r], s = row_params[r].tail_s, b = row_params[r].tail_b;
-      v4f t = *reinterpret_cast<const v4f*>(tile + r * pitch + c);
-      const v4f q = RESIDUAL == kOtherResidual ? other[i] : reg[i];
+    const uint32_t r = lead + turn_row, v = sub + k * lanes, c = 4 * v;
+    const bool here = r < nrows && c < len;
+    const GateRow g = row_params[min(r, nrows - 1)];
+    v4f t = WHOLE ? tile[min(r, nrows - 1) * pitch + min(v, pitch - 1)] : front(reg[i], g);
+    if (RESIDUAL == kOtherResidual && !WHOLE && i % kTurn == 0) {
+      uint32_t k_ahead = k, turn_ahead = turn_row;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        t[j] = t[j] * g;
-        if (RESIDUAL != kNoResidual) {
-          t[j] = t[j] * s;
-          t[j] = t[j] + b;
-          // Eltwise SUM with unit coefficients: Set(0), then y += 1 * input, input by input
-          float u = 0.0f + (p.residual_first ? q[j] : t[j]);
-          u = u + (p.residual_first ? t[j] : q[j]);
-          t[j] = u > 0 ? u : 0;
-          if (VEC || c + j < len) total += static_cast<double>(t[j]);
-        }
+      for (int n = 0; n < kTurn; ++n) {
+        other[n] = vector(res, k_ahead, turn_ahead);
+        step(k_ahead, turn_ahead);
       }
-      float* at = y + static_cast<uint64_t>(row0 + r) * len + c;
+    }
+    v4f q = RESIDUAL == kOtherResidual && !WHOLE ? other[i % kTurn] : reg[i];
+    if (RESIDUAL == kOtherResidual) arrange(q, c);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      t[j] = t[j] * g.gate;
+      if (RESIDUAL != kNoResidual) {
+        t[j] = t[j] * g.tail_s;
+        t[j] = t[j] + g.tail_b;
+        // Eltwise SUM with unit coefficients: Set(0), then y += 1 * input, input by input
+        float u = 0.0f + (p.residual_first ? q[j] : t[j]);
+        u = u + (p.residual_first ? t[j] : q[j]);
+        t[j] = u > 0 ? u : 0;
+        if (mean) total += static_cast<double>(here && (VEC || c + j < len) ? t[j] : 0.f);
+      }
+    }
+    if (here) {
+      float* at = y + static_cast<uint64_t>(row0) * len + (r * len + c);
       if (VEC) {
         store4_stream(at, t);
       } else if (c + 4 <= len) {
@@ -179,25 +286,21 @@ __global__ __launch_bounds__(kBlock) void squeeze_gate_kernel(const float* x, co
           if (c + j < len) at[j] = t[j];
       }
     }
-    if (++k == pieces) {
-      if (RESIDUAL != kNoResidual && mean) {  // the row is complete: every lane of the wave is here
-        total += dpp_f64<kDppXor1>(total);
-        total += dpp_f64<kDppXor2>(total);
-        total += dpp_f64<kDppHalfMirror>(total);
-        total += dpp_f64<kDppMirror>(total);
-        if (log2_lanes > 4) total += __shfl_xor(total, 16, kWave);
-        if (log2_lanes > 5) total += __shfl_xor(total, 32, kWave);
-        if (log2_lanes > 6) {
-          if ((threadIdx.x & (kWave - 1)) == 0 && r < nrows) part[r][threadIdx.x / kWave] = total;
-        } else if (sub == 0 && r < nrows) {
-          mean[row0 + r] = static_cast<float>(total / static_cast<double>(static_cast<int>(len)));
-        }
-        total = 0.0;
+    if (RESIDUAL != kNoResidual && mean && k + 1 == pieces) {  // the row is complete: every lane of the wave is here
+      total += dpp_f64<kDppXor1>(total);
+      total += dpp_f64<kDppXor2>(total);
+      total += dpp_f64<kDppHalfMirror>(total);
+      total += dpp_f64<kDppMirror>(total);
+      if (log2_lanes > 4) total += __shfl_xor(total, 16, kWave);
+      if (log2_lanes > 5) total += __shfl_xor(total, 32, kWave);
+      if (log2_lanes > 6) {
+        if ((threadIdx.x & (kWave - 1)) == 0 && r < nrows) part[r][threadIdx.x / kWave] = total;
+      } else if (sub == 0 && r < nrows) {
+        mean[row0 + r] = static_cast<float>(total / static_cast<double>(static_cast<int>(len)));
       }
-      k = 0, c = 4 * sub, r += turn_rows;
-    } else {
-      c += 4 * lanes;
+      total = 0.0;
     }
+    step(k, turn_row);
   }
   if (RESIDUAL != kNoResidual && mean && log2_lanes > 6) {
     __syncthreads();
@@ -211,9 +314,15 @@ __global__ __launch_bounds__(kBlock) void squeeze_gate_kernel(const float* x, co
 
 // How a shape is cut.
 struct GateShape {
-  uint32_t log2_lanes, pieces, group, pitch;
+  uint32_t log2_lanes, pieces, group, chunk, pitch;
   int slots;
 };
+
+// Six workgroups on a CU.  Rows that do not fit whole go through LDS in chunks (four of the
+// 112x112 planes' rows per CU instead of three, [16,64,112,112] 124 -> 81 us; with 18 KB
+// [32,512,28,28] would be cut too, 26.0 -> 28.1), unless there are no more than two
+// workgroups per CU to hold.
+constexpr uint32_t kGateTileBytes = 26000, kGateMaxTileBytes = 62000, kGateCus = 256;
 
 // Lanes per row: as many as a row has vectors, up to a wave; the whole workgroup where
 // a wave would take more than eight steps over a row, and where there are so few rows
@@ -226,12 +335,20 @@ inline GateShape gate_shape(uint32_t rows, uint32_t len) {
   if (nv > 16 && rows < 1024) g.log2_lanes = 8;
   const uint32_t lanes = 1u << g.log2_lanes, turn_rows = kBlock >> g.log2_lanes;
   g.pieces = (nv + lanes - 1) / lanes;
-  g.slots = g.pieces <= 8 ? 8 : 16;
-  uint32_t turns = static_cast<uint32_t>(g.slots) / g.pieces;
+  uint32_t turns = g.pieces <= 8 ? 8 / g.pieces : 1;
   if (turns * turn_rows > kGateMaxRows) turns = kGateMaxRows / turn_rows;
   while (turns > 1 && (rows + turns * turn_rows - 1) / (turns * turn_rows) < 1024u) --turns;
+  const uint32_t used = turns * g.pieces;
+  g.slots = used <= 1 ? 1 : used <= 4 ? 4 : used <= 8 ? 8 : 16;
   g.group = turns * turn_rows;
-  g.pitch = 4 * (nv | 1u);  // an odd number of 128-bit pieces: the summing lanes meet different banks
+  // LDS holds equal chunks of the rows, as few as fit the tile; the pitch is an odd
+  // number of vectors, so that the summing lanes meet different banks.
+  for (uint32_t chunks = 1;; ++chunks) {
+    g.chunk = (g.pieces + chunks - 1) / chunks;
+    g.pitch = (g.chunk * lanes < nv ? g.chunk * lanes : nv) | 1u;
+    const uint32_t bytes = g.group * g.pitch * static_cast<uint32_t>(sizeof(v4f));
+    if (bytes <= (rows <= 2 * kGateCus * g.group ? kGateMaxTileBytes : kGateTileBytes) || g.chunk == 1) break;
+  }
   return g;
 }
 
@@ -241,18 +358,36 @@ using namespace shdw;
 
 namespace {
 
-template <int SLOTS, bool VEC>
+template <int SLOTS, bool VEC, bool WHOLE>
 void launch_gate(const GateShape& g, uint32_t rows, uint32_t len, const float* x, const float* res, float* y, float* mean,
                  const GateParams& p, hipStream_t st) {
   const uint32_t grid = (rows + g.group - 1) / g.group;
-  const size_t lds = static_cast<size_t>(g.group) * g.pitch * sizeof(float);
-#define SHDW_LAUNCH(R)                                                                                          \
-  squeeze_gate_kernel<SLOTS, VEC, R><<<grid, kBlock, lds, st>>>(x, res, y, mean, rows, len, g.group, g.log2_lanes, \
-                                                                g.pieces, g.pitch, p)
+  const size_t lds = static_cast<size_t>(g.group) * g.pitch * sizeof(v4f);
+#define SHDW_LAUNCH(R)                                                                                           \
+  squeeze_gate_kernel<SLOTS, VEC, WHOLE, R><<<grid, kBlock, lds, st>>>(x, res, y, mean, rows, len, g.group,      \
+                                                                       g.log2_lanes, g.pieces, g.chunk, g.pitch, p)
   if (!res) SHDW_LAUNCH(kNoResidual);
   else if (res == x) SHDW_LAUNCH(kSameResidual);
   else SHDW_LAUNCH(kOtherResidual);
 #undef SHDW_LAUNCH
+}
+
+template <int SLOTS, bool VEC>
+void launch_gate(const GateShape& g, uint32_t rows, uint32_t len, const float* x, const float* res, float* y, float* mean,
+                 const GateParams& p, hipStream_t st) {
+  if (g.chunk == g.pieces) launch_gate<SLOTS, VEC, true>(g, rows, len, x, res, y, mean, p, st);
+  else launch_gate<SLOTS, VEC, false>(g, rows, len, x, res, y, mean, p, st);
+}
+
+template <bool VEC>
+void launch_gate(const GateShape& g, uint32_t rows, uint32_t len, const float* x, const float* res, float* y, float* mean,
+                 const GateParams& p, hipStream_t st) {
+  switch (g.slots) {
+    case 1: launch_gate<1, VEC, true>(g, rows, len, x, res, y, mean, p, st); break;
+    case 4: launch_gate<4, VEC>(g, rows, len, x, res, y, mean, p, st); break;
+    case 8: launch_gate<8, VEC>(g, rows, len, x, res, y, mean, p, st); break;
+    default: launch_gate<16, VEC>(g, rows, len, x, res, y, mean, p, st);
+  }
 }
 
 }  // namespace
@@ -272,12 +407,7 @@ extern "C" int shdw_hip_squeeze_gate(int n, int channel, int inner_num, const fl
   const bool vec = len % 4 == 0 && aligned16(x) && aligned16(y) && (!residual || aligned16(residual));
   const GateShape g = gate_shape(rows, len);
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (g.slots == 8) {
-    if (vec) launch_gate<8, true>(g, rows, len, x, residual, y, mean, p, st);
-    else launch_gate<8, false>(g, rows, len, x, residual, y, mean, p, st);
-  } else {
-    if (vec) launch_gate<16, true>(g, rows, len, x, residual, y, mean, p, st);
-    else launch_gate<16, false>(g, rows, len, x, residual, y, mean, p, st);
-  }
+  if (vec) launch_gate<true>(g, rows, len, x, residual, y, mean, p, st);
+  else launch_gate<false>(g, rows, len, x, residual, y, mean, p, st);
   return launch_status();
 }

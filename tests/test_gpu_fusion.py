@@ -478,3 +478,21 @@ def test_squeeze_gate_window_of_the_first_run(gpu):
             assert isinstance(errors[1], str)
         else:
             assert_bit_exact(errors[0], errors[1], "another window")
+
+
+@pytest.mark.parametrize("spread", [1, 40, 120])
+def test_squeeze_gate_quotients(gpu, spread):
+    """(x - mean) / deviation over magnitudes for which the kernel's reciprocal form holds, up to its limits, and
+    past them, where it divides; zeros of both signs and deviations with an all-ones significand among them."""
+    shape = (4, 64, 9, 12)
+    net = gate_net(shape, ["t"], tail=False, front="bn+scale")
+    weights, feed = bn_data(shape)
+    rng = np.random.default_rng(spread)
+    mean, variance = weights[0], weights[1]
+    mean[::2] = 0
+    variance[:] = (2.0 ** rng.uniform(-spread / 2, spread / 2, variance.shape)).astype(F)
+    variance[:8] = np.nextafter(F(4), F(0))
+    x = (normal(81, shape) * 2.0 ** rng.integers(-spread, spread + 1, shape)).astype(F)
+    x[0, ::3, 0, :4] = [0.0, -0.0, 1e-42, -1e-42]
+    run_all(net, weights, {"x": x, "r": x}, ["t"],
+            expect_fused=["bn(BatchNorm) + sc(Scale) + squeeze(Pooling) + gate(Activate) + mul(Binary) -> t"])
