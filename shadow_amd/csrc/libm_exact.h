@@ -859,6 +859,8 @@ SHDW_LIBM_FN bool powf_is_ordinary(uint32_t ix, uint32_t iy) {
 // place at the end, so several of these can run side by side in one lane; any
 // other ix and y give some number and no fault.
 // log_tab is kPowfLog2Tab or a copy of it in faster memory, as tab is of kExp2fTab.
+// IN_RANGE: |y log2 x| < 126 is known, and nothing is put in place.
+template <bool IN_RANGE>
 SHDW_LIBM_FN float powf_ordinary(uint32_t ix, float y, uint32_t sign_bias, const uint64_t* tab,
                                  const PowfLog2Entry* log_tab) {
   // log2(x)
@@ -898,6 +900,7 @@ SHDW_LIBM_FN float powf_ordinary(uint32_t ix, float y, uint32_t sign_bias, const
   res = __builtin_fma(zz, rr2, res);
   res = res * sc;
   float out = static_cast<float>(res);
+  if (IN_RANGE) return out;
   // |y log2 x| >= 126: past the largest float, below half the smallest, or the smallest itself
   const bool far = (d2u(ylogx) >> 47 & 0xffff) >= (d2u(126.0) >> 47);
   const bool over = far && ylogx > 0x1.fffffffd1d571p+6;
@@ -910,7 +913,7 @@ SHDW_LIBM_FN float powf_ordinary(uint32_t ix, float y, uint32_t sign_bias, const
 }
 
 SHDW_LIBM_FN float powf_ordinary(uint32_t ix, float y, uint32_t sign_bias, const uint64_t* tab) {
-  return powf_ordinary(ix, y, sign_bias, tab, kPowfLog2Tab);
+  return powf_ordinary<false>(ix, y, sign_bias, tab, kPowfLog2Tab);
 }
 
 SHDW_LIBM_FN float exact_powf(float x, float y, const uint64_t* tab) {

@@ -51,15 +51,34 @@ SHDW_DEVICE void lrn_stage_tables(LrnTables* t) {
   __syncthreads();
 }
 
-// powf(scale, y) for the scales of a round.  The straight path for all of them (any
-// bits may go in, see powf_ordinary); then, if some lane holds a scale that is not a
-// positive normal number, the whole function for those, one instance of its code.
-SHDW_DEVICE void lrn_powers(const float (&scale)[kLrnRound], float y, const LrnTables* t,
+// powf(scale, y) for the scales of a round.  Where every scale of the wave lies in
+// [2^-100, 2^100] and 0 < |y| <= 1.25 (`small_power`; LRN's scales are near k, its power
+// -0.75), |y log2 scale| is below 126 and nothing of powf's special cases can apply:
+// two comparisons on the round's extremes stand for the tests of each of the eight
+// (a quarter of the instructions: [44,96,55,55] 39.1 -> 33.3 us, [64,256,56,56] 137 -> 118,
+// held to five waves a SIMD; with the registers it likes, four, 38.1 and 118).  Otherwise the straight
+// path with its range tests for all of them (any bits may go in, see powf_ordinary);
+// then, if some lane holds a scale that is not a positive normal number, the whole
+// function for those, one instance of its code.
+SHDW_DEVICE void lrn_powers(const float (&scale)[kLrnRound], float y, bool small_power, const LrnTables* t,
                             float (&power)[kLrnRound]) {
+  uint32_t lo = __float_as_uint(scale[0]), hi = lo;  // as bits: negative numbers and NaN lie above every positive one
+#pragma unroll
+  for (uint32_t j = 1; j < kLrnRound; ++j) {
+    lo = min(lo, __float_as_uint(scale[j]));
+    hi = max(hi, __float_as_uint(scale[j]));
+  }
+  if (small_power && __builtin_amdgcn_ballot_w64(!(lo >= __float_as_uint(0x1p-100f) && hi <= __float_as_uint(0x1p100f))) == 0) {
+#pragma unroll
+    for (uint32_t j = 0; j < kLrnRound; ++j)
+      power[j] = libm::powf_ordinary<true>(__float_as_uint(scale[j]), y, 0u, t->exp2, t->log2);
+    return;
+  }
+  asm volatile("");  // keeps the compiler from working out both forms side by side
   bool plain = true;
 #pragma unroll
   for (uint32_t j = 0; j < kLrnRound; ++j) {
-    power[j] = libm::powf_ordinary(__float_as_uint(scale[j]), y, 0u, t->exp2, t->log2);
+    power[j] = libm::powf_ordinary<false>(__float_as_uint(scale[j]), y, 0u, t->exp2, t->log2);
     plain = plain && libm::powf_is_ordinary(__float_as_uint(scale[j]), __float_as_uint(y));
   }
   if (__builtin_amdgcn_ballot_w64(!plain) == 0) return;
@@ -119,7 +138,7 @@ SHDW_DEVICE void lrn_round(const float* in, float* out, uint32_t head0, uint32_t
 #pragma unroll
   for (int t = 0; t < SIZE; ++t) prev[t] = entering[kLrnRound - SIZE + t];
   if (!finish) return;  // a round in front of this workgroup's share: only the sum had to pass through it
-  lrn_powers(scale, neg_beta, tables, power);
+  lrn_powers(scale, neg_beta, neg_beta != 0.f && __builtin_fabsf(neg_beta) <= 1.25f, tables, power);
 #pragma unroll
   for (uint32_t j = 0; j < kLrnRound; ++j) {
     const uint32_t head = head0 + j;
@@ -128,7 +147,7 @@ SHDW_DEVICE void lrn_round(const float* in, float* out, uint32_t head0, uint32_t
 }
 
 template <int SIZE>
-__global__ __launch_bounds__(kBlock) void lrn_window_kernel(const float* x, float* y, uint32_t positions,
+__global__ __launch_bounds__(kBlock, 5) void lrn_window_kernel(const float* x, float* y, uint32_t positions,
                                                             uint32_t step, uint32_t channels, FastDiv f_step,
                                                             float alpha_over_size, float neg_beta, float k) {
   __shared__ LrnTables tables;
@@ -210,7 +229,7 @@ __global__ __launch_bounds__(kBlock) void lrn_across_channels_kernel(
       }
     }
     if (head0 < first) continue;  // in front of this workgroup's share: only the sum had to pass through
-    lrn_powers(scale, neg_beta, &tables, power);
+    lrn_powers(scale, neg_beta, neg_beta != 0.f && __builtin_fabsf(neg_beta) <= 1.25f, &tables, power);
 #pragma unroll
     for (uint32_t j = 0; j < kLrnRound; ++j) {
       const uint32_t head = head0 + j;

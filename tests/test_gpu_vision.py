@@ -136,6 +136,17 @@ def test_lrn_scales_below_one_and_negative(gpu):
         assert_bit_exact(gpuops.lrn(x, shape, 5, alpha, 0.75, k), want, "lrn alpha %g k %g" % (alpha, k))
 
 
+@pytest.mark.parametrize("beta", [0.75, -1.25, 1.25, 1.2500001, 3.0, 0.0])
+def test_lrn_scales_at_the_ends_of_the_short_powers(gpu, beta):
+    """Scales of exactly k around 2^-100 and 2^100, where the kernel turns to the powers with range tests."""
+    shape = (2, 9, 5, 7)
+    x = normal(92, int(np.prod(shape)))
+    for e in (-126, -101, -100, -99, 0, 99, 100, 101, 127):
+        for k in (2.0 ** e, float(np.nextafter(F(2.0 ** e), F(np.inf))), float(np.nextafter(F(2.0 ** e), F(0)))):
+            want, _ = oracle.lrn(x, shape, 3, 0.0, beta, k)
+            assert_bit_exact(gpuops.lrn(x, shape, 3, 0.0, beta, k), want, "k %g beta %g" % (k, beta))
+
+
 def test_lrn_argument_errors(gpu):
     lib = gpu
     buf = shadow_amd.Buffer(4 * 2 * 3 * 4 * 4)
