@@ -99,6 +99,11 @@ int shdw_hip_mem_info(size_t* free_bytes, size_t* total_bytes);
 int shdw_hip_memcpy_h2d(void* dst, const void* src, size_t bytes, void* stream);
 /* ref: shadow/core/allocator.cu:20-27 (read: D2H; blocking when stream==NULL) */
 int shdw_hip_memcpy_d2h(void* dst, const void* src, size_t bytes, void* stream);
+/* The same for a few kilobytes that the host waits for: a kernel stores them in
+ * `staging` (shdw_hip_host_malloc, at least `bytes` long), the stream is waited for and
+ * they are copied to dst.  bytes and src must be multiples of 4, otherwise, and while the
+ * stream is being captured, it is shdw_hip_memcpy_d2h. */
+int shdw_hip_memcpy_d2h_staged(void* dst, const void* src, size_t bytes, void* staging, void* stream);
 /* ref: shadow/core/allocator.cu:38-45 (copy: D2D; blocking when stream==NULL) */
 int shdw_hip_memcpy_d2d(void* dst, const void* src, size_t bytes, void* stream);
 /* Pinned host staging memory for the two calls above; Shadow reads back into a

@@ -48,6 +48,7 @@ SIGNATURES = {
     "shdw_hip_free": (_I, [_V]),
     "shdw_hip_memcpy_h2d": (_I, [_V, _V, _Z, _V]),
     "shdw_hip_memcpy_d2h": (_I, [_V, _V, _Z, _V]),
+    "shdw_hip_memcpy_d2h_staged": (_I, [_V, _V, _Z, _V, _V]),
     "shdw_hip_memcpy_d2d": (_I, [_V, _V, _Z, _V]),
     "shdw_hip_host_malloc": (_I, [c_void_pp, _Z]),
     "shdw_hip_host_free": (_I, [_V]),

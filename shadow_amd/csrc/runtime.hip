@@ -2,6 +2,7 @@
 // that Shadow's GPUAllocator / GPUContext sit on.
 #include <hip/hip_runtime.h>
 
+#include <cstdint>
 #include <cstdio>
 #include <cstring>
 
@@ -103,6 +104,23 @@ int shdw_hip_memcpy_h2d(void* dst, const void* src, size_t bytes, void* stream) 
 }
 int shdw_hip_memcpy_d2h(void* dst, const void* src, size_t bytes, void* stream) {
   return copy(dst, src, bytes, hipMemcpyDeviceToHost, stream);
+}
+// 1 KB into pageable memory takes the runtime 26 us; the kernel, the wait and the host's own copy 17.
+int shdw_hip_memcpy_d2h_staged(void* dst, const void* src, size_t bytes, void* staging, void* stream) {
+  if (bytes == 0) return SHDW_OK;
+  if (!dst || !src || !staging) return SHDW_E_INVALID_ARGUMENT;
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  const hipError_t asked = hipStreamIsCapturing(as_stream(stream), &capture);
+  if (asked != hipSuccess) (void)hipGetLastError();
+  if (asked != hipSuccess || capture != hipStreamCaptureStatusNone || (bytes | reinterpret_cast<uintptr_t>(src)) % 4 != 0 ||
+      bytes / 4 > INT32_MAX)
+    return copy(dst, src, bytes, hipMemcpyDeviceToHost, stream);
+  const int code = shdw_hip_copy(static_cast<int>(bytes / 4), static_cast<const float*>(src), static_cast<float*>(staging), stream);
+  if (code != SHDW_OK) return code;
+  const hipError_t e = hipStreamSynchronize(as_stream(stream));
+  if (e != hipSuccess) return rc(e);
+  std::memcpy(dst, staging, bytes);
+  return SHDW_OK;
 }
 int shdw_hip_memcpy_d2d(void* dst, const void* src, size_t bytes, void* stream) {
   return copy(dst, src, bytes, hipMemcpyDeviceToDevice, stream);

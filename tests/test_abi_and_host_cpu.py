@@ -176,6 +176,9 @@ def test_entry_points_validate_before_touching_the_device():
     assert lib.shdw_hip_batch_norm_scale_residual_relu(16, 2, 8, p, p, p, 1.0, 0.0, p, p, None, 0, p, p, None) == E
     assert lib.shdw_hip_batch_norm_scale_residual_relu(15, 2, 8, p, p, p, 1.0, 0.0, p, p, p, 0, p, p, None) == E
     assert lib.shdw_hip_batch_norm_scale_residual_relu(0, 2, 8, p, p, p, 1.0, 0.0, p, p, p, 0, p, p, None) == 0
+    assert lib.shdw_hip_memcpy_d2h_staged(p, p, 4, None, None) == E
+    assert lib.shdw_hip_memcpy_d2h_staged(None, p, 4, p, None) == E
+    assert lib.shdw_hip_memcpy_d2h_staged(None, None, 0, None, None) == 0
     gate = lib.shdw_hip_squeeze_gate
     assert gate(16, 2, 8, p, p, None, 1.0, 0.0, p, p, 1, p, p, p, 0, p, p, None) == E       # half of the statistics
     assert gate(16, 2, 8, p, p, p, 1.0, 0.0, p, p, 1, None, None, p, 0, p, p, None) == E    # a residual without a scale

@@ -213,3 +213,15 @@ def test_running_errors(gpu):
             nw.forward({"other": inputs["data"]})
         with pytest.raises(ShadowError, match="Unknown blob"):
             nw.blob("missing")
+
+
+@pytest.mark.parametrize("count", [1, 1023, 4096, 4097])
+def test_results_read_back_around_the_staging_size(gpu, count):
+    """Results of up to 16 KB come back through pinned memory, larger ones by the runtime's copy."""
+    text = "\n".join(["[m]", "[{out_blob, v_s, [y]}]", "[]", "[Input] | [in] | [0 1 1] | [] | [x] | [{x, v_i, [%d]}]" % count,
+                      "[Unary] | [neg] | [1 1 1] | [x] | [y] | [{operation, s_i, [13]}]"]) + "\n"
+    x = normal(5, count)
+    with shadow_amd.Network(text, []) as net:
+        for k in range(3):
+            net.forward({"x": x + np.float32(k)})
+            assert np.array_equal(net.blob("y"), -(x + np.float32(k)))
