@@ -510,6 +510,10 @@ static bool plan_pool_band(const PoolArgs& p, int target_outputs, BandArgs* a) {
 // vectors per row, so that a load instruction covers every other 16 bytes, ran
 // at 59 us on [64,64,112,112] where the band kernel takes 49 and this one 43;
 // workgroups of 64 or 1024 lanes 47 to 48 us, XCD-contiguous numbering no change.)
+// Bound by the latency of its requests and then by memory: with the wave-end
+// column fetched in a branch per row the rows' loads waited for one another,
+// 22.1 us for the 3x3 maximum of [32,64,112,112] (128 MB) against 19.6, and
+// 13.4 against 11.3 for the 3x3 average at stride 1 below on its result.
 struct HalveArgs {
   int in_h, in_w, out_h, out_w;
   FastDiv f_pairs;  // lanes per output row: in_w / 4
@@ -534,8 +538,8 @@ SHDW_DEVICE float neighbour(float own, float from) {
 template <bool MAX, int K, int PAD>
 __global__ __launch_bounds__(kHalveLanes) void pool_halve_kernel(const float* x, float* y, uint32_t tasks,
                                                                  HalveArgs p) {
-  const uint32_t t = blockIdx.x * kHalveLanes + threadIdx.x;
-  if (t >= tasks) return;
+  const uint32_t own_task = blockIdx.x * kHalveLanes + threadIdx.x;
+  const uint32_t t = min(own_task, tasks - 1);  // lanes without a task repeat the last one up to the store
   uint32_t rest, v, plane, r;
   fd_divmod(t, p.f_pairs, rest, v);
   fd_divmod(rest, p.f_out_h, plane, r);
@@ -550,22 +554,33 @@ __global__ __launch_bounds__(kHalveLanes) void pool_halve_kernel(const float* x,
   const int halo_abs = 4 * static_cast<int>(v) + kHaloCol;
   const bool halo_valid = K == 3 && halo_abs >= 0 && halo_abs < p.in_w;
   const uint32_t lane = threadIdx.x & (kWave - 1);
-  const bool fetch_halo = halo_valid && lane == (PAD ? 0u : static_cast<uint32_t>(kWave - 1));
+  const int h_last = p.in_h - 1;
+  // Every request before anything is used, and none in a branch: all lanes ask for
+  // the column of the lane at the wave's end, which then is one address.
+  v4f q[K];
+  float halo[K];
+#pragma unroll
+  for (int i = 0; i < K; ++i) q[i] = load4(img + min(max(h_first + i, 0), h_last) * p.in_w);
+  if (K == 3) {
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+      const uint32_t at = static_cast<uint32_t>(img - x) + min(max(h_first + i, 0), h_last) * p.in_w + (halo_valid ? kHaloCol : 0);
+      halo[i] = x[__builtin_amdgcn_readlane(at, PAD ? 0 : kWave - 1)];
+    }
+  }
+  const bool at_end = lane == (PAD ? 0u : static_cast<uint32_t>(kWave - 1));
   float acc[2];
   acc[0] = acc[1] = MAX ? -FLT_MAX : 0.f;
 #pragma unroll
   for (int i = 0; i < K; ++i) {
     const int ri = h_first + i;
     const bool row_valid = ri >= 0 && ri < p.in_h;
-    const float* row = img + min(max(ri, 0), p.in_h - 1) * p.in_w;
-    const v4f q = load4(row);
     float cells[kCells];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) cells[kAt + e] = q[e];
+    for (int e = 0; e < 4; ++e) cells[kAt + e] = q[i][e];
     if (K == 3) {
-      float own = neutral;
-      if (fetch_halo) own = row[kHaloCol];
-      const float h = PAD ? neighbour<-1>(own, q[3]) : neighbour<+1>(own, q[0]);
+      const float own = at_end ? halo[i] : neutral;
+      const float h = PAD ? neighbour<-1>(own, q[i][3]) : neighbour<+1>(own, q[i][0]);
       cells[PAD ? 0 : 4] = halo_valid ? h : neutral;
     }
     // a row above or below the input leaves the running values as they are,
@@ -587,6 +602,7 @@ __global__ __launch_bounds__(kHalveLanes) void pool_halve_kernel(const float* x,
     const int pool_size = (h_end_pad - h_first) * (w_end_pad - w_first);
     res[j] = MAX ? acc[j] : acc[j] / static_cast<float>(pool_size);
   }
+  if (own_task >= tasks) return;
   typedef float v2f __attribute__((ext_vector_type(2)));
   float* dst = y + ((plane * static_cast<uint32_t>(p.out_h) + r) * static_cast<uint32_t>(p.out_w) + 2 * v);
   __builtin_nontemporal_store(v2f{res[0], res[1]}, reinterpret_cast<v2f*>(dst));
@@ -602,17 +618,26 @@ template <bool MAX>
 __global__ __launch_bounds__(kHalveLanes) void pool_same_kernel(const float* x, float* y, uint32_t tasks,
                                                                 HalveArgs p) {
   // runs of eight workgroups on one XCD: every input row is read for three output rows
-  const uint32_t t = xcd_runs(blockIdx.x, gridDim.x, 3) * kHalveLanes + threadIdx.x;
-  if (t >= tasks) return;
+  const uint32_t own_task = xcd_runs(blockIdx.x, gridDim.x, 3) * kHalveLanes + threadIdx.x;
+  const uint32_t t = min(own_task, tasks - 1);
   uint32_t rest, v, plane, r;
   fd_divmod(t, p.f_pairs, rest, v);
   fd_divmod(rest, p.f_out_h, plane, r);
   const float neutral = MAX ? -FLT_MAX : 0.f;
   const uint32_t lane = threadIdx.x & (kWave - 1);
   const bool left_valid = v > 0, right_valid = 4 * v + 4 < static_cast<uint32_t>(p.in_w);
-  const bool fetch_left = left_valid && lane == 0, fetch_right = right_valid && lane == kWave - 1;
   const float* img = x + plane * static_cast<uint32_t>(p.in_h * p.in_w) + 4 * v;
   const int h_first = static_cast<int>(r) - 1;
+  v4f q3[3];
+  float left[3], right[3];  // the columns beside the wave's vectors, requested as above
+#pragma unroll
+  for (int i = 0; i < 3; ++i) q3[i] = load4(img + min(max(h_first + i, 0), p.in_h - 1) * p.in_w);
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    const uint32_t at = static_cast<uint32_t>(img - x) + min(max(h_first + i, 0), p.in_h - 1) * p.in_w;
+    left[i] = x[__builtin_amdgcn_readlane(at - (left_valid ? 1 : 0), 0)];
+    right[i] = x[__builtin_amdgcn_readlane(at + (right_valid ? 4 : 0), kWave - 1)];
+  }
   float acc[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) acc[j] = MAX ? -FLT_MAX : 0.f;
@@ -620,11 +645,8 @@ __global__ __launch_bounds__(kHalveLanes) void pool_same_kernel(const float* x, 
   for (int i = 0; i < 3; ++i) {
     const int ri = h_first + i;
     const bool row_valid = ri >= 0 && ri < p.in_h;
-    const float* row = img + min(max(ri, 0), p.in_h - 1) * p.in_w;
-    const v4f q = load4(row);
-    float own_l = neutral, own_r = neutral;
-    if (fetch_left) own_l = row[-1];
-    if (fetch_right) own_r = row[4];
+    const v4f q = q3[i];
+    const float own_l = lane == 0 ? left[i] : neutral, own_r = lane == kWave - 1 ? right[i] : neutral;
     const float hl = neighbour<-1>(own_l, q[3]), hr = neighbour<+1>(own_r, q[0]);
     const float cells[6] = {left_valid ? hl : neutral, q[0], q[1], q[2], q[3], right_valid ? hr : neutral};
 #pragma unroll
@@ -644,6 +666,7 @@ __global__ __launch_bounds__(kHalveLanes) void pool_same_kernel(const float* x, 
     const int pool_size = (h_end_pad - h_first) * (w_end_pad - w_first);
     res[j] = MAX ? acc[j] : acc[j] / static_cast<float>(pool_size);
   }
+  if (own_task >= tasks) return;
   store4_stream(y + ((plane * static_cast<uint32_t>(p.out_h) + r) * static_cast<uint32_t>(p.out_w) + 4 * v), res);
 }
 
