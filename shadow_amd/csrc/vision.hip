@@ -208,7 +208,7 @@ __global__ __launch_bounds__(kBlock) void pool_window_kernel(const float* x, flo
 // input reads a pad cell, a cell above or below reads the spare row, and the
 // unrolled K x K walk needs no predicates at all.
 constexpr int kBandTileFloats = 8192;  // upper bound of the dynamic LDS tile (32 KB)
-constexpr int kBandBatch = 4;
+constexpr int kBandBatch = 8;
 constexpr int kBandMaxPad = 64;        // wider clipping goes to the direct kernel
 constexpr int kPoolBandOutputs = 512;  // outputs a workgroup aims for (measured best of 256..4096)
 constexpr int kBandWideMinCols = 3;    // windows this wide at a column stride of 1: four outputs per lane
@@ -387,8 +387,13 @@ SHDW_DEVICE void band_windows_wide(const float* tile, float* y, const BandArgs& 
 // A workgroup walks `bands_per_group` consecutive bands.  PIPE (every span
 // starts 16-byte aligned and in_w % 4 == 0): the next band's 128-bit loads are
 // issued into registers before the current band's windows are walked, so HBM
-// requests stay in flight during the LDS phase.  Otherwise each band is staged
-// on its own with scalar loads.
+// requests stay in flight during the LDS phase.  Otherwise the same with single
+// floats, up to eight a lane ahead and the rest of a longer span behind them.
+// Lanes beyond a span take its last elements again: a branch around each load
+// has the compiler wait for the one before it.  3x3 maximum by two of
+// [44,96,55,55] behind an LRN 18.4 -> about 15 us (the pair 49.3 -> 47.2); the
+// single floats keep the non-temporal hint, without it the pair takes 50.8, the
+// LRN's own input no longer being in the cache for the next pass.
 constexpr int kBandMaxRegs = kBandTileFloats / 4 / kBlock;  // vectors per lane for a full tile
 static_assert(kBandMaxRegs == 8, "the launch switch covers up to 8 staged vectors per lane");
 constexpr uint32_t kBandGroupsWanted = 4096;
@@ -411,12 +416,13 @@ __global__ __launch_bounds__(kBlock) void pool_band_kernel(const float* x, float
   __syncthreads();
   if (PIPE) {
     v4f reg[kBandRegs];
-    BandSpan cur = band_span(p, x, g0);
+    const auto request = [&](const BandSpan& bs) {
+      if (bs.span == 0) return;  // every window of the band in the padding
 #pragma unroll
-    for (int k = 0; k < kBandRegs; ++k) {
-      const uint32_t v = k * kBlock + threadIdx.x;
-      if (4 * v < cur.span) reg[k] = load4_stream(cur.src + 4ull * v);
-    }
+      for (int k = 0; k < kBandRegs; ++k) reg[k] = load4_stream(bs.src + min(4u * (k * kBlock + threadIdx.x), bs.span - 4));
+    };
+    BandSpan cur = band_span(p, x, g0);
+    request(cur);
     for (uint32_t g = g0; g < g1; ++g) {
 #pragma unroll
       for (int k = 0; k < kBandRegs; ++k) {
@@ -427,35 +433,42 @@ __global__ __launch_bounds__(kBlock) void pool_band_kernel(const float* x, float
       const BandSpan walk = cur;
       if (g + 1 < g1) {
         cur = band_span(p, x, g + 1);
-#pragma unroll
-        for (int k = 0; k < kBandRegs; ++k) {
-          const uint32_t v = k * kBlock + threadIdx.x;
-          if (4 * v < cur.span) reg[k] = load4_stream(cur.src + 4ull * v);
-        }
+        request(cur);
       }
       if (p.wide) band_windows_wide<MAX, K>(tile, y, p, walk);
       else band_windows<MAX, K>(tile, y, p, walk);
       __syncthreads();  // the tile is rewritten next
     }
   } else {
+    float reg[kBandBatch];
+    const auto request = [&](const BandSpan& bs, uint32_t t0) {
+      if (bs.span == 0) return;
+#pragma unroll
+      for (int k = 0; k < kBandBatch; ++k) reg[k] = __builtin_nontemporal_load(bs.src + min(t0 + k * kBlock + threadIdx.x, bs.span - 1));
+    };
+    const auto keep = [&](const BandSpan& bs, uint32_t t0) {
+#pragma unroll
+      for (int k = 0; k < kBandBatch; ++k) {
+        const uint32_t t = t0 + k * kBlock + threadIdx.x;
+        if (t < bs.span) tile[band_slot(p, t)] = reg[k];
+      }
+    };
+    BandSpan cur = band_span(p, x, g0);
+    request(cur, 0);
     for (uint32_t g = g0; g < g1; ++g) {
-      const BandSpan bs = band_span(p, x, g);
-      for (uint32_t t0 = 0; t0 < bs.span; t0 += kBandBatch * kBlock) {
-        float reg[kBandBatch];
-#pragma unroll
-        for (int k = 0; k < kBandBatch; ++k) {
-          const uint32_t t = t0 + k * kBlock + threadIdx.x;
-          if (t < bs.span) reg[k] = __builtin_nontemporal_load(bs.src + t);
-        }
-#pragma unroll
-        for (int k = 0; k < kBandBatch; ++k) {
-          const uint32_t t = t0 + k * kBlock + threadIdx.x;
-          if (t < bs.span) tile[band_slot(p, t)] = reg[k];
-        }
+      keep(cur, 0);
+      for (uint32_t t0 = kBandBatch * kBlock; t0 < cur.span; t0 += kBandBatch * kBlock) {
+        request(cur, t0);
+        keep(cur, t0);
       }
       __syncthreads();
-      if (p.wide) band_windows_wide<MAX, K>(tile, y, p, bs);
-      else band_windows<MAX, K>(tile, y, p, bs);
+      const BandSpan walk = cur;
+      if (g + 1 < g1) {
+        cur = band_span(p, x, g + 1);
+        request(cur, 0);
+      }
+      if (p.wide) band_windows_wide<MAX, K>(tile, y, p, walk);
+      else band_windows<MAX, K>(tile, y, p, walk);
       __syncthreads();
     }
   }
