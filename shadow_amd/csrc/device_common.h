@@ -28,17 +28,27 @@ constexpr int kStream = 64;
 
 #define SHDW_DEVICE __device__ __forceinline__
 
-// 128-bit streaming accesses, the one place that states their cache policy.
-// Stores carry the non-temporal hint: a plain store leaves dirty lines in L2 that
-// are written back when the kernel ends (broadcast of 67 MB of output 11.4 us
-// with the hint, 13.0 to 19.2 without; 103 MB copy 19.3 against 31.9).  Loads do
-// not: a line that a plain load fetched stays in the 256 MB Infinity Cache, where
-// the next operator on the same tensor finds it (operators read what the one
-// before them read or wrote), and the per-channel parameters stay in L2 either
-// way.  Seven operators over one 205 MB tensor 434 -> 420 us, five reductions of
-// one 51 MB tensor 50.3 -> 48.2 us, three norms of one 51 MB tensor 64.9 -> 58.1 us,
-// grid sampling of a 26 MB tensor 17.4 -> 13.4 us.
-SHDW_DEVICE v4f load4_stream(const float* p) { return *reinterpret_cast<const v4f*>(p); }
+// Streaming accesses: whose cache lines one wave asks for, once.  Both directions
+// carry the non-temporal hint, every such access through these functions.
+// Stores: a plain store leaves dirty lines in L2 that are written back when the
+// kernel ends (broadcast of 67 MB of output 11.4 us with the hint, 13.0 to 19.2
+// without; 103 MB copy 19.3 against 31.9).
+// Loads: without the hint an operand that is new, or that the operator before has
+// just written, arrives more slowly from 12 MB on, whatever the kernel: ReLU of 12.8 /
+// 51 / 205 MB 5.1 / 17.0 / 62.6 us with it and 5.4 / 17.5 / 65.1 without, the sum of two of
+// 51 MB 24.3 and 26.2, 7x7 averages of 205 MB 31.8 and 34.8, group norms of 205 MB 76.5 and
+// 80.8; behind the kernel that wrote the operand the same (ReLU 16.9 and 17.8, sum 24.5 and
+// 26.2).  Plain loads pay only where several operators read one tensor of up to 256 MB one
+// after another (ReLU of 51 MB 15.6 against 16.6), which a kernel cannot know.
+// Lines that several waves share are for load4 and load4_any below: operands that are
+// read again, and rows that start anywhere in a line where short pieces of them go to
+// different waves (channel shuffle of 49-element rows, 103 MB: 20.9 us plain, 23.2 with the
+// hint; the transposes in movers.hip; 3x3 pooling bands of 27-wide rows 23.4 and 25.7).
+template <class T>
+SHDW_DEVICE T load_stream(const T* p) {
+  return __builtin_nontemporal_load(p);
+}
+SHDW_DEVICE v4f load4_stream(const float* p) { return load_stream(reinterpret_cast<const v4f*>(p)); }  // 128 bits
 SHDW_DEVICE void store4_stream(float* p, v4f v) {
   __builtin_nontemporal_store(v, reinterpret_cast<v4f*>(p));
 }
@@ -51,7 +61,7 @@ SHDW_DEVICE v4f load4(const float* p) { return *reinterpret_cast<const v4f*>(p);
 // 73 us, where four 4-byte accesses per lane need 172 us.
 typedef float v4f_unaligned __attribute__((ext_vector_type(4), aligned(4)));
 SHDW_DEVICE v4f load4_stream_any(const float* p) {
-  return *reinterpret_cast<const v4f_unaligned*>(p);
+  return __builtin_nontemporal_load(reinterpret_cast<const v4f_unaligned*>(p));  // T would lose the alignment
 }
 SHDW_DEVICE v4f load4_any(const float* p) { return *reinterpret_cast<const v4f_unaligned*>(p); }
 SHDW_DEVICE void store4_stream_any(float* p, v4f v) {

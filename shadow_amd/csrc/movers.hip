@@ -57,7 +57,7 @@ __global__ __launch_bounds__(kStream) void copy_chunks_any_kernel(const float* s
   const float* s = src + static_cast<uint64_t>(n) * src_pitch + src_off + first;
   float* d = dst + static_cast<uint64_t>(n) * dst_pitch + dst_off + first;
   if (first + 4 <= chunk) {
-    store4_stream_any(d, load4_stream_any(s));
+    store4_stream_any(d, load4_any(s));  // chunks share lines (103 MB: 19.4 us, 20.0 streamed)
   } else {
     for (uint32_t j = 0; first + j < chunk; ++j) d[j] = s[j];
   }
@@ -127,7 +127,7 @@ __global__ __launch_bounds__(kStream) void rows_pick_any_kernel(const float* x, 
   const float* src = x + s * inner + first;
   if (first + 4 <= inner) {
     const v4f zero = {0.f, 0.f, 0.f, 0.f};
-    store4_stream_any(dst, s < 0 ? zero : load4_stream_any(src));
+    store4_stream_any(dst, s < 0 ? zero : load4_any(src));  // rows share lines ([256,1024,7,7] 30.4 us, 33.2 streamed)
   } else {
     for (uint32_t j = 0; first + j < inner; ++j) dst[j] = s < 0 ? 0.f : src[j];
   }
@@ -151,11 +151,11 @@ __global__ __launch_bounds__(kStream) void rows_pick_flat_kernel(const float* x,
     int64_t s = map.source(r);
     v4f v;
     if (p + 4 <= inner) {
-      v = s < 0 ? v4f{0.f, 0.f, 0.f, 0.f} : load4_stream_any(x + s * inner + p);
+      v = s < 0 ? v4f{0.f, 0.f, 0.f, 0.f} : load4_any(x + s * inner + p);  // rows share lines
     } else {
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        v[j] = s < 0 ? 0.f : __builtin_nontemporal_load(x + s * inner + p);
+        v[j] = s < 0 ? 0.f : x[s * inner + p];
         if (++p == inner) p = 0, s = map.source(++r);  // never past the last row: 4 i + 3 < n
       }
     }
@@ -272,6 +272,17 @@ __global__ __launch_bounds__(kBlock) void permute_generic_kernel(const float* x,
   }
 }
 
+// Whether the pieces of rows that a transposition's tiles read share cache lines with
+// other tiles' pieces, or their vectors straddle lines: such rows are read with plain
+// loads.  Not where rows are whole units (64 bytes for the 64 x 64 tiles, lines for the
+// longer and fewer pieces of the thin ones), and not where a tile takes rows whole, by whole
+// vectors.  [64,128,729] 10.1 us plain and 12.1 with the hint, [64,3000,63] 27.9 and 32.3,
+// [64,200,1444] 39.5 and 44.2, [64,126,400] 8.3 and 9.2; on the other side [64,256,3136] 72.5
+// and 70.6, [64,3000,48] 17.3 and 16.8, [64,128,784] 9.8 and 9.6, [64,16,3136] 7.6 and 6.9.
+static bool shared_rows(const float* x, uint32_t cols, uint32_t tile_cols, uint32_t unit) {
+  return !aligned16(x) || !(cols % unit == 0 || (cols <= tile_cols && cols % 4 == 0));
+}
+
 // Transposition with one thin side (interleaved <-> planar images: [H*W][3] <->
 // [3][H*W]): the 64 x 64 tiles below would be 3 wide, nine tenths of every
 // workgroup idle ([4.3M][3] -> [3][4.3M]: 229 us per 51 MB).  Here a tile takes the
@@ -288,7 +299,8 @@ constexpr uint32_t kThinTileFloats = 8192;  // 32 KB
 // 22 us for thin = 17); the tile rows get a pitch of thin + 1 instead (21 us), and
 // the contiguous side, whose vectors no longer sit on 16 bytes in LDS, moves its
 // four floats one by one there.
-template <bool COLS_THIN, bool PAD>
+// SHARED: the planar rows are read with plain loads, see shared_rows().
+template <bool COLS_THIN, bool PAD, bool SHARED>
 __global__ __launch_bounds__(kBlock) void transpose_thin_kernel(const float* x, float* y, uint32_t big,
                                                                  FastDiv f_thin, uint32_t span,
                                                                  FastDiv f_tiles) {
@@ -337,7 +349,8 @@ __global__ __launch_bounds__(kBlock) void transpose_thin_kernel(const float* x, 
   } else {
     for (uint32_t u = threadIdx.x; u < thin * quads; u += kBlock) {
       const uint32_t i = u / quads, q = u - i * quads;
-      const v4f r = load4_stream_any(planar_src + static_cast<uint64_t>(i) * big + 4 * q);
+      const float* src = planar_src + static_cast<uint64_t>(i) * big + 4 * q;
+      const v4f r = SHARED ? load4_any(src) : load4_stream_any(src);
 #pragma unroll
       for (int k = 0; k < 4; ++k) tile[(4 * q + k) * pitch + i] = r[k];
     }
@@ -368,6 +381,8 @@ constexpr int kTile = 64;
 // multiples of four, odd pointers); the last vector of a row that is not whole
 // moves float by float.  One float per lane instead ran at 2.2 to 2.7 times a
 // copy ([24][129][4148] -> [24][4148][129]: 38 us per 51 MB).
+// SHARED: plain loads, see shared_rows().
+template <bool SHARED>
 __global__ __launch_bounds__(kBlock) void transpose_kernel(const float* x, float* y, uint32_t rows,
                                                             uint32_t cols, uint32_t tiles_c,
                                                             FastDiv f_tiles) {
@@ -384,11 +399,11 @@ __global__ __launch_bounds__(kBlock) void transpose_kernel(const float* x, float
     if (r < rows && c < cols) {
       const float* src = x + plane + static_cast<uint64_t>(r) * cols + c;
       if (c + 4 <= cols) {
-        const v4f v = load4_stream_any(src);
+        const v4f v = SHARED ? load4_any(src) : load4_stream_any(src);
 #pragma unroll
         for (int j = 0; j < 4; ++j) tile[k][4 * q + j] = v[j];
       } else {
-        for (uint32_t j = 0; c + j < cols; ++j) tile[k][4 * q + j] = __builtin_nontemporal_load(src + j);
+        for (uint32_t j = 0; c + j < cols; ++j) tile[k][4 * q + j] = src[j];
       }
     }
   }
@@ -920,7 +935,7 @@ __global__ __launch_bounds__(kStream) void resize_double_nearest_kernel(const fl
   const uint32_t t = blockIdx.x * kStream + threadIdx.x;
   if (t >= tasks) return;
   typedef float v2f __attribute__((ext_vector_type(2)));
-  const v2f v = __builtin_nontemporal_load(reinterpret_cast<const v2f*>(x) + t);
+  const v2f v = load_stream(reinterpret_cast<const v2f*>(x) + t);
   uint32_t row, o;  // row counts input rows over all planes; o the lane's place in the row
   fd_divmod(t, p.f_vecs, row, o);
   float* dst = y + 2 * row * p.out_w + 4 * o;
@@ -1189,14 +1204,21 @@ int shdw_hip_permute(int num_axes, const int* in_shape, const int* order, const 
       if (span && groups <= INT32_MAX) {
         const FastDiv ft = make_fastdiv(tiles), fthin = make_fastdiv(thin);
         const uint32_t g = static_cast<uint32_t>(groups);
+        // tiles of a side of up to 15 rows keep 512 and more of the other, little of it shared:
+        // [64,3,50625] 18.6 us plain and 18.4 with the hint, [64,8,12321] 11.0 both
+        const bool shared = thin >= 16 && shared_rows(x, big, span, 32);
         if (cols_thin && pad)
-          transpose_thin_kernel<true, true><<<g, kBlock, 0, st>>>(x, y, big, fthin, span, ft);
+          transpose_thin_kernel<true, true, false><<<g, kBlock, 0, st>>>(x, y, big, fthin, span, ft);
         else if (cols_thin)
-          transpose_thin_kernel<true, false><<<g, kBlock, 0, st>>>(x, y, big, fthin, span, ft);
+          transpose_thin_kernel<true, false, false><<<g, kBlock, 0, st>>>(x, y, big, fthin, span, ft);
+        else if (pad && shared)
+          transpose_thin_kernel<false, true, true><<<g, kBlock, 0, st>>>(x, y, big, fthin, span, ft);
         else if (pad)
-          transpose_thin_kernel<false, true><<<g, kBlock, 0, st>>>(x, y, big, fthin, span, ft);
+          transpose_thin_kernel<false, true, false><<<g, kBlock, 0, st>>>(x, y, big, fthin, span, ft);
+        else if (shared)
+          transpose_thin_kernel<false, false, true><<<g, kBlock, 0, st>>>(x, y, big, fthin, span, ft);
         else
-          transpose_thin_kernel<false, false><<<g, kBlock, 0, st>>>(x, y, big, fthin, span, ft);
+          transpose_thin_kernel<false, false, false><<<g, kBlock, 0, st>>>(x, y, big, fthin, span, ft);
         return launch_status();
       }
     }
@@ -1205,7 +1227,10 @@ int shdw_hip_permute(int num_axes, const int* in_shape, const int* order, const 
     if (groups <= INT32_MAX) {
       const FastDiv ft = make_fastdiv(tiles_r * tiles_c);
       const uint32_t g = static_cast<uint32_t>(groups);
-      transpose_kernel<<<g, kBlock, 0, st>>>(x, y, rows, cols, tiles_c, ft);
+      if (shared_rows(x, cols, kTile, 16))
+        transpose_kernel<true><<<g, kBlock, 0, st>>>(x, y, rows, cols, tiles_c, ft);
+      else
+        transpose_kernel<false><<<g, kBlock, 0, st>>>(x, y, rows, cols, tiles_c, ft);
       return launch_status();
     }
   }

@@ -343,12 +343,12 @@ __global__ __launch_bounds__(kBlock) void reduce_strided_short_kernel(const floa
   const uint32_t n = VEC ? min(4u, inner - 4 * c) : 1u;
   auto fetch = [&](uint32_t r) -> v4f {
     const float* src = p + static_cast<uint64_t>(r) * inner;
-    if (!VEC) return v4f{__builtin_nontemporal_load(src), 0.f, 0.f, 0.f};
+    if (!VEC) return v4f{load_stream(src), 0.f, 0.f, 0.f};
     if (n == 4) return load4_stream_any(src);  // any dword address: rows need not be whole vectors
     v4f v = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int j = 0; j < 3; ++j)
-      if (static_cast<uint32_t>(j) < n) v[j] = __builtin_nontemporal_load(src + j);
+      if (static_cast<uint32_t>(j) < n) v[j] = load_stream(src + j);
     return v;
   };
   uint32_t r = 0;
@@ -493,11 +493,11 @@ __global__ __launch_bounds__(kWave * WAVES) void reduce_strided_kernel(
     for (; r + 3 * kWaves < r_end; r += 4 * kWaves) {
       float v[4];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) v[u] = __builtin_nontemporal_load(p + static_cast<size_t>(r + u * kWaves) * inner);
+      for (int u = 0; u < 4; ++u) v[u] = load_stream(p + static_cast<size_t>(r + u * kWaves) * inner);
 #pragma unroll
       for (int u = 0; u < 4; ++u) acc.add(v[u], r + u * kWaves);
     }
-    for (; r < r_end; r += kWaves) acc.add(__builtin_nontemporal_load(p + static_cast<size_t>(r) * inner), r);
+    for (; r < r_end; r += kWaves) acc.add(load_stream(p + static_cast<size_t>(r) * inner), r);
   }
   if (w > 0) lds[w - 1][lane] = acc.pack();
   __syncthreads();

@@ -144,7 +144,7 @@ __global__ __launch_bounds__(kBlock) void softmax_columns_reg_kernel(const float
   float v[DMAX];
 #pragma unroll
   for (int c = 0; c < DMAX; ++c)
-    if (c < DFULL || c < dim) v[c] = __builtin_nontemporal_load(xc + static_cast<uint64_t>(c) * inner);
+    if (c < DFULL || c < dim) v[c] = load_stream(xc + static_cast<uint64_t>(c) * inner);
   float max_val = -FLT_MAX;
 #pragma unroll
   for (int c = 0; c < DMAX; ++c)
@@ -467,7 +467,7 @@ __global__ __launch_bounds__(kBlock) void normalize_columns_reg_kernel(const flo
   float v[DMAX];
 #pragma unroll
   for (int c = 0; c < DMAX; ++c)
-    if (c < dim) v[c] = __builtin_nontemporal_load(xc + static_cast<uint64_t>(c) * inner);
+    if (c < dim) v[c] = load_stream(xc + static_cast<uint64_t>(c) * inner);
   double acc = 0;
 #pragma unroll
   for (int c = 0; c < DMAX; ++c)
@@ -515,7 +515,7 @@ SHDW_DEVICE void quad_load(const float* xc, const QuadLane& q, uint32_t dim, uin
         v[c] = v4f{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int k = 0; k < 3; ++k)
-          if (static_cast<uint32_t>(k) < q.n) v[c][k] = __builtin_nontemporal_load(xc + static_cast<uint64_t>(c) * inner + k);
+          if (static_cast<uint32_t>(k) < q.n) v[c][k] = load_stream(xc + static_cast<uint64_t>(c) * inner + k);
       }
     }
   }
@@ -881,10 +881,6 @@ struct TileLane {
     c0 = threadIdx.x / LANES_PER_ROW;
     valid = j < width ? min(4u, width - j) : 0u;
   }
-  // KEEP: leave the lines in the Infinity Cache (Softmax, [16,150,72,72] 28.9 -> 25.9 us);
-  // Normalize streams past it, which leaves it to the score maps of a detection head
-  // (the head's five operators 64.0 us, 66.9 us with the feature map kept).
-  template <bool KEEP>
   SHDW_DEVICE void load(const float* xs, v4f (&r)[kTilePerLane]) const {
     if (valid == 0) return;
 #pragma unroll
@@ -893,7 +889,7 @@ struct TileLane {
       if (c >= dim) continue;
       const float* src = xs + static_cast<uint64_t>(c) * inner + j;
       if (!TAIL || valid == 4) {
-        r[u] = KEEP ? load4_stream_any(src) : __builtin_nontemporal_load(reinterpret_cast<const v4f_unaligned*>(src));
+        r[u] = load4_stream_any(src);
       } else {
         r[u] = v4f{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -974,7 +970,7 @@ __global__ __launch_bounds__(kBlock) void normalize_tile_kernel(const float* x, 
   const uint64_t base = static_cast<uint64_t>(n) * dim * inner + p0;
   const TileLane<TS_SHIFT, ROWS> lane(width, dim, inner);
   v4f r[kTilePerLane];
-  lane.template load<false>(x + base, r);
+  lane.load(x + base, r);
   // the tile holds the terms of the sums, fp32 values that widen exactly: the folding wave's chain sets the
   // pace of a tall, narrow tile, and every instruction taken off it is time off the tile
   lane.park(lds, r, [p](const v4f& v) {
@@ -1091,7 +1087,7 @@ __global__ __launch_bounds__(kBlock) void softmax_tile_kernel(const float* x, fl
   const uint64_t base = static_cast<uint64_t>(n) * dim * inner + p0;
   const Lane lane(width, dim, inner);
   v4f r[kTilePerLane];
-  lane.template load<true>(x + base, r);
+  lane.load(x + base, r);
   if (lane.valid != 0) {
     v4f m = {-FLT_MAX, -FLT_MAX, -FLT_MAX, -FLT_MAX};
     bool nan[4] = {false, false, false, false};
@@ -1474,7 +1470,7 @@ struct RowStream {
       } else {
 #pragma unroll
         for (int k = 0; k < 3; ++k)
-          if (static_cast<uint32_t>(k) < n) reg[i][k] = __builtin_nontemporal_load(src + k);
+          if (static_cast<uint32_t>(k) < n) reg[i][k] = load_stream(src + k);
       }
     }
   }
@@ -1674,7 +1670,7 @@ struct TallTile {
         } else {
 #pragma unroll
           for (int e = 0; e < 3; ++e)
-            if (static_cast<uint32_t>(e) < valid) v[i][e] = __builtin_nontemporal_load(src + e);
+            if (static_cast<uint32_t>(e) < valid) v[i][e] = load_stream(src + e);
         }
       }
   }
@@ -1875,7 +1871,7 @@ struct LongSlab {
       } else {
 #pragma unroll
         for (int j = 0; j < 3; ++j)
-          if (e + j < cells) v[i][j] = __builtin_nontemporal_load(src + e + j);
+          if (e + j < cells) v[i][j] = load_stream(src + e + j);
       }
     }
   }

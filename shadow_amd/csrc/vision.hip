@@ -444,7 +444,7 @@ __global__ __launch_bounds__(kBlock) void pool_band_kernel(const float* x, float
     const auto request = [&](const BandSpan& bs, uint32_t t0) {
       if (bs.span == 0) return;
 #pragma unroll
-      for (int k = 0; k < kBandBatch; ++k) reg[k] = __builtin_nontemporal_load(bs.src + min(t0 + k * kBlock + threadIdx.x, bs.span - 1));
+      for (int k = 0; k < kBandBatch; ++k) reg[k] = load_stream(bs.src + min(t0 + k * kBlock + threadIdx.x, bs.span - 1));
     };
     const auto keep = [&](const BandSpan& bs, uint32_t t0) {
 #pragma unroll
@@ -1105,7 +1105,7 @@ __global__ __launch_bounds__(kBlock) void pool_plane_kernel(const float* x, floa
             uint32_t r, c;
             fd_divmod(t, fc, r, c);
             slot[k] = r * pitch + c;
-            reg[k] = __builtin_nontemporal_load(base + static_cast<uint64_t>(r) * len + c0 + c);
+            reg[k] = load_stream(base + static_cast<uint64_t>(r) * len + c0 + c);
           }
         }
 #pragma unroll
@@ -1202,11 +1202,11 @@ __global__ __launch_bounds__(kBlock) void pool_rows_stream_kernel(const float* x
       if (row0 + g >= rows || c >= len) continue;
       const float* src = x + static_cast<uint64_t>(row0 + g) * len + c;
       if (c + 4 <= len) {
-        reg[i] = __builtin_nontemporal_load(reinterpret_cast<const v4f_unaligned*>(src));
+        reg[i] = load4_stream_any(src);
       } else {
 #pragma unroll
         for (int k = 0; k < 3; ++k)
-          if (c + k < len) reg[i][k] = __builtin_nontemporal_load(src + k);
+          if (c + k < len) reg[i][k] = load_stream(src + k);
       }
     }
   };

@@ -134,6 +134,24 @@ def test_permute_op(ws, shape, order):
     assert_bit_exact(got, want, "permute")
 
 
+@pytest.mark.parametrize("shape", [(2, 70, 784), (2, 70, 786), (2, 70, 60), (2, 70, 63),      # 64 x 64 tiles: either kind of load
+                                   (2, 126, 416), (2, 126, 400), (2, 24, 352), (2, 24, 361),  # thin tiles of long rows
+                                   (2, 16, 352), (2, 16, 361), (2, 12, 361), (2, 361, 24), (2, 361, 23)])
+@pytest.mark.parametrize("x_off", [0, 1])
+def test_transposes_of_rows_in_whole_lines_and_not(gpu, shape, x_off):
+    """Rows whose pieces share cache lines are loaded otherwise than rows of whole lines; pointers off the vector
+    boundary count among the former.  Same bits."""
+    x = with_specials(normal(95, shape), 95).reshape(shape)
+    dx, dy = shadow_amd.Buffer(x.nbytes + 16), shadow_amd.Buffer(x.nbytes)
+    dx.upload(x, 4 * x_off)
+    lib = shadow_amd.hip()
+    shadow_amd.check(lib.shdw_hip_permute(3, shadow_amd.ints(list(shape)), shadow_amd.ints([0, 2, 1]), dx.ptr + 4 * x_off,
+                                          dy.ptr, None))
+    shadow_amd.check(lib.shdw_hip_stream_sync(None))
+    assert_bit_exact(dy.download(count=x.size).reshape(shape[0], shape[2], shape[1]), np.ascontiguousarray(x.swapaxes(1, 2)),
+                     "%s + %d" % (shape, x_off))
+
+
 @pytest.mark.parametrize("type_", [0, 1])
 # rows that are whole vectors and rows that are not (26, 38, 6 and 9 floats: a lane's four source floats run
 # over the end of a row, a channel and an image), strides 1 to 4, a tensor that is no whole vectors
