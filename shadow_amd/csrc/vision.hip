@@ -208,7 +208,6 @@ __global__ __launch_bounds__(kBlock) void pool_window_kernel(const float* x, flo
 // input reads a pad cell, a cell above or below reads the spare row, and the
 // unrolled K x K walk needs no predicates at all.
 constexpr int kBandTileFloats = 8192;  // upper bound of the dynamic LDS tile (32 KB)
-constexpr int kBandBatch = 8;
 constexpr int kBandMaxPad = 64;        // wider clipping goes to the direct kernel
 constexpr int kPoolBandOutputs = 512;  // outputs a workgroup aims for (measured best of 256..4096)
 constexpr int kBandWideMinCols = 3;    // windows this wide at a column stride of 1: four outputs per lane
@@ -384,26 +383,29 @@ SHDW_DEVICE void band_windows_wide(const float* tile, float* y, const BandArgs& 
   }
 }
 
-// A workgroup walks `bands_per_group` consecutive bands.  PIPE (every span
+// A workgroup walks `bands_per_group` consecutive bands.  kBandVectors (every span
 // starts 16-byte aligned and in_w % 4 == 0): the next band's 128-bit loads are
 // issued into registers before the current band's windows are walked, so HBM
 // requests stay in flight during the LDS phase.  Otherwise the same with single
-// floats, up to eight a lane ahead and the rest of a longer span behind them.
-// Lanes beyond a span take its last elements again: a branch around each load
-// has the compiler wait for the one before it.  3x3 maximum by two of
-// [44,96,55,55] behind an LRN 18.4 -> about 15 us (the pair 49.3 -> 47.2); the
-// single floats keep the non-temporal hint, without it the pair takes 50.8, the
-// LRN's own input no longer being in the cache for the next pass.
+// floats, as many a lane ahead as a band has, up to eight, and the rest of a longer
+// span behind them.  Lanes beyond a span take its last elements again: a branch
+// around each load has the compiler wait for the one before it.
+// Single floats are plain loads (kBandFloatsKept) where the rows that neighbouring bands
+// share are a sixteenth of what a band reads or more, and the input is 24 MB or more;
+// elsewhere they carry the hint of the streams.  Operands new in every call, hint / plain:
+// [16,64,225,225] 3x3 at stride 1 132.8 / 122.2 us, [64,64,113,113] 5x5 at stride 1 134.8 / 125.6,
+// [16,64,225,225] 3x3 by two 55.0 / 52.0; [44,96,55,55] 3x3 by two 16.3 / 16.0 (a 37th shared:
+// left with the hint); under 24 MB [16,64,35,35] 3x3 at stride 1 5.8 / 6.1.
+enum { kBandVectors, kBandFloats, kBandFloatsKept };
+constexpr uint64_t kBandKeptBytes = 24u << 20;
 constexpr int kBandMaxRegs = kBandTileFloats / 4 / kBlock;  // vectors per lane for a full tile
 static_assert(kBandMaxRegs == 8, "the launch switch covers up to 8 staged vectors per lane");
 constexpr uint32_t kBandGroupsWanted = 4096;
 constexpr uint32_t kBandMaxWalk = 16;
 
-// REGS: 128-bit vectors a lane stages per band (PIPE only; 0 otherwise).
-template <bool MAX, int K, int REGS>
+// REGS: vectors or floats a lane requests ahead per band.
+template <bool MAX, int K, int KIND, int REGS>
 __global__ __launch_bounds__(kBlock) void pool_band_kernel(const float* x, float* y, BandArgs p) {
-  constexpr bool PIPE = REGS > 0;
-  constexpr int kBandRegs = PIPE ? REGS : 1;
   extern __shared__ __align__(16) float tile[];  // (tile_rows + 1) x pitch
   const uint32_t g0 = blockIdx.x * p.bands_per_group;
   const uint32_t g1 = min(g0 + p.bands_per_group, p.total_bands);
@@ -414,18 +416,18 @@ __global__ __launch_bounds__(kBlock) void pool_band_kernel(const float* x, float
       *reinterpret_cast<v4f*>(tile + t) = v4f{neutral, neutral, neutral, neutral};
   }
   __syncthreads();
-  if (PIPE) {
-    v4f reg[kBandRegs];
+  if (KIND == kBandVectors) {
+    v4f reg[REGS];
     const auto request = [&](const BandSpan& bs) {
       if (bs.span == 0) return;  // every window of the band in the padding
 #pragma unroll
-      for (int k = 0; k < kBandRegs; ++k) reg[k] = load4_stream(bs.src + min(4u * (k * kBlock + threadIdx.x), bs.span - 4));
+      for (int k = 0; k < REGS; ++k) reg[k] = load4_stream(bs.src + min(4u * (k * kBlock + threadIdx.x), bs.span - 4));
     };
     BandSpan cur = band_span(p, x, g0);
     request(cur);
     for (uint32_t g = g0; g < g1; ++g) {
 #pragma unroll
-      for (int k = 0; k < kBandRegs; ++k) {
+      for (int k = 0; k < REGS; ++k) {
         const uint32_t v = k * kBlock + threadIdx.x;
         if (4 * v < cur.span) *reinterpret_cast<v4f*>(tile + band_slot(p, 4 * v)) = reg[k];
       }
@@ -440,15 +442,18 @@ __global__ __launch_bounds__(kBlock) void pool_band_kernel(const float* x, float
       __syncthreads();  // the tile is rewritten next
     }
   } else {
-    float reg[kBandBatch];
+    float reg[REGS];
     const auto request = [&](const BandSpan& bs, uint32_t t0) {
       if (bs.span == 0) return;
 #pragma unroll
-      for (int k = 0; k < kBandBatch; ++k) reg[k] = load_stream(bs.src + min(t0 + k * kBlock + threadIdx.x, bs.span - 1));
+      for (int k = 0; k < REGS; ++k) {
+        const float* from = bs.src + min(t0 + k * kBlock + threadIdx.x, bs.span - 1);
+        reg[k] = KIND == kBandFloatsKept ? *from : load_stream(from);
+      }
     };
     const auto keep = [&](const BandSpan& bs, uint32_t t0) {
 #pragma unroll
-      for (int k = 0; k < kBandBatch; ++k) {
+      for (int k = 0; k < REGS; ++k) {
         const uint32_t t = t0 + k * kBlock + threadIdx.x;
         if (t < bs.span) tile[band_slot(p, t)] = reg[k];
       }
@@ -457,7 +462,7 @@ __global__ __launch_bounds__(kBlock) void pool_band_kernel(const float* x, float
     request(cur, 0);
     for (uint32_t g = g0; g < g1; ++g) {
       keep(cur, 0);
-      for (uint32_t t0 = kBandBatch * kBlock; t0 < cur.span; t0 += kBandBatch * kBlock) {
+      for (uint32_t t0 = REGS * kBlock; t0 < cur.span; t0 += REGS * kBlock) {
         request(cur, t0);
         keep(cur, t0);
       }
@@ -1442,20 +1447,28 @@ static int run_pooling(bool three_d, const int* in_shape, int pool_type, const i
       a.bands_per_group = per;
       const uint32_t g = (a.total_bands + per - 1) / per;
       const bool pipe = p.in_w % 4 == 0 && aligned16(x);
+      const int shared = a.bands_per_plane > 1 ? std::max(p.kh - p.sh, 0) : 0;  // rows that two bands read
+      const bool kept = 16 * shared >= a.tile_rows &&
+                        static_cast<uint64_t>(in_shape[0]) * in_shape[1] * p.in_h * p.in_w * sizeof(float) >= kBandKeptBytes;
       const int k = p.kh == p.kw && (p.kh == 2 || p.kh == 3 || (p.kh == 5 && a.wide)) ? p.kh : 0;
-      const int vecs = (a.tile_rows * p.in_w / 4 + kBlock - 1) / kBlock;  // per lane and band
-      const int regs = !pipe ? 0 : (vecs <= 2 ? 2 : (vecs <= 3 ? 3 : (vecs <= 4 ? 4 : (vecs <= 6 ? 6 : 8))));
-      if (pl->chosen(SHDW_PATH_POOL_BAND, 100 * regs + k, g)) return SHDW_OK;
-#define SHDW_LAUNCH_BAND(MAXV, KV)                                                              \
+      const int steps = (a.tile_rows * p.in_w / (pipe ? 4 : 1) + kBlock - 1) / kBlock;  // per lane and band
+      const int regs = steps <= 2 ? 2 : (steps <= 3 ? 3 : (steps <= 4 ? 4 : (steps <= 6 ? 6 : 8)));
+      if (pl->chosen(SHDW_PATH_POOL_BAND, (pipe ? 100 * regs : 0) + k, g)) return SHDW_OK;
+#define SHDW_LAUNCH_BAND_REGS(MAXV, KV, KINDV)                                                  \
   do {                                                                                           \
     switch (regs) {                                                                              \
-      case 0: pool_band_kernel<MAXV, KV, 0><<<g, kBlock, lds, st>>>(x, y, a); break;             \
-      case 2: pool_band_kernel<MAXV, KV, 2><<<g, kBlock, lds, st>>>(x, y, a); break;             \
-      case 3: pool_band_kernel<MAXV, KV, 3><<<g, kBlock, lds, st>>>(x, y, a); break;             \
-      case 4: pool_band_kernel<MAXV, KV, 4><<<g, kBlock, lds, st>>>(x, y, a); break;             \
-      case 6: pool_band_kernel<MAXV, KV, 6><<<g, kBlock, lds, st>>>(x, y, a); break;             \
-      default: pool_band_kernel<MAXV, KV, 8><<<g, kBlock, lds, st>>>(x, y, a); break;            \
+      case 2: pool_band_kernel<MAXV, KV, KINDV, 2><<<g, kBlock, lds, st>>>(x, y, a); break;      \
+      case 3: pool_band_kernel<MAXV, KV, KINDV, 3><<<g, kBlock, lds, st>>>(x, y, a); break;      \
+      case 4: pool_band_kernel<MAXV, KV, KINDV, 4><<<g, kBlock, lds, st>>>(x, y, a); break;      \
+      case 6: pool_band_kernel<MAXV, KV, KINDV, 6><<<g, kBlock, lds, st>>>(x, y, a); break;      \
+      default: pool_band_kernel<MAXV, KV, KINDV, 8><<<g, kBlock, lds, st>>>(x, y, a); break;     \
     }                                                                                            \
+  } while (0)
+#define SHDW_LAUNCH_BAND(MAXV, KV)                                                              \
+  do {                                                                                           \
+    if (pipe) SHDW_LAUNCH_BAND_REGS(MAXV, KV, kBandVectors);                                     \
+    else if (kept) SHDW_LAUNCH_BAND_REGS(MAXV, KV, kBandFloatsKept);                             \
+    else SHDW_LAUNCH_BAND_REGS(MAXV, KV, kBandFloats);                                           \
   } while (0)
       if (pool_type == 0) {
         if (k == 3)
@@ -1477,6 +1490,7 @@ static int run_pooling(bool three_d, const int* in_shape, int pool_type, const i
           SHDW_LAUNCH_BAND(false, 0);
       }
 #undef SHDW_LAUNCH_BAND
+#undef SHDW_LAUNCH_BAND_REGS
       return launch_status();
     }
   }

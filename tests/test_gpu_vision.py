@@ -725,6 +725,25 @@ def test_pooling_on_pointers_off_the_vector_boundary(gpu, pool, shape, kernel, s
     assert_bit_exact(got, want.ravel(), "pooling")
 
 
+# rows that are no whole vectors: two, three, four, six and eight floats a lane ahead, spans past that; above and below
+# 24 MB of input, where the loads change; walks of several bands
+@pytest.mark.parametrize("pool", [0, 1])
+@pytest.mark.parametrize("shape,kernel,stride,pad", [
+    ((3, 2, 55, 55), 2, 1, 0), ((2, 3, 35, 35), 2, 1, 0), ((2, 2, 30, 31), 3, 1, 1), ((2, 2, 35, 35), 3, 1, 1),
+    ((3, 2, 55, 55), 3, 2, 0), ((1, 2, 225, 225), 5, 1, 2), ((65, 32, 55, 55), 2, 1, 0), ((70, 30, 55, 55), 3, 2, 0),
+    ((165, 32, 35, 35), 3, 1, 1), ((42, 3, 225, 225), 5, 1, 2)])
+def test_pooling_bands_of_single_floats(gpu, pool, shape, kernel, stride, pad):
+    x = with_specials(normal(64, shape), 64).reshape(shape)
+    want = oracle.pooling_op(x, pool, [kernel], [stride], [pad], full_pooling=False)
+    path, variant, grid = ctypes.c_int(), ctypes.c_int(), ctypes.c_uint()
+    assert gpu.shdw_hip_pooling2d_plan(shadow_amd.ints(list(shape)), pool, kernel, kernel, stride, stride, pad, pad,
+                                       shadow_amd.ints(list(want.shape)), ctypes.byref(path), ctypes.byref(variant),
+                                       ctypes.byref(grid)) == 0
+    assert path.value == 24 and variant.value < 100  # a band of single floats
+    got = gpuops.pooling(x, shape, pool, [kernel] * 2, [stride] * 2, [pad] * 2, want.shape)
+    assert_bit_exact(got, want.ravel(), "band %s" % (shape,))
+
+
 def test_pooling_op_errors(ws):
     ws.set_blob("x", np.zeros((2, 3, 8, 8), F))
     with pytest.raises(ShadowError, match="Check Failed"):
