@@ -101,8 +101,9 @@ int shdw_hip_memcpy_h2d(void* dst, const void* src, size_t bytes, void* stream);
 int shdw_hip_memcpy_d2h(void* dst, const void* src, size_t bytes, void* stream);
 /* The same for a few kilobytes that the host waits for: a kernel stores them in
  * `staging` (shdw_hip_host_malloc, at least `bytes` long), the stream is waited for and
- * they are copied to dst.  bytes and src must be multiples of 4, otherwise, and while the
- * stream is being captured, it is shdw_hip_memcpy_d2h. */
+ * they are copied to dst.  bytes and src must be multiples of 4, src memory of the current
+ * device and both ranges inside their allocations; otherwise, and while the stream is being
+ * captured, it is shdw_hip_memcpy_d2h. */
 int shdw_hip_memcpy_d2h_staged(void* dst, const void* src, size_t bytes, void* staging, void* stream);
 /* ref: shadow/core/allocator.cu:38-45 (copy: D2D; blocking when stream==NULL) */
 int shdw_hip_memcpy_d2d(void* dst, const void* src, size_t bytes, void* stream);

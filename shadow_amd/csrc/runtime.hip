@@ -20,6 +20,23 @@ int copy(void* dst, const void* src, size_t bytes, hipMemcpyKind kind, void* str
   if (stream == nullptr) return rc(hipMemcpy(dst, src, bytes, kind));
   return rc(hipMemcpyAsync(dst, src, bytes, kind, as_stream(stream)));
 }
+// Whether `bytes` from p on lie in one allocation of the given kind that kernels of the current
+// device reach.  The runtime's copies look this up themselves and return an error, or let the host
+// copy; a kernel would fault.
+bool reachable(const void* p, size_t bytes, hipMemoryType kind) {
+  hipPointerAttribute_t attributes;
+  hipDeviceptr_t base = nullptr;
+  size_t size = 0;
+  int device = -1;
+  if (hipPointerGetAttributes(&attributes, p) != hipSuccess || hipGetDevice(&device) != hipSuccess ||
+      hipMemGetAddressRange(&base, &size, const_cast<void*>(p)) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  const size_t offset = static_cast<const char*>(p) - static_cast<const char*>(base);
+  return attributes.type == kind && (kind == hipMemoryTypeHost || attributes.device == device) && offset <= size &&
+         bytes <= size - offset;
+}
 }  // namespace
 
 extern "C" {
@@ -113,7 +130,7 @@ int shdw_hip_memcpy_d2h_staged(void* dst, const void* src, size_t bytes, void* s
   const hipError_t asked = hipStreamIsCapturing(as_stream(stream), &capture);
   if (asked != hipSuccess) (void)hipGetLastError();
   if (asked != hipSuccess || capture != hipStreamCaptureStatusNone || (bytes | reinterpret_cast<uintptr_t>(src)) % 4 != 0 ||
-      bytes / 4 > INT32_MAX)
+      bytes / 4 > INT32_MAX || !reachable(src, bytes, hipMemoryTypeDevice) || !reachable(staging, bytes, hipMemoryTypeHost))
     return copy(dst, src, bytes, hipMemcpyDeviceToHost, stream);
   const int code = shdw_hip_copy(static_cast<int>(bytes / 4), static_cast<const float*>(src), static_cast<float*>(staging), stream);
   if (code != SHDW_OK) return code;

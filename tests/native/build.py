@@ -29,7 +29,14 @@ def build():
     _run([hipcc, "--offload-arch=gfx950", "-O3", "-std=c++17", "-ffp-contract=off",
           "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-Wno-unused-command-line-argument",
           os.path.join(HERE, "launch_shapes.hip"), "-o", shapes])
-    return [out, shapes]
+    root = os.path.dirname(os.path.dirname(HERE))
+    readback = os.path.join(HERE, "readback")
+    _run(["g++", "-std=c++17", "-O1", "-D__HIP_PLATFORM_AMD__", "-I", os.path.join(root, "include"),
+          "-I", os.path.join(root, "shadow_amd", "host"), "-isystem", os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include"),
+          "-x", "c++", os.path.join(HERE, "readback.cpp"), os.path.join(root, "shadow_amd", "csrc", "runtime.hip"),
+          os.path.join(root, "shadow_amd", "host", "src", "device_hip.cpp"),
+          "-Wl,--unresolved-symbols=ignore-all", "-o", readback])
+    return [out, shapes, readback]
 
 
 if __name__ == "__main__":
