@@ -48,7 +48,10 @@ class HipAllocator : public Allocator {
   // With the device chosen: the staging memory belongs to it.
   void set_stream(void* stream) override {
     stream_ = stream;
-    if (staging_ == nullptr && shdw_hip_host_malloc(&staging_, kStagingBytes) != 0) staging_ = nullptr;
+    if (staging_ == nullptr && shdw_hip_host_malloc(&staging_, kStagingBytes) != 0) {
+      staging_ = nullptr;           // reads then go by the runtime's copy
+      (void)shdw_hip_last_error();  // and the next launch is not to report this
+    }
   }
   ~HipAllocator() override {
     if (staging_ != nullptr) shdw_hip_host_free(staging_);

@@ -108,6 +108,7 @@ int main() {
     pinned_result = hipErrorOutOfMemory;
     auto allocator = Shadow::GetAllocator<Shadow::DeviceType::kGPU>();
     allocator->set_stream(nullptr);
+    expect("no pinned memory leaves no error for the next launch", last_error == hipSuccess);
     kernels = copies = 0;
     allocator->read(512, device_memory, dst);
     expect("without pinned memory reads go by the runtime's copy", kernels == 0 && copies == 1);
