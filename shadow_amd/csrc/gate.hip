@@ -11,7 +11,7 @@
 // x + (-0)).  The plane sum is fp32, front to back, by one lane, as Vision::Pooling
 // adds; the mean at the end is fp64, rounded once after the divide.
 //
-// What bounds it: 25 KB of LDS a workgroup leave six on a CU, whose loads, ordered
+// What bounds it: five workgroups on a CU (LDS and registers), whose loads, ordered
 // sums (784 dependent additions: 3 us) and stores overlap each other's, and 30 vector
 // instructions an element.  One block with its tail takes, per call: [32,512,28,28]
 // (103 MB) 27 us, where its five launches took 78; [64,64,56,56] 43; [64,512,14,14]
@@ -23,6 +23,7 @@
 
 #include "../../include/shadow_hip.h"
 #include "device_common.h"
+#include "gate_shape.h"
 #include "launch.h"
 #include "libm_exact.h"
 
@@ -68,8 +69,6 @@ struct GateParams {
 };
 
 enum { kNoResidual = 0, kOtherResidual = 1, kSameResidual = 2 };
-
-constexpr uint32_t kGateMaxRows = 64;  // per workgroup: a lane of one wave each in the ordered sum
 
 // Waves per SIMD that the registers are held to: what a lane's vectors leave room for.
 constexpr int gate_waves(int slots) { return slots == 16 ? 4 : slots == 8 ? 5 : 6; }
@@ -312,46 +311,6 @@ __global__ __launch_bounds__(kBlock, gate_waves(SLOTS)) void squeeze_gate_kernel
   }
 }
 
-// How a shape is cut.
-struct GateShape {
-  uint32_t log2_lanes, pieces, group, chunk, pitch;
-  int slots;
-};
-
-// Six workgroups on a CU.  Rows that do not fit whole go through LDS in chunks (four of the
-// 112x112 planes' rows per CU instead of three, [16,64,112,112] 124 -> 81 us; with 18 KB
-// [32,512,28,28] would be cut too, 26.0 -> 28.1), unless there are no more than two
-// workgroups per CU to hold.
-constexpr uint32_t kGateTileBytes = 26000, kGateMaxTileBytes = 62000, kGateCus = 256;
-
-// Lanes per row: as many as a row has vectors, up to a wave; the whole workgroup where
-// a wave would take more than eight steps over a row, and where there are so few rows
-// that a row per wave would leave CUs idle.  Rows per workgroup: what eight vectors per
-// lane hold, fewer while that leaves under 1024 workgroups (four per CU).
-inline GateShape gate_shape(uint32_t rows, uint32_t len) {
-  const uint32_t nv = (len + 3) / 4;
-  GateShape g{};
-  g.log2_lanes = nv <= 16 ? 4 : nv <= 32 ? 5 : nv <= 512 ? 6 : 8;
-  if (nv > 16 && rows < 1024) g.log2_lanes = 8;
-  const uint32_t lanes = 1u << g.log2_lanes, turn_rows = kBlock >> g.log2_lanes;
-  g.pieces = (nv + lanes - 1) / lanes;
-  uint32_t turns = g.pieces <= 8 ? 8 / g.pieces : 1;
-  if (turns * turn_rows > kGateMaxRows) turns = kGateMaxRows / turn_rows;
-  while (turns > 1 && (rows + turns * turn_rows - 1) / (turns * turn_rows) < 1024u) --turns;
-  const uint32_t used = turns * g.pieces;
-  g.slots = used <= 1 ? 1 : used <= 4 ? 4 : used <= 8 ? 8 : 16;
-  g.group = turns * turn_rows;
-  // LDS holds equal chunks of the rows, as few as fit the tile; the pitch is an odd
-  // number of vectors, so that the summing lanes meet different banks.
-  for (uint32_t chunks = 1;; ++chunks) {
-    g.chunk = (g.pieces + chunks - 1) / chunks;
-    g.pitch = (g.chunk * lanes < nv ? g.chunk * lanes : nv) | 1u;
-    const uint32_t bytes = g.group * g.pitch * static_cast<uint32_t>(sizeof(v4f));
-    if (bytes <= (rows <= 2 * kGateCus * g.group ? kGateMaxTileBytes : kGateTileBytes) || g.chunk == 1) break;
-  }
-  return g;
-}
-
 }  // namespace shdw
 
 using namespace shdw;
@@ -372,6 +331,10 @@ void launch_gate(const GateShape& g, uint32_t rows, uint32_t len, const float* x
 #undef SHDW_LAUNCH
 }
 
+// Four vectors a lane of every row and the rows' odd pitch stay below the tile: never cut.
+static_assert((4 * kBlock + kGateMaxRows) * sizeof(v4f) <= kGateTileBytes, "rows of up to four vectors a lane lie whole in LDS");
+static_assert(kBlock == kGateLanes && sizeof(v4f) == kGateVectorBytes, "gate_shape.h counts in these");
+
 template <int SLOTS, bool VEC>
 void launch_gate(const GateShape& g, uint32_t rows, uint32_t len, const float* x, const float* res, float* y, float* mean,
                  const GateParams& p, hipStream_t st) {
@@ -384,7 +347,7 @@ void launch_gate(const GateShape& g, uint32_t rows, uint32_t len, const float* x
                  const GateParams& p, hipStream_t st) {
   switch (g.slots) {
     case 1: launch_gate<1, VEC, true>(g, rows, len, x, res, y, mean, p, st); break;
-    case 4: launch_gate<4, VEC>(g, rows, len, x, res, y, mean, p, st); break;
+    case 4: launch_gate<4, VEC, true>(g, rows, len, x, res, y, mean, p, st); break;
     case 8: launch_gate<8, VEC>(g, rows, len, x, res, y, mean, p, st); break;
     default: launch_gate<16, VEC>(g, rows, len, x, res, y, mean, p, st);
   }

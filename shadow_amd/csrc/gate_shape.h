@@ -1,0 +1,57 @@
+// How the gated block's kernel (gate.hip) cuts a shape: host code without HIP, so that
+// tests/test_gate_shape_cpu.py can go over shapes without a device.
+#ifndef SHADOW_AMD_CSRC_GATE_SHAPE_H_
+#define SHADOW_AMD_CSRC_GATE_SHAPE_H_
+
+#include <cstdint>
+
+namespace shdw {
+
+constexpr uint32_t kGateMaxRows = 64;  // per workgroup: a lane of one wave each in the ordered sum
+constexpr uint32_t kGateLanes = 256, kGateVectorBytes = 16;
+
+// How a shape is cut.
+struct GateShape {
+  uint32_t log2_lanes, pieces, group, chunk, pitch;
+  int slots;
+};
+
+// Five workgroups on a CU: the tile and 2.5 KB of parameters, table and partial sums each
+// (28.5 KB of 160), as many as the registers of eight vectors a lane leave room for
+// (gate_waves).  Rows that do not fit whole go through LDS in chunks (four of the
+// 112x112 planes' rows per CU instead of three, [16,64,112,112] 124 -> 81 us; with 18 KB
+// eight 28x28 planes would be cut too, [32,512,28,28] 26.0 -> 28.1), unless there are no
+// more than two workgroups per CU to hold.
+constexpr uint32_t kGateTileBytes = 26000, kGateMaxTileBytes = 62000, kGateCus = 256;
+
+// Lanes per row: as many as a row has vectors, up to a wave; the whole workgroup where
+// a wave would take more than eight steps over a row, and where there are so few rows
+// that a row per wave would leave CUs idle.  Rows per workgroup: what eight vectors per
+// lane hold, fewer while that leaves under 1024 workgroups (four per CU).
+inline GateShape gate_shape(uint32_t rows, uint32_t len) {
+  const uint32_t nv = (len + 3) / 4;
+  GateShape g{};
+  g.log2_lanes = nv <= 16 ? 4 : nv <= 32 ? 5 : nv <= 512 ? 6 : 8;
+  if (nv > 16 && rows < 1024) g.log2_lanes = 8;
+  const uint32_t lanes = 1u << g.log2_lanes, turn_rows = kGateLanes >> g.log2_lanes;
+  g.pieces = (nv + lanes - 1) / lanes;
+  uint32_t turns = g.pieces <= 8 ? 8 / g.pieces : 1;
+  if (turns * turn_rows > kGateMaxRows) turns = kGateMaxRows / turn_rows;
+  while (turns > 1 && (rows + turns * turn_rows - 1) / (turns * turn_rows) < 1024u) --turns;
+  const uint32_t used = turns * g.pieces;
+  g.slots = used <= 1 ? 1 : used <= 4 ? 4 : used <= 8 ? 8 : 16;
+  g.group = turns * turn_rows;
+  // LDS holds equal chunks of the rows, as few as fit the tile; the pitch is an odd
+  // number of vectors, so that the summing lanes meet different banks.
+  for (uint32_t chunks = 1;; ++chunks) {
+    g.chunk = (g.pieces + chunks - 1) / chunks;
+    g.pitch = (g.chunk * lanes < nv ? g.chunk * lanes : nv) | 1u;
+    const uint32_t bytes = g.group * g.pitch * kGateVectorBytes;
+    if (bytes <= (rows <= 2 * kGateCus * g.group ? kGateMaxTileBytes : kGateTileBytes) || g.chunk == 1) break;
+  }
+  return g;
+}
+
+}  // namespace shdw
+
+#endif  // SHADOW_AMD_CSRC_GATE_SHAPE_H_

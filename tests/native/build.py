@@ -36,7 +36,9 @@ def build():
           "-x", "c++", os.path.join(HERE, "readback.cpp"), os.path.join(root, "shadow_amd", "csrc", "runtime.hip"),
           os.path.join(root, "shadow_amd", "host", "src", "device_hip.cpp"),
           "-Wl,--unresolved-symbols=ignore-all", "-o", readback])
-    return [out, shapes, readback]
+    gate = os.path.join(HERE, "gate_shape.so")
+    _run(["g++", "-std=c++17", "-O2", "-fPIC", "-shared", os.path.join(HERE, "gate_shape.cpp"), "-o", gate])
+    return [out, shapes, readback, gate]
 
 
 if __name__ == "__main__":

@@ -1,0 +1,27 @@
+// gate_shape (shadow_amd/csrc/gate_shape.h) for tests/test_gate_shape_cpu.py.
+#include "../../shadow_amd/csrc/gate_shape.h"
+
+extern "C" void gate_shape(unsigned rows, unsigned len, unsigned* out) {
+  const shdw::GateShape g = shdw::gate_shape(rows, len);
+  const unsigned all[] = {g.log2_lanes, g.pieces, g.group, g.chunk, g.pitch, static_cast<unsigned>(g.slots)};
+  for (int k = 0; k < 6; ++k) out[k] = all[k];
+}
+
+// The first length in [1, last] whose cut breaks what the kernel relies on, or 0.
+extern "C" unsigned gate_shape_scan(unsigned rows, unsigned last) {
+  for (unsigned len = 1; len <= last; ++len) {
+    const shdw::GateShape g = shdw::gate_shape(rows, len);
+    const unsigned nv = (len + 3) / 4, lanes = 1u << g.log2_lanes, turn_rows = 256u >> g.log2_lanes;
+    const unsigned turns = g.group / turn_rows, kept = g.chunk * lanes < nv ? g.chunk * lanes : nv;
+    const bool ok = (g.slots == 1 || g.slots == 4 || g.slots == 8 || g.slots == 16) &&
+                    turns >= 1 && g.group == turns * turn_rows && g.group <= shdw::kGateMaxRows &&
+                    turns * g.pieces <= static_cast<unsigned>(g.slots) &&             // every vector has a slot
+                    g.pieces * lanes >= nv && g.chunk >= 1 && g.chunk <= g.pieces &&  // every column a piece
+                    g.pitch >= kept && g.pitch % 2 == 1 &&
+                    g.group * g.pitch * 16u + 2560u <= 65536u &&                      // LDS of a workgroup
+                    (g.slots >= 8 || g.chunk == g.pieces) &&                          // the forms that are launched
+                    (g.log2_lanes <= 6 || g.group <= shdw::kGateMaxRows / 8);         // partial sums of a row's waves
+    if (!ok) return len;
+  }
+  return 0;
+}

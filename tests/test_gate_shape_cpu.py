@@ -1,0 +1,40 @@
+"""How the gated block's kernel cuts a shape (shadow_amd/csrc/gate_shape.h): what every cut has to
+keep to, and which form the shapes of the GPU tests get."""
+import ctypes
+import os
+
+import pytest
+
+from tests.native import build
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+
+@pytest.fixture(scope="module")
+def native():
+    path = os.path.join(HERE, "native", "gate_shape.so")
+    if not os.path.exists(path):
+        build.build()
+    return ctypes.CDLL(path)
+
+
+@pytest.mark.parametrize("rows", [1, 2, 255, 512, 513, 1023, 1024, 1025, 2047, 2048, 4096, 4097, 8192, 16384, 65536, 1 << 20])
+def test_every_cut_fits_the_kernel(native, rows):
+    assert native.gate_shape_scan(rows, 15360) == 0
+
+
+def cut(native, rows, length):
+    out = (ctypes.c_uint * 6)()
+    native.gate_shape(rows, length, out)
+    lanes, pieces, group, chunk, _, slots = out
+    return {"lanes": 1 << lanes, "turns": group * (1 << lanes) // 256, "slots": slots, "chunked": chunk != pieces,
+            "cut_group": rows % group != 0}
+
+
+def test_forms_of_the_gpu_shapes(native):
+    """The shapes of test_gpu_gate.py reach the forms they are there for."""
+    from tests.test_gpu_gate import FORMS
+    for (n, c, h, w), form in FORMS.items():
+        got = cut(native, n * c, h * w)
+        assert {k: got[k] for k in form} == form, (n, c, h, w, got)
+    assert {f["slots"] for f in FORMS.values()} == {1, 4, 8, 16}

@@ -428,8 +428,8 @@ GATE = "bn(BatchNorm) + sc(Scale) + act(Activate) + squeeze(Pooling) + gate(Acti
 GATE_TAIL = " + sc2(Scale) + add(Eltwise) + relu(Activate)"
 
 
-# rows that are whole vectors and not, a quarter of a wave to a workgroup per row, several rows and
-# one per workgroup, the last workgroup cut, one vector and sixteen per lane, the longest row and past it
+# the model's side of it: rows that are whole vectors and not, a quarter of a wave to a workgroup per row, the longest row
+# and past it.  The kernel's forms: test_gpu_gate.py.
 @pytest.mark.parametrize("shape", [SHAPE, (2, 8, 4, 8), (5, 3, 1, 1), (1, 16, 14, 14), (1040, 2, 5, 6), (1031, 1, 8, 8),
                                    (530, 2, 9, 9), (515, 2, 28, 28), (1030, 1, 27, 29), (513, 2, 45, 45),
                                    (2, 3, 60, 61), (1100, 1, 60, 60), (1, 2, 100, 101), (1, 2, 120, 128), (1, 2, 124, 124)])
@@ -438,6 +438,14 @@ def test_squeeze_gate(gpu, shape):
     feed["r"] = normal(77, shape)
     run_all(gate_net(shape, ["e", "pool"]), weights, feed, ["e", "pool"], fp64=("pool",),
             expect_fused=[GATE + GATE_TAIL + " + gap(Reduce) -> e, pool"])
+
+
+def test_squeeze_gate_of_volumes(gpu):
+    """Five axes: the average is Pooling's over all three spatial ones."""
+    shape = (2, 3, 4, 5, 6)
+    weights, feed = bn_data(shape)
+    feed = {"x": normal(82, shape, 2.0), "r": normal(83, shape)}
+    run_all(gate_net(shape, ["e"], residual="r", mean=False), weights, feed, ["e"], expect_fused=[GATE + GATE_TAIL + " -> e"])
 
 
 @pytest.mark.parametrize("shape", [SHAPE, (2, 8, 4, 8)])

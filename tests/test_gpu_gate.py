@@ -1,0 +1,147 @@
+"""shdw_hip_squeeze_gate through the C ABI, every form its kernel has: rows whole in LDS and in
+chunks, one and several rows a lane, last groups cut short, one to sixteen vectors a lane,
+each with rows of whole vectors and not, and with x, another tensor or nothing as the
+residual.  Bit for bit against the operators of the oracle; the plane means, 64-bit sums
+in another order, to 1e-5.  tests/test_gate_shape_cpu.py checks that the shapes reach the
+forms named here."""
+import numpy as np
+import pytest
+
+import oracle
+import shadow_amd
+from shadow_amd import Buffer
+from tests.helpers import assert_bit_exact, assert_rel_close, normal, uniform, with_specials
+
+pytestmark = pytest.mark.gpu
+F = np.float32
+
+FORMS = {
+    (516, 1, 84, 84): {"lanes": 256, "turns": 1, "slots": 8, "chunked": True},
+    (516, 1, 81, 81): {"lanes": 256, "turns": 1, "slots": 8, "chunked": True},
+    (2060, 1, 44, 44): {"lanes": 64, "turns": 1, "slots": 8, "chunked": True},
+    (2060, 1, 45, 45): {"lanes": 64, "turns": 1, "slots": 8, "chunked": True},
+    (2061, 1, 60, 60): {"lanes": 256, "turns": 2, "slots": 8, "chunked": True, "cut_group": True},
+    (2061, 1, 59, 61): {"lanes": 256, "turns": 2, "slots": 8, "chunked": True, "cut_group": True},
+    (600, 1, 112, 112): {"lanes": 256, "turns": 1, "slots": 16, "chunked": True},
+    (600, 1, 111, 113): {"lanes": 256, "turns": 1, "slots": 16, "chunked": True},
+    (3, 2, 112, 112): {"lanes": 256, "turns": 1, "slots": 16, "chunked": False},
+    (3, 2, 111, 113): {"lanes": 256, "turns": 1, "slots": 16, "chunked": False},
+    (8201, 1, 28, 28): {"lanes": 64, "turns": 2, "slots": 8, "chunked": False, "cut_group": True},
+    (8201, 1, 27, 29): {"lanes": 64, "turns": 2, "slots": 8, "chunked": False, "cut_group": True},
+    (4101, 1, 31, 33): {"lanes": 64, "turns": 1, "slots": 4, "chunked": False, "cut_group": True},
+    (32801, 1, 7, 8): {"lanes": 16, "turns": 2, "slots": 4, "chunked": False, "cut_group": True},
+    (32801, 1, 5, 6): {"lanes": 16, "turns": 2, "slots": 4, "chunked": False, "cut_group": True},
+    (21867, 3, 2, 2): {"lanes": 16, "turns": 4, "slots": 4, "chunked": False, "cut_group": True},
+    (1366, 3, 9, 9): {"lanes": 32, "turns": 1, "slots": 1, "chunked": False, "cut_group": True},
+    (5, 3, 9, 9): {"lanes": 256, "turns": 1, "slots": 1, "chunked": False},
+    (4099, 1, 1, 3): {"lanes": 16, "turns": 1, "slots": 1, "chunked": False, "cut_group": True},
+    (4099, 1, 1, 1): {"lanes": 16, "turns": 1, "slots": 1, "chunked": False, "cut_group": True},
+}
+
+
+class Case:
+    """Inputs of one shape; parts that are left out are None."""
+
+    def __init__(self, shape, residual="other", stats=True, scale=True, bias=True, relu=True, tail_scale=True, tail_bias=True,
+                 special=False):
+        c = shape[1]
+        self.shape, self.relu = shape, relu
+        self.x = normal(70, shape, 2.0)
+        if special:
+            self.x = with_specials(self.x, 3).reshape(shape)
+        self.stats = (normal(71, c, 0.3), uniform(72, c, 0.2, 3.0)) if stats else (None, None)
+        self.scale = uniform(73, c, 0.5, 1.5) if scale else None
+        self.bias = normal(74, c, 0.3) if bias else None
+        tail = residual is not None
+        self.tail = (uniform(75, c, 0.5, 1.5) if tail and tail_scale else None, normal(76, c, 0.3) if tail and tail_bias else None)
+        self.residual = {"x": self.x, "other": normal(77, shape), "first": normal(77, shape), None: None}[residual]
+        self.first = residual == "first"
+
+    def want(self):
+        shape, c = self.shape, self.shape[1]
+        inner = int(np.prod(shape[2:]))
+        with np.errstate(all="ignore"):
+            f = self.x
+            if self.stats[0] is not None:
+                f = oracle.batch_norm(f.ravel(), *self.stats, c, inner, F(0.5), F(1e-3)).reshape(shape)
+            if self.scale is not None or self.bias is not None:
+                f = oracle.scale_bias(f.ravel(), self.scale, self.bias, c, inner).reshape(shape)
+            if self.relu:
+                f = oracle.activate_op(f, 1)
+            y = oracle.binary_op(f, oracle.activate_op(oracle.pooling_op(f, 1, global_pooling=True), 3), operation=2)
+            if self.residual is None:
+                return y, None
+            t = oracle.scale_bias(y.ravel(), *self.tail, c, inner).reshape(shape)
+            y = oracle.activate_op(oracle.eltwise_op([self.residual, t] if self.first else [t, self.residual], 1), 1)
+            return y, oracle.reduce_op(y, 4, list(range(2, len(shape))))
+
+    def run(self, lib, alias=None, off=(0, 0, 0), mean=True):
+        """alias: 'x' or 'residual', which y then is; off: floats that x, the residual and y are off the vector boundary."""
+        def buffer(a, at=0):
+            if a is None:
+                return None
+            b = Buffer(4 * (a.size + 4))
+            b.upload(np.ascontiguousarray(a, F).ravel(), 4 * at)
+            kept.append(b)
+            return b.ptr + 4 * at
+
+        kept, n, c = [], self.x.size, self.shape[1]
+        x = buffer(self.x, off[0])
+        res = x if self.residual is self.x else buffer(self.residual, off[1])
+        y_buf = Buffer(4 * (n + 4))
+        y = {"x": x, "residual": res, None: y_buf.ptr + 4 * off[2]}[alias]
+        m_buf = Buffer(4 * (n // int(np.prod(self.shape[2:])))) if self.residual is not None and mean else None
+        shadow_amd.check(lib.shdw_hip_squeeze_gate(
+            n, c, int(np.prod(self.shape[2:])), x, buffer(self.stats[0]), buffer(self.stats[1]), 0.5, 1e-3, buffer(self.scale),
+            buffer(self.bias), int(self.relu), buffer(self.tail[0]), buffer(self.tail[1]), res, int(self.first), y,
+            m_buf.ptr if m_buf else None, None))
+        shadow_amd.check(lib.shdw_hip_stream_sync(None))
+        if alias is None:
+            got = y_buf.download(count=n, offset_bytes=4 * off[2])
+        else:
+            where = kept[0] if alias == "x" or self.residual is self.x else kept[1]
+            got = where.download(count=n, offset_bytes=4 * (off[0] if where is kept[0] else off[1]))
+        return got, None if m_buf is None else m_buf.download(count=m_buf.nbytes // 4)
+
+    def check(self, lib, what, **how):
+        (got, mean), (want, want_mean) = self.run(lib, **how), self.want()
+        assert_bit_exact(got, want.ravel(), what)
+        if mean is not None:
+            assert assert_rel_close(mean, want_mean.ravel(), 1e-5, what + " mean") == 0
+
+
+@pytest.mark.parametrize("residual", ["x", "other", "first", None])
+@pytest.mark.parametrize("shape", sorted(FORMS))
+def test_every_form(gpu, shape, residual):
+    Case(shape, residual).check(gpu, "%s %s" % (shape, residual))
+
+
+# whole and chunked, whole vectors and not
+ALIASED = [(8201, 1, 28, 28), (8201, 1, 27, 29), (2060, 1, 44, 44), (2060, 1, 45, 45), (600, 1, 111, 113), (5, 3, 9, 9), (4099, 1, 1, 3)]
+
+
+@pytest.mark.parametrize("alias,residual", [("x", "x"), ("x", "other"), ("residual", "other"), ("residual", "first"), ("x", None)])
+@pytest.mark.parametrize("shape", ALIASED)
+def test_result_in_place_of_an_operand(gpu, shape, alias, residual):
+    Case(shape, residual).check(gpu, "%s y is %s, residual %s" % (shape, alias, residual), alias=alias)
+
+
+@pytest.mark.parametrize("off", [(1, 0, 0), (0, 2, 0), (0, 0, 3), (1, 1, 1)])
+@pytest.mark.parametrize("shape", [(8201, 1, 28, 28), (2060, 1, 44, 44), (21867, 3, 2, 2)])
+def test_pointers_off_the_vector_boundary(gpu, shape, off):
+    Case(shape, "other").check(gpu, "%s off %s" % (shape, off), off=off)
+
+
+@pytest.mark.parametrize("shape", [(6, 5, 7, 9), (2, 3, 8, 12), (2, 3, 4, 5, 6)])
+@pytest.mark.parametrize("parts", [
+    dict(stats=False, scale=False, bias=False, relu=False), dict(stats=False, scale=False, bias=False),  # ReLU alone
+    dict(scale=False, bias=False), dict(scale=False, bias=False, relu=False),                            # BatchNorm alone
+    dict(stats=False, bias=False), dict(stats=False, scale=False), dict(scale=False), dict(bias=False, relu=False)])
+@pytest.mark.parametrize("tail", [dict(residual=None), dict(tail_bias=False), dict(tail_scale=False, residual="first")])
+def test_parts_left_out(gpu, shape, parts, tail):
+    """Fronts and tails of any parts, special values among the elements, volumes as well as planes."""
+    Case(shape, special=True, **parts, **{"residual": "other", **tail}).check(gpu, "%s %s %s" % (shape, parts, tail))
+
+
+def test_no_mean_asked_for(gpu):
+    Case((2060, 1, 45, 45), "x").check(gpu, "no mean", mean=False)
