@@ -29,7 +29,7 @@ constexpr int kStream = 64;
 #define SHDW_DEVICE __device__ __forceinline__
 
 // Streaming accesses: whose cache lines one wave asks for, once.  Both directions
-// carry the non-temporal hint, every such access through these functions.
+// carry the non-temporal hint; loads get it through these functions alone.
 // Stores: a plain store leaves dirty lines in L2 that are written back when the
 // kernel ends (broadcast of 67 MB of output 11.4 us with the hint, 13.0 to 19.2
 // without; 103 MB copy 19.3 against 31.9).
@@ -40,10 +40,13 @@ constexpr int kStream = 64;
 // 80.8; behind the kernel that wrote the operand the same (ReLU 16.9 and 17.8, sum 24.5 and
 // 26.2).  Plain loads pay only where several operators read one tensor of up to 256 MB one
 // after another (ReLU of 51 MB 15.6 against 16.6), which a kernel cannot know.
-// Lines that several waves share are for load4 and load4_any below: operands that are
-// read again, and rows that start anywhere in a line where short pieces of them go to
-// different waves (channel shuffle of 49-element rows, 103 MB: 20.9 us plain, 23.2 with the
-// hint; the transposes in movers.hip; 3x3 pooling bands of 27-wide rows 23.4 and 25.7).
+// load4 and load4_any below are for lines that are asked for more than once: operands that
+// the kernel, or the call's next one, reads again (normalisation of 513 and more values in
+// two walks, 103 MB: rows of 512 28.8 us plain, 32.9 with the hint, [16,4096,196] 73.7 and
+// 86.7; SSDNormalize per item of [8,256,56,56] 18.6 and 20.3), and rows that start anywhere
+// in a line where short pieces of them go to different waves (channel shuffle of 49-element
+// rows, 103 MB: 20.9 us plain, 23.2 with the hint; the transposes in movers.hip; 3x3 pooling
+// bands of 225-wide rows 122 and 133).
 template <class T>
 SHDW_DEVICE T load_stream(const T* p) {
   return __builtin_nontemporal_load(p);

@@ -599,7 +599,7 @@ __global__ __launch_bounds__(kBlock) void ssd_row_partials_kernel(const float* x
     for (; t + (kAhead - 1) * kBlock < stop; t += kAhead * kBlock) {
       v4f q[kAhead];
 #pragma unroll
-      for (int u = 0; u < kAhead; ++u) q[u] = load4_stream(xr + 4ull * (t + u * kBlock));
+      for (int u = 0; u < kAhead; ++u) q[u] = load4(xr + 4ull * (t + u * kBlock));  // read again by the scaling
 #pragma unroll
       for (int u = 0; u < kAhead; ++u) {
 #pragma unroll
@@ -610,7 +610,7 @@ __global__ __launch_bounds__(kBlock) void ssd_row_partials_kernel(const float* x
       }
     }
     for (; t < stop; t += kBlock) {
-      const v4f q = load4_stream(xr + 4ull * t);
+      const v4f q = load4(xr + 4ull * t);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const float sq = q[j] * q[j];

@@ -1466,7 +1466,7 @@ struct RowStream {
       if (n == 0) continue;
       const float* src = x + static_cast<uint64_t>(row0 + row_of(lane, i)) * len + c0 + col_of(lane, i);
       if (n == 4) {
-        reg[i] = load4_stream_any(src);
+        reg[i] = load4_any(src);  // both walks ask for it
       } else {
 #pragma unroll
         for (int k = 0; k < 3; ++k)
@@ -1666,7 +1666,7 @@ struct TallTile {
       if (has(k, i)) {
         const float* src = x + base + static_cast<uint64_t>(row(k, i)) * inner;
         if (valid == 4) {
-          v[i] = load4_stream_any(src);
+          v[i] = load4_any(src);  // every walk asks for it
         } else {
 #pragma unroll
           for (int e = 0; e < 3; ++e)
@@ -1867,7 +1867,7 @@ struct LongSlab {
     for (int i = 0; i < kLongLoads; ++i) {
       const uint32_t e = first(i);
       if (e + 4 <= cells) {
-        v[i] = load4_stream_any(src + e);
+        v[i] = load4_any(src + e);  // every walk asks for it
       } else {
 #pragma unroll
         for (int j = 0; j < 3; ++j)
