@@ -32,8 +32,10 @@ HIPCC = os.environ.get("HIPCC", shutil.which("hipcc") or "/opt/rocm/bin/hipcc")
 # 14 dwords; a struct by value ends the list) are put into SGPRs as a wave starts instead of
 # being fetched by its first instruction, so a streaming wave's first load goes out about
 # 0.2 us earlier.  Kernels therefore take pointers and counts first, functors and structs
-# last.  [16,32,128,256] broadcasts 65.6 -> 64.1 us for five, five reductions of
-# [32,512,28,28] 48.3 -> 47.1, a decoder stage 59.5 -> 57.6, three poolings 58.0 -> 57.1.
+# last.  [16,32,128,256] broadcasts 67.4 -> 65.9 us for five, five reductions of
+# [32,512,28,28] 50.6 -> 49.7, a decoder stage 63.2 -> 62.0, three poolings 52.8 -> 52.0,
+# three softmaxes 46.0 -> 45.2; not all kernels gain: softmax of [12845,1000,1] 50.1 -> 51.6,
+# the 56x56 averages of [16,256,56,56] 21.5 -> 22.0.
 HIP_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=off",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",

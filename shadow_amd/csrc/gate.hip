@@ -14,8 +14,8 @@
 // What bounds it: five workgroups on a CU (LDS and registers), whose loads, ordered
 // sums (784 dependent additions: 3 us) and stores overlap each other's, and 30 vector
 // instructions an element.  One block with its tail takes, per call: [32,512,28,28]
-// (103 MB) 27 us, where its five launches took 78; [64,64,56,56] 43; [64,512,14,14]
-// 11.9; [64,1024,7,7] 8.5; [16,64,112,112] 80 (its sums are 12 544 long).  With loads in
+// (103 MB) 27 us, where its five launches took 78; [64,64,56,56] 44; [64,512,14,14]
+// 12.1; [64,1024,7,7] 8.8; [16,64,112,112] 80 (its sums are 12 544 long).  With loads in
 // branches of their own, a division per element, LDS reads next to the additions that
 // use them and rows whole in LDS whatever their length: 29, 43, 13.9, 11.3 and 112; with the residual
 // another tensor than x 35 -> 27.5, 49 -> 44, 15.1 -> 12.0, 12.3 -> 8.2, 116 -> 80.
