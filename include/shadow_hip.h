@@ -312,7 +312,7 @@ int shdw_hip_batch_norm_scale_residual_relu(int n, int channel, int inner_num, c
  * leaves its step out.  Every step is rounded as in the operators; the average of f
  * is the fp32 sum in order of Pooling, the mean the fp64 sum of Reduce.  y may alias
  * x or the residual.  inner_num > SHDW_SQUEEZE_GATE_MAX_INNER returns
- * SHDW_E_UNSUPPORTED (a workgroup holds a plane in its registers, sixteen vectors a lane).
+ * SHDW_E_UNSUPPORTED (a workgroup holds a plane in its registers, up to fifteen vectors a lane).
  * ref: shadow/operators/kernels/{batch_norm,scale,activate,pooling,binary,reduce}.cpp,
  *      eltwise.hpp:37-44 */
 #define SHDW_SQUEEZE_GATE_MAX_INNER 15360
