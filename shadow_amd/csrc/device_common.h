@@ -131,6 +131,55 @@ SHDW_DEVICE void fd_divmod(uint32_t n, const FastDiv& f, uint32_t& q, uint32_t& 
 }
 
 // ---------------------------------------------------------------------------
+// Division by a divisor that many dividends share.  t / d, correctly rounded, is the
+// fp64 product t * r rounded to fp32, with r within 2^-52 of 1 / d: the product is then
+// within 2^-51 of the quotient, and a quotient of two fp32 numbers that is a normal fp32
+// number lies on no midpoint between two of them and no nearer to one than 2^-49 of its
+// size (|A 2^k - M B| >= 1 for a dividend A, a divisor B of 24 bits and a midpoint M of 25).
+// Subnormal quotients can lie on a midpoint: a wave that holds one divides.  Zeros in
+// the dividends need no division; a wave looks twice before it divides for them.
+// Four instructions an element where a division takes eleven, one of them at half rate.
+// ---------------------------------------------------------------------------
+// 1 / d in fp64: the hardware's estimate (2^-22 or better) and two Newton steps; as the
+// estimate where those are undefined (0, infinite, NaN), so that t * r is t / d there too.
+SHDW_DEVICE double reciprocal(float d) {
+  const double dd = static_cast<double>(d), r0 = __builtin_amdgcn_rcp(dd);
+  double r = __builtin_fma(__builtin_fma(-dd, r0, 1.0), r0, r0);
+  r = __builtin_fma(__builtin_fma(-dd, r, 1.0), r, r);
+  return r == r ? r : r0;
+}
+
+// t[j] / d[j] for N dividends of a lane, r[j] = reciprocal(d[j]); every lane of the wave
+// that runs this must hold some dividend.
+template <int N, class D, class R>
+SHDW_DEVICE void quotients(float (&t)[N], D&& d, R&& r) {
+  constexpr float kLeast = 0x1p-126f;
+  float q[N];
+#pragma unroll
+  for (int j = 0; j < N; ++j) q[j] = static_cast<float>(static_cast<double>(t[j]) * r(j));
+  float lo = __builtin_fabsf(q[0]);
+#pragma unroll
+  for (int j = 1; j < N; ++j) lo = __builtin_fminf(lo, __builtin_fabsf(q[j]));
+  if (__builtin_amdgcn_ballot_w64(!(lo >= kLeast)) != 0) {
+    bool whole = true;
+#pragma unroll
+    for (int j = 0; j < N; ++j) whole = whole && (t[j] == 0.f || __builtin_fabsf(q[j]) >= kLeast);
+    if (__builtin_amdgcn_ballot_w64(!whole) != 0) {
+      asm volatile("");  // keeps the compiler from evaluating both sides
+#pragma unroll
+      for (int j = 0; j < N; ++j) q[j] = t[j] / d(j);
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < N; ++j) t[j] = q[j];
+}
+SHDW_DEVICE v4f quotients4(v4f t, float d, double r) {
+  float q[4] = {t[0], t[1], t[2], t[3]};
+  quotients(q, [d](int) { return d; }, [r](int) { return r; });
+  return v4f{q[0], q[1], q[2], q[3]};
+}
+
+// ---------------------------------------------------------------------------
 // wave64 exchange.  Steps 1..8 stay inside a row of 16 lanes and use DPP
 // (no LDS traffic); 16 and 32 cross rows and go through ds_bpermute.
 // ---------------------------------------------------------------------------

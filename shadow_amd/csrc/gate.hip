@@ -12,9 +12,11 @@
 // adds; the mean at the end is fp64, rounded once after the divide.
 //
 // What bounds it: five workgroups on a CU (LDS and registers), whose loads, ordered
-// sums (784 dependent additions: 3 us) and stores overlap each other's, and 30 vector
-// instructions an element.  One block with its tail takes, per call: [32,512,28,28]
-// (103 MB) 27 us, where its five launches took 78; [64,64,56,56] 44; [64,512,14,14]
+// sums (784 dependent additions: 3 us; without them [32,512,28,28] takes 22.9 us instead of
+// 27) and stores overlap each other's, and 20 vector instructions an element.  One block
+// with its tail takes, per call: [32,512,28,28]
+// (103 MB) 26.5 us (28.7 with the quotients in fp32 and the row's parameters read for every
+// vector), where its five launches took 78; [64,64,56,56] 44; [64,512,14,14]
 // 12.1; [64,1024,7,7] 8.8; [16,64,112,112] 80 (its sums are 12 544 long).  With loads in
 // branches of their own, a division per element, LDS reads next to the additions that
 // use them and rows whole in LDS whatever their length: 29, 43, 13.9, 11.3 and 112; with the residual
@@ -33,38 +35,15 @@ namespace shdw {
 
 // Per-row parameters, as the rows' lanes leave them in LDS.
 struct alignas(16) GateRow {
-  float m, d, rd, s, b, tail_s, tail_b, gate;  // rd = 1 / d, or 0 where d is out of range for quotients4
+  float m, d;
+  double r;  // 1 / d
+  float s, b, tail_s, tail_b, gate;
 };
-
-// t / d, correctly rounded, by the reciprocal rd of d rounded to nearest: an estimate
-// and two corrections from the exact remainder (Markstein, "Computation of elementary
-// functions on the IBM RISC System/6000 processor", 1990; the second is needed because
-// the estimate may be two last places off).  Nothing may overflow or lose bits on the
-// way: |d| in [2^-30, 2^30], |t| in [2^-60, 2^60] (NaN passes); a wave with any other
-// element divides.  5 instructions an element instead of the 11 of a division.
-SHDW_DEVICE v4f quotients4(v4f t, float d, float rd) {
-  const float a0 = __builtin_fabsf(t[0]), a1 = __builtin_fabsf(t[1]), a2 = __builtin_fabsf(t[2]), a3 = __builtin_fabsf(t[3]);
-  const float lo = __builtin_fminf(__builtin_fminf(a0, a1), __builtin_fminf(a2, a3));
-  const float hi = __builtin_fmaxf(__builtin_fmaxf(a0, a1), __builtin_fmaxf(a2, a3));
-  if (__builtin_amdgcn_ballot_w64(!(lo >= 0x1p-60f && hi <= 0x1p60f && rd != 0.f)) == 0) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      float q = t[j] * rd;
-      q = __builtin_fmaf(__builtin_fmaf(-d, q, t[j]), rd, q);
-      t[j] = __builtin_fmaf(__builtin_fmaf(-d, q, t[j]), rd, q);
-    }
-  } else {
-    asm volatile("");  // keeps the compiler from evaluating both sides
-#pragma unroll
-    for (int j = 0; j < 4; ++j) t[j] = t[j] / d;
-  }
-  return t;
-}
 
 struct GateParams {
   const float *stat_mean, *stat_variance, *scale, *bias, *tail_scale, *tail_bias;
   float scale_factor, eps, plane;
-  int relu, residual_first;
+  int relu;
   FastDiv channel;
 };
 
@@ -121,17 +100,17 @@ SHDW_DEVICE float add_in_order(float sum, const v4f* row, uint32_t cols) {
 
 // L = 2^log2_lanes lanes share a row, so a workgroup takes 256 / L rows per turn and
 // `pieces` steps of 4 L columns per row; slot i of a lane's SLOTS vectors is a piece of
-// a turn, the same for all lanes.  Every vector is requested before anything else
-// happens, and without a branch (a branch around a load has the compiler copy the
-// registers of the loads before it, and wait for them): lanes with nothing to load take
-// the row's or the group's last vector again.  WHOLE: the front's result stays in LDS;
-// otherwise LDS holds `chunk` pieces of the rows at a time and the front is taken again
-// on the way out.
-template <int SLOTS, bool VEC, bool WHOLE, int RESIDUAL>
+// a turn, the same for all lanes, and slots from `used` on hold nothing.  Every vector is
+// requested before anything else happens, and without a branch (a branch around a load has
+// the compiler copy the registers of the loads before it, and wait for them): lanes with
+// nothing to load take the row's or the group's last vector again.  WHOLE: the front's
+// result stays in LDS; otherwise LDS holds `chunk` pieces of the rows at a time and the
+// front is taken again on the way out.  ONE: one turn, a lane's vectors are of one row.
+template <int SLOTS, bool VEC, bool WHOLE, bool ONE, int RESIDUAL>
 __global__ __launch_bounds__(kBlock, gate_waves(SLOTS)) void squeeze_gate_kernel(const float* x, const float* res, float* y, float* mean,
                                                               uint32_t rows, uint32_t len, uint32_t group,
                                                               uint32_t log2_lanes, uint32_t pieces, uint32_t chunk,
-                                                              uint32_t pitch, GateParams p) {
+                                                              uint32_t pitch, uint32_t used, GateParams p) {
   extern __shared__ v4f tile[];  // a chunk of the group's rows, pitch vectors apart
   __shared__ uint64_t tab[32];
   __shared__ GateRow row_params[kGateMaxRows];
@@ -143,13 +122,15 @@ __global__ __launch_bounds__(kBlock, gate_waves(SLOTS)) void squeeze_gate_kernel
   const uint32_t last = len < 4 ? 0 : len - 4;  // of a row's columns that a vector can start at
 
   const auto step = [&](uint32_t& k, uint32_t& turn_row) {
-    if (++k == pieces) k = 0, turn_row += turn_rows;
+    if (++k == pieces && !ONE) k = 0, turn_row += turn_rows;
   };
+  // addresses: one for the group, the same for all lanes, and a lane's 32-bit offset
   const auto vector = [&](const float* src, uint32_t k, uint32_t turn_row) {
-    const float* at = src + static_cast<uint64_t>(row0) * len + min(lead + turn_row, nrows - 1) * len +
-                      min(4 * (sub + k * lanes), last);
-    if (VEC) return load4_stream(at);
-    if (len >= 4) return load4_stream_any(at);
+    const float* from = src + static_cast<uint64_t>(row0) * len;
+    const uint32_t offset = min(lead + turn_row, nrows - 1) * len + min(4 * (sub + k * lanes), last);
+    if (VEC) return load4_stream(from + offset);
+    if (len >= 4) return load4_stream_any(from + offset);
+    const float* at = from + offset;
     return v4f{at[0], at[len > 1 ? 1 : 0], at[len > 2 ? 2 : 0], 0.f};
   };
   const auto request = [&](const float* src, v4f* to) {
@@ -178,11 +159,11 @@ __global__ __launch_bounds__(kBlock, gate_waves(SLOTS)) void squeeze_gate_kernel
   v4f reg[SLOTS], other[kTurn];
   request(x, reg);
   if (threadIdx.x < nrows) {
-    GateRow g{0.f, 1.f, 1.f, 1.f, -0.f, 1.f, -0.f, 0.f};
+    GateRow g{0.f, 1.f, 1.0, 1.f, -0.f, 1.f, -0.f, 0.f};
     if (p.stat_mean) {
       g.m = stat_mean * p.scale_factor;
       g.d = __builtin_sqrtf(__builtin_fabsf(stat_variance * p.scale_factor) + p.eps);
-      g.rd = g.d >= 0x1p-30f && g.d <= 0x1p30f ? 1.f / g.d : 0.f;
+      g.r = reciprocal(g.d);
     }
     if (p.scale) g.s = scale;
     if (p.bias) g.b = bias;
@@ -193,17 +174,21 @@ __global__ __launch_bounds__(kBlock, gate_waves(SLOTS)) void squeeze_gate_kernel
   if (threadIdx.x < 32) tab[threadIdx.x] = entry;
   __syncthreads();
 
+  // max(t, 0) stands for t > 0 ? t : 0: both make 0 of NaN and of -0, and t, a sum, is no signalling NaN
   const auto front = [&](v4f t, const GateRow& g) {
     if (p.stat_mean) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) t[j] = t[j] - g.m;
-      t = quotients4(t, g.d, g.rd);
+      t = quotients4(t, g.d, g.r);
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       t[j] = t[j] * g.s;
       t[j] = t[j] + g.b;
-      if (p.relu) t[j] = t[j] > 0 ? t[j] : 0;
+    }
+    if (p.relu) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) t[j] = __builtin_fmaxf(t[j], 0.f);
     }
     return t;
   };
@@ -213,6 +198,7 @@ __global__ __launch_bounds__(kBlock, gate_waves(SLOTS)) void squeeze_gate_kernel
   // do not meet on one SIMD.
   const uint32_t walked = threadIdx.x & (kWave - 1);
   const bool walks = threadIdx.x / kWave == ((blockIdx.x / kXcds) & 3u) && walked < nrows;
+  GateRow g = row_params[min(lead, nrows - 1)];
   float sum = 0.f;
   for (uint32_t k0 = 0; k0 < pieces; k0 += chunk) {
     if (!WHOLE && k0) __syncthreads();
@@ -221,9 +207,10 @@ __global__ __launch_bounds__(kBlock, gate_waves(SLOTS)) void squeeze_gate_kernel
 #pragma unroll
     for (int i = 0; i < SLOTS; ++i) {
       const uint32_t r = lead + turn_row, v = sub + k * lanes;
-      if (WHOLE || k - k0 < chunk) {
+      if (!ONE && k == 0) g = row_params[min(r, nrows - 1)];
+      if (i < used && (WHOLE || k - k0 < chunk)) {
         arrange(reg[i], 4 * v);
-        const v4f t = front(reg[i], row_params[min(r, nrows - 1)]);
+        const v4f t = front(reg[i], g);
         if (r < nrows && 4 * v < len) tile[r * pitch + v - k0 * lanes] = t;
       }
       step(k, turn_row);
@@ -234,7 +221,9 @@ __global__ __launch_bounds__(kBlock, gate_waves(SLOTS)) void squeeze_gate_kernel
     if (walks) {
       const v4f* mine = tile + walked * pitch;
       const uint32_t cols = WHOLE ? len : min(len - 4 * k0 * lanes, 4 * chunk * lanes);
+      __builtin_amdgcn_s_setprio(3);  // nothing else of the workgroup moves meanwhile: 26.9 -> 26.4 us on [32,512,28,28]
       sum = add_in_order(sum, mine, cols);
+      __builtin_amdgcn_s_setprio(0);
     }
     if (WHOLE) break;
   }
@@ -242,13 +231,14 @@ __global__ __launch_bounds__(kBlock, gate_waves(SLOTS)) void squeeze_gate_kernel
   __syncthreads();
 
   asm("" : "+v"(sub), "+v"(lead));  // the slots' offsets are taken again instead of kept
+  if (ONE) g = row_params[min(lead, nrows - 1)];
   double total = 0.0;
   uint32_t k = 0, turn_row = 0;
 #pragma unroll
   for (int i = 0; i < SLOTS; ++i) {
+    if (i >= used) continue;
     const uint32_t r = lead + turn_row, v = sub + k * lanes, c = 4 * v;
-    const bool here = r < nrows && c < len;
-    const GateRow g = row_params[min(r, nrows - 1)];
+    if (!ONE && k == 0) g = row_params[min(r, nrows - 1)];
     v4f t = WHOLE ? tile[min(r, nrows - 1) * pitch + min(v, pitch - 1)] : front(reg[i], g);
     if (RESIDUAL == kOtherResidual && !WHOLE && i % kTurn == 0) {
       uint32_t k_ahead = k, turn_ahead = turn_row;
@@ -260,44 +250,53 @@ __global__ __launch_bounds__(kBlock, gate_waves(SLOTS)) void squeeze_gate_kernel
     }
     v4f q = RESIDUAL == kOtherResidual && !WHOLE ? other[i % kTurn] : reg[i];
     if (RESIDUAL == kOtherResidual) arrange(q, c);
+    // Eltwise SUM with unit coefficients is Set(0), then y += 1 * input, input by input: behind
+    // the ReLU neither the 0 in front nor which input comes first can be told from t + q.
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       t[j] = t[j] * g.gate;
       if (RESIDUAL != kNoResidual) {
         t[j] = t[j] * g.tail_s;
         t[j] = t[j] + g.tail_b;
-        // Eltwise SUM with unit coefficients: Set(0), then y += 1 * input, input by input
-        float u = 0.0f + (p.residual_first ? q[j] : t[j]);
-        u = u + (p.residual_first ? t[j] : q[j]);
-        t[j] = u > 0 ? u : 0;
-        if (mean) total += static_cast<double>(here && (VEC || c + j < len) ? t[j] : 0.f);
+        t[j] = __builtin_fmaxf(t[j] + q[j], 0.f);
       }
     }
-    if (here) {
-      float* at = y + static_cast<uint64_t>(row0) * len + (r * len + c);
+    if (r < nrows && c < len) {
+      float* to = y + static_cast<uint64_t>(row0) * len;
+      const uint32_t offset = r * len + c;
       if (VEC) {
-        store4_stream(at, t);
+        store4_stream(to + offset, t);
       } else if (c + 4 <= len) {
-        store4_stream_any(at, t);
+        store4_stream_any(to + offset, t);
       } else {
 #pragma unroll
         for (int j = 0; j < 3; ++j)
-          if (c + j < len) at[j] = t[j];
+          if (c + j < len) to[offset + j] = t[j];
       }
     }
-    if (RESIDUAL != kNoResidual && mean && k + 1 == pieces) {  // the row is complete: every lane of the wave is here
-      total += dpp_f64<kDppXor1>(total);
-      total += dpp_f64<kDppXor2>(total);
-      total += dpp_f64<kDppHalfMirror>(total);
-      total += dpp_f64<kDppMirror>(total);
-      if (log2_lanes > 4) total += __shfl_xor(total, 16, kWave);
-      if (log2_lanes > 5) total += __shfl_xor(total, 32, kWave);
-      if (log2_lanes > 6) {
-        if ((threadIdx.x & (kWave - 1)) == 0 && r < nrows) part[r][threadIdx.x / kWave] = total;
-      } else if (sub == 0 && r < nrows) {
-        mean[row0 + r] = static_cast<float>(total / static_cast<double>(static_cast<int>(len)));
+    if (RESIDUAL != kNoResidual && mean) {
+      const auto add = [&](int j) { total += static_cast<double>(t[j]); };
+      if (k + 1 < pieces || VEC) {
+        if (k + 1 < pieces || c < len) add(0), add(1), add(2), add(3);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (c + j < len) add(j);
       }
-      total = 0.0;
+      if (k + 1 == pieces) {  // the row is complete: every lane of the wave is here
+        total += dpp_f64<kDppXor1>(total);
+        total += dpp_f64<kDppXor2>(total);
+        total += dpp_f64<kDppHalfMirror>(total);
+        total += dpp_f64<kDppMirror>(total);
+        if (log2_lanes > 4) total += __shfl_xor(total, 16, kWave);
+        if (log2_lanes > 5) total += __shfl_xor(total, 32, kWave);
+        if (log2_lanes > 6) {
+          if ((threadIdx.x & (kWave - 1)) == 0 && r < nrows) part[r][threadIdx.x / kWave] = total;
+        } else if (sub == 0 && r < nrows) {
+          mean[row0 + r] = static_cast<float>(total / static_cast<double>(static_cast<int>(len)));
+        }
+        total = 0.0;
+      }
     }
     step(k, turn_row);
   }
@@ -317,14 +316,16 @@ using namespace shdw;
 
 namespace {
 
-template <int SLOTS, bool VEC, bool WHOLE>
+uint32_t used_slots(const GateShape& g) { return (g.group << g.log2_lanes) / kBlock * g.pieces; }
+
+template <int SLOTS, bool VEC, bool WHOLE, bool ONE>
 void launch_gate(const GateShape& g, uint32_t rows, uint32_t len, const float* x, const float* res, float* y, float* mean,
                  const GateParams& p, hipStream_t st) {
   const uint32_t grid = (rows + g.group - 1) / g.group;
   const size_t lds = static_cast<size_t>(g.group) * g.pitch * sizeof(v4f);
 #define SHDW_LAUNCH(R)                                                                                           \
-  squeeze_gate_kernel<SLOTS, VEC, WHOLE, R><<<grid, kBlock, lds, st>>>(x, res, y, mean, rows, len, g.group,      \
-                                                                       g.log2_lanes, g.pieces, g.chunk, g.pitch, p)
+  squeeze_gate_kernel<SLOTS, VEC, WHOLE, ONE, R><<<grid, kBlock, lds, st>>>(x, res, y, mean, rows, len, g.group, \
+                                                                            g.log2_lanes, g.pieces, g.chunk, g.pitch, used_slots(g), p)
   if (!res) SHDW_LAUNCH(kNoResidual);
   else if (res == x) SHDW_LAUNCH(kSameResidual);
   else SHDW_LAUNCH(kOtherResidual);
@@ -335,21 +336,28 @@ void launch_gate(const GateShape& g, uint32_t rows, uint32_t len, const float* x
 static_assert((4 * kBlock + kGateMaxRows) * sizeof(v4f) <= kGateTileBytes, "rows of up to four vectors a lane lie whole in LDS");
 static_assert(kBlock == kGateLanes && sizeof(v4f) == kGateVectorBytes, "gate_shape.h counts in these");
 
-template <int SLOTS, bool VEC>
+template <int SLOTS, bool VEC, bool ONE>
 void launch_gate(const GateShape& g, uint32_t rows, uint32_t len, const float* x, const float* res, float* y, float* mean,
                  const GateParams& p, hipStream_t st) {
-  if (g.chunk == g.pieces) launch_gate<SLOTS, VEC, true>(g, rows, len, x, res, y, mean, p, st);
-  else launch_gate<SLOTS, VEC, false>(g, rows, len, x, res, y, mean, p, st);
+  if (g.chunk == g.pieces) launch_gate<SLOTS, VEC, true, ONE>(g, rows, len, x, res, y, mean, p, st);
+  else launch_gate<SLOTS, VEC, false, ONE>(g, rows, len, x, res, y, mean, p, st);
 }
 
 template <bool VEC>
 void launch_gate(const GateShape& g, uint32_t rows, uint32_t len, const float* x, const float* res, float* y, float* mean,
                  const GateParams& p, hipStream_t st) {
+  const bool one = used_slots(g) == g.pieces;  // one and sixteen slots are of one turn in any case
   switch (g.slots) {
-    case 1: launch_gate<1, VEC, true>(g, rows, len, x, res, y, mean, p, st); break;
-    case 4: launch_gate<4, VEC, true>(g, rows, len, x, res, y, mean, p, st); break;
-    case 8: launch_gate<8, VEC>(g, rows, len, x, res, y, mean, p, st); break;
-    default: launch_gate<16, VEC>(g, rows, len, x, res, y, mean, p, st);
+    case 1: launch_gate<1, VEC, true, true>(g, rows, len, x, res, y, mean, p, st); break;
+    case 4:
+      if (one) launch_gate<4, VEC, true, true>(g, rows, len, x, res, y, mean, p, st);
+      else launch_gate<4, VEC, true, false>(g, rows, len, x, res, y, mean, p, st);
+      break;
+    case 8:
+      if (one) launch_gate<8, VEC, true>(g, rows, len, x, res, y, mean, p, st);
+      else launch_gate<8, VEC, false>(g, rows, len, x, res, y, mean, p, st);
+      break;
+    default: launch_gate<16, VEC, true>(g, rows, len, x, res, y, mean, p, st);
   }
 }
 
@@ -366,7 +374,7 @@ extern "C" int shdw_hip_squeeze_gate(int n, int channel, int inner_num, const fl
   if (n == 0) return SHDW_OK;
   const uint32_t rows = static_cast<uint32_t>(n / inner_num), len = static_cast<uint32_t>(inner_num);
   const GateParams p{stat_mean, stat_variance, scale, bias, tail_scale, tail_bias, scale_factor, eps,
-                     static_cast<float>(inner_num), relu, residual_first, make_fastdiv(static_cast<uint32_t>(channel))};
+                     static_cast<float>(inner_num), relu, make_fastdiv(static_cast<uint32_t>(channel))};
   const bool vec = len % 4 == 0 && aligned16(x) && aligned16(y) && (!residual || aligned16(residual));
   const GateShape g = gate_shape(rows, len);
   hipStream_t st = static_cast<hipStream_t>(stream);
