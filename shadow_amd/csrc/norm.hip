@@ -15,9 +15,10 @@
 // boundary.  Rows of up to 32768 elements stay in registers between the three
 // passes (one HBM read, one write); longer rows are re-read, from L2.
 //
-// The kernels are close to VALU-bound (two fp64 accumulations and an IEEE
-// division per element), so the affine step avoids per-element index
-// arithmetic: LayerNorm's parameters are loaded as vectors by row position,
+// The kernels are close to VALU-bound (two fp64 accumulations and a quotient per
+// element; with a division of fp32 in place of the shared reciprocal [16,256,56,56] as
+// 512 / 4096 rows takes 20.2 / 20.6 us instead of 15.0 / 19.4), so the affine step avoids
+// per-element index arithmetic: LayerNorm's parameters are loaded as vectors by row position,
 // GroupNorm's channel is computed once per 128-bit vector.
 #include <hip/hip_runtime.h>
 
@@ -106,32 +107,20 @@ SHDW_DEVICE float norm_affine1(const NormArgs& p, uint32_t i, float v) {
   return affine1(v, p.scale[c], p.bias[c]);
 }
 
-SHDW_DEVICE double wave_sum(double v) {
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off);
-  return v;
-}
-
 // Sum over the LANES lanes that own a row, result in each of them.  LANES <= 64:
 // the lanes are neighbours inside one wave; more: whole waves, through `slots`.
 template <int LANES>
 SHDW_DEVICE double row_sum(double v, double* slots) {
-  if (LANES <= 16) {
-    // inside a row of 16 lanes the exchanges are DPP moves (no LDS traffic); after
-    // each step the lanes that have met hold the same sum, so the mirrors of the
-    // last two steps pair every lane with one from the other half
-    if (LANES >= 2) v += dpp_f64<kDppXor1>(v);
-    if (LANES >= 4) v += dpp_f64<kDppXor2>(v);
-    if (LANES >= 8) v += dpp_f64<kDppHalfMirror>(v);
-    if (LANES >= 16) v += dpp_f64<kDppMirror>(v);
-    return v;
-  }
-  if (LANES <= kWave) {
-#pragma unroll
-    for (int off = LANES / 2; off >= 1; off >>= 1) v += __shfl_xor(v, off);
-    return v;
-  }
-  v = wave_sum(v);
+  // inside a row of 16 lanes the exchanges are DPP moves (no LDS traffic); after
+  // each step the lanes that have met hold the same sum, so the mirrors of the
+  // last two steps pair every lane with one from the other half
+  if (LANES >= 2) v += dpp_f64<kDppXor1>(v);
+  if (LANES >= 4) v += dpp_f64<kDppXor2>(v);
+  if (LANES >= 8) v += dpp_f64<kDppHalfMirror>(v);
+  if (LANES >= 16) v += dpp_f64<kDppMirror>(v);
+  if (LANES >= 32) v += __shfl_xor(v, 16);
+  if (LANES >= 64) v += __shfl_xor(v, 32);
+  if (LANES <= kWave) return v;
   __syncthreads();  // slots may still be read from the previous sum
   if ((threadIdx.x & 63) == 0) slots[threadIdx.x >> 6] = v;
   __syncthreads();
@@ -142,7 +131,7 @@ SHDW_DEVICE double row_sum(double v, double* slots) {
 }
 
 // The row (<= REGS * 4 * LANES elements) is held in REGS vectors per lane.
-// LANES = 16, 32 or 64: 16, 8 or 4 rows per 256-lane workgroup, no barriers (a
+// LANES = 4 to 64: 64 to 4 rows per 256-lane workgroup, no barriers (a
 // wave-per-row layout leaves 3/4 of the lanes idle on rows of 64 floats: 85 us
 // per 58 MB, and rows of 49 went through the one-workgroup-per-row kernel at
 // 307 us).  LANES = 256 or 1024: one row per workgroup of that size.
@@ -173,9 +162,11 @@ __global__ __launch_bounds__(LANES <= kWave ? kBlock : LANES, LANES == kBigBlock
 #pragma unroll
   for (int k = 0; k < REGS; ++k) {
     const uint32_t first = 4 * (k * LANES + lane), c = count(k);
-    if (c == 4) {
-      reg[k] = TAIL ? load4_stream_any(xr + first) : load4_stream(xr + first);
-    } else if (TAIL && c > 0) {
+    if (!TAIL) {  // lanes past the row's end take its last vector again
+      reg[k] = load4_stream(xr + min(first, p.inner - 4));
+    } else if (c == 4) {
+      reg[k] = load4_stream_any(xr + first);
+    } else if (c > 0) {
       reg[k] = v4f{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int j = 0; j < 3; ++j)
@@ -186,12 +177,11 @@ __global__ __launch_bounds__(LANES <= kWave ? kBlock : LANES, LANES == kBigBlock
 #pragma unroll
   for (int k = 0; k < REGS; ++k) {
     const uint32_t c = count(k);
+    if (c == 0) continue;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      if (j < c) {
-        const float t = p.alpha * reg[k][j];
-        acc += static_cast<double>(t);
-      }
+      const float t = p.alpha * reg[k][j];
+      acc += static_cast<double>(!TAIL || j < c ? t : 0.f);
     }
   }
   const float mean = static_cast<float>(row_sum<LANES>(acc, slots));
@@ -199,20 +189,20 @@ __global__ __launch_bounds__(LANES <= kWave ? kBlock : LANES, LANES == kBigBlock
 #pragma unroll
   for (int k = 0; k < REGS; ++k) {
     const uint32_t c = count(k);
+    if (c == 0) continue;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      if (j < c) {
-        const float val = reg[k][j] - mean;
-        reg[k][j] = val;
-        const float sq = val * val;
-        const float t = p.alpha * sq;
-        acc += static_cast<double>(t);
-      }
+      const float val = reg[k][j] - mean;
+      reg[k][j] = val;
+      const float sq = val * val;
+      const float t = p.alpha * sq;
+      acc += static_cast<double>(!TAIL || j < c ? t : 0.f);
     }
   }
   const float variance = static_cast<float>(row_sum<LANES>(acc, slots));
   const float ve = variance + p.eps;
   const float denom = __builtin_sqrtf(ve);
+  const double recip = reciprocal(denom);
   // One lookup per row where the row shares its scale and bias; only in the
   // forms of up to 64 lanes per row (the host asks for it only there): the
   // 1024-lane form has no register to spare for it.
@@ -224,9 +214,7 @@ __global__ __launch_bounds__(LANES <= kWave ? kBlock : LANES, LANES == kBigBlock
   for (int k = 0; k < REGS; ++k) {
     const uint32_t first = 4 * (k * LANES + lane), c = count(k);
     if (c == 0) continue;
-    v4f r;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) r[j] = reg[k][j] / denom;
+    v4f r = quotients4(reg[k], denom, recip);
     if (row_affine) r = norm_row_affine4(ra, r);
     if (!TAIL) {
       if (!row_affine) r = norm_affine4(p, static_cast<uint32_t>(base) + first, first, r);
@@ -351,12 +339,11 @@ __global__ __launch_bounds__(kBlock) void norm_rows_lds_kernel(const float* x, f
   const float variance = static_cast<float>(row_sum<L>(acc, nullptr));
   const float ve = variance + p.eps;
   const float denom = __builtin_sqrtf(ve);
+  const double recip = reciprocal(denom);
   if (r < nrows) {
     const uint32_t first = static_cast<uint32_t>(base) + r * inner;  // global index of the row
     const RowAffine ra = norm_row_affine(p, first);
-    auto finish = [&](uint32_t pos, float v) -> float {
-      const float val = v - mean;
-      float q = val / denom;
+    auto finish = [&](uint32_t pos, float q) -> float {
       if (p.affine == kAffineRow) q = affine1(q, ra.s, ra.b);
       else if (p.affine == kAffineRowPos) q = affine1(q, sc[c_begin + pos], bi[c_begin + pos]);
       else if (p.affine != kAffineNone) q = norm_affine1(p, first + c_begin + pos, q);
@@ -365,13 +352,14 @@ __global__ __launch_bounds__(kBlock) void norm_rows_lds_kernel(const float* x, f
     for (c = 0; c + 4 <= n; c += 4) {
       float v[4];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) v[k] = mine[c + k];
+      for (int k = 0; k < 4; ++k) v[k] = mine[c + k] - mean;
+      quotients(v, [&](int) { return denom; }, [&](int) { return recip; });
 #pragma unroll
       for (int k = 0; k < 4; ++k) v[k] = finish(c + k, v[k]);
 #pragma unroll
       for (int k = 0; k < 4; ++k) mine[c + k] = v[k];
     }
-    for (; c < n; ++c) mine[c] = finish(c, mine[c]);
+    for (; c < n; ++c) mine[c] = finish(c, (mine[c] - mean) / denom);
   }
   __syncthreads();
 
@@ -425,16 +413,15 @@ __global__ __launch_bounds__(kBlock) void norm_rows_stream_kernel(const float* x
   const float variance = static_cast<float>(row_sum<kBlock>(acc, slots));
   const float ve = variance + p.eps;
   const float denom = __builtin_sqrtf(ve);
+  const double recip = reciprocal(denom);
   const RowAffine ra = norm_row_affine(p, static_cast<uint32_t>(base));
   for (uint32_t t = threadIdx.x; t < steps; t += kBlock) {
     if (VEC) {
       const v4f q = load4(xr + 4ull * t);
       v4f r;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float val = q[j] - mean;
-        r[j] = val / denom;
-      }
+      for (int j = 0; j < 4; ++j) r[j] = q[j] - mean;
+      r = quotients4(r, denom, recip);
       r = p.affine == kAffineRow ? norm_row_affine4(ra, r)
                                  : norm_affine4(p, static_cast<uint32_t>(base) + 4 * t, 4 * t, r);
       store4_stream(yr + 4ull * t, r);
@@ -513,6 +500,7 @@ __global__ __launch_bounds__(kBlock) void norm_rows_split_kernel(const float* x,
   const float variance = static_cast<float>(fold_partials(row_squares, splits, slots));
   const float ve = variance + p.eps;
   const float denom = __builtin_sqrtf(ve);
+  const double recip = reciprocal(denom);
   float* yr = y + base;
   const RowAffine ra = norm_row_affine(p, static_cast<uint32_t>(base));
   if (VEC) {
@@ -520,10 +508,8 @@ __global__ __launch_bounds__(kBlock) void norm_rows_split_kernel(const float* x,
       const v4f q = load4(xr + 4ull * t);
       v4f r;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float val = q[j] - mean;
-        r[j] = val / denom;
-      }
+      for (int j = 0; j < 4; ++j) r[j] = q[j] - mean;
+      r = quotients4(r, denom, recip);
       r = p.affine == kAffineRow ? norm_row_affine4(ra, r)
                                  : norm_affine4(p, static_cast<uint32_t>(base) + 4 * t, 4 * t, r);
       store4_stream(yr + 4ull * t, r);
@@ -794,6 +780,20 @@ int shdw_hip_group_norm_ws(int outer_num, int inner_num, float eps, const float*
   }
   // workgroups of 256 lanes holding 256 / lanes rows each
   auto groups = [rows](uint32_t lanes) { return (rows + kBlock / lanes - 1) / (kBlock / lanes); };
+  // Short rows of whole vectors from registers, eight lanes a row (every lane of a row of 16
+  // does the once-a-row work again): 12.8 M elements in rows of 64 / 128 / 256 take 19.1 / 19.4 /
+  // 17.9 us, through LDS 23.5 / 24.0 / 24.1.  Not where a lane's vectors are in pieces of
+  // lines, which the stores then send one by one (rows of 196: 41 us against 20), nor where
+  // rows are shorter than three vectors (rows of 4 and 8: 43 and 24 against 23 and 20).
+  const bool whole_lines = p.inner % 32 == 0 || (p.inner % 16 == 0 && p.inner <= 64) || (p.inner >= 12 && p.inner <= 32);
+  if (vec && nvec <= 64 && rows >= 1024 && whole_lines) {
+    if (nvec <= 4) norm_rows_reg_kernel<1, 4, false><<<groups(4), kBlock, 0, st>>>(x, y, p);
+    else if (nvec <= 8) norm_rows_reg_kernel<1, 8, false><<<groups(8), kBlock, 0, st>>>(x, y, p);
+    else if (nvec <= 16) norm_rows_reg_kernel<2, 8, false><<<groups(8), kBlock, 0, st>>>(x, y, p);
+    else if (nvec <= 32) norm_rows_reg_kernel<4, 8, false><<<groups(8), kBlock, 0, st>>>(x, y, p);
+    else norm_rows_reg_kernel<8, 8, false><<<groups(8), kBlock, 0, st>>>(x, y, p);
+    return launch_status();
+  }
   if (p.inner <= kNormLdsMaxInner && rows >= 1024) {
     // short rows through LDS, L lanes per row (any row length, any dword address)
     if (!scale)
@@ -856,6 +856,11 @@ int shdw_hip_group_norm_ws(int outer_num, int inner_num, float eps, const float*
     norm_rows_reg_kernel<4, kWave, false><<<groups(kWave), kBlock, 0, st>>>(x, y, p);
   } else if (nvec <= 8 * kWave && rows >= 2048) {
     norm_rows_reg_kernel<8, kWave, false><<<groups(kWave), kBlock, 0, st>>>(x, y, p);
+  } else if (nvec > 3 * kBlock && nvec <= 15 * kWave && rows >= 2048) {
+    // A wave a row where 256 lanes would leave a part of their last step idle, no barrier: rows of
+    // 3136 and 3600 (12.8 M elements) 17.5 and 18.1 us, with 256 lanes 19.4 and 21.1; of 4096 and
+    // 2500, which fill the 256 lanes or need three steps, 20.4 and 23.7 against 19.5 and 20.4.
+    norm_rows_reg_kernel<16, kWave, false><<<groups(kWave), kBlock, 0, st>>>(x, y, p);
   } else if (nvec <= 2 * kBlock) {
     norm_rows_reg_kernel<2, kBlock, false><<<rows, kBlock, 0, st>>>(x, y, p);
   } else if (nvec <= 4 * kBlock) {
