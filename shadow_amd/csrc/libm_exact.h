@@ -90,18 +90,19 @@ SHDW_LIBM_FN float expf_main(float x, const uint64_t* tab) {
   const double InvLn2N = 0x1.71547652b82fep+5;  // 32 / ln 2
   const double Shift = 0x1.8p+52;
   const double xd = static_cast<double>(x);
-  const double z = InvLn2N * xd;
-  double kd = z + Shift;
+  // The library rounds InvLn2N * xd before it adds Shift and sums the polynomial as
+  // (c0 r + c1) r^2 + (c2 r + 1); the fused addition and Horner's form are two operations
+  // shorter and round to the same float for every x of the range above.
+  double kd = __builtin_fma(InvLn2N, xd, Shift);
   const uint64_t ki = d2u(kd);
   kd -= Shift;
   const double r = __builtin_fma(InvLn2N, xd, -kd);
   const double s = u2d(tab[ki & 31] + (ki << 47));
   const double c0 = 0x1.c6af84b912394p-20, c1 = 0x1.ebfce50fac4f3p-13,
                c2 = 0x1.62e42ff0c52d6p-6;
-  const double p = __builtin_fma(c0, r, c1);
-  const double r2 = r * r;
-  double y = __builtin_fma(c2, r, 1.0);
-  y = __builtin_fma(p, r2, y);
+  double y = __builtin_fma(c0, r, c1);
+  y = __builtin_fma(y, r, c2);
+  y = __builtin_fma(y, r, 1.0);
   y = y * s;
   return static_cast<float>(y);
 }
@@ -113,6 +114,12 @@ SHDW_LIBM_FN float exact_expf(float x, const uint64_t* tab) {
   res = (x > 0x1.62e42ep6f) ? __builtin_inff() : res;  // overflow (and +inf)
   res = (x < -0x1.9fe368p6f) ? 0.0f : res;             // underflow to zero (and -inf)
   return res;
+}
+
+// The same for x that is never above zero (or NaN): Softmax's x - max.
+SHDW_LIBM_FN float exact_expf_nonpositive(float x, const uint64_t* tab) {
+  const float res = expf_main(x, tab);
+  return (x < -0x1.9fe368p6f) ? 0.0f : res;
 }
 
 SHDW_LIBM_FN float exact_expm1f(float x) {

@@ -32,6 +32,16 @@ constexpr int kSlabMaxFloats = 15 * 1024;  // slab + per-column statistics, 60 K
 // std::max(a, b) of libstdc++: b only when a < b.
 SHDW_DEVICE float std_max(float a, float b) { return a < b ? b : a; }
 
+// The largest of m, a and b for Softmax, whose maximum may be taken in any order (see
+// softmax_slab_kernel): one instruction for two elements, where compare-and-select is two for
+// each, and no canonicalisation of the operands in front of it (a NaN among them may go either
+// way, as may the sign of a zero).
+SHDW_DEVICE float max3_any_order(float m, float a, float b) {
+  float r;
+  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(m), "v"(a), "v"(b));
+  return r;
+}
+
 // ---------------------------------------------------------------------------
 // Softmax (shadow/operators/kernels/softmax.cpp:10-42)
 // ---------------------------------------------------------------------------
@@ -845,13 +855,10 @@ __global__ __launch_bounds__(kBlock) void normalize_packed_kernel(const float* x
 
 // Columns of 65 to 1024 elements over a wide inner extent: a workgroup owns a
 // tile of TS = 64, 32 or 16 neighbouring positions with all their `dim` elements,
-// 64 KB at most, so x is read from HBM once.  Each lane keeps its share of the
-// tile (16 vectors of 4 positions at most) in registers and also parks it in
-// LDS; wave 0 folds the TS columns from LDS in index order, one column per lane,
-// and hands the TS results over in the first tile row (nobody else reads the
-// tile, and the fold is done with it); after the barrier every lane finishes
-// its registers.  Only one SIMD pays for the serial fold, the other waves of
-// the CU keep their SIMDs free for the other resident workgroups.
+// 64 KB at most, in its lanes' registers (16 vectors of 4 positions each at most),
+// so x is read from HBM once.  Normalize's fp64 sums are added up where they are
+// (normalize_tile_kernel); Softmax's fp32 running sums have to be walked in index
+// order, out of LDS, by one wave, one column per lane (softmax_tile_kernel).
 //
 // Rows of the tile start wherever inner and the tile offset put them, so the
 // 128-bit global accesses are only 4-byte aligned (the hardware splits the ones
@@ -881,13 +888,18 @@ struct TileLane {
     c0 = threadIdx.x / LANES_PER_ROW;
     valid = j < width ? min(4u, width - j) : 0u;
   }
+  // Two steps of rows at a time (u and u + 1, u even), left out where no lane has a row in them: a
+  // test of uniform values, so no lane mask is set up.  Lanes whose row is past the end take the
+  // last one again.
+  SHDW_DEVICE bool step(int u) const { return (u & ~1) * STEP < dim; }
+  SHDW_DEVICE bool has(int u) const { return c0 + u * STEP < dim; }
+  SHDW_DEVICE uint32_t row(int u) const { return min(c0 + u * STEP, dim - 1); }
   SHDW_DEVICE void load(const float* xs, v4f (&r)[kTilePerLane]) const {
     if (valid == 0) return;
 #pragma unroll
     for (int u = 0; u < kTilePerLane; ++u) {
-      const uint32_t c = c0 + u * STEP;
-      if (c >= dim) continue;
-      const float* src = xs + static_cast<uint64_t>(c) * inner + j;
+      if (!step(u)) continue;
+      const float* src = xs + static_cast<uint64_t>(row(u)) * inner + j;
       if (!TAIL || valid == 4) {
         r[u] = load4_stream_any(src);
       } else {
@@ -897,19 +909,6 @@ struct TileLane {
           if (k < valid) r[u][k] = src[k];
       }
     }
-  }
-  // f(v): what the folding lanes are to find in the tile for the vector v
-  template <typename F>
-  SHDW_DEVICE void park(float* lds, const v4f (&r)[kTilePerLane], F f) const {
-    if (valid == 0) return;
-#pragma unroll
-    for (int u = 0; u < kTilePerLane; ++u) {
-      const uint32_t c = c0 + u * STEP;
-      if (c < dim) *reinterpret_cast<v4f*>(lds + (c << TS_SHIFT) + j) = f(r[u]);
-    }
-  }
-  SHDW_DEVICE void park(float* lds, const v4f (&r)[kTilePerLane]) const {
-    park(lds, r, [](const v4f& v) { return v; });
   }
   SHDW_DEVICE void store(float* ys, uint32_t u, v4f v) const {
     const uint32_t c = c0 + u * STEP;
@@ -928,6 +927,22 @@ struct TileLane {
       for (int k = 0; k < 3; ++k)
         if (k < valid) dst[k] = v[k];
     }
+  }
+};
+
+// The quotients of a lane's vectors by the four statistics of its positions.
+struct TileQuotients {
+  v4f d;
+  double r[4];
+  SHDW_DEVICE TileQuotients(const float* divisors, const double* reciprocals) {
+    d = *reinterpret_cast<const v4f*>(divisors);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) r[k] = reciprocals[k];
+  }
+  SHDW_DEVICE v4f operator()(const v4f& v) const {
+    float q[4] = {v[0], v[1], v[2], v[3]};
+    quotients(q, [this](int k) { return d[k]; }, [this](int k) { return r[k]; });
+    return v4f{q[0], q[1], q[2], q[3]};
   }
 };
 
@@ -955,46 +970,126 @@ SHDW_DEVICE T fold_tile_column(const float* column, uint32_t dim, T acc, F f) {
   return acc;
 }
 
-// p other than 1 and 2 is not taken here: powf per element inside the serial
-// fold would dominate.
+// Whether a sum of non-negative terms in fp64 that were added in another order than the
+// reference's gives the reference's value all the same: both orders' sums are within
+// (terms - 1 + 25) 2^-53 of the true one (a lane adds up to 16, and 9 more additions join
+// the lanes), so what norm_finish makes of either lies within `slack` of what it makes of the
+// other before it rounds to fp32; where the two ends of that interval round to the same
+// number the order cannot show.  About one column in 2^18 of 512 random terms has to be
+// added again in order.  NaN is never settled, nor is a sum with a negative eps.
+template <int PMODE>
+SHDW_DEVICE bool norm_settled(double acc, float eps, uint32_t terms) {
+  if (PMODE == 3 && !(eps >= 0.f)) return false;
+  const double slack = static_cast<double>(terms + 64) * 0x1p-53;
+  const double v = PMODE == 3 ? __builtin_sqrt(acc + static_cast<double>(eps)) : acc;
+  return static_cast<float>(v * (1.0 - slack)) == static_cast<float>(v * (1.0 + slack));
+}
+
+// Sum over the lanes of a wave that are `LANES` apart (4, 8 or 16).
+template <int LANES>
+SHDW_DEVICE double strided_lane_sum(double v) {
+  if (LANES <= 4) v += dpp_f64<kDppRor4>(v);
+  if (LANES <= 8) v += dpp_f64<kDppRor8>(v);
+  v += __shfl_xor(v, 16);
+  v += __shfl_xor(v, 32);
+  return v;
+}
+
+// Memory-bound: every lane adds up the terms of its own rows in registers and the partial sums
+// meet over the lanes and the four waves, so the tile itself needs no LDS and a CU holds four
+// workgroups of a [.,512,.] column tile (128 VGPRs).  With the columns walked in order out of
+// 64 KB of LDS (two workgroups a CU, one wave of four at work for 512 dependent additions) and
+// divisions [16,512,38,38], 94.6 MB, took 32.3 us; now 20.6.  p other than 1 and 2 is not taken here: powf per
+// element in order would dominate.
 template <int PMODE, int SM, int TS_SHIFT, int ROWS>
 __global__ __launch_bounds__(kBlock) void normalize_tile_kernel(const float* x, float* y, uint32_t dim,
-                                                                 uint32_t inner, FastDiv f_tiles, float p,
-                                                                 float eps, const float* scale) {
-  extern __shared__ __align__(16) float lds[];
+                                                                 uint32_t inner, const float* scale, float p,
+                                                                 float eps, FastDiv f_tiles) {
+  using Lane = TileLane<TS_SHIFT, ROWS>;
   constexpr uint32_t TS = 1u << TS_SHIFT;
+  constexpr int kWaves = kBlock / kWave;
+  __shared__ __align__(16) double partial[kWaves][TS];
+  __shared__ __align__(16) double recip[TS];
+  __shared__ __align__(16) float handed[TS];
+  __shared__ __align__(16) float chunk[Lane::STEP * TS];
+  __shared__ uint32_t unsettled;
   uint32_t n, tile;
   fd_divmod(xcd_contiguous(blockIdx.x, gridDim.x), f_tiles, n, tile);
   const uint32_t p0 = tile << TS_SHIFT;
   const uint32_t width = min(TS, inner - p0);
   const uint64_t base = static_cast<uint64_t>(n) * dim * inner + p0;
-  const TileLane<TS_SHIFT, ROWS> lane(width, dim, inner);
+  const Lane lane(width, dim, inner);
+  auto term = [p](float v) { return static_cast<float>(norm_term<PMODE>(v, p)); };  // an fp32 value, widened exactly
   v4f r[kTilePerLane];
   lane.load(x + base, r);
-  // the tile holds the terms of the sums, fp32 values that widen exactly: the folding wave's chain sets the
-  // pace of a tall, narrow tile, and every instruction taken off it is time off the tile
-  lane.park(lds, r, [p](const v4f& v) {
-    return v4f{static_cast<float>(norm_term<PMODE>(v[0], p)), static_cast<float>(norm_term<PMODE>(v[1], p)),
-               static_cast<float>(norm_term<PMODE>(v[2], p)), static_cast<float>(norm_term<PMODE>(v[3], p))};
-  });
-  __syncthreads();
-  if (threadIdx.x < width) {  // width <= TS <= 64: lanes of wave 0, one column each
-    const float* column = lds + threadIdx.x;
-    const double acc =
-        fold_tile_column<TS_SHIFT>(column, dim, 0.0, [](double a, float t) { return a + static_cast<double>(t); });
-    lds[threadIdx.x] = norm_finish<PMODE>(acc, p, eps);
+  float factor[kTilePerLane];
+  if (SM == kSsdChannelScale) {
+#pragma unroll
+    for (int u = 0; u < kTilePerLane; ++u)
+      if (lane.step(u)) factor[u] = scale[lane.row(u)];
+  }
+  double acc[4] = {0, 0, 0, 0};
+  if (lane.valid != 0) {
+#pragma unroll
+    for (int u = 0; u < kTilePerLane; ++u) {
+      if (!lane.step(u)) continue;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) acc[k] += static_cast<double>(lane.has(u) ? term(r[u][k]) : 0.f);
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < 4; ++k) acc[k] = strided_lane_sum<Lane::LANES_PER_ROW>(acc[k]);
+  if (threadIdx.x % kWave < Lane::LANES_PER_ROW) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) partial[threadIdx.x / kWave][lane.j + k] = acc[k];
   }
   __syncthreads();
+  if (threadIdx.x < kWave) {  // all of wave 0, so that its lanes agree on the flag
+    bool settled = true;
+    if (threadIdx.x < width) {
+      double sum = partial[0][threadIdx.x];
+#pragma unroll
+      for (int w = 1; w < kWaves; ++w) sum += partial[w][threadIdx.x];
+      const float d = norm_finish<PMODE>(sum, p, eps);
+      handed[threadIdx.x] = d;
+      recip[threadIdx.x] = reciprocal(d);
+      settled = norm_settled<PMODE>(sum, eps, dim);
+    }
+    const uint64_t seen = __builtin_amdgcn_ballot_w64(!settled);
+    if (threadIdx.x == 0) unsettled = seen != 0;
+  }
+  __syncthreads();
+  if (unsettled != 0) {  // the whole workgroup: the sums in index order, STEP rows at a time
+    double sum = 0;
+#pragma unroll
+    for (int u = 0; u < kTilePerLane; ++u) {
+      if (u * Lane::STEP >= dim) continue;
+      if (lane.valid != 0 && lane.has(u))
+        *reinterpret_cast<v4f*>(chunk + (lane.c0 << TS_SHIFT) + lane.j) = v4f{term(r[u][0]), term(r[u][1]), term(r[u][2]), term(r[u][3])};
+      __syncthreads();
+      if (threadIdx.x < width) {
+        const uint32_t rows = min(Lane::STEP, dim - u * Lane::STEP);
+        for (uint32_t c = 0; c < rows; ++c) sum += static_cast<double>(chunk[(c << TS_SHIFT) + threadIdx.x]);
+      }
+      __syncthreads();
+    }
+    if (threadIdx.x < width) {
+      const float d = norm_finish<PMODE>(sum, p, eps);
+      handed[threadIdx.x] = d;
+      recip[threadIdx.x] = reciprocal(d);
+    }
+    __syncthreads();
+  }
   if (lane.valid == 0) return;
-  const v4f d = *reinterpret_cast<const v4f*>(lds + lane.j);
+  const TileQuotients q(handed + lane.j, recip + lane.j);
 #pragma unroll
   for (int u = 0; u < kTilePerLane; ++u) {
-    const uint32_t c = lane.c0 + u * lane.STEP;
-    if (c >= dim) continue;
-    v4f q;
+    if (!lane.has(u)) continue;
+    const uint32_t c = lane.c0 + u * Lane::STEP;
+    v4f v = q(r[u]);
 #pragma unroll
-    for (int k = 0; k < 4; ++k) q[k] = ssd_scaled<SM>(r[u][k] / d[k], scale, c);
-    lane.store(y + base, u, q);
+    for (int k = 0; k < 4; ++k) v[k] = SM == kSsdChannelScale ? v[k] * factor[u] : ssd_scaled<SM>(v[k], scale, c);
+    lane.store(y + base, u, v);
   }
 }
 
@@ -1022,18 +1117,17 @@ static void launch_normalize_tile_ts(int outer_num, int dim, int inner_num, floa
                                      const float* scale, float* y, hipStream_t st) {
   const uint32_t tiles = (static_cast<uint32_t>(inner_num) + (1u << TS_SHIFT) - 1) >> TS_SHIFT;
   const uint32_t grid = static_cast<uint32_t>(outer_num) * tiles;
-  const size_t bytes = (static_cast<size_t>(dim) << TS_SHIFT) * sizeof(float);
   const uint32_t d = static_cast<uint32_t>(dim), in = static_cast<uint32_t>(inner_num);
   const FastDiv ft = make_fastdiv(tiles);
   switch (tile_rows(inner_num, y)) {
     case kRowsSector:
-      normalize_tile_kernel<PMODE, SM, TS_SHIFT, kRowsSector><<<grid, kBlock, bytes, st>>>(x, y, d, in, ft, p, eps, scale);
+      normalize_tile_kernel<PMODE, SM, TS_SHIFT, kRowsSector><<<grid, kBlock, 0, st>>>(x, y, d, in, scale, p, eps, ft);
       break;
     case kRowsQuad:
-      normalize_tile_kernel<PMODE, SM, TS_SHIFT, kRowsQuad><<<grid, kBlock, bytes, st>>>(x, y, d, in, ft, p, eps, scale);
+      normalize_tile_kernel<PMODE, SM, TS_SHIFT, kRowsQuad><<<grid, kBlock, 0, st>>>(x, y, d, in, scale, p, eps, ft);
       break;
     default:
-      normalize_tile_kernel<PMODE, SM, TS_SHIFT, kRowsAny><<<grid, kBlock, bytes, st>>>(x, y, d, in, ft, p, eps, scale);
+      normalize_tile_kernel<PMODE, SM, TS_SHIFT, kRowsAny><<<grid, kBlock, 0, st>>>(x, y, d, in, scale, p, eps, ft);
   }
 }
 
@@ -1042,12 +1136,10 @@ static int normalize_tile_shift(int dim);
 template <int PMODE, int SM>
 static void launch_normalize_tile(int outer_num, int dim, int inner_num, float p, float eps, const float* x,
                                   const float* scale, float* y, hipStream_t st) {
-  // 64 positions per tile row while the tile stays within 32 KB (four and more
-  // workgroups per CU), else 32, up to 64 KB: rows of 16 positions (64 bytes)
-  // cost more than the lower occupancy does.  [64,256,56,56]: 85 us with 64
-  // positions (64 KB), 80 us with 32; [64,512,38,38]: 105 us with 32 (64 KB),
-  // 115 us with 16.  Softmax, with its four barriers per tile, takes the widest
-  // tile that fits.
+  // 64 positions per tile row while a lane has at most eight vectors of them (up to 128 rows),
+  // else 32, up to 16 vectors, else 16.  Measured when the columns were walked out of a tile in
+  // LDS: [64,256,56,56] 85 us with 64 positions, 80 us with 32; [64,512,38,38] 105 us with 32, 115
+  // with 16.  Softmax takes the widest tile that fits.
   const int shift = normalize_tile_shift(dim);
   if (shift == 6)
     launch_normalize_tile_ts<PMODE, SM, 6>(outer_num, dim, inner_num, p, eps, x, scale, y, st);
@@ -1057,28 +1149,39 @@ static void launch_normalize_tile(int outer_num, int dim, int inner_num, float p
     launch_normalize_tile_ts<PMODE, SM, 4>(outer_num, dim, inner_num, p, eps, x, scale, y, st);
 }
 
+// Maximum over the lanes of a wave that are `LANES` apart (4, 8 or 16).
+template <int LANES>
+SHDW_DEVICE float strided_lane_max(float m) {
+  if (LANES <= 4) m = max3_any_order(m, m, dpp_f32<kDppRor4>(m));
+  if (LANES <= 8) m = max3_any_order(m, m, dpp_f32<kDppRor8>(m));
+  m = max3_any_order(m, m, __shfl_xor(m, 16));
+  return max3_any_order(m, m, __shfl_xor(m, 32));
+}
+
 // Softmax on the same tile layout (65 <= dim <= 1024).  The lanes hold x, later
-// exp(x - max), in registers.  Behind the tile lie the exp table, a row that
-// hands the maxima and later the sums over, and a flag.
+// exp(x - max), in registers.  Behind the tile lie the exp table and what is handed from
+// lane to lane: the waves' maxima, and later the sums and their reciprocals.
 //
-// The running maximum max = std_max(x[c], max), started at -FLT_MAX, is the
-// largest element whatever the order as long as no element is NaN (a NaN takes
-// the maximum over and the next element takes it back, so then the order
-// counts; which of two zeros wins does not change exp(x - max)).  Every lane
-// therefore takes the maximum of its own rows, the STEP partial maxima per
-// position meet in the first tile rows and one lane per position folds them; a
-// lane that met a NaN hands a NaN over instead, and a tile with one anywhere
-// parks x and walks the columns in index order like the sums.  The sum of the
-// exponentials is an fp32 running sum and always walks.
+// The maxima are taken in any order: from the lanes' own rows, then over the lanes and the
+// waves (a NaN anywhere in a column makes all of it NaN whatever the maximum was).  The sum of
+// the exponentials is an fp32 running sum and is always walked in index order, by one wave; which
+// of the four changes from one group of 256 workgroups to the next, since wave i of every
+// workgroup of a CU is on the same SIMD and walks that share one take turns.
+//
+// [16,150,72,72], 99.5 MB: 23.6 us.  Its vector instructions bound it together with the rounds of
+// load, walk and store (the exponential 17 an element, the quotient 4); 28.4 us with the maxima by
+// compare and select, a division and the longer exponential, and five barriers.
 template <int TS_SHIFT, int ROWS>
 __global__ __launch_bounds__(kBlock) void softmax_tile_kernel(const float* x, float* y, uint32_t dim,
                                                                uint32_t inner, FastDiv f_tiles) {
   extern __shared__ __align__(16) float lds[];
   constexpr uint32_t TS = 1u << TS_SHIFT;
+  constexpr uint32_t kWaves = kBlock / kWave;
   using Lane = TileLane<TS_SHIFT, ROWS>;
   uint64_t* tab = reinterpret_cast<uint64_t*>(lds + (dim << TS_SHIFT));  // after the tile, 16-byte aligned
-  float* handed = reinterpret_cast<float*>(tab + 32);
-  uint32_t* any_nan = reinterpret_cast<uint32_t*>(handed + TS);
+  float* maxima = reinterpret_cast<float*>(tab + 32);                    // [wave][TS]
+  double* recip = reinterpret_cast<double*>(tab + 32);                   // [TS], when the maxima have been read
+  float* handed = reinterpret_cast<float*>(recip + TS);                  // [TS]
   if (threadIdx.x < 32) tab[threadIdx.x] = libm::kExp2fTab[threadIdx.x];
   uint32_t n, tile;
   fd_divmod(xcd_contiguous(blockIdx.x, gridDim.x), f_tiles, n, tile);
@@ -1086,90 +1189,69 @@ __global__ __launch_bounds__(kBlock) void softmax_tile_kernel(const float* x, fl
   const uint32_t width = min(TS, inner - p0);
   const uint64_t base = static_cast<uint64_t>(n) * dim * inner + p0;
   const Lane lane(width, dim, inner);
+  const uint32_t wave = threadIdx.x / kWave;
   v4f r[kTilePerLane];
   lane.load(x + base, r);
+  v4f m = {-FLT_MAX, -FLT_MAX, -FLT_MAX, -FLT_MAX};
   if (lane.valid != 0) {
-    v4f m = {-FLT_MAX, -FLT_MAX, -FLT_MAX, -FLT_MAX};
-    bool nan[4] = {false, false, false, false};
 #pragma unroll
-    for (int u = 0; u < kTilePerLane; ++u) {
-      if (lane.c0 + u * Lane::STEP >= dim) continue;
+    for (int u = 0; u < kTilePerLane; u += 2) {
+      if (!lane.step(u)) continue;
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const float v = r[u][k];
-        nan[k] |= v != v;
-        m[k] = m[k] < v ? v : m[k];
-      }
+      for (int k = 0; k < 4; ++k) m[k] = max3_any_order(m[k], r[u][k], r[u + 1][k]);
     }
-#pragma unroll
-    for (int k = 0; k < 4; ++k) m[k] = nan[k] ? __builtin_nanf("") : m[k];
-    *reinterpret_cast<v4f*>(lds + (lane.c0 << TS_SHIFT) + lane.j) = m;  // row c0 < STEP <= 64 < dim
   }
+#pragma unroll
+  for (int k = 0; k < 4; ++k) m[k] = strided_lane_max<Lane::LANES_PER_ROW>(m[k]);
+  if (threadIdx.x % kWave < Lane::LANES_PER_ROW) *reinterpret_cast<v4f*>(maxima + wave * TS + lane.j) = m;
   __syncthreads();
-  if (threadIdx.x < kWave) {  // all of wave 0, so that its lanes agree on the flag
-    float m = -FLT_MAX;
-    bool nan = false;
-    if (threadIdx.x < width) {
-      const uint32_t groups = min(Lane::STEP, dim);
-      for (uint32_t g = 0; g < groups; ++g) {
-        const float v = lds[(g << TS_SHIFT) + threadIdx.x];
-        nan |= v != v;
-        m = m < v ? v : m;
-      }
-      handed[threadIdx.x] = m;
-    }
-    const uint64_t seen = __builtin_amdgcn_ballot_w64(nan);
-    if (threadIdx.x == 0) *any_nan = seen != 0;
-  }
-  __syncthreads();
-  if (*any_nan != 0) {  // the whole workgroup: the maxima in index order
-    lane.park(lds, r);
-    __syncthreads();
-    if (threadIdx.x < width) {
-      const float* column = lds + threadIdx.x;
-      handed[threadIdx.x] = fold_tile_column<TS_SHIFT>(column, dim, -FLT_MAX,
-                                                      [](float m, float v) { return std_max(v, m); });
-    }
-    __syncthreads();
-  }
   if (lane.valid != 0) {
-    const v4f m = *reinterpret_cast<const v4f*>(handed + lane.j);
 #pragma unroll
-    for (int u = 0; u < kTilePerLane; ++u) {
-      if (lane.c0 + u * lane.STEP >= dim) continue;
+    for (uint32_t w = 0; w < kWaves; ++w) {
+      const v4f other = *reinterpret_cast<const v4f*>(maxima + w * TS + lane.j);
 #pragma unroll
-      for (int k = 0; k < 4; ++k) r[u][k] = libm::exact_expf(r[u][k] - m[k], tab);
+      for (int k = 0; k < 4; ++k) m[k] = max3_any_order(m[k], m[k], other[k]);
+    }
+#pragma unroll
+    for (int u = 0; u < kTilePerLane; u += 2) {  // eight exponentials, each a chain, side by side
+      if (!lane.step(u)) continue;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) r[u + k / 4][k % 4] = libm::exact_expf_nonpositive(r[u + k / 4][k % 4] - m[k % 4], tab);
+#pragma unroll
+      for (int k = 0; k < 2; ++k)
+        if (lane.has(u + k)) *reinterpret_cast<v4f*>(lds + ((lane.c0 + (u + k) * Lane::STEP) << TS_SHIFT) + lane.j) = r[u + k];
     }
   }
-  lane.park(lds, r);
   __syncthreads();  // also: every lane has its maxima before the sums replace them
-  if (threadIdx.x < width) {
-    const float* column = lds + threadIdx.x;
-    handed[threadIdx.x] = fold_tile_column<TS_SHIFT>(column, dim, 0.f, [](float a, float v) { return a + v; });
+  if (wave == blockIdx.x / kBlock % kWaves) {
+    const uint32_t pos = threadIdx.x % kWave;
+    if (pos < width) {
+      __builtin_amdgcn_s_setprio(3);
+      const float sum = fold_tile_column<TS_SHIFT>(lds + pos, dim, 0.f, [](float a, float v) { return a + v; });
+      handed[pos] = sum;
+      recip[pos] = reciprocal(sum);
+      __builtin_amdgcn_s_setprio(0);
+    }
   }
   __syncthreads();
   if (lane.valid == 0) return;
-  const v4f d = *reinterpret_cast<const v4f*>(handed + lane.j);
+  const TileQuotients q(handed + lane.j, recip + lane.j);
 #pragma unroll
-  for (int u = 0; u < kTilePerLane; ++u) {
-    if (lane.c0 + u * lane.STEP >= dim) continue;
-    v4f q;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) q[k] = r[u][k] / d[k];
-    lane.store(y + base, u, q);
-  }
+  for (int u = 0; u < kTilePerLane; ++u)
+    if (lane.has(u)) lane.store(y + base, u, q(r[u]));
 }
 
 constexpr size_t kExpTabBytes = 32 * sizeof(uint64_t);
-constexpr size_t kSoftmaxTileExtraBytes = kExpTabBytes + 64 * sizeof(float) + 16;  // table, hand-over row, flag
-// (32 positions of 512 channels, or 16 of 1024, plus the exp table: 64 KB + 256 bytes, two workgroups per CU all the same)
+// the exp table and the maxima of four waves, whose place the sums (fp32) and their reciprocals (fp64) take
+// (32 positions of 512 channels, or 16 of 1024, with it: 66 KB at most, two workgroups per CU all the same)
+static size_t softmax_tile_extra_bytes(int ts) { return kExpTabBytes + static_cast<size_t>(kBlock / kWave) * ts * sizeof(float); }
 
 template <int TS_SHIFT>
 static void launch_softmax_tile_ts(int outer_num, int dim, int inner_num, const float* x, float* y,
                                    hipStream_t st) {
   const uint32_t tiles = (static_cast<uint32_t>(inner_num) + (1u << TS_SHIFT) - 1) >> TS_SHIFT;
   const uint32_t grid = static_cast<uint32_t>(outer_num) * tiles;
-  const size_t bytes = (static_cast<size_t>(dim) << TS_SHIFT) * sizeof(float) + kSoftmaxTileExtraBytes;
+  const size_t bytes = (static_cast<size_t>(dim) << TS_SHIFT) * sizeof(float) + softmax_tile_extra_bytes(1 << TS_SHIFT);
   const uint32_t d = static_cast<uint32_t>(dim), in = static_cast<uint32_t>(inner_num);
   const FastDiv ft = make_fastdiv(tiles);
   switch (tile_rows(inner_num, y)) {
