@@ -205,6 +205,7 @@ SHDW_DEVICE uint32_t dpp_u32(uint32_t v) {
 
 constexpr int kDppXor1 = 0xB1;        // quad_perm [1,0,3,2]
 constexpr int kDppXor2 = 0x4E;        // quad_perm [2,3,0,1]
+constexpr int kDppWaveShr1 = 0x138;    // lane i takes lane i - 1, lane 0 keeps its own
 constexpr int kDppRor4 = 0x124;        // lane i takes lane i - 4 (modulo 16) inside 16
 constexpr int kDppRor8 = 0x128;        // lane i <-> i + 8 (modulo 16) inside 16
 constexpr int kDppHalfMirror = 0x141;  // lane i <-> 7-i inside 8

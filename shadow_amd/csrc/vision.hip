@@ -1172,98 +1172,106 @@ static void launch_pool_plane(const float* x, float* y, uint32_t rows, uint32_t 
 }
 
 // Whole-plane average over rows of any length, without a barrier: every wave of a
-// workgroup works by itself on G consecutive rows, which it walks in chunks of
-// W = 4096 / G columns.  All lanes fetch a chunk (16 vectors each, 16 KB per wave)
-// and lay it down in the wave's LDS rows; lane g < G then adds row g's columns in
-// index order (an fp32 running sum has no other order; a dependent addition takes
-// six clocks, so a row of 3136 takes 8 us whatever else happens) while the next
-// chunk is already on its way.  A wave never waits for another wave, so a CU's
-// eight resident waves overlap each other's fetches and folds.  G shrinks as the
-// rows get longer and fewer: what matters is enough waves in flight (16 KB each)
-// to cover HBM's latency, not how many lanes of a wave fold.  The four waves of a
-// workgroup exist for their placement only: one per SIMD.  Single-wave
-// workgroups were measured to pile up on one SIMD of a CU when only four of
-// them fit the launch, and waves that share a SIMD take turns at every addition.
-// The LDS pitch of W + 4 floats keeps 128-bit accesses aligned and puts the
-// folding lanes on distinct banks.
-constexpr int kStreamVectors = 16;  // per lane and chunk
+// workgroup works by itself on G consecutive rows, in chunks of W = 32 * 64 / G
+// columns.  An fp32 running sum has no order but the index order, so a row costs a
+// chain of as many dependent additions, 2.8 ns each (9 us for 3136), and a wave alone
+// on its SIMD issues nothing faster than that whatever it issues: what counts is to
+// issue little besides the additions.  A chunk passes through the wave's LDS once, so
+// that every one of the 64 / G lanes of a row holds 32 consecutive columns of it in
+// registers; the sum then visits these lanes in turn, 32 additions each, and moves to
+// the next with the first of them (a DPP operand).  All lanes add all the time, each to
+// what its neighbour had, and the one whose turn it is has the row's sum.  The next
+// chunk is on its way meanwhile.  Columns past the end are zeros, which leave a sum that
+// starts at +0 as it is.  The four waves of a workgroup exist for their placement only:
+// one per SIMD.  Single-wave workgroups were measured to pile up on one SIMD of a CU when
+// only four of them fit the launch.
+// With one lane of a row reading its columns from LDS in steps of 64 (a read for four
+// additions, its latency exposed once a step) 2048 rows of 3136 took 18.0 us.
+constexpr int kSpan = 32;              // columns of a lane and chunk
+constexpr int kSpanPitch = kSpan + 4;  // in LDS: 128-bit accesses of 16 neighbouring lanes on distinct banks
+constexpr int kStreamVectors = kSpan / 4;  // per lane and chunk
 constexpr int kStreamWaves = kBlock / kWave;
 
 template <int G>
 __global__ __launch_bounds__(kBlock) void pool_rows_stream_kernel(const float* x, float* y, uint32_t rows,
                                                                    uint32_t len, float pool_size) {
-  constexpr uint32_t W = 256u * kStreamVectors / G, VW = W / 4, PITCH = W + 4;
-  __shared__ __align__(16) float tiles[kStreamWaves * G * PITCH];
-  const uint32_t lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-  float* tile = tiles + wave * (G * PITCH);
+  constexpr uint32_t L = kWave / G, W = kSpan * L, VW = W / 4;
+  __shared__ __align__(16) float tiles[kStreamWaves][kWave * kSpanPitch];
+  const uint32_t lane = threadIdx.x % kWave;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  float* tile = tiles[wave];
   const uint32_t row0 = (blockIdx.x * kStreamWaves + wave) * G;
   if (row0 >= rows) return;  // the whole wave
   v4f reg[kStreamVectors];
+  // No branch around a load: vectors past the end of a row take its last four elements (rows
+  // have 256 and more), rows past the end take the last row.
   auto request = [&](uint32_t c0) {
+    const float* at = x + static_cast<uint64_t>(row0) * len;
+    const uint32_t last_row = rows - 1 - row0;
 #pragma unroll
     for (int i = 0; i < kStreamVectors; ++i) {
       const uint32_t v = lane + kWave * i;
-      const uint32_t g = v / VW, c = c0 + 4 * (v % VW);
-      if (row0 + g >= rows || c >= len) continue;
-      const float* src = x + static_cast<uint64_t>(row0 + g) * len + c;
-      if (c + 4 <= len) {
-        reg[i] = load4_stream_any(src);
-      } else {
-#pragma unroll
-        for (int k = 0; k < 3; ++k)
-          if (c + k < len) reg[i][k] = load_stream(src + k);
-      }
+      reg[i] = load4_stream_any(at + (min(v / VW, last_row) * len + min(c0 + 4 * (v % VW), len - 4)));
     }
   };
   float sum = 0.f;
+  uint32_t turns = 0;
   request(0);
   for (uint32_t c0 = 0; c0 < len; c0 += W) {
+    auto slot = [&](int i) {
+      const uint32_t v = lane + kWave * i, c = 4 * (v % VW);
+      return tile + (v / VW * L + c / kSpan) * kSpanPitch + c % kSpan;
+    };
+    if (c0 + W <= len) {
 #pragma unroll
-    for (int i = 0; i < kStreamVectors; ++i) {
-      const uint32_t v = lane + kWave * i;
-      *reinterpret_cast<v4f*>(tile + (v / VW) * PITCH + 4 * (v % VW)) = reg[i];
+      for (int i = 0; i < kStreamVectors; ++i) *reinterpret_cast<v4f*>(slot(i)) = reg[i];
+    } else {
+#pragma unroll
+      for (int i = 0; i < kStreamVectors; ++i) {
+        const uint32_t c = c0 + 4 * ((lane + kWave * i) % VW);
+        const uint32_t moved = c - min(c, len - 4);  // by how much the vector was moved to the front
+        *reinterpret_cast<v4f*>(slot(i)) = moved == 0 ? reg[i] : v4f{0.f, 0.f, 0.f, 0.f};
+        if (moved - 1 < 3) {  // the row ends inside it
+#pragma unroll
+          for (int k = 1; k < 4; ++k)
+            if (k >= moved) slot(i)[k - moved] = reg[i][k];
+        }
+      }
     }
     __builtin_amdgcn_wave_barrier();
     if (c0 + W < len) request(c0 + W);
-    if (lane < G) {
-      const uint32_t cols = min(W, len - c0);
-      const float* mine = tile + lane * PITCH;
-      // 64 values per step, read with sixteen 128-bit reads and then added in order.  One set of
-      // registers: with two sets taking turns (the next step's reads behind this step's additions) the
-      // compiler copied one set into the other every turn, 32 moves per 64 additions, and a wave
-      // alone on its SIMD issues an instruction every 2.8 ns whatever it is; the LDS latency that is
-      // exposed instead is a twentieth of a step's additions.
-      constexpr int kAhead = 16, kStep = 4 * kAhead;
-      uint32_t c = 0;
-      for (; c + kStep <= cols; c += kStep) {
-        v4f q[kAhead];
+    v4f mine[kStreamVectors];
 #pragma unroll
-        for (int k = 0; k < kAhead; ++k) q[k] = *reinterpret_cast<const v4f*>(mine + c + 4 * k);
+    for (int i = 0; i < kStreamVectors; ++i) mine[i] = *reinterpret_cast<const v4f*>(tile + lane * kSpanPitch + 4 * i);
+    if (c0 != 0) sum = __shfl(sum, lane | (L - 1));  // from the last lane of the row to its first
+    turns = min(L, (len - c0 + kSpan - 1) / kSpan);
 #pragma unroll
-        for (int k = 0; k < kStep; ++k) sum += q[k / 4][k % 4];
-      }
-      for (; c < cols; ++c) sum += mine[c];
+    for (int k = 0; k < kSpan; ++k) sum += mine[k / 4][k % 4];
+    for (uint32_t t = 1; t < turns; ++t) {
+      sum = dpp_f32<kDppWaveShr1>(sum);
+#pragma unroll
+      for (int k = 0; k < kSpan; ++k) sum += mine[k / 4][k % 4];
     }
     __builtin_amdgcn_wave_barrier();
   }
-  if (lane < G && row0 + lane < rows) y[row0 + lane] = sum / pool_size;
+  const uint32_t row = row0 + lane / L;
+  if (lane % L == turns - 1 && row < rows) y[row] = sum / pool_size;
 }
 
 // From this row length on the whole-plane average takes the streaming kernel
-// (per 51 MB, against pool_plane_kernel: 28x28 planes 15.1 / 23.5 us, 56x56 planes
-// 24.6 / 59 us; 14x14 planes 13.2 / 14.2 us but 45.8 / 42.0 us per 205 MB, 7x7 planes
-// 12.6 / 12.7 and 44.1 / 39.6 us).
+// (per 51 MB, against pool_plane_kernel: 28x28 planes 10.7 / 23.5 us, 56x56 planes
+// 14.5 / 59 us; 14x14 planes, before the sum went from lane to lane, 13.2 / 14.2 us but
+// 45.8 / 42.0 us per 205 MB).  Few rows as well: [1,3,224,224] 126 us against 630.
 constexpr int kPlaneStreamMinLen = 256;
-// Few rows as well: a wave per row walks at 5 ns per element where the workgroup form above, which stages
-// a chunk, meets at a barrier and then walks it, takes 10 to 18 ([1,3,224,224]: 252 us against 630 us,
-// 64 planes of 56x56: 29 against 30).
-// Rows per wave: as many as leave 1536 waves and more (six per CU), so long and few rows get a wave
-// each.  Measured per 51 MB: 16x16 planes 10.2 us with 32 rows per wave (12.7 with 16), 20x20 11.7 with
-// 16 (14.6 with 8), 28x28 13.1 with 8 (17.2 with 4, 13.7 with 16), 40x40 16.6 with 4 (21.7 with 2),
-// 56x56 21.3 with 2 (26.3 with 4, 33.9 with 1).
+// Rows per wave: up to eight while there are 512 waves (two a CU) and more.  Every wave issues all
+// the additions of a row whatever the number of its rows, so few rows go one to a wave and many
+// eight, from where on memory bounds the launch and shorter row pieces do not help it.  With 1 / 2
+// / 4 / 8 / 16 rows per wave: 512 rows of 12544 36.7 / 36.3 / 40.5 / 47.6 / 73.6 us, 2048 of 3136
+// 13.4 / 13.4 / 12.6 / 14.1 / 21.1, 4096 of 3136 23.8 / 15.2 / 14.5 / 14.8 / 21.8, 16384 of 784
+// 24.2 / 14.8 / 11.8 / 10.7 / 11.1, 50200 of 256 33.3 / 18.3 / 11.9 / 9.9 / 10.1.
 static int stream_rows_per_wave(uint32_t rows) {
   int g = 1;
-  while (g < 64 && rows / static_cast<uint32_t>(2 * g) >= 1536u) g <<= 1;
+  while (g < 8 && rows / static_cast<uint32_t>(2 * g) >= 512u) g <<= 1;
   return g;
 }
 
@@ -1273,9 +1281,6 @@ static void launch_pool_rows_stream(const float* x, float* y, uint32_t rows, uin
   const uint32_t per_wg = static_cast<uint32_t>(g) * kStreamWaves;
   const uint32_t grid = (rows + per_wg - 1) / per_wg;
   switch (g) {
-    case 64: pool_rows_stream_kernel<64><<<grid, kBlock, 0, st>>>(x, y, rows, len, size); break;
-    case 32: pool_rows_stream_kernel<32><<<grid, kBlock, 0, st>>>(x, y, rows, len, size); break;
-    case 16: pool_rows_stream_kernel<16><<<grid, kBlock, 0, st>>>(x, y, rows, len, size); break;
     case 8: pool_rows_stream_kernel<8><<<grid, kBlock, 0, st>>>(x, y, rows, len, size); break;
     case 4: pool_rows_stream_kernel<4><<<grid, kBlock, 0, st>>>(x, y, rows, len, size); break;
     case 2: pool_rows_stream_kernel<2><<<grid, kBlock, 0, st>>>(x, y, rows, len, size); break;

@@ -1,0 +1,36 @@
+"""Whole-plane averages of 256 and more elements: the sum of a plane goes from lane to lane, 32
+elements each, in chunks of 32 * 64 / G columns for G = 1, 2, 4 or 8 planes a wave."""
+import numpy as np
+import pytest
+
+import oracle
+from tests import gpuops
+from tests.helpers import assert_bit_exact, normal, with_specials
+
+pytestmark = pytest.mark.gpu
+
+# planes either side of where G changes (1024, 2048, 4096) and of whole waves and workgroups;
+# lengths either side of a lane's span, of a chunk and of whole vectors
+PLANES = [1, 3, 1023, 1025, 2047, 2050, 4095, 4097, 4129]
+LENGTHS = [256, 257, 287, 289, 511, 514, 1023, 1027, 2048, 2049, 4099]
+
+
+@pytest.mark.parametrize("length", LENGTHS)
+@pytest.mark.parametrize("planes", PLANES)
+def test_whole_plane_average(gpu, planes, length):
+    x = normal(planes + length, planes * length, 2.0)
+    shape, out = (1, planes, 1, length), (1, planes, 1, 1)
+    want = oracle.pooling(x, shape, 1, (1, length), (1, 1), (0, 0), out)
+    assert_bit_exact(gpuops.pooling(x, shape, 1, (1, length), (1, 1), (0, 0), out, offset=planes % 4), want, "average")
+
+
+@pytest.mark.parametrize("length", [256, 515, 2051])
+def test_whole_plane_average_of_special_values(gpu, length):
+    shape, out = (5, 7, length), (5, 7, 1)
+    x = with_specials(normal(3, 35 * length, 2.0), 3).reshape(shape)
+    x[1] = -0.0
+    x[2] = np.float32(1e-42)
+    x[3, :, -1] = np.inf
+    args = ((5, 7, 1, length), 1, (1, length), (1, 1), (0, 0), (5, 7, 1, 1))
+    with np.errstate(all="ignore"):
+        assert_bit_exact(gpuops.pooling(x, *args), oracle.pooling(x, *args), "average")
