@@ -10,8 +10,9 @@
 // channels) or in LDS (a column of `size` floats per lane, no two lanes share a
 // bank row), the centre of the window is multiplied as soon as its scale is
 // known, x is read once and y written once.  Neighbouring lanes hold neighbouring
-// positions, so every load and store of a wave is one run of 256 bytes.  y may be x: a lane has read every channel of a round, and all
-// before it, when it writes the channels the round finishes, which lie behind them.
+// positions, so every load and store of a wave is one run of 256 bytes.  y may be x: a lane
+// has read every channel of a round, and all before it, when it writes the channels the
+// round finishes, which lie behind them.
 #include <hip/hip_runtime.h>
 
 #include <climits>
@@ -94,90 +95,121 @@ SHDW_DEVICE void lrn_powers(const float (&scale)[kLrnRound], float y, bool small
   }
 }
 
+// ---- windows of 1, 3, 5 and 7 channels: the window lives in registers ----
+// A workgroup owns 64 positions and goes through their channels in spans of four rounds, a
+// wave each.  Every lane has the channels of its round at once, those of the next span
+// on their way during the powers; the waves take turns at the walk, which is short (two dependent
+// additions a channel), each handing the sum and the last SIZE channels to the next through
+// LDS; then all of them work out their powers, which are most of the work, at the same time.
+// Bound by the vector ALUs: 30 instructions a power, two thirds of them fp64.  With one wave
+// walking all channels of its positions, and up to eight workgroups sharing the rounds of a
+// position where there are few (each walking from the first channel on): [44,96,55,55]
+// 38.8 -> 30.1 us, [16,256,56,56] 48.8 -> 30.8, [64,256,56,56] 118 -> 90, [68,256,27,27] 51.3 ->
+// 33.9, [1,96,55,55] 14.6 -> 8.0.  Rounds of 16 and 24 channels: 37.8 and 37.6 on the first.
+//
+// Round c0 finishes channels c0 .. c0 + 7, for which the sum takes in channel c + post and
+// lets go of channel c - post - 1: own[j] is channel c0 + post + j, prev[t] channel
+// c0 + post - SIZE + t.  y may be x: what a span writes lies behind everything that later
+// spans read, and inside a span all is read before the last of its barriers.
+constexpr int kLrnWaves = kBlock / kWave;
+
+template <int SIZE>
+struct LrnHand {
+  float accum[kWave], prev[SIZE][kWave];
+};
+
+// EDGE: the first segments and those that reach past the last channel, with the tests of the
+// reference's three loops (the same for all lanes); the segments between them need none.
+template <int SIZE, bool EDGE>
+SHDW_DEVICE float lrn_walk(const float (&own)[kLrnRound], const float (&prev)[SIZE],
+                           float (&scale)[kLrnRound], float accum, uint32_t c0, uint32_t channels,
+                           float alpha_over_size, float k) {
+  constexpr uint32_t post = (SIZE - 1) / 2;
+#pragma unroll
+  for (int j = 0; j < static_cast<int>(kLrnRound); ++j) {
+    const uint32_t c = c0 + j;
+    if (!EDGE || c + post < channels) accum += own[j] * own[j];
+    if (!EDGE || (c > post && c < channels)) {
+      const float leaving = j >= SIZE ? own[j >= SIZE ? j - SIZE : 0] : prev[j < SIZE ? j : 0];
+      accum -= leaving * leaving;
+    }
+    scale[j] = k + accum * alpha_over_size;
+  }
+  return accum;
+}
+
+template <int SIZE>
+__global__ __launch_bounds__(kBlock, 5) void lrn_window_kernel(const float* x, float* y, uint32_t positions, uint32_t step,
+                                                               uint32_t channels, float alpha_over_size, float neg_beta,
+                                                               float k, FastDiv f_step) {
+  constexpr int SEG = kLrnRound;
+  static_assert(SIZE % 2 == 1 && SIZE <= SEG, "the window must fit into a round");
+  constexpr uint32_t post = (SIZE - 1) / 2;
+  __shared__ LrnTables tables;
+  __shared__ LrnHand<SIZE> hand;
+  lrn_stage_tables(&tables);
+  const uint32_t lane = threadIdx.x % kWave;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const uint32_t p = blockIdx.x * kWave + lane, at = min(p, positions - 1);
+  const uint32_t b = fd_div(at, f_step);
+  const size_t base = static_cast<size_t>(b) * channels * step + (at - b * step);
+  const float* in = x + base;
+  float* out = y + base;
+  float ahead[SEG];  // the next span's, on their way during the powers
+  auto request = [&](uint32_t c0) {
+#pragma unroll
+    for (int j = 0; j < SEG; ++j) ahead[j] = in[static_cast<size_t>(min(c0 + post + j, channels - 1)) * step];
+  };
+  request(wave * SEG);
+  for (uint32_t span = 0; span < channels; span += kLrnWaves * SEG) {
+    const uint32_t c0 = span + wave * SEG;
+    float own[SEG], prev[SIZE], scale[SEG];
+#pragma unroll
+    for (int j = 0; j < SEG; ++j) own[j] = ahead[j];
+    if (c0 == 0) {
+#pragma unroll
+      for (int t = 0; t < SIZE; ++t) prev[t] = t + static_cast<int>(post) >= SIZE ? in[static_cast<size_t>(t + post - SIZE) * step] : 0.f;
+    }
+    for (uint32_t turn = 0; turn < kLrnWaves; ++turn) {
+      if (wave == turn && c0 < channels) {  // the same for the whole wave
+        float accum = 0.f;
+        if (c0 == 0) {
+#pragma unroll
+          for (int t = SIZE - static_cast<int>(post); t < SIZE; ++t) accum += prev[t] * prev[t];
+        } else {
+          accum = hand.accum[lane];
+#pragma unroll
+          for (int t = 0; t < SIZE; ++t) prev[t] = hand.prev[t][lane];
+        }
+        if (c0 > post && c0 + post + SEG <= channels)
+          accum = lrn_walk<SIZE, false>(own, prev, scale, accum, c0, channels, alpha_over_size, k);
+        else
+          accum = lrn_walk<SIZE, true>(own, prev, scale, accum, c0, channels, alpha_over_size, k);
+        hand.accum[lane] = accum;
+#pragma unroll
+        for (int t = 0; t < SIZE; ++t) hand.prev[t][lane] = own[SEG - SIZE + t];
+      }
+      __syncthreads();
+    }
+    if (span + kLrnWaves * SEG < channels) request(c0 + kLrnWaves * SEG);
+    if (c0 >= channels) continue;
+    float power[SEG];
+    lrn_powers(scale, neg_beta, neg_beta != 0.f && __builtin_fabsf(neg_beta) <= 1.25f, &tables, power);
+#pragma unroll
+    for (int j = 0; j < SEG; ++j) {
+      const float centre = j >= static_cast<int>(post) ? own[j >= static_cast<int>(post) ? j - post : 0]
+                                                       : prev[j < static_cast<int>(post) ? SIZE - post + j : 0];
+      if (c0 + j < channels && p < positions) out[static_cast<size_t>(c0 + j) * step] = centre * power[j];
+    }
+  }
+}
+
 // The channels of the round that starts at head0 (zeros past the last one).
 SHDW_DEVICE void lrn_fetch(const float* in, uint32_t head0, uint32_t channels, uint32_t step,
                            float (&values)[kLrnRound]) {
 #pragma unroll
   for (uint32_t j = 0; j < kLrnRound; ++j)
     values[j] = head0 + j < channels ? in[static_cast<size_t>(head0 + j) * step] : 0.f;
-}
-
-// ---- windows of 1, 3, 5 and 7 channels: the window lives in registers ----
-// prev[t] is channel head0 - SIZE + t, the last SIZE channels of the round before.
-// EDGE: the first round and those that reach past the last channel, with the tests
-// of the reference's three loops; the rounds between them need none.
-// `round` holds the channels of this round on entry and those of the next on
-// return: they are asked for before the powers and arrive while those are worked
-// out.  (The channels this round writes lie behind all of them, y may be x.)
-template <int SIZE, bool EDGE>
-SHDW_DEVICE void lrn_round(const float* in, float* out, uint32_t head0, uint32_t channels, uint32_t step,
-                           float (&round)[kLrnRound], float (&prev)[SIZE], float& accum, float alpha_over_size,
-                           float neg_beta, float k, const LrnTables* tables, bool finish) {
-  static_assert(SIZE % 2 == 1 && SIZE <= static_cast<int>(kLrnRound), "the window must fit into a round");
-  constexpr uint32_t post = (SIZE - 1) / 2;
-  const uint32_t steps = channels + post;  // step `head` takes channel head in and finishes channel head - post
-  float entering[kLrnRound], scale[kLrnRound], centre[kLrnRound], power[kLrnRound];
-#pragma unroll
-  for (uint32_t j = 0; j < kLrnRound; ++j) entering[j] = round[j];
-  lrn_fetch(in, head0 + kLrnRound, channels, step, round);
-#pragma unroll
-  for (uint32_t j = 0; j < kLrnRound; ++j) {
-    const uint32_t head = head0 + j;  // the same for every lane, and so is every test on it
-    scale[j] = 1.f;
-    centre[j] = 0.f;
-    if (!EDGE || head < channels) accum += entering[j] * entering[j];
-    if (!EDGE || (head >= SIZE && head < steps)) {
-      const float leaving = j >= SIZE ? entering[j >= SIZE ? j - SIZE : 0] : prev[j < SIZE ? j : 0];
-      accum -= leaving * leaving;
-    }
-    if (!EDGE || (head >= post && head < steps)) {
-      scale[j] = k + accum * alpha_over_size;
-      centre[j] = j >= post ? entering[j >= post ? j - post : 0] : prev[j < post ? SIZE - post + j : 0];
-    }
-  }
-#pragma unroll
-  for (int t = 0; t < SIZE; ++t) prev[t] = entering[kLrnRound - SIZE + t];
-  if (!finish) return;  // a round in front of this workgroup's share: only the sum had to pass through it
-  lrn_powers(scale, neg_beta, neg_beta != 0.f && __builtin_fabsf(neg_beta) <= 1.25f, tables, power);
-#pragma unroll
-  for (uint32_t j = 0; j < kLrnRound; ++j) {
-    const uint32_t head = head0 + j;
-    if (!EDGE || (head >= post && head < steps)) out[static_cast<size_t>(head - post) * step] = centre[j] * power[j];
-  }
-}
-
-template <int SIZE>
-__global__ __launch_bounds__(kBlock, 5) void lrn_window_kernel(const float* x, float* y, uint32_t positions,
-                                                            uint32_t step, uint32_t channels, FastDiv f_step,
-                                                            float alpha_over_size, float neg_beta, float k) {
-  __shared__ LrnTables tables;
-  lrn_stage_tables(&tables);
-  const uint32_t p = blockIdx.x * kBlock + threadIdx.x;
-  if (p >= positions) return;
-  const uint32_t b = fd_div(p, f_step);
-  const size_t base = static_cast<size_t>(b) * channels * step + (p - b * step);
-  const float* in = x + base;
-  float* out = y + base;
-  float prev[SIZE], round[kLrnRound];
-#pragma unroll
-  for (int t = 0; t < SIZE; ++t) prev[t] = 0.f;
-  float accum = 0.f;
-  const uint32_t steps = channels + (SIZE - 1) / 2;
-  // gridDim.y workgroups share the rounds of a position: each walks the sum from the
-  // first channel on, which is cheap, and works out the powers of its own rounds only
-  const uint32_t rounds = (steps + kLrnRound - 1) / kLrnRound;
-  const uint32_t first = blockIdx.y * rounds / gridDim.y * kLrnRound;
-  const uint32_t end = (blockIdx.y + 1) * rounds / gridDim.y * kLrnRound;
-  lrn_fetch(in, 0, channels, step, round);
-  for (uint32_t head0 = 0; head0 < end; head0 += kLrnRound) {
-    const bool finish = head0 >= first;
-    if (head0 >= SIZE && head0 + kLrnRound <= channels)
-      lrn_round<SIZE, false>(in, out, head0, channels, step, round, prev, accum, alpha_over_size, neg_beta, k, &tables,
-                             finish);
-    else
-      lrn_round<SIZE, true>(in, out, head0, channels, step, round, prev, accum, alpha_over_size, neg_beta, k, &tables,
-                            finish);
-  }
 }
 
 // ---- any window up to kLrnMaxSize channels: the window lives in LDS ----
@@ -264,10 +296,21 @@ extern "C" int shdw_hip_lrn(const int* in_shape, int size, float alpha, float be
   hipStream_t st = static_cast<hipStream_t>(stream);
   const uint32_t grid = grid_for(positions), chan = static_cast<uint32_t>(channels);
   const FastDiv f_step = make_fastdiv(step);
+  if (size <= 7) {
+    const dim3 share((positions + kWave - 1) / kWave);
+#define SHDW_LRN(S) \
+  lrn_window_kernel<S><<<share, kBlock, 0, st>>>(x, y, positions, step, chan, alpha_over_size, -beta, k, f_step)
+    if (size == 1) SHDW_LRN(1);
+    else if (size == 3) SHDW_LRN(3);
+    else if (size == 5) SHDW_LRN(5);
+    else SHDW_LRN(7);
+#undef SHDW_LRN
+    return launch_status();
+  }
   // A tensor with few positions has few waves, and each walks all the channels one round after
   // the other (82 us for 256 channels, however few the waves).  Up to eight workgroups then share
   // the rounds of a position, about 4096 waves in all and four rounds each at the least; measured
-  // on 12.8 M elements: [16,256,56,56] (784 waves) 82 -> 65, 56, 60, 77 us with 2, 4, 8, 16 shares,
+  // on 12.8 M elements, with windows in registers: [16,256,56,56] (784 waves) 82 -> 65, 56, 60, 77 us with 2, 4, 8, 16 shares,
   // [44,96,55,55] (2080 waves) 49 -> 42, 47, 55; [64,256,56,56] (3136 waves) 141 -> 139, 149.
   // In place a workgroup would overwrite what another still has to read: one share.
   const uint32_t waves = (positions + kWave - 1) / kWave;
@@ -277,21 +320,8 @@ extern "C" int shdw_hip_lrn(const int* in_shape, int size, float alpha, float be
   shares = shares > most ? most : shares;
   shares = shares > rounds / 4 ? rounds / 4 : shares;
   if (x == y || shares < 1) shares = 1;
-#define SHDW_LRN(S) \
-  lrn_window_kernel<S><<<dim3(grid, shares), kBlock, 0, st>>>(x, y, positions, step, chan, f_step, alpha_over_size, -beta, k)
-  if (size == 1) {
-    SHDW_LRN(1);
-  } else if (size == 3) {
-    SHDW_LRN(3);
-  } else if (size == 5) {
-    SHDW_LRN(5);
-  } else if (size == 7) {
-    SHDW_LRN(7);
-  } else {
-    const size_t lds = static_cast<size_t>(size) * kBlock * sizeof(float);
-    lrn_across_channels_kernel<<<dim3(grid, shares), kBlock, lds, st>>>(x, y, positions, step, chan, f_step,
-                                                          static_cast<uint32_t>(size), alpha_over_size, -beta, k);
-  }
-#undef SHDW_LRN
+  const size_t lds = static_cast<size_t>(size) * kBlock * sizeof(float);
+  lrn_across_channels_kernel<<<dim3(grid, shares), kBlock, lds, st>>>(x, y, positions, step, chan, f_step,
+                                                        static_cast<uint32_t>(size), alpha_over_size, -beta, k);
   return launch_status();
 }

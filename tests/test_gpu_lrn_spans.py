@@ -1,0 +1,36 @@
+"""LRN with windows of one to seven channels: four waves of a workgroup share the channels of 64
+positions, eight each, and hand the running sum on."""
+import numpy as np
+import pytest
+
+import oracle
+from tests import gpuops
+from tests.helpers import assert_bit_exact, normal
+
+pytestmark = pytest.mark.gpu
+
+
+# channels either side of a round, of a span of four and of whole spans; positions either side of a wave
+@pytest.mark.parametrize("channels", [3, 7, 8, 9, 10, 24, 31, 32, 33, 34, 63, 66, 97, 129])
+@pytest.mark.parametrize("positions", [1, 63, 65, 130])
+@pytest.mark.parametrize("size", [1, 3, 5, 7])
+def test_lrn_spans(gpu, channels, positions, size):
+    shape = (2, channels, 1, positions)
+    x = normal(channels + size, 2 * channels * positions, 4.0)
+    want = oracle.lrn(x, shape, size, 1e-2, 0.75, 1.0)[0]
+    assert_bit_exact(gpuops.lrn(x, shape, size, 1e-2, 0.75, 1.0), want, "lrn")
+    assert_bit_exact(gpuops.lrn(x, shape, size, 1e-2, 0.75, 1.0, inplace=True), want, "lrn in place")
+
+
+@pytest.mark.parametrize("channels", [9, 35, 70])
+def test_lrn_spans_of_special_values(gpu, channels):
+    shape = (1, channels, 5, 30)
+    x = normal(channels, channels * 150, 1.0).reshape(channels, 150).copy()
+    x[channels // 2, :40] = np.inf
+    x[0, 30:60] = np.nan
+    x[channels - 1, 50:90] = 1e30
+    x[:, 100:] = 0.0
+    with np.errstate(all="ignore"):
+        for k in (1.0, 0.0, -0.5):
+            want = oracle.lrn(x, shape, 5, 1e-1, 0.75, k)[0]
+            assert_bit_exact(gpuops.lrn(x, shape, 5, 1e-1, 0.75, k), want, "k = %g" % k)
