@@ -87,7 +87,7 @@ __global__ __launch_bounds__(kWave) void softmax_columns_kernel(const float* x, 
 #pragma unroll
     for (int u = 0; u < kColumnBatch; ++u) v[u] = xc[static_cast<uint64_t>(c0 + u) * inner];
 #pragma unroll
-    for (int u = 0; u < kColumnBatch; ++u) v[u] = libm::exact_expf(v[u] - max_val, tab);
+    for (int u = 0; u < kColumnBatch; ++u) v[u] = libm::exact_expf_nonpositive(v[u] - max_val, tab);
 #pragma unroll
     for (int u = 0; u < kColumnBatch; ++u) {
       yc[static_cast<uint64_t>(c0 + u) * inner] = v[u];
@@ -102,7 +102,7 @@ __global__ __launch_bounds__(kWave) void softmax_columns_kernel(const float* x, 
 #pragma unroll
     for (int u = 0; u < kColumnBatch; ++u) {
       if (c0 + u < dim) {
-        const float e = libm::exact_expf(v[u] - max_val, tab);
+        const float e = libm::exact_expf_nonpositive(v[u] - max_val, tab);
         yc[static_cast<uint64_t>(c0 + u) * inner] = e;
         sum += e;
       }
@@ -163,7 +163,7 @@ __global__ __launch_bounds__(kBlock) void softmax_columns_reg_kernel(const float
 #pragma unroll
   for (int c = 0; c < DMAX; ++c) {
     if (c < DFULL || c < dim) {
-      v[c] = libm::exact_expf(v[c] - max_val, tab);
+      v[c] = libm::exact_expf_nonpositive(v[c] - max_val, tab);
       sum += v[c];
     }
   }
@@ -273,21 +273,60 @@ SHDW_DEVICE float block_max_any_order(float m, float* scratch4) {
   return m;
 }
 
-// Front-to-back sum of lds[0..n) by the calling lane, 128-bit LDS reads.
-template <class ACC>
-SHDW_DEVICE ACC sequential_sum(const float* lds, uint32_t n) {
-  ACC sum = 0;
+// Front-to-back fp32 sum of lds[0..n) by a whole wave, the result in all its lanes: a lane holds 16
+// consecutive elements of a chunk of 1024 and the sum goes from lane to lane, as in
+// pool_rows_stream_kernel (by one lane out of LDS, eight 128-bit reads at a time, softmax of [16,1000]
+// takes 7.2 us, so 5.6; [8192,4096] 120 and 99).  lds is 16-byte aligned and readable up to the next multiple of four.
+SHDW_DEVICE float wave_ordered_sum(const float* lds, uint32_t n) {
+  constexpr uint32_t kSpan = 16, kChunk = kWave * kSpan;
+  const uint32_t lane = threadIdx.x % kWave;
+  float sum = 0.f;
+  for (uint32_t c0 = 0; c0 < n; c0 += kChunk) {
+    const uint32_t first = c0 + lane * kSpan, last = (n - 1) & ~3u;
+    float v[kSpan];
+#pragma unroll
+    for (uint32_t k = 0; k < kSpan; k += 4) {
+      const v4f q = *reinterpret_cast<const v4f*>(lds + min(first + k, last));
+#pragma unroll
+      for (uint32_t j = 0; j < 4; ++j) v[k + j] = first + k + j < n ? q[j] : 0.f;  // a sum that starts at +0 stays as it is
+    }
+    const uint32_t turns = min(static_cast<uint32_t>(kWave), (n - c0 + kSpan - 1) / kSpan);
+    auto turn = [&]() {
+#pragma unroll
+      for (uint32_t k = 0; k < kSpan; ++k) sum += v[k];
+    };
+    turn();
+    uint32_t t = 1;
+    for (; t + 4 <= turns; t += 4) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        sum = dpp_f32<kDppWaveShr1>(sum);
+        turn();
+      }
+    }
+    for (; t < turns; ++t) {
+      sum = dpp_f32<kDppWaveShr1>(sum);
+      turn();
+    }
+    sum = __shfl(sum, turns - 1);
+  }
+  return sum;
+}
+
+// Front-to-back fp64 sum of lds[0..n) by the calling lane, 128-bit LDS reads.
+SHDW_DEVICE double sequential_sum(const float* lds, uint32_t n) {
+  double sum = 0;
   const v4f* l4 = reinterpret_cast<const v4f*>(lds);
   const uint32_t q = n / 4;
 #pragma unroll 8
   for (uint32_t c = 0; c < q; ++c) {
     const v4f v = l4[c];
-    sum += static_cast<ACC>(v[0]);
-    sum += static_cast<ACC>(v[1]);
-    sum += static_cast<ACC>(v[2]);
-    sum += static_cast<ACC>(v[3]);
+    sum += static_cast<double>(v[0]);
+    sum += static_cast<double>(v[1]);
+    sum += static_cast<double>(v[2]);
+    sum += static_cast<double>(v[3]);
   }
-  for (uint32_t c = 4 * q; c < n; ++c) sum += static_cast<ACC>(lds[c]);
+  for (uint32_t c = 4 * q; c < n; ++c) sum += static_cast<double>(lds[c]);
   return sum;
 }
 
@@ -314,12 +353,20 @@ __global__ __launch_bounds__(kBlock) void softmax_slab_kernel(const float* x, fl
     float m = -FLT_MAX;
     for (uint32_t t = threadIdx.x; t < slab; t += kBlock) m = std_max(lds[t], m);
     m = block_max_any_order(m, wave_max);
-    for (uint32_t t = threadIdx.x; t < slab; t += kBlock) lds[t] = libm::exact_expf(lds[t] - m, tab);
+    for (uint32_t t = threadIdx.x; t < slab; t += kBlock) lds[t] = libm::exact_expf_nonpositive(lds[t] - m, tab);
     __syncthreads();
-    if (threadIdx.x == 0) stat[0] = sequential_sum<float>(lds, slab);
+    if (threadIdx.x < kWave) {
+      const float sum = wave_ordered_sum(lds, slab);
+      if (threadIdx.x == 0) wave_max[0] = sum;  // behind the barrier everyone has read the maxima
+    }
     __syncthreads();
-    const float sum = stat[0];
-    for (uint32_t t = threadIdx.x; t < slab; t += kBlock) ys[t] = lds[t] / sum;
+    const float sum = wave_max[0];
+    const double recip = reciprocal(sum);
+    for (uint32_t t = threadIdx.x; t < slab; t += kBlock) {
+      float q[1] = {lds[t]};
+      quotients(q, [&](int) { return sum; }, [&](int) { return recip; });
+      ys[t] = q[0];
+    }
     return;
   }
   // inner < 64 here.  The maxima in any order as well (a NaN in a column makes all
@@ -345,7 +392,7 @@ __global__ __launch_bounds__(kBlock) void softmax_slab_kernel(const float* x, fl
   __syncthreads();
   for (uint32_t t = threadIdx.x; t < slab; t += kBlock) {
     const uint32_t s = t - fd_div(t, f_inner) * inner;
-    lds[t] = libm::exact_expf(lds[t] - stat[s], tab);
+    lds[t] = libm::exact_expf_nonpositive(lds[t] - stat[s], tab);
   }
   __syncthreads();
   if (threadIdx.x < inner) {
@@ -566,7 +613,7 @@ __global__ __launch_bounds__(kBlock) void softmax_quads_reg_kernel(const float* 
     if (c < dim) {
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
-        v[c][k] = libm::exact_expf(v[c][k] - max_val[k], tab);
+        v[c][k] = libm::exact_expf_nonpositive(v[c][k] - max_val[k], tab);
         sum[k] += v[c][k];
       }
     }
@@ -629,7 +676,7 @@ __global__ __launch_bounds__(kBlock) void normalize_slab_kernel(const float* x, 
   stage_slab(lds, xs, slab, [p](float v) { return static_cast<float>(norm_term<PMODE>(v, p)); });
   __syncthreads();
   if (inner == 1) {
-    if (threadIdx.x == 0) stat[0] = norm_finish<PMODE>(sequential_sum<double>(lds, slab), p, eps);
+    if (threadIdx.x == 0) stat[0] = norm_finish<PMODE>(sequential_sum(lds, slab), p, eps);
   } else {
     if (threadIdx.x < inner) {  // inner < 64 here
       double acc = 0;
@@ -817,7 +864,7 @@ __global__ __launch_bounds__(kBlock) void softmax_packed_kernel(const float* x, 
     stat[q] = m;
   }
   __syncthreads();
-  packed_update(lds, sp, [&](float v, uint32_t cq, uint32_t) { return libm::exact_expf(v - stat[cq], tab); });
+  packed_update(lds, sp, [&](float v, uint32_t cq, uint32_t) { return libm::exact_expf_nonpositive(v - stat[cq], tab); });
   __syncthreads();
   if (q < sp.ncols) {
     float sum = 0.f;
@@ -1268,11 +1315,10 @@ static void launch_softmax_tile_ts(int outer_num, int dim, int inner_num, const 
 // kernels) a CU has eight such walks in flight and 255 of 256 lanes wait for
 // each.  Here every wave works by itself, without a barrier, on R consecutive
 // rows (R a power of two, R * pitch floats of LDS: one contiguous piece of x):
-// all 64 lanes stage them, 64 / R lanes share a row for the maximum (any order,
-// see softmax_slab_kernel), the exponentials and the division, the first lane
-// of each row adds it up front to back, and the piece goes back as it came.  A
-// wave never waits for another, so a CU has 8 or 16 of them, each with R walks,
-// at different points of their work.  The four waves of a workgroup exist for
+// all 64 lanes stage them, 64 / R lanes share a row for the elementwise part, the
+// row is added up front to back, and the piece goes back as it came.  A wave never
+// waits for another, so a CU has 8 or 16 of them, each with R walks, at different
+// points of their work.  The four waves of a workgroup exist for
 // their placement, one per SIMD (see pool_rows_stream_kernel).
 // ---------------------------------------------------------------------------
 constexpr uint32_t kRowsMinDim = 17;
@@ -1398,7 +1444,7 @@ __global__ __launch_bounds__(kBlock) void softmax_short_rows_kernel(const float*
         for (uint32_t c = 0; c < dim; ++c) m = std_max(col[c * inner], m);
         float sum = 0.f;
         for (uint32_t c = 0; c < dim; ++c) {
-          const float v = libm::exact_expf(col[c * inner] - m, tab);
+          const float v = libm::exact_expf_nonpositive(col[c * inner] - m, tab);
           col[c * inner] = v;
           sum += v;
         }
@@ -1415,7 +1461,7 @@ __global__ __launch_bounds__(kBlock) void softmax_short_rows_kernel(const float*
     float sum = 0.f;
 #pragma unroll
     for (int c = 0; c < D; ++c) {
-      e[c] = libm::exact_expf(e[c] - m, tab);
+      e[c] = libm::exact_expf_nonpositive(e[c] - m, tab);
       sum += e[c];
     }
 #pragma unroll
@@ -1430,39 +1476,107 @@ __global__ __launch_bounds__(kBlock) void softmax_short_rows_kernel(const float*
   if (lane < 3 && rest < cells) ys[rest] = tile[place(rest)];
 }
 
-template <int TILE>
-__global__ __launch_bounds__(kBlock) void softmax_rows_kernel(const float* x, float* y, uint32_t rows, WaveRows w) {
-  __shared__ __align__(16) float tiles[kBlock / kWave][TILE];
-  __shared__ float stats[kBlock / kWave][kWave];
+// Softmax: the lanes of a row hold `span` consecutive elements each, in registers from the maximum
+// to the quotients, side by side (one exponential after the other, each waiting for its value from
+// LDS and its table entry, took most of a wave's time).  The ordered sum goes from lane to lane, as
+// in pool_rows_stream_kernel.  The wave's piece passes through LDS on the way in and out, since a
+// lane's share of it starts anywhere; rows of an odd length lie there as they do in memory
+// (WHOLE: moved 128 bits at a time), others one element apart, and a span is odd too, so that
+// neighbouring lanes meet different banks.
+// [139712,21,1], 23.5 MB: 11.7 -> 8.5 us; [600000,21,1] 33.4 -> 24.7, [4096,1000,1] 20.9 -> 16.2,
+// [262144,49,1] 30.6 -> 25.6.
+constexpr int kRowsSpan = 36;  // at most: 1023 elements over 32 lanes, made odd
+
+template <bool WHOLE>
+__global__ __launch_bounds__(kBlock, 4) void softmax_rows_kernel(const float* x, float* y, uint32_t rows, uint32_t span,
+                                                              uint32_t tile_floats, WaveRows w) {
+  extern __shared__ __align__(16) float lds[];
   __shared__ uint64_t tab[32];
   if (threadIdx.x < 32) tab[threadIdx.x] = libm::kExp2fTab[threadIdx.x];
   __syncthreads();  // the only one: from here on every wave is on its own
-  const uint32_t lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-  float* tile = tiles[wave];
-  float* stat = stats[wave];
+  const uint32_t lane = threadIdx.x % kWave;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  float* tile = lds + wave * tile_floats;
   const uint32_t row0 = (blockIdx.x * (kBlock / kWave) + wave) * w.rows_per_wave;
   if (row0 >= rows) return;  // the whole wave
   const uint32_t nrows = min(w.rows_per_wave, rows - row0), cells = nrows * w.dim;
   const uint64_t base = static_cast<uint64_t>(row0) * w.dim;
-  rows_stage_in(tile, x + base, cells, w, lane);
-  __builtin_amdgcn_wave_barrier();
-  const uint32_t group = 1u << w.group_log2;
-  const uint32_t r = lane >> w.group_log2, sub = lane & (group - 1);
-  float* mine = tile + (r < nrows ? r : 0) * w.pitch;  // rows past the end: their lanes read row 0 and write nothing
-  float m = -FLT_MAX;
-  for (uint32_t c = sub; c < w.dim; c += group) m = std_max(mine[c], m);
-  for (uint32_t off = 1; off < group; off <<= 1) m = std_max(__shfl_xor(m, off), m);  // all 64 lanes are here
-  __builtin_amdgcn_wave_barrier();
-  if (r < nrows)
-    for (uint32_t c = sub; c < w.dim; c += group) mine[c] = libm::exact_expf(mine[c] - m, tab);
-  __builtin_amdgcn_wave_barrier();
-  if (sub == 0 && r < nrows) {
-    float sum = 0.f;
-    walk_column(mine, 1, w.dim, [&](float a) { sum += a; });
-    stat[r] = sum;
+  const uint32_t nvec = cells / 4, rest = 4 * nvec + lane;  // 17 elements and more: a vector at least
+  constexpr int kMost = 8;                                  // vectors of a lane: 2048 floats a wave at most
+  if (WHOLE) {
+    v4f reg[kMost];
+#pragma unroll
+    for (int k = 0; k < kMost; ++k)
+      if (k * kWave < nvec) reg[k] = load4_stream_any(x + base + 4 * min(k * kWave + lane, nvec - 1));
+#pragma unroll
+    for (int k = 0; k < kMost; ++k)
+      if (k * kWave + lane < nvec) *reinterpret_cast<v4f*>(tile + 4 * (k * kWave + lane)) = reg[k];
+    if (rest < cells) tile[rest] = x[base + rest];
+  } else {
+    rows_stage_in(tile, x + base, cells, w, lane);
   }
   __builtin_amdgcn_wave_barrier();
-  rows_stage_out(tile, y + base, cells, w, lane, [&](float e, uint32_t rr, uint32_t) { return e / stat[rr]; });
+  const uint32_t group = 1u << w.group_log2, r = lane >> w.group_log2, sub = lane & (group - 1);
+  const uint32_t c0 = sub * span;
+  const uint32_t n = r < nrows && c0 < w.dim ? min(span, w.dim - c0) : 0u;  // elements of this lane
+  // lanes without any read row 0, which does not matter; a span is read in whole fours, past the row's end
+  float* mine = tile + (n ? r * w.pitch + c0 : 0u);
+  float v[kRowsSpan];
+#pragma unroll
+  for (int k = 0; k < kRowsSpan; k += 4) {
+    if (k >= span) continue;
+#pragma unroll
+    for (int j = k; j < k + 4; ++j) v[j] = j < n ? mine[j] : -__builtin_inff();  // its exponential is 0, which adds nothing
+  }
+  float m = -FLT_MAX;
+#pragma unroll
+  for (int k = 0; k < kRowsSpan; k += 4) {
+    if (k >= span) continue;
+    m = max3_any_order(m, v[k], v[k + 1]);
+    m = max3_any_order(m, v[k + 2], v[k + 3]);
+  }
+  if (group >= 2) m = max3_any_order(m, m, dpp_f32<kDppXor1>(m));
+  if (group >= 4) m = max3_any_order(m, m, dpp_f32<kDppXor2>(m));
+  if (group >= 8) m = max3_any_order(m, m, dpp_f32<kDppHalfMirror>(m));
+  if (group >= 16) m = max3_any_order(m, m, dpp_f32<kDppMirror>(m));
+  if (group >= 32) m = max3_any_order(m, m, __shfl_xor(m, 16));
+#pragma unroll
+  for (int k = 0; k < kRowsSpan; k += 4) {
+    if (k >= span) continue;
+#pragma unroll
+    for (int j = k; j < k + 4; ++j) v[j] = libm::exact_expf_nonpositive(v[j] - m, tab);
+  }
+  float sum = 0.f;
+  const uint32_t turns = (w.dim + span - 1) / span;
+  for (uint32_t t = 0; t < turns; ++t) {
+    if (t > 0) sum = dpp_f32<kDppWaveShr1>(sum);
+#pragma unroll
+    for (int k = 0; k < kRowsSpan; k += 4) {
+      if (k >= span) continue;
+#pragma unroll
+      for (int j = k; j < k + 4; ++j) sum += v[j];
+    }
+  }
+  if (group > 1) sum = __shfl(sum, (lane & ~(group - 1)) + turns - 1);
+  const double recip = reciprocal(sum);
+#pragma unroll
+  for (int k = 0; k < kRowsSpan; k += 4) {
+    if (k >= span) continue;
+    const v4f q = quotients4(v4f{v[k], v[k + 1], v[k + 2], v[k + 3]}, sum, recip);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (k + j < n) mine[k + j] = q[j];
+  }
+  __builtin_amdgcn_wave_barrier();
+  if (WHOLE) {
+#pragma unroll
+    for (int k = 0; k < kMost; ++k)
+      if (k * kWave + lane < nvec)
+        store4_stream_any(y + base + 4 * (k * kWave + lane), *reinterpret_cast<const v4f*>(tile + 4 * (k * kWave + lane)));
+    if (rest < cells) y[base + rest] = tile[rest];
+  } else {
+    rows_stage_out(tile, y + base, cells, w, lane, [](float e, uint32_t, uint32_t) { return e; });
+  }
 }
 
 // PMODE 1, 2 (Normalize) and 3 (SSDNormalize per position); the terms of the sum are formed by the walking lane.
@@ -1505,6 +1619,27 @@ static bool wave_rows(int dim, WaveRows* w) {
   while ((r << w->group_log2) < kWave) ++w->group_log2;
   w->f_dim = make_fastdiv(d);
   return true;
+}
+
+// More waves where there are few: 32 rows a wave instead of 64 under 8192 waves, and from there half as
+// many, down to four, while there are not 1024.  With 64 / 32 / 16 / 8 / 4 rows a wave: [31768,21]
+// 6.2 / 5.2 / 5.0 / 6.1 / 8.9 us, [139712,21] 9.5 / 8.5 / 10.6 / 16.5 / 29.6, [1500000,24] 59 / 73 / 94;
+// with 16 / 8 / 4 [2000,91] 6.3 / 5.9 / 5.4, [1024,64] 6.1 / 5.5 / 5.2.
+static void fewer_rows_per_wave(uint32_t rows, WaveRows* w) {
+  auto fewer = [&](uint32_t least_rows, uint32_t waves) {
+    while (w->rows_per_wave > least_rows && rows / w->rows_per_wave < waves) w->rows_per_wave /= 2, ++w->group_log2;
+  };
+  fewer(32, 8192);
+  fewer(4, 1024);
+}
+
+static void launch_softmax_rows(uint32_t rows, const WaveRows& w, uint32_t grid, const float* x, float* y, hipStream_t st) {
+  const uint32_t group = 1u << w.group_log2;
+  const uint32_t span = group > 1 ? ((w.dim + group - 1) / group) | 1u : w.dim;
+  const uint32_t tile = (w.rows_per_wave * w.pitch + kRowsSpan + 3) & ~3u;  // a lane's last four may lie behind the last row
+  const size_t bytes = static_cast<size_t>(kBlock / kWave) * tile * sizeof(float);
+  if (w.pitch == w.dim) softmax_rows_kernel<true><<<grid, kBlock, bytes, st>>>(x, y, rows, span, tile, w);
+  else softmax_rows_kernel<false><<<grid, kBlock, bytes, st>>>(x, y, rows, span, tile, w);
 }
 
 // ---------------------------------------------------------------------------
@@ -1818,7 +1953,7 @@ __global__ __launch_bounds__(kBlock) void softmax_tall_kernel(const float* x, fl
       if (t.has(k, i)) {
         v4f ex;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) ex[e] = libm::exact_expf(reg[i][e] - max_val[e], tab);
+        for (int e = 0; e < 4; ++e) ex[e] = libm::exact_expf_nonpositive(reg[i][e] - max_val[e], tab);
         *reinterpret_cast<v4f*>(buf + t.slot(i)) = ex;
       }
     __syncthreads();
@@ -1848,7 +1983,7 @@ __global__ __launch_bounds__(kBlock) void softmax_tall_kernel(const float* x, fl
         if (t.has(k + j, i)) {
           v4f q;
 #pragma unroll
-          for (int e = 0; e < 4; ++e) q[e] = libm::exact_expf(w[j][i][e] - max_val[e], tab) / total[e];
+          for (int e = 0; e < 4; ++e) q[e] = libm::exact_expf_nonpositive(w[j][i][e] - max_val[e], tab) / total[e];
           t.store(y, t.row(k + j, i), q);
         }
   }
@@ -2042,7 +2177,7 @@ __global__ __launch_bounds__(kBlock) void softmax_long_slab_kernel(const float* 
     for (int i = 0; i < kLongLoads; ++i) {
       v4f ex;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) ex[j] = libm::exact_expf(reg[i][j] - max_val[i][j], tab);
+      for (int j = 0; j < 4; ++j) ex[j] = libm::exact_expf_nonpositive(reg[i][j] - max_val[i][j], tab);
       *reinterpret_cast<v4f*>(buf + LongSlab::first(i)) = ex;  // slots past the chunk's cells are never walked
     }
     __syncthreads();
@@ -2067,7 +2202,7 @@ __global__ __launch_bounds__(kBlock) void softmax_long_slab_kernel(const float* 
   for (uint32_t k = 0; k < chunks; k += 2) {
     t.load(k, v);
     t.load(k + 1, v2);
-    auto quotient = [&](float a, int i, int j) { return libm::exact_expf(a - max_val[i][j], tab) / total[i][j]; };
+    auto quotient = [&](float a, int i, int j) { return libm::exact_expf_nonpositive(a - max_val[i][j], tab) / total[i][j]; };
     t.store(k, v, quotient);
     t.store(k + 1, v2, quotient);
   }
@@ -2224,7 +2359,7 @@ static int column_geometry(int outer_num, int dim, int inner_num, ColumnGeometry
   g->columns = static_cast<uint32_t>(columns);
   const int64_t slab = static_cast<int64_t>(dim) * inner_num;
   g->use_slab = inner_num < 64 && slab + inner_num <= kSlabMaxFloats;
-  g->slab_bytes = static_cast<uint32_t>((slab + inner_num) * sizeof(float));
+  g->slab_bytes = static_cast<uint32_t>((slab + inner_num + 3) / 4 * 4 * sizeof(float));  // whole vectors: wave_ordered_sum
   return SHDW_OK;
 }
 
@@ -2264,8 +2399,9 @@ static int run_softmax(int outer_num, int dim, int inner_num, const float* x, fl
   if (WaveRows w; rows_apply(outer_num, dim, inner_num) && dim <= kRowsSoftmaxMaxDim &&
                   wave_rows<kRowsSmallTile>(dim, &w)) {
     const uint32_t rows = static_cast<uint32_t>(outer_num);
+    fewer_rows_per_wave(rows, &w);
     if (pl->chosen(SHDW_PATH_ROWS, static_cast<int>(w.rows_per_wave), rows_grid(rows, w))) return SHDW_OK;
-    softmax_rows_kernel<kRowsSmallTile><<<pl->grid, kBlock, 0, st>>>(x, y, rows, w);
+    launch_softmax_rows(rows, w, pl->grid, x, y, st);
     return launch_status();
   }
   // slabs with inner > 1 walk their columns in loops, one exponential after the other: ahead of the packed
@@ -2292,7 +2428,11 @@ static int run_softmax(int outer_num, int dim, int inner_num, const float* x, fl
     softmax_quads_reg_kernel<kQuadMaxDim><<<pl->grid, kBlock, 0, st>>>(x, y, quads, d, inner, fq);
     return launch_status();
   }
-  if (const uint32_t group = packed_group(dim, inner_num)) {
+  // Fewer rows than the forms above take: a workgroup each, whose lanes share the row, where the packed
+  // kernel walks a row with one lane for the maximum and one for the sum ([1,256,1] 3.3 us against 7.0, [256,64,1]
+  // 3.3 / 16.3, [1000,200,1] 4.1 / 19.8, [1000,18,1] 3.7 / 8.1).
+  const bool few_rows = inner_num == 1 && outer_num < kRowsMinRows && g.use_slab;
+  if (const uint32_t group = few_rows ? 0u : packed_group(dim, inner_num)) {
     const uint32_t slabs = static_cast<uint32_t>(outer_num);
     if (pl->chosen(SHDW_PATH_PACKED, static_cast<int>(group), (slabs + group - 1) / group)) return SHDW_OK;
     softmax_packed_kernel<<<pl->grid, kBlock, packed_bytes(dim, inner_num, group), st>>>(
