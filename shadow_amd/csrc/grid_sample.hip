@@ -61,6 +61,10 @@ __global__ __launch_bounds__(kBlock) void grid_sample_kernel(const float* x, con
   const size_t in_plane = static_cast<size_t>(in_h) * in_w;
   const float* src = x + (static_cast<size_t>(b) * channel + c0) * in_plane;
   float* dst = y + (static_cast<size_t>(b) * channel + c0) * out_plane + s;
+  // Stores carry the streams' hint, and the reads of a whole share of channels are under way before
+  // the first of them is used: bilinear [64,256,56,56] 119 -> 68.5 us, [8,64,112,112] 12.6 -> 11.0,
+  // of which the reads' part is 119 -> 107 and 12.6 -> 12.0.
+  const auto store = [&](int c, float v) { __builtin_nontemporal_store(v, dst + static_cast<size_t>(c) * out_plane); };
   const float src_h_f = (gy + 1) / 2.f * static_cast<float>(in_h - 1);
   const float src_w_f = (gx + 1) / 2.f * static_cast<float>(in_w - 1);
   if (MODE == 0) {
@@ -68,9 +72,14 @@ __global__ __launch_bounds__(kBlock) void grid_sample_kernel(const float* x, con
     int src_w = to_int_as_x86(__builtin_roundf(src_w_f));
     const bool outside = PAD == 0 && (src_h < 0 || src_w < 0 || src_h > in_h - 1 || src_w > in_w - 1);
     const size_t cell = static_cast<size_t>(clamp_index(src_h, in_h)) * in_w + clamp_index(src_w, in_w);
-    for (int c = 0; c < count; ++c) {
-      const float v = src[c * in_plane + cell];
-      dst[static_cast<size_t>(c) * out_plane] = outside ? 0.f : v;
+    if (count == kGridChannels) {
+      float v[kGridChannels];
+#pragma unroll
+      for (int c = 0; c < kGridChannels; ++c) v[c] = src[c * in_plane + cell];
+#pragma unroll
+      for (int c = 0; c < kGridChannels; ++c) store(c, outside ? 0.f : v[c]);
+    } else {
+      for (int c = 0; c < count; ++c) store(c, outside ? 0.f : src[c * in_plane + cell]);
     }
     return;
   }
@@ -96,15 +105,22 @@ __global__ __launch_bounds__(kBlock) void grid_sample_kernel(const float* x, con
     const int left = w0 < in_w - 2 ? w0 : in_w - 2;
     const bool w0_first = w0 == left, w1_first = w1 == left;
     const size_t r0 = static_cast<size_t>(h0) * in_w + left, r1 = static_cast<size_t>(h1) * in_w + left;
-    for (int c = 0; c < count; ++c) {
-      const float* plane = src + c * in_plane;
-      const v2f_unaligned top = *reinterpret_cast<const v2f_unaligned*>(plane + r0);
-      const v2f_unaligned bottom = *reinterpret_cast<const v2f_unaligned*>(plane + r1);
+    const auto finish = [&](int c, v2f_unaligned top, v2f_unaligned bottom) {
       const float v0 = w0_first ? top[0] : top[1], v1 = w0_first ? bottom[0] : bottom[1];
       const float v2 = w1_first ? top[0] : top[1], v3 = w1_first ? bottom[0] : bottom[1];
       float v = k0 * v0 + k1 * v1 + k2 * v2 + k3 * v3;
       v = nan ? __builtin_nanf("") : v;
-      dst[static_cast<size_t>(c) * out_plane] = outside ? 0.f : v;
+      store(c, outside ? 0.f : v);
+    };
+    const auto pair = [&](int c, size_t at) { return *reinterpret_cast<const v2f_unaligned*>(src + c * in_plane + at); };
+    if (count == kGridChannels) {  // all of a lane's reads under way at once
+      v2f_unaligned top[kGridChannels], bottom[kGridChannels];
+#pragma unroll
+      for (int c = 0; c < kGridChannels; ++c) top[c] = pair(c, r0), bottom[c] = pair(c, r1);
+#pragma unroll
+      for (int c = 0; c < kGridChannels; ++c) finish(c, top[c], bottom[c]);
+    } else {
+      for (int c = 0; c < count; ++c) finish(c, pair(c, r0), pair(c, r1));
     }
     return;
   }
@@ -114,7 +130,7 @@ __global__ __launch_bounds__(kBlock) void grid_sample_kernel(const float* x, con
     const float* plane = src + c * in_plane;
     float v = k0 * plane[i0] + k1 * plane[i1] + k2 * plane[i2] + k3 * plane[i3];
     v = nan ? __builtin_nanf("") : v;
-    dst[static_cast<size_t>(c) * out_plane] = outside ? 0.f : v;
+    store(c, outside ? 0.f : v);
   }
 }
 
