@@ -138,7 +138,10 @@ SHDW_DEVICE float lrn_walk(const float (&own)[kLrnRound], const float (&prev)[SI
   return accum;
 }
 
-template <int SIZE>
+// STREAM: the stores carry the streams' hint; not where rows of positions start inside a vector, whose
+// pieces of lines would leave one by one ([44,96,55,55] 32.6 us plain, 34.0 with it, [68,256,27,27] 35.0
+// and 40.5; [64,256,56,56] 93.2 and 82.1, [256,64,14,14] 11.8 and 10.5).
+template <int SIZE, bool STREAM>
 __global__ __launch_bounds__(kBlock, 5) void lrn_window_kernel(const float* x, float* y, uint32_t positions, uint32_t step,
                                                                uint32_t channels, float alpha_over_size, float neg_beta,
                                                                float k, FastDiv f_step) {
@@ -199,7 +202,11 @@ __global__ __launch_bounds__(kBlock, 5) void lrn_window_kernel(const float* x, f
     for (int j = 0; j < SEG; ++j) {
       const float centre = j >= static_cast<int>(post) ? own[j >= static_cast<int>(post) ? j - post : 0]
                                                        : prev[j < static_cast<int>(post) ? SIZE - post + j : 0];
-      if (c0 + j < channels && p < positions) out[static_cast<size_t>(c0 + j) * step] = centre * power[j];
+      if (c0 + j < channels && p < positions) {
+        float* to = out + static_cast<size_t>(c0 + j) * step;
+        if (STREAM) __builtin_nontemporal_store(centre * power[j], to);
+        else *to = centre * power[j];
+      }
     }
   }
 }
@@ -298,8 +305,10 @@ extern "C" int shdw_hip_lrn(const int* in_shape, int size, float alpha, float be
   const FastDiv f_step = make_fastdiv(step);
   if (size <= 7) {
     const dim3 share((positions + kWave - 1) / kWave);
-#define SHDW_LRN(S) \
-  lrn_window_kernel<S><<<share, kBlock, 0, st>>>(x, y, positions, step, chan, alpha_over_size, -beta, k, f_step)
+    const bool stream = step % 4 == 0 && aligned16(y);
+#define SHDW_LRN(S)                                                                                                             \
+  stream ? lrn_window_kernel<S, true><<<share, kBlock, 0, st>>>(x, y, positions, step, chan, alpha_over_size, -beta, k, f_step) \
+         : lrn_window_kernel<S, false><<<share, kBlock, 0, st>>>(x, y, positions, step, chan, alpha_over_size, -beta, k, f_step)
     if (size == 1) SHDW_LRN(1);
     else if (size == 3) SHDW_LRN(3);
     else if (size == 5) SHDW_LRN(5);
