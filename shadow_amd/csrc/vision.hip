@@ -302,7 +302,7 @@ SHDW_DEVICE void band_windows(const float* tile, float* y, const BandArgs& p, co
         }
       }
       const int pool_size = (h_end_pad - h_first) * (w_end_pad - w_first);
-      dst[hl * p.out_w + w] = MAX ? max_val : sum_val / static_cast<float>(pool_size);
+      __builtin_nontemporal_store(MAX ? max_val : sum_val / static_cast<float>(pool_size), dst + (hl * p.out_w + w));
     }
   }
 }
@@ -386,7 +386,11 @@ SHDW_DEVICE void band_windows_wide(const float* tile, float* y, const BandArgs& 
 // A workgroup walks `bands_per_group` consecutive bands.  kBandVectors (every span
 // starts 16-byte aligned and in_w % 4 == 0): the next band's 128-bit loads are
 // issued into registers before the current band's windows are walked, so HBM
-// requests stay in flight during the LDS phase.  Otherwise the same with single
+// requests stay in flight during the LDS phase.  kBandSpan (any other rows, where no
+// window needs padding cells beside them, so that the tile is the span as it lies in memory):
+// the same from any dword address ([44,96,55,55] 3x3 by two 15.7 us with single floats, 14.5 so, its
+// average 16.6 and 14.6; before the outputs carried the streams' hint 16.6 and 18.4).
+// Otherwise the same with single
 // floats, as many a lane ahead as a band has, up to eight, and the rest of a longer
 // span behind them.  Lanes beyond a span take its last elements again: a branch
 // around each load has the compiler wait for the one before it.
@@ -396,7 +400,7 @@ SHDW_DEVICE void band_windows_wide(const float* tile, float* y, const BandArgs& 
 // [16,64,225,225] 3x3 at stride 1 132.8 / 122.2 us, [64,64,113,113] 5x5 at stride 1 134.8 / 125.6,
 // [16,64,225,225] 3x3 by two 55.0 / 52.0; [44,96,55,55] 3x3 by two 16.3 / 16.0 (a 37th shared:
 // left with the hint); under 24 MB [16,64,35,35] 3x3 at stride 1 5.8 / 6.1.
-enum { kBandVectors, kBandFloats, kBandFloatsKept };
+enum { kBandVectors, kBandSpan, kBandFloats, kBandFloatsKept };
 constexpr uint64_t kBandKeptBytes = 24u << 20;
 constexpr int kBandMaxRegs = kBandTileFloats / 4 / kBlock;  // vectors per lane for a full tile
 static_assert(kBandMaxRegs == 8, "the launch switch covers up to 8 staged vectors per lane");
@@ -411,25 +415,35 @@ __global__ __launch_bounds__(kBlock) void pool_band_kernel(const float* x, float
   const uint32_t g1 = min(g0 + p.bands_per_group, p.total_bands);
   {
     const float neutral = MAX ? -FLT_MAX : 0.f;
-    const uint32_t cells = static_cast<uint32_t>(p.tile_rows + 1) * p.pitch;  // multiple of 4
+    const uint32_t cells = static_cast<uint32_t>(p.tile_rows + 1) * p.pitch;  // up to three of the spare floats behind it too
     for (uint32_t t = 4 * threadIdx.x; t < cells; t += 4 * kBlock)
       *reinterpret_cast<v4f*>(tile + t) = v4f{neutral, neutral, neutral, neutral};
   }
   __syncthreads();
-  if (KIND == kBandVectors) {
+  if (KIND == kBandVectors || KIND == kBandSpan) {
     v4f reg[REGS];
     const auto request = [&](const BandSpan& bs) {
       if (bs.span == 0) return;  // every window of the band in the padding
 #pragma unroll
-      for (int k = 0; k < REGS; ++k) reg[k] = load4_stream(bs.src + min(4u * (k * kBlock + threadIdx.x), bs.span - 4));
+      for (int k = 0; k < REGS; ++k) {
+        const float* from = bs.src + min(4u * (k * kBlock + threadIdx.x), bs.span - 4);
+        reg[k] = KIND == kBandVectors ? load4_stream(from) : load4_stream_any(from);
+      }
     };
     BandSpan cur = band_span(p, x, g0);
     request(cur);
     for (uint32_t g = g0; g < g1; ++g) {
 #pragma unroll
       for (int k = 0; k < REGS; ++k) {
-        const uint32_t v = k * kBlock + threadIdx.x;
-        if (4 * v < cur.span) *reinterpret_cast<v4f*>(tile + band_slot(p, 4 * v)) = reg[k];
+        const uint32_t t = 4 * (k * kBlock + threadIdx.x);
+        if (KIND == kBandVectors) {
+          if (t < cur.span) *reinterpret_cast<v4f*>(tile + band_slot(p, t)) = reg[k];
+        } else if (t + 4 <= cur.span) {
+          *reinterpret_cast<v4f*>(tile + t) = reg[k];
+        } else if (t < cur.span) {  // the span's last four, of which the lane before wrote some
+#pragma unroll
+          for (int j = 0; j < 4; ++j) tile[cur.span - 4 + j] = reg[k][j];
+        }
       }
       __syncthreads();
       const BandSpan walk = cur;
@@ -486,11 +500,12 @@ static bool plan_pool_band(const PoolArgs& p, int target_outputs, BandArgs* a) {
   const int over_r = (p.out_w - 1) * p.sw - p.pw + p.kw - p.in_w;
   const int pad_l = (p.pw + 3) & ~3, pad_r = over_r > 0 ? (over_r + 3) & ~3 : 0;
   if (pad_l > kBandMaxPad || pad_r > kBandMaxPad) return false;
-  const int pitch = pad_l + ((p.in_w + 3) & ~3) + pad_r;
+  const bool wide = p.sw == 1 && p.kw >= kBandWideMinCols && p.out_w >= 16;
+  // without padding cells the tile is the span as it lies in memory (but for 128-bit reads of rows)
+  const int pitch = pad_l + pad_r == 0 && !wide ? p.in_w : pad_l + ((p.in_w + 3) & ~3) + pad_r;
   const int rows_cap = kBandTileFloats / pitch - 1;  // one row is the spare
   if (rows_cap < p.kh) return false;
   const int band_cap = (rows_cap - p.kh) / p.sh + 1;
-  const bool wide = p.sw == 1 && p.kw >= kBandWideMinCols && p.out_w >= 16;
   if (wide) target_outputs *= 4;
   int band = (target_outputs + p.out_w - 1) / p.out_w;
   band = band < 1 ? 1 : band;
@@ -1456,7 +1471,8 @@ static int run_pooling(bool three_d, const int* in_shape, int pool_type, const i
       const bool kept = 16 * shared >= a.tile_rows &&
                         static_cast<uint64_t>(in_shape[0]) * in_shape[1] * p.in_h * p.in_w * sizeof(float) >= kBandKeptBytes;
       const int k = p.kh == p.kw && (p.kh == 2 || p.kh == 3 || (p.kh == 5 && a.wide)) ? p.kh : 0;
-      const int steps = (a.tile_rows * p.in_w / (pipe ? 4 : 1) + kBlock - 1) / kBlock;  // per lane and band
+      const bool span = !pipe && a.pitch == p.in_w && p.in_w >= 4;
+      const int steps = ((a.tile_rows * p.in_w + (pipe || span ? 3 : 0)) / (pipe || span ? 4 : 1) + kBlock - 1) / kBlock;  // per lane and band
       const int regs = steps <= 2 ? 2 : (steps <= 3 ? 3 : (steps <= 4 ? 4 : (steps <= 6 ? 6 : 8)));
       if (pl->chosen(SHDW_PATH_POOL_BAND, (pipe ? 100 * regs : 0) + k, g)) return SHDW_OK;
 #define SHDW_LAUNCH_BAND_REGS(MAXV, KV, KINDV)                                                  \
@@ -1472,6 +1488,7 @@ static int run_pooling(bool three_d, const int* in_shape, int pool_type, const i
 #define SHDW_LAUNCH_BAND(MAXV, KV)                                                              \
   do {                                                                                           \
     if (pipe) SHDW_LAUNCH_BAND_REGS(MAXV, KV, kBandVectors);                                     \
+    else if (span) SHDW_LAUNCH_BAND_REGS(MAXV, KV, kBandSpan);                                   \
     else if (kept) SHDW_LAUNCH_BAND_REGS(MAXV, KV, kBandFloatsKept);                             \
     else SHDW_LAUNCH_BAND_REGS(MAXV, KV, kBandFloats);                                           \
   } while (0)
