@@ -300,10 +300,14 @@ constexpr uint32_t kThinTileFloats = 8192;  // 32 KB
 // the contiguous side, whose vectors no longer sit on 16 bytes in LDS, moves its
 // four floats one by one there.
 // SHARED: the planar rows are read with plain loads, see shared_rows().
+// From a planar side a lane asks for all its vectors of the tile before it lays the first one down
+// ([64,16,3136] 7.7 -> 5.5 us, [64,3,50625] 18.8 -> 15.8, [64,126,400] 6.2 -> 5.6); from the contiguous
+// side that is slower ([64,1444,84] 18.0 and 21.6, [64,50625,3] 18.9 and 23.7).
 template <bool COLS_THIN, bool PAD, bool SHARED>
 __global__ __launch_bounds__(kBlock) void transpose_thin_kernel(const float* x, float* y, uint32_t big,
                                                                  FastDiv f_thin, uint32_t span,
                                                                  FastDiv f_tiles) {
+  constexpr int kAhead = kThinTileFloats / 4 / kBlock;  // vectors of a lane
   __shared__ __align__(16) float tile[kThinTileFloats];  // [span][pitch], the interleaved side's order
   const uint32_t thin = f_thin.d, pitch = PAD ? thin + 1 : thin;
   uint32_t b, t;
@@ -347,12 +351,24 @@ __global__ __launch_bounds__(kBlock) void transpose_thin_kernel(const float* x, 
       planar_dst[static_cast<uint64_t>(j) * big + r] = tile[r * pitch + j];
     }
   } else {
-    for (uint32_t u = threadIdx.x; u < thin * quads; u += kBlock) {
-      const uint32_t i = u / quads, q = u - i * quads;
-      const float* src = planar_src + static_cast<uint64_t>(i) * big + 4 * q;
-      const v4f r = SHARED ? load4_any(src) : load4_stream_any(src);
+    // all of a lane's vectors under way at once; lanes past the last one take it again
+    const uint32_t vectors = thin * quads;
+    v4f reg[kAhead];
+    uint32_t at[kAhead];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) tile[(4 * q + k) * pitch + i] = r[k];
+    for (int s = 0; s < kAhead; ++s) {
+      if (s * kBlock >= vectors) continue;
+      const uint32_t u = min(s * kBlock + threadIdx.x, vectors - 1);
+      const uint32_t i = u / quads, q = u - i * quads;
+      const float* src = planar_src + (static_cast<uint64_t>(i) * big + 4 * q);
+      reg[s] = SHARED ? load4_any(src) : load4_stream_any(src);
+      at[s] = 4 * q * pitch + i;
+    }
+#pragma unroll
+    for (int s = 0; s < kAhead; ++s) {
+      if (s * kBlock + threadIdx.x >= vectors) continue;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) tile[at[s] + k * pitch] = reg[s][k];
     }
     const uint32_t rest = n - 4 * quads;
     for (uint32_t u = threadIdx.x; u < thin * rest; u += kBlock) {
@@ -1198,7 +1214,10 @@ int shdw_hip_permute(int num_axes, const int* in_shape, const int* order, const 
       const bool cols_thin = cols <= rows;
       const uint32_t thin = cols_thin ? cols : rows, big = cols_thin ? rows : cols;
       const bool pad = thin % 8 == 0;
-      const uint32_t span = (kThinTileFloats / (thin + (pad ? 1 : 0))) & ~63u;
+      uint32_t span = (kThinTileFloats / (thin + (pad ? 1 : 0))) & ~63u;
+      // shorter tiles while there are under two a CU: [16,361,126] 6.7 -> 4.9 us, [1,65536,3] 6.0 -> 4.7,
+      // [64,400,126] 8.5 -> 6.5; the other way they are level
+      while (span > 32 && static_cast<uint64_t>(batch) * ((big + span - 1) / span) < 512) span = span / 2 & ~31u;
       const uint32_t tiles = span ? (big + span - 1) / span : 0;  // span 0: a padded side of 128 does not fit
       const int64_t groups = static_cast<int64_t>(batch) * tiles;
       if (span && groups <= INT32_MAX) {
