@@ -17,7 +17,8 @@
 // with its tail takes, per call: [32,512,28,28]
 // (103 MB) 26.5 us (28.7 with the quotients in fp32 and the row's parameters read for every
 // vector), where its five launches took 78; [64,64,56,56] 44; [64,512,14,14]
-// 12.1; [64,1024,7,7] 8.8; [16,64,112,112] 80 (its sums are 12 544 long).  With loads in
+// 12.1; [64,1024,7,7] 8.8; [16,64,112,112] 72 and [16,64,96,96] 54, both in chunks (their sums
+// are 12 544 and 9216 long).  With loads in
 // branches of their own, a division per element, LDS reads next to the additions that
 // use them and rows whole in LDS whatever their length: 29, 43, 13.9, 11.3 and 112; with the residual
 // another tensor than x 35 -> 27.5, 49 -> 44, 15.1 -> 12.0, 12.3 -> 8.2, 116 -> 80.
@@ -198,16 +199,21 @@ __global__ __launch_bounds__(kBlock, gate_waves(SLOTS)) void squeeze_gate_kernel
   // do not meet on one SIMD.
   const uint32_t walked = threadIdx.x & (kWave - 1);
   const bool walks = threadIdx.x / kWave == ((blockIdx.x / kXcds) & 3u) && walked < nrows;
-  GateRow g = row_params[min(lead, nrows - 1)];
+  GateRow g;
   float sum = 0.f;
   for (uint32_t k0 = 0; k0 < pieces; k0 += chunk) {
     if (!WHOLE && k0) __syncthreads();
     asm("" : "+v"(sub), "+v"(lead));
+    // Read again for every chunk: of a row's parameters that stay the same the compiler takes the front of
+    // all slots ahead of the chunks, and spills what does not fit (500 bytes a lane of sixteen
+    // vectors: [16,64,112,112] 92 us instead of 72, [16,64,96,96] 75 instead of 54).
+    if (ONE) g = row_params[min(lead, nrows - 1)];
     uint32_t k = 0, turn_row = 0;
 #pragma unroll
     for (int i = 0; i < SLOTS; ++i) {
       const uint32_t r = lead + turn_row, v = sub + k * lanes;
-      if (!ONE && k == 0) g = row_params[min(r, nrows - 1)];
+      // for every vector where rows go in chunks: kept from piece to piece they do not fit beside the vectors
+      if (!ONE && (k == 0 || !WHOLE)) g = row_params[min(r, nrows - 1)];
       if (i < used && (WHOLE || k - k0 < chunk)) {
         arrange(reg[i], 4 * v);
         const v4f t = front(reg[i], g);
@@ -238,7 +244,7 @@ __global__ __launch_bounds__(kBlock, gate_waves(SLOTS)) void squeeze_gate_kernel
   for (int i = 0; i < SLOTS; ++i) {
     if (i >= used) continue;
     const uint32_t r = lead + turn_row, v = sub + k * lanes, c = 4 * v;
-    if (!ONE && k == 0) g = row_params[min(r, nrows - 1)];
+    if (!ONE && (k == 0 || !WHOLE)) g = row_params[min(r, nrows - 1)];
     v4f t = WHOLE ? tile[min(r, nrows - 1) * pitch + min(v, pitch - 1)] : front(reg[i], g);
     if (RESIDUAL == kOtherResidual && !WHOLE && i % kTurn == 0) {
       uint32_t k_ahead = k, turn_ahead = turn_row;
