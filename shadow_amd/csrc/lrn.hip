@@ -96,16 +96,17 @@ SHDW_DEVICE void lrn_powers(const float (&scale)[kLrnRound], float y, bool small
 }
 
 // ---- windows of 1, 3, 5 and 7 channels: the window lives in registers ----
-// A workgroup owns 64 positions and goes through their channels in spans of four rounds, a
-// wave each.  Every lane has the channels of its round at once, those of the next span
+// One, two or four waves of a workgroup own 64 positions and go through their channels in spans
+// of a round each.  Every lane has the channels of its round at once, those of the next span
 // on their way during the powers; the waves take turns at the walk, which is short (two dependent
 // additions a channel), each handing the sum and the last SIZE channels to the next through
 // LDS; then all of them work out their powers, which are most of the work, at the same time.
-// Bound by the vector ALUs: 30 instructions a power, two thirds of them fp64.  With one wave
+// Bound by the vector ALUs: the powers, fp64 for the most part.  With one wave
 // walking all channels of its positions, and up to eight workgroups sharing the rounds of a
 // position where there are few (each walking from the first channel on): [44,96,55,55]
-// 38.8 -> 30.1 us, [16,256,56,56] 48.8 -> 30.8, [64,256,56,56] 118 -> 90, [68,256,27,27] 51.3 ->
-// 33.9, [1,96,55,55] 14.6 -> 8.0.  Rounds of 16 and 24 channels: 37.8 and 37.6 on the first.
+// 36.9 -> 28.9 us, [16,256,56,56] 48.6 -> 31.5, [64,256,56,56] 122 -> 92, [64,256,27,27] 50.0 ->
+// 30.6, [1,96,55,55] 14.8 -> 8.8, [512,8,56,56] 48.0 -> 27.5, [100,40,56,56] 31.3 -> 24.0.  Rounds of 16
+// and 24 channels: 37.8 and 37.6 on the first.
 //
 // Round c0 finishes channels c0 .. c0 + 7, for which the sum takes in channel c + post and
 // lets go of channel c - post - 1: own[j] is channel c0 + post + j, prev[t] channel
@@ -138,10 +139,13 @@ SHDW_DEVICE float lrn_walk(const float (&own)[kLrnRound], const float (&prev)[SI
   return accum;
 }
 
+// WAVES: how many of the workgroup's four waves share the channels of 64 positions; the others have positions
+// of their own (see the rule at launch_windows).
+//
 // STREAM: the stores carry the streams' hint; not where rows of positions start inside a vector, whose
 // pieces of lines would leave one by one ([44,96,55,55] 32.6 us plain, 34.0 with it, [68,256,27,27] 35.0
 // and 40.5; [64,256,56,56] 93.2 and 82.1, [256,64,14,14] 11.8 and 10.5).
-template <int SIZE, bool STREAM>
+template <int SIZE, int WAVES, bool STREAM>
 __global__ __launch_bounds__(kBlock, 5) void lrn_window_kernel(const float* x, float* y, uint32_t positions, uint32_t step,
                                                                uint32_t channels, float alpha_over_size, float neg_beta,
                                                                float k, FastDiv f_step) {
@@ -149,11 +153,13 @@ __global__ __launch_bounds__(kBlock, 5) void lrn_window_kernel(const float* x, f
   static_assert(SIZE % 2 == 1 && SIZE <= SEG, "the window must fit into a round");
   constexpr uint32_t post = (SIZE - 1) / 2;
   __shared__ LrnTables tables;
-  __shared__ LrnHand<SIZE> hand;
+  __shared__ LrnHand<SIZE> hands[kLrnWaves / WAVES];
   lrn_stage_tables(&tables);
   const uint32_t lane = threadIdx.x % kWave;
-  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  const uint32_t p = blockIdx.x * kWave + lane, at = min(p, positions - 1);
+  const uint32_t in_group = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const uint32_t wave = in_group % WAVES;
+  LrnHand<SIZE>& hand = hands[in_group / WAVES];
+  const uint32_t p = (blockIdx.x * (kLrnWaves / WAVES) + in_group / WAVES) * kWave + lane, at = min(p, positions - 1);
   const uint32_t b = fd_div(at, f_step);
   const size_t base = static_cast<size_t>(b) * channels * step + (at - b * step);
   const float* in = x + base;
@@ -164,7 +170,7 @@ __global__ __launch_bounds__(kBlock, 5) void lrn_window_kernel(const float* x, f
     for (int j = 0; j < SEG; ++j) ahead[j] = in[static_cast<size_t>(min(c0 + post + j, channels - 1)) * step];
   };
   request(wave * SEG);
-  for (uint32_t span = 0; span < channels; span += kLrnWaves * SEG) {
+  for (uint32_t span = 0; span < channels; span += WAVES * SEG) {
     const uint32_t c0 = span + wave * SEG;
     float own[SEG], prev[SIZE], scale[SEG];
 #pragma unroll
@@ -173,7 +179,7 @@ __global__ __launch_bounds__(kBlock, 5) void lrn_window_kernel(const float* x, f
 #pragma unroll
       for (int t = 0; t < SIZE; ++t) prev[t] = t + static_cast<int>(post) >= SIZE ? in[static_cast<size_t>(t + post - SIZE) * step] : 0.f;
     }
-    for (uint32_t turn = 0; turn < kLrnWaves; ++turn) {
+    for (uint32_t turn = 0; turn < WAVES; ++turn) {
       if (wave == turn && c0 < channels) {  // the same for the whole wave
         float accum = 0.f;
         if (c0 == 0) {
@@ -192,9 +198,9 @@ __global__ __launch_bounds__(kBlock, 5) void lrn_window_kernel(const float* x, f
 #pragma unroll
         for (int t = 0; t < SIZE; ++t) hand.prev[t][lane] = own[SEG - SIZE + t];
       }
-      __syncthreads();
+      if (WAVES > 1) __syncthreads();
     }
-    if (span + kLrnWaves * SEG < channels) request(c0 + kLrnWaves * SEG);
+    if (c0 + WAVES * SEG < channels) request(c0 + WAVES * SEG);
     if (c0 >= channels) continue;
     float power[SEG];
     lrn_powers(scale, neg_beta, neg_beta != 0.f && __builtin_fabsf(neg_beta) <= 1.25f, &tables, power);
@@ -281,6 +287,41 @@ __global__ __launch_bounds__(kBlock) void lrn_across_channels_kernel(
 
 using namespace shdw;
 
+namespace {
+
+template <int SIZE, int WAVES>
+void launch_windows(const float* x, float* y, uint32_t positions, uint32_t step, uint32_t channels, float alpha_over_size,
+                    float neg_beta, float k, bool stream, hipStream_t st) {
+  constexpr uint32_t kOwned = kLrnWaves / WAVES * kWave;
+  const uint32_t grid = positions / kOwned + (positions % kOwned != 0);
+  const FastDiv f_step = make_fastdiv(step);
+  if (stream) lrn_window_kernel<SIZE, WAVES, true><<<grid, kBlock, 0, st>>>(x, y, positions, step, channels, alpha_over_size, neg_beta, k, f_step);
+  else lrn_window_kernel<SIZE, WAVES, false><<<grid, kBlock, 0, st>>>(x, y, positions, step, channels, alpha_over_size, neg_beta, k, f_step);
+}
+
+// One wave for 64 positions works without barriers and leaves no wave without a round, four finish soonest and
+// share the SIMDs out most evenly: one from where on the SIMDs' shares of the runs of 64 (runs / 1024, rounded up)
+// differ by an eighth at most, two from where on four are more than the chip holds at a time (5120), no more than
+// there are rounds; and four where a walk over many channels would outlast the others.  With 1 / 2 / 4 waves,
+// by runs: 23437 of 8 channels 26.6 / 37.1 / 58.6 us, 11718 of 16 24.7 / 26.4 / 41.5, 4687 of 40 25.1 / 26.6 / 32.1,
+// 4000 of 96 42.1 / 44.1 / 46.5; 3332 of 64 28.4 / 26.3 / 26.9, 3136 of 40 18.5 / 18.3 / 20.7, 3136 of 64
+// 29.6 / 26.7 / 27.0, of 96 42.1 / 39.4 / 36.2, of 256 103.6 / 92.8 / 88.5; 2079 of 96 34.4 / 28.7 / 30.0, 1400 of 96
+// 27.4 / 19.7 / 20.9; 1200 of 96 26.3 / 19.1 / 16.0, 732 of 256 48.7 / 36.0 / 28.6.
+template <int SIZE>
+void launch_windows(const float* x, float* y, uint32_t positions, uint32_t step, uint32_t channels, float alpha_over_size,
+                    float neg_beta, float k, bool stream, hipStream_t st) {
+  constexpr uint32_t kResident = 5120, kEven = 3584;
+  const uint32_t runs = (positions + kWave - 1) / kWave, rounds = (channels + kLrnRound - 1) / kLrnRound;
+  if (rounds == 1 || (runs > kEven && rounds <= 16))
+    launch_windows<SIZE, 1>(x, y, positions, step, channels, alpha_over_size, neg_beta, k, stream, st);
+  else if (rounds == 2 || (runs > kResident / 4 && (runs <= kResident / 2 || rounds <= 8)))
+    launch_windows<SIZE, 2>(x, y, positions, step, channels, alpha_over_size, neg_beta, k, stream, st);
+  else
+    launch_windows<SIZE, 4>(x, y, positions, step, channels, alpha_over_size, neg_beta, k, stream, st);
+}
+
+}  // namespace
+
 extern "C" int shdw_hip_lrn(const int* in_shape, int size, float alpha, float beta, float k, const float* x,
                             float* y, void* stream) {
   if (!in_shape || size < 1 || size % 2 == 0) return SHDW_E_INVALID_ARGUMENT;
@@ -304,16 +345,11 @@ extern "C" int shdw_hip_lrn(const int* in_shape, int size, float alpha, float be
   const uint32_t grid = grid_for(positions), chan = static_cast<uint32_t>(channels);
   const FastDiv f_step = make_fastdiv(step);
   if (size <= 7) {
-    const dim3 share((positions + kWave - 1) / kWave);
     const bool stream = step % 4 == 0 && aligned16(y);
-#define SHDW_LRN(S)                                                                                                             \
-  stream ? lrn_window_kernel<S, true><<<share, kBlock, 0, st>>>(x, y, positions, step, chan, alpha_over_size, -beta, k, f_step) \
-         : lrn_window_kernel<S, false><<<share, kBlock, 0, st>>>(x, y, positions, step, chan, alpha_over_size, -beta, k, f_step)
-    if (size == 1) SHDW_LRN(1);
-    else if (size == 3) SHDW_LRN(3);
-    else if (size == 5) SHDW_LRN(5);
-    else SHDW_LRN(7);
-#undef SHDW_LRN
+    if (size == 1) launch_windows<1>(x, y, positions, step, chan, alpha_over_size, -beta, k, stream, st);
+    else if (size == 3) launch_windows<3>(x, y, positions, step, chan, alpha_over_size, -beta, k, stream, st);
+    else if (size == 5) launch_windows<5>(x, y, positions, step, chan, alpha_over_size, -beta, k, stream, st);
+    else launch_windows<7>(x, y, positions, step, chan, alpha_over_size, -beta, k, stream, st);
     return launch_status();
   }
   // A tensor with few positions has few waves, and each walks all the channels one round after

@@ -1,5 +1,5 @@
-"""LRN with windows of one to seven channels: four waves of a workgroup share the channels of 64
-positions, eight each, and hand the running sum on."""
+"""LRN with windows of one to seven channels: one, two or four waves of a workgroup share the channels of
+64 positions, eight each, and hand the running sum on."""
 import numpy as np
 import pytest
 
@@ -34,3 +34,15 @@ def test_lrn_spans_of_special_values(gpu, channels):
         for k in (1.0, 0.0, -0.5):
             want = oracle.lrn(x, shape, 5, 1e-1, 0.75, k)[0]
             assert_bit_exact(gpuops.lrn(x, shape, 5, 1e-1, 0.75, k), want, "k = %g" % k)
+
+
+# one, two and four waves for 64 positions: either side of 1280, 2560 and 3584 runs of 64, of 8, 16, 64 and 128 channels
+@pytest.mark.parametrize("channels,positions", [(8, 3 * 27400), (17, 3 * 27305), (17, 3 * 27312), (33, 3 * 54612), (65, 3 * 54617), (9, 3 * 54700),
+                                                (20, 3 * 76458), (20, 3 * 76461), (40, 3 * 76470), (137, 3 * 27400), (137, 3 * 54617)])
+@pytest.mark.parametrize("size", [1, 5, 7])
+def test_lrn_spans_of_many_positions(gpu, channels, positions, size):
+    shape = (1, channels, 3, positions // 3)
+    x = normal(channels + size, channels * positions, 4.0)
+    want = oracle.lrn(x, shape, size, 1e-2, 0.75, 1.0)[0]
+    assert_bit_exact(gpuops.lrn(x, shape, size, 1e-2, 0.75, 1.0), want, "lrn")
+    assert_bit_exact(gpuops.lrn(x, shape, size, 1e-2, 0.75, 1.0, inplace=True), want, "lrn in place")
