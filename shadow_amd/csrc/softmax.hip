@@ -956,20 +956,26 @@ struct TileLane {
   SHDW_DEVICE bool step(int u) const { return (u & ~1) * STEP < dim; }
   SHDW_DEVICE bool has(int u) const { return c0 + u * STEP < dim; }
   SHDW_DEVICE uint32_t row(int u) const { return min(c0 + u * STEP, dim - 1); }
-  SHDW_DEVICE void load(const float* xs, v4f (&r)[kTilePerLane]) const {
+  // A lane whose four positions reach past the row's end takes the row's last four, without a branch
+  // around each load (a row has sixteen and more), and moves its own to the front: [8,1024,361] 12.5 -> 10.6 us
+  // (p = 2), [34,271,158] 8.3 -> 7.1, with 1, 2 or 3 single floats in such lanes before.
+  SHDW_DEVICE v4f to_front(v4f v, uint32_t moved) const {
+    if (TAIL && (moved & 1u)) v = v4f{v[1], v[2], v[3], v[3]};
+    if (TAIL && (moved & 2u)) v = v4f{v[2], v[3], v[3], v[3]};
+    return v;
+  }
+  template <int N>
+  SHDW_DEVICE void load(const float* xs, v4f (&r)[N]) const {
     if (valid == 0) return;
+    const uint32_t moved = 4 - valid;
+    const float* from = xs + j - moved;
 #pragma unroll
-    for (int u = 0; u < kTilePerLane; ++u) {
-      if (!step(u)) continue;
-      const float* src = xs + static_cast<uint64_t>(row(u)) * inner + j;
-      if (!TAIL || valid == 4) {
-        r[u] = load4_stream_any(src);
-      } else {
-        r[u] = v4f{0.f, 0.f, 0.f, 0.f};
+    for (int u = 0; u < N; ++u)
+      if (step(u)) r[u] = load4_stream_any(from + static_cast<uint64_t>(row(u)) * inner);
+    if (TAIL && moved) {
 #pragma unroll
-        for (int k = 0; k < 3; ++k)
-          if (k < valid) r[u][k] = src[k];
-      }
+      for (int u = 0; u < N; ++u)
+        if (step(u)) r[u] = to_front(r[u], moved);
     }
   }
   SHDW_DEVICE void store(float* ys, uint32_t u, v4f v) const {
@@ -1064,12 +1070,13 @@ SHDW_DEVICE double strided_lane_sum(double v) {
 // divisions [16,512,38,38], 94.6 MB, took 32.3 us; now 20.6.  p other than 1 and 2 is not taken here: powf per
 // element in order would dominate.
 template <int PMODE, int SM, int TS_SHIFT, int ROWS>
-__global__ __launch_bounds__(kBlock) void normalize_tile_kernel(const float* x, float* y, uint32_t dim,
+__global__ __launch_bounds__(kBlock, TS_SHIFT == 6 ? 7 : SM == kSsdChannelScale ? 4 : 5) void normalize_tile_kernel(const float* x, float* y, uint32_t dim,
                                                                  uint32_t inner, const float* scale, float p,
                                                                  float eps, FastDiv f_tiles) {
   using Lane = TileLane<TS_SHIFT, ROWS>;
   constexpr uint32_t TS = 1u << TS_SHIFT;
   constexpr int kWaves = kBlock / kWave;
+  constexpr int kPerLane = TS_SHIFT == 6 ? kTilePerLane / 2 : kTilePerLane;  // tiles of 64 positions have up to 128 rows
   __shared__ __align__(16) double partial[kWaves][TS];
   __shared__ __align__(16) double recip[TS];
   __shared__ __align__(16) float handed[TS];
@@ -1082,22 +1089,23 @@ __global__ __launch_bounds__(kBlock) void normalize_tile_kernel(const float* x, 
   const uint64_t base = static_cast<uint64_t>(n) * dim * inner + p0;
   const Lane lane(width, dim, inner);
   auto term = [p](float v) { return static_cast<float>(norm_term<PMODE>(v, p)); };  // an fp32 value, widened exactly
-  v4f r[kTilePerLane];
+  v4f r[kPerLane];
   lane.load(x + base, r);
-  float factor[kTilePerLane];
-  if (SM == kSsdChannelScale) {
-#pragma unroll
-    for (int u = 0; u < kTilePerLane; ++u)
-      if (lane.step(u)) factor[u] = scale[lane.row(u)];
-  }
   double acc[4] = {0, 0, 0, 0};
   if (lane.valid != 0) {
 #pragma unroll
-    for (int u = 0; u < kTilePerLane; ++u) {
+    for (int u = 0; u < kPerLane; ++u) {
       if (!lane.step(u)) continue;
 #pragma unroll
       for (int k = 0; k < 4; ++k) acc[k] += static_cast<double>(lane.has(u) ? term(r[u][k]) : 0.f);
     }
+  }
+  // the rows' factors are asked for when the rows are through: [16,512,38,38] 18.6 -> 17.2 us, [1,512,1444] 9.5 -> 7.8
+  float factor[kPerLane];
+  if (SM == kSsdChannelScale) {
+#pragma unroll
+    for (int u = 0; u < kPerLane; ++u)
+      if (lane.step(u)) factor[u] = scale[lane.row(u)];
   }
 #pragma unroll
   for (int k = 0; k < 4; ++k) acc[k] = strided_lane_sum<Lane::LANES_PER_ROW>(acc[k]);
@@ -1124,7 +1132,7 @@ __global__ __launch_bounds__(kBlock) void normalize_tile_kernel(const float* x, 
   if (unsettled != 0) {  // the whole workgroup: the sums in index order, STEP rows at a time
     double sum = 0;
 #pragma unroll
-    for (int u = 0; u < kTilePerLane; ++u) {
+    for (int u = 0; u < kPerLane; ++u) {
       if (u * Lane::STEP >= dim) continue;
       if (lane.valid != 0 && lane.has(u))
         *reinterpret_cast<v4f*>(chunk + (lane.c0 << TS_SHIFT) + lane.j) = v4f{term(r[u][0]), term(r[u][1]), term(r[u][2]), term(r[u][3])};
@@ -1145,7 +1153,7 @@ __global__ __launch_bounds__(kBlock) void normalize_tile_kernel(const float* x, 
   if (lane.valid == 0) return;
   const TileQuotients q(handed + lane.j, recip + lane.j);
 #pragma unroll
-  for (int u = 0; u < kTilePerLane; ++u) {
+  for (int u = 0; u < kPerLane; ++u) {
     if (!lane.has(u)) continue;
     const uint32_t c = lane.c0 + u * Lane::STEP;
     v4f v = q(r[u]);
@@ -1198,8 +1206,9 @@ static int normalize_tile_shift(int dim);
 template <int PMODE, int SM>
 static void launch_normalize_tile(int outer_num, int dim, int inner_num, float p, float eps, const float* x,
                                   const float* scale, float* y, hipStream_t st) {
-  // 64 positions per tile row while a lane has at most eight vectors of them (up to 128 rows),
-  // else 32, up to 16 vectors, else 16.  Measured when the columns were walked out of a tile in
+  // 64 positions per tile row while a lane has at most eight vectors of them (up to 128 rows; the kernel
+  // holds no more of these, so that eight waves fit a SIMD: [32,96,3025] 18.9 -> 13.7 us, [16,128,5625]
+  // 22.2 -> 17.2 with a factor a row), else 32, up to 16 vectors, else 16.  Measured when the columns were walked out of a tile in
   // LDS: [64,256,56,56] 85 us with 64 positions, 80 us with 32; [64,512,38,38] 105 us with 32, 115
   // with 16.  Softmax takes the widest tile that fits.
   const int shift = normalize_tile_shift(dim);

@@ -10,8 +10,9 @@ from tests.helpers import assert_bit_exact, normal, uniform
 
 F = np.float32
 # (outer, dim, inner): one row more than the steps of the lanes, a last step with rows missing, whole
-# tiles; positions that end inside a lane's four, on multiples of 4 and of 16
-SHAPES = [(2, 65, 16), (1, 65, 4097), (3, 129, 37), (2, 255, 64), (2, 512, 100), (1, 511, 1444), (2, 513, 65), (1, 1024, 80)]
+# tiles; positions that end one, two and three into a lane's four, on multiples of 4 and of 16
+SHAPES = [(2, 65, 16), (1, 65, 4097), (3, 129, 37), (2, 255, 64), (2, 512, 100), (1, 511, 1444), (2, 513, 65), (1, 1024, 80),
+          (2, 100, 67), (2, 128, 130), (3, 300, 46), (2, 600, 83), (1, 1000, 78)]
 
 
 def tied_column(dim, squares):
