@@ -1041,17 +1041,20 @@ SHDW_DEVICE T fold_tile_column(const float* column, uint32_t dim, T acc, F f) {
 // Whether a sum of non-negative terms in fp64 that were added in another order than the
 // reference's gives the reference's value all the same: both orders' sums are within
 // (terms - 1 + 25) 2^-53 of the true one (a lane adds up to 16, and 9 more additions join
-// the lanes), so what norm_finish makes of either lies within `slack` of what it makes of the
-// other before it rounds to fp32; where the two ends of that interval round to the same
-// number the order cannot show.  About one column in 2^18 of 512 random terms has to be
-// added again in order.  NaN is never settled, nor is a sum with a negative eps.
+// the lanes), so the reference's lies between the two ends below, and what norm_finish makes of it
+// between what it makes of them, since every operation there is monotonic.  Where that is the
+// same number the order cannot show; a NaN among the terms is NaN in any order.  About one
+// column in 2^18 of 512 random terms is left.
 template <int PMODE>
-SHDW_DEVICE bool norm_settled(double acc, float eps, uint32_t terms) {
-  if (PMODE == 3 && !(eps >= 0.f)) return false;
+SHDW_DEVICE bool norm_settled(double acc, float p, float eps, uint32_t terms) {
   const double slack = static_cast<double>(terms + 64) * 0x1p-53;
-  const double v = PMODE == 3 ? __builtin_sqrt(acc + static_cast<double>(eps)) : acc;
-  return static_cast<float>(v * (1.0 - slack)) == static_cast<float>(v * (1.0 + slack));
+  const float lo = norm_finish<PMODE>(acc * (1.0 - slack), p, eps), hi = norm_finish<PMODE>(acc * (1.0 + slack), p, eps);
+  return lo == hi || hi != hi;
 }
+
+// The same of a sum whose terms are all 0 or at least `least`: they are multiples of the last place of
+// `least`, more than 2^-24 of it, so below 2^29 times it every partial sum is exact in any order.
+SHDW_DEVICE bool norm_exact(double acc, float least) { return acc <= static_cast<double>(least) * 0x1p29; }
 
 // Sum over the lanes of a wave that are `LANES` apart (4, 8 or 16).
 template <int LANES>
@@ -1063,12 +1066,27 @@ SHDW_DEVICE double strided_lane_sum(double v) {
   return v;
 }
 
+// Maximum over the lanes of a wave that are `LANES` apart (4, 8 or 16).
+template <int LANES>
+SHDW_DEVICE float strided_lane_max(float m) {
+  if (LANES <= 4) m = max3_any_order(m, m, dpp_f32<kDppRor4>(m));
+  if (LANES <= 8) m = max3_any_order(m, m, dpp_f32<kDppRor8>(m));
+  m = max3_any_order(m, m, __shfl_xor(m, 16));
+  return max3_any_order(m, m, __shfl_xor(m, 32));
+}
+
 // Memory-bound: every lane adds up the terms of its own rows in registers and the partial sums
 // meet over the lanes and the four waves, so the tile itself needs no LDS and a CU holds four
 // workgroups of a [.,512,.] column tile (128 VGPRs).  With the columns walked in order out of
 // 64 KB of LDS (two workgroups a CU, one wave of four at work for 512 dependent additions) and
-// divisions [16,512,38,38], 94.6 MB, took 32.3 us; now 20.6.  p other than 1 and 2 is not taken here: powf per
+// divisions [16,512,38,38], 94.6 MB, took 30.2 us; now 17.3.  p other than 1 and 2 is not taken here: powf per
 // element in order would dominate.
+//
+// A column whose sum the bound cannot settle is one of whole numbers more often than not (a sum past 2^24
+// that is odd lies between two floats), exact in every order: the workgroup looks for the least term of
+// each column, and only if that does not settle all of them adds up in order.  18-bit numbers, p = 1, on
+// [16,512,38,38] 17.8 us (always in order 23.4), one column that needs the order on [2,512,400] 14.8 (others 7.5),
+// every column on [16,512,38,38] 25.5.
 template <int PMODE, int SM, int TS_SHIFT, int ROWS>
 __global__ __launch_bounds__(kBlock, TS_SHIFT == 6 ? 7 : SM == kSsdChannelScale ? 4 : 5) void normalize_tile_kernel(const float* x, float* y, uint32_t dim,
                                                                  uint32_t inner, const float* scale, float p,
@@ -1081,7 +1099,7 @@ __global__ __launch_bounds__(kBlock, TS_SHIFT == 6 ? 7 : SM == kSsdChannelScale 
   __shared__ __align__(16) double recip[TS];
   __shared__ __align__(16) float handed[TS];
   __shared__ __align__(16) float chunk[Lane::STEP * TS];
-  __shared__ uint32_t unsettled;
+  __shared__ uint64_t unsettled;  // a bit a position
   uint32_t n, tile;
   fd_divmod(xcd_contiguous(blockIdx.x, gridDim.x), f_tiles, n, tile);
   const uint32_t p0 = tile << TS_SHIFT;
@@ -1123,12 +1141,46 @@ __global__ __launch_bounds__(kBlock, TS_SHIFT == 6 ? 7 : SM == kSsdChannelScale 
       const float d = norm_finish<PMODE>(sum, p, eps);
       handed[threadIdx.x] = d;
       recip[threadIdx.x] = reciprocal(d);
-      settled = norm_settled<PMODE>(sum, eps, dim);
+      settled = norm_settled<PMODE>(sum, p, eps, dim);
+      partial[0][threadIdx.x] = sum;
     }
     const uint64_t seen = __builtin_amdgcn_ballot_w64(!settled);
-    if (threadIdx.x == 0) unsettled = seen != 0;
+    if (threadIdx.x == 0) unsettled = seen;
   }
   __syncthreads();
+  if (unsettled != 0) {  // the whole workgroup
+    float least[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) least[k] = __builtin_inff();
+    if (lane.valid != 0) {
+#pragma unroll
+      for (int u = 0; u < kPerLane; ++u) {
+        if (!lane.step(u)) continue;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {  // the last row may come up again
+          const float t = term(r[u][k]);
+          least[k] = t > 0.f ? __builtin_fminf(least[k], t) : least[k];
+        }
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) least[k] = -strided_lane_max<Lane::LANES_PER_ROW>(-least[k]);
+    if (threadIdx.x % kWave < Lane::LANES_PER_ROW)
+      *reinterpret_cast<v4f*>(chunk + threadIdx.x / kWave * TS + lane.j) = v4f{least[0], least[1], least[2], least[3]};
+    __syncthreads();
+    if (threadIdx.x < kWave) {
+      bool settled = true;
+      if (threadIdx.x < width && (unsettled >> threadIdx.x & 1u)) {
+        float l = chunk[threadIdx.x];
+#pragma unroll
+        for (int w = 1; w < kWaves; ++w) l = __builtin_fminf(l, chunk[w * TS + threadIdx.x]);
+        settled = norm_exact(partial[0][threadIdx.x], l);
+      }
+      const uint64_t seen = __builtin_amdgcn_ballot_w64(!settled);
+      if (threadIdx.x == 0) unsettled = seen;
+    }
+    __syncthreads();
+  }
   if (unsettled != 0) {  // the whole workgroup: the sums in index order, STEP rows at a time
     double sum = 0;
 #pragma unroll
@@ -1137,10 +1189,9 @@ __global__ __launch_bounds__(kBlock, TS_SHIFT == 6 ? 7 : SM == kSsdChannelScale 
       if (lane.valid != 0 && lane.has(u))
         *reinterpret_cast<v4f*>(chunk + (lane.c0 << TS_SHIFT) + lane.j) = v4f{term(r[u][0]), term(r[u][1]), term(r[u][2]), term(r[u][3])};
       __syncthreads();
-      if (threadIdx.x < width) {
-        const uint32_t rows = min(Lane::STEP, dim - u * Lane::STEP);
-        for (uint32_t c = 0; c < rows; ++c) sum += static_cast<double>(chunk[(c << TS_SHIFT) + threadIdx.x]);
-      }
+      if (threadIdx.x < width)
+        sum = fold_tile_column<TS_SHIFT>(chunk + threadIdx.x, min(Lane::STEP, dim - u * Lane::STEP), sum,
+                                         [](double a, float t) { return a + static_cast<double>(t); });
       __syncthreads();
     }
     if (threadIdx.x < width) {
@@ -1218,15 +1269,6 @@ static void launch_normalize_tile(int outer_num, int dim, int inner_num, float p
     launch_normalize_tile_ts<PMODE, SM, 5>(outer_num, dim, inner_num, p, eps, x, scale, y, st);
   else
     launch_normalize_tile_ts<PMODE, SM, 4>(outer_num, dim, inner_num, p, eps, x, scale, y, st);
-}
-
-// Maximum over the lanes of a wave that are `LANES` apart (4, 8 or 16).
-template <int LANES>
-SHDW_DEVICE float strided_lane_max(float m) {
-  if (LANES <= 4) m = max3_any_order(m, m, dpp_f32<kDppRor4>(m));
-  if (LANES <= 8) m = max3_any_order(m, m, dpp_f32<kDppRor8>(m));
-  m = max3_any_order(m, m, __shfl_xor(m, 16));
-  return max3_any_order(m, m, __shfl_xor(m, 32));
 }
 
 // Softmax on the same tile layout (65 <= dim <= 1024).  The lanes hold x, later

@@ -77,3 +77,39 @@ def test_zeros_infinities_and_nans_in_columns(gpu, outer, dim, inner):
         want = oracle.ssd_normalize(x, outer, dim, inner, False, True, 1e-10, None)
         assert_bit_exact(gpuops.ssd_normalize(x, outer, dim, inner, False, True, 1e-10, None), want, "ssd")
         assert_bit_exact(gpuops.softmax(x, outer, dim, inner), oracle.softmax(x, outer, dim, inner), "softmax")
+
+
+def whole_columns(outer, dim, inner, largest):
+    """Whole numbers, every third column's sum made odd and past 2^24: exactly between two floats or next to it."""
+    x = np.random.default_rng(11).integers(0, largest, (outer, dim, inner)).astype(F)
+    over = np.sum(x, axis=1, dtype=np.float64)
+    x[:, 7, ::3] += ((1 + np.float64(1 << 24) - over[:, ::3]).clip(0) // 2 * 2 + (over[:, ::3] + 1) % 2).astype(F)
+    x[:, dim - 1, ::5] = 0
+    return x
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("outer,dim,inner", SHAPES)
+def test_sums_that_are_exact_in_any_order(gpu, outer, dim, inner):
+    """Alone and beside columns that have to be added in order."""
+    for largest in (2, 256, 1 << 18):
+        x = whole_columns(outer, dim, inner, largest)
+        for y in (x, np.where(np.arange(inner) % 16 == 3, tied_column(dim, False)[:, None], x).astype(F)):
+            want = oracle.normalize(y, outer, dim, inner, 1.0, 1e-12)
+            assert_bit_exact(gpuops.normalize(y, outer, dim, inner, 1.0, 1e-12), want, "p = 1, below %d" % largest)
+        y = np.sqrt(x).astype(F) if largest == 2 else x
+        want = oracle.normalize(y, outer, dim, inner, 2.0, 1e-12)
+        assert_bit_exact(gpuops.normalize(y, outer, dim, inner, 2.0, 1e-12), want, "p = 2, below %d" % largest)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("outer,dim,inner", SHAPES)
+def test_negative_eps_next_to_the_sum(gpu, outer, dim, inner):
+    """sum + eps is 0, negative or a few last places of the sum."""
+    x = columns(outer, dim, inner, True)
+    x[:, :, 1::2] = F(2.0 ** -5)
+    eps = dim * 2.0 ** -10
+    with np.errstate(all="ignore"):
+        for e in (-1.0, -eps, -eps * (1 + 2.0 ** -20), -eps * (1 - 2.0 ** -20), -1e9):
+            want = oracle.ssd_normalize(x, outer, dim, inner, False, True, e, None)
+            assert_bit_exact(gpuops.ssd_normalize(x, outer, dim, inner, False, True, e, None), want, "eps %g" % e)
