@@ -560,7 +560,7 @@ enum {
   SHDW_PATH_POOL_PLANE = 21,        /* global pooling, planes in LDS */
   SHDW_PATH_POOL_PLANE_STREAM = 22, /* global average of long planes, streamed */
   SHDW_PATH_POOL_SMALL_PLANES = 23, /* whole planes in LDS; variant = 100 * separable + window unrolled for (0: loops) */
-  SHDW_PATH_POOL_BAND = 24,         /* bands of input rows in LDS; variant = 100 * registers per lane + window unrolled for */
+  SHDW_PATH_POOL_BAND = 24,         /* bands of input rows in LDS; variant = window unrolled for + 100 * (vectors a lane, padding cells in LDS) or 10 * (vectors a lane, rows as they lie) or 0 (single floats) */
   SHDW_PATH_POOL_WINDOW = 25,       /* a lane per output, windows from memory */
   SHDW_PATH_POOL_HALVE = 26,        /* 3x3 / 2x2 at stride 2, output rows half as long as input rows of 4 m columns: no staging; variant = window side */
   SHDW_PATH_POOL_SAME = 27          /* 3x3 at stride 1 with pad 1 on rows of 4 m columns: no staging */

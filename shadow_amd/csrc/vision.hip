@@ -252,8 +252,8 @@ SHDW_DEVICE uint32_t band_slot(const BandArgs& p, uint32_t t) {
 }
 
 // K > 0: square K x K window, fully unrolled, all LDS reads in flight together.
-// K = 0: any window, clipped loops.
-template <bool MAX, int K>
+// K = 0: any window, clipped loops.  STREAM: the outputs carry the streams' hint.
+template <bool MAX, int K, bool STREAM>
 SHDW_DEVICE void band_windows(const float* tile, float* y, const BandArgs& p, const BandSpan& bs) {
   // Lane -> (output row, output column) by shift and mask: w_lanes is a power
   // of two >= min(out_w, 256).  A lane keeps its column(s), so everything that
@@ -302,7 +302,9 @@ SHDW_DEVICE void band_windows(const float* tile, float* y, const BandArgs& p, co
         }
       }
       const int pool_size = (h_end_pad - h_first) * (w_end_pad - w_first);
-      __builtin_nontemporal_store(MAX ? max_val : sum_val / static_cast<float>(pool_size), dst + (hl * p.out_w + w));
+      const float out = MAX ? max_val : sum_val / static_cast<float>(pool_size);
+      if (STREAM) __builtin_nontemporal_store(out, dst + (hl * p.out_w + w));
+      else dst[hl * p.out_w + w] = out;
     }
   }
 }
@@ -388,19 +390,29 @@ SHDW_DEVICE void band_windows_wide(const float* tile, float* y, const BandArgs& 
 // issued into registers before the current band's windows are walked, so HBM
 // requests stay in flight during the LDS phase.  kBandSpan (any other rows, where no
 // window needs padding cells beside them, so that the tile is the span as it lies in memory):
-// the same from any dword address ([44,96,55,55] 3x3 by two 15.7 us with single floats, 14.5 so, its
-// average 16.6 and 14.6; before the outputs carried the streams' hint 16.6 and 18.4).
-// Otherwise the same with single
+// the same from any dword address ([44,96,55,55] 3x3 by two 15.8 us with single floats, 14.3 so, its
+// average 16.5 and 14.3).  Otherwise the same with single
 // floats, as many a lane ahead as a band has, up to eight, and the rest of a longer
 // span behind them.  Lanes beyond a span take its last elements again: a branch
 // around each load has the compiler wait for the one before it.
-// Single floats are plain loads (kBandFloatsKept) where the rows that neighbouring bands
-// share are a sixteenth of what a band reads or more, and the input is 24 MB or more;
-// elsewhere they carry the hint of the streams.  Operands new in every call, hint / plain:
-// [16,64,225,225] 3x3 at stride 1 132.8 / 122.2 us, [64,64,113,113] 5x5 at stride 1 134.8 / 125.6,
-// [16,64,225,225] 3x3 by two 55.0 / 52.0; [44,96,55,55] 3x3 by two 16.3 / 16.0 (a 37th shared:
-// left with the hint); under 24 MB [16,64,35,35] 3x3 at stride 1 5.8 / 6.1.
-enum { kBandVectors, kBandSpan, kBandFloats, kBandFloatsKept };
+//
+// Loads carry the hint of the streams but for rows that neighbouring bands share: spans with any such rows, or of
+// inputs under 24 MB (kBandSpanKept), single floats where a sixteenth of what a band reads is shared and the
+// input is 24 MB and more (kBandFloatsKept).  Outputs carry it but for inputs under 24 MB, spans and single floats
+// that are read plainly, and vectors of which a sixteenth is shared, where the window's walk is unrolled (the other
+// walks take long enough for it not to matter); outputs of band_windows_wide are stored plainly.  Operands
+// new in every call, hint / plain:
+//   single floats, loads: [16,64,225,225] 3x3 at stride 1 132.8 / 122.2 us, [64,64,113,113] 5x5 at stride 1
+//     134.8 / 125.6; under 24 MB [16,64,35,35] 3x3 at stride 1 5.8 / 6.1;
+//   spans, loads and stores: 3x3 by two of [16,64,225,225] 51.1 / 48.7, [4,32,300,301] 13.2 / 12.6, [32,64,111,111]
+//     24.4 / 23.8, [44,96,55,55] 14.4 / 14.2, [16,32,75,75] 6.4 / 5.8; without shared rows 2x2 by two of [64,64,113,113]
+//     46.6 / 48.6, of [64,64,112,110] 46.2 / 47.2, 4x4 by four of [2,3,500,501] 4.6 / 4.3;
+//   single floats with one column of padding, stores: 3x3 by two of [44,96,55,55] 14.8 / 16.0, [32,64,111,111]
+//     25.4 / 26.4; read plainly [16,64,225,225] 51.2 / 49.2; small, 4x4 by four of [2,3,500,501] 5.3 / 5.0;
+//   vectors, stores: 2x2 at stride 1 of [64,64,112,112] 101.6 / 94.9, 3x3 by two of [8,64,400,400] 87.3 / 83.4,
+//     [16,64,228,228] 53.9 / 53.0; 5x5 by two of [16,64,224,224] 91.1 / 92.2, 7x7 by two of [64,32,96,96] 58.4 / 59.7;
+//     without shared rows 4x4 by four of [64,64,112,112] 40.1 / 41.2, 3x3 by three of [16,64,100,100] 11.0 / 10.5.
+enum { kBandVectors, kBandVectorsPlainOut, kBandSpan, kBandSpanKept, kBandFloats, kBandFloatsPlainOut, kBandFloatsKept };
 constexpr uint64_t kBandKeptBytes = 24u << 20;
 constexpr int kBandMaxRegs = kBandTileFloats / 4 / kBlock;  // vectors per lane for a full tile
 static_assert(kBandMaxRegs == 8, "the launch switch covers up to 8 staged vectors per lane");
@@ -420,14 +432,16 @@ __global__ __launch_bounds__(kBlock) void pool_band_kernel(const float* x, float
       *reinterpret_cast<v4f*>(tile + t) = v4f{neutral, neutral, neutral, neutral};
   }
   __syncthreads();
-  if (KIND == kBandVectors || KIND == kBandSpan) {
+  constexpr bool kVectors = KIND == kBandVectors || KIND == kBandVectorsPlainOut;
+  constexpr bool kStreamOut = KIND == kBandVectors || KIND == kBandSpan || KIND == kBandFloats;
+  if (kVectors || KIND == kBandSpan || KIND == kBandSpanKept) {
     v4f reg[REGS];
     const auto request = [&](const BandSpan& bs) {
       if (bs.span == 0) return;  // every window of the band in the padding
 #pragma unroll
       for (int k = 0; k < REGS; ++k) {
         const float* from = bs.src + min(4u * (k * kBlock + threadIdx.x), bs.span - 4);
-        reg[k] = KIND == kBandVectors ? load4_stream(from) : load4_stream_any(from);
+        reg[k] = kVectors ? load4_stream(from) : KIND == kBandSpan ? load4_stream_any(from) : load4_any(from);
       }
     };
     BandSpan cur = band_span(p, x, g0);
@@ -436,7 +450,7 @@ __global__ __launch_bounds__(kBlock) void pool_band_kernel(const float* x, float
 #pragma unroll
       for (int k = 0; k < REGS; ++k) {
         const uint32_t t = 4 * (k * kBlock + threadIdx.x);
-        if (KIND == kBandVectors) {
+        if (kVectors) {
           if (t < cur.span) *reinterpret_cast<v4f*>(tile + band_slot(p, t)) = reg[k];
         } else if (t + 4 <= cur.span) {
           *reinterpret_cast<v4f*>(tile + t) = reg[k];
@@ -452,7 +466,7 @@ __global__ __launch_bounds__(kBlock) void pool_band_kernel(const float* x, float
         request(cur);
       }
       if (p.wide) band_windows_wide<MAX, K>(tile, y, p, walk);
-      else band_windows<MAX, K>(tile, y, p, walk);
+      else band_windows<MAX, K, kStreamOut>(tile, y, p, walk);
       __syncthreads();  // the tile is rewritten next
     }
   } else {
@@ -487,7 +501,7 @@ __global__ __launch_bounds__(kBlock) void pool_band_kernel(const float* x, float
         request(cur, 0);
       }
       if (p.wide) band_windows_wide<MAX, K>(tile, y, p, walk);
-      else band_windows<MAX, K>(tile, y, p, walk);
+      else band_windows<MAX, K, kStreamOut>(tile, y, p, walk);
       __syncthreads();
     }
   }
@@ -1468,13 +1482,14 @@ static int run_pooling(bool three_d, const int* in_shape, int pool_type, const i
       const uint32_t g = (a.total_bands + per - 1) / per;
       const bool pipe = p.in_w % 4 == 0 && aligned16(x);
       const int shared = a.bands_per_plane > 1 ? std::max(p.kh - p.sh, 0) : 0;  // rows that two bands read
-      const bool kept = 16 * shared >= a.tile_rows &&
-                        static_cast<uint64_t>(in_shape[0]) * in_shape[1] * p.in_h * p.in_w * sizeof(float) >= kBandKeptBytes;
+      const bool small = static_cast<uint64_t>(in_shape[0]) * in_shape[1] * p.in_h * p.in_w * sizeof(float) < kBandKeptBytes;
       const int k = p.kh == p.kw && (p.kh == 2 || p.kh == 3 || (p.kh == 5 && a.wide)) ? p.kh : 0;
       const bool span = !pipe && a.pitch == p.in_w && p.in_w >= 4;
+      const bool kept = span ? shared > 0 || small : 16 * shared >= a.tile_rows && !small;
+      const bool plain_out = !a.wide && (small || (pipe ? k > 0 && 16 * shared >= a.tile_rows : kept));
       const int steps = ((a.tile_rows * p.in_w + (pipe || span ? 3 : 0)) / (pipe || span ? 4 : 1) + kBlock - 1) / kBlock;  // per lane and band
       const int regs = steps <= 2 ? 2 : (steps <= 3 ? 3 : (steps <= 4 ? 4 : (steps <= 6 ? 6 : 8)));
-      if (pl->chosen(SHDW_PATH_POOL_BAND, (pipe ? 100 * regs : 0) + k, g)) return SHDW_OK;
+      if (pl->chosen(SHDW_PATH_POOL_BAND, (pipe ? 100 * regs : span ? 10 * regs : 0) + k, g)) return SHDW_OK;
 #define SHDW_LAUNCH_BAND_REGS(MAXV, KV, KINDV)                                                  \
   do {                                                                                           \
     switch (regs) {                                                                              \
@@ -1487,10 +1502,13 @@ static int run_pooling(bool three_d, const int* in_shape, int pool_type, const i
   } while (0)
 #define SHDW_LAUNCH_BAND(MAXV, KV)                                                              \
   do {                                                                                           \
-    if (pipe) SHDW_LAUNCH_BAND_REGS(MAXV, KV, kBandVectors);                                     \
-    else if (span) SHDW_LAUNCH_BAND_REGS(MAXV, KV, kBandSpan);                                   \
-    else if (kept) SHDW_LAUNCH_BAND_REGS(MAXV, KV, kBandFloatsKept);                             \
-    else SHDW_LAUNCH_BAND_REGS(MAXV, KV, kBandFloats);                                           \
+    if (pipe && plain_out) SHDW_LAUNCH_BAND_REGS(MAXV, KV, kBandVectorsPlainOut);               \
+    else if (pipe) SHDW_LAUNCH_BAND_REGS(MAXV, KV, kBandVectors);                               \
+    else if (span && kept) SHDW_LAUNCH_BAND_REGS(MAXV, KV, kBandSpanKept);                      \
+    else if (span) SHDW_LAUNCH_BAND_REGS(MAXV, KV, kBandSpan);                                  \
+    else if (kept) SHDW_LAUNCH_BAND_REGS(MAXV, KV, kBandFloatsKept);                            \
+    else if (plain_out) SHDW_LAUNCH_BAND_REGS(MAXV, KV, kBandFloatsPlainOut);                   \
+    else SHDW_LAUNCH_BAND_REGS(MAXV, KV, kBandFloats);                                          \
   } while (0)
       if (pool_type == 0) {
         if (k == 3)
