@@ -138,9 +138,11 @@ SHDW_DEVICE double row_sum(double v, double* slots) {
 // TAIL = false: inner % 4 == 0 and 16-byte aligned pointers.  TAIL = true: any
 // row length on any dword address; a lane's vector may end inside its four
 // positions, whole vectors still move as (unaligned) 128-bit accesses.
+// BY_STEP: steps that no lane has are left out, and the loads go out one after the other for
+// the test of it.
 constexpr int kBigBlock = 1024;
 
-template <int REGS, int LANES, bool TAIL>
+template <int REGS, int LANES, bool TAIL, bool BY_STEP = false>
 // Two 1024-lane workgroups per CU are 8 waves per SIMD, at most 64 registers
 // per lane (the second launch bound asks for that; unasked the compiler took
 // 67 and left room for one workgroup).  Eight vectors of a ragged row: seven waves a SIMD (unasked
@@ -160,18 +162,22 @@ __global__ __launch_bounds__(LANES <= kWave ? kBlock : LANES, LANES == kBigBlock
     return first >= p.inner ? 0u : min(4u, p.inner - first);
   };
   v4f reg[REGS];
+  if (!TAIL) {  // lanes past the row's end take its last vector again
 #pragma unroll
-  for (int k = 0; k < REGS; ++k) {
-    const uint32_t first = 4 * (k * LANES + lane), c = count(k);
-    if (!TAIL) {  // lanes past the row's end take its last vector again
-      reg[k] = load4_stream(xr + min(first, p.inner - 4));
-    } else if (c == 4) {
-      reg[k] = load4_stream_any(xr + first);
-    } else if (c > 0) {
-      reg[k] = v4f{0.f, 0.f, 0.f, 0.f};
+    for (int k = 0; k < REGS; ++k)
+      if (!BY_STEP || 4u * k * LANES < p.inner) reg[k] = load4_stream(xr + min(4 * (k * LANES + lane), p.inner - 4));
+  } else {
 #pragma unroll
-      for (int j = 0; j < 3; ++j)
-        if (j < c) reg[k][j] = xr[first + j];
+    for (int k = 0; k < REGS; ++k) {
+      const uint32_t first = 4 * (k * LANES + lane), c = count(k);
+      if (c == 4) {
+        reg[k] = load4_stream_any(xr + first);
+      } else if (c > 0) {
+        reg[k] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+          if (j < c) reg[k][j] = xr[first + j];
+      }
     }
   }
   double acc = 0;
@@ -866,6 +872,11 @@ int shdw_hip_group_norm_ws(int outer_num, int inner_num, float eps, const float*
     norm_rows_reg_kernel<2, kBlock, false><<<rows, kBlock, 0, st>>>(x, y, p);
   } else if (nvec <= 4 * kBlock) {
     norm_rows_reg_kernel<4, kBlock, false><<<rows, kBlock, 0, st>>>(x, y, p);
+  } else if (nvec <= 8 * kBlock && p.affine == kAffineRowPos && rows >= 1024) {
+    // LayerNorm of long rows, as many as fill the chip: with all loads / by step [1568,8192] 23.1 / 20.0 us, [1568,6000]
+    // 18.8 / 16.2, [2048,5120] 21.1 / 14.8, [3000,8192] 40.3 / 38.4; [500,8192] 7.9 / 9.0, and without parameters
+    // [3000,8192] 34.3 / 37.7, by channels 37.9 / 38.9.
+    norm_rows_reg_kernel<8, kBlock, false, true><<<rows, kBlock, 0, st>>>(x, y, p);
   } else if (nvec <= 8 * kBlock) {
     norm_rows_reg_kernel<8, kBlock, false><<<rows, kBlock, 0, st>>>(x, y, p);
   } else if (nvec <= 4 * kBigBlock) {
