@@ -532,6 +532,21 @@ __global__ __launch_bounds__(kBlock) void norm_rows_split_kernel(const float* x,
 
 constexpr uint32_t kNormSplitMaxRows = 512, kNormSplitMinInner = 32768, kNormSplitMinChunk = 8192;
 
+// Whether norm_rows_reg_kernel<16, kWave> (four waves a SIMD, a row each) shares its rows out evenly enough: no more
+// than the chip's 1024 SIMDs hold at a time, and four fifths of these busy in the last turn of three or four, without
+// scale and bias fifteen sixteenths of any.  With 256 lanes / a wave a row, InstanceNorm
+// and plain: 4096 rows of 3136 19.9 / 18.4 and 19.7 / 19.1 us, of 3600 23.7 / 22.0 and 23.6 / 22.5, of 3840 23.2 / 22.5 and
+// 23.5 / 23.2, 3840 of 3136 18.9 / 17.5 and 18.6 / 19.0, 3500 of 3600 21.2 / 19.5 and 20.9 / 22.3, 3300 of 3136
+// 16.9 / 16.5 and 16.5 / 18.0, 3072 of 3136 15.9 / 14.5 and 15.8 / 14.1; 4160 of 3136 20.3 / 23.1 and 20.0 / 21.8,
+// 2500 of 3136 13.8 / 13.6 and 13.4 / 13.7, 2100 of 3136 11.3 / 13.4 and 11.2 / 12.8, 2048 of 3136 9.2 / 10.9 and
+// 10.2 / 10.0, 8000 of 3136 35.0 / 39.4 and 34.7 / 36.4.
+static bool even_rows(uint32_t rows, bool affine) {
+  constexpr uint32_t kSimds = 1024;
+  if (rows > 4 * kSimds) return false;
+  const uint32_t places = (rows + kSimds - 1) / kSimds * kSimds;
+  return affine ? rows >= 2560 && 5 * rows >= 4 * places : 16 * rows >= 15 * places;
+}
+
 // Slices per row: enough for about a thousand workgroups, each with at least
 // 8192 elements; 1 where rows are many or short.
 static uint32_t norm_row_splits(int64_t rows, int64_t inner) {
@@ -863,10 +878,8 @@ int shdw_hip_group_norm_ws(int outer_num, int inner_num, float eps, const float*
     norm_rows_reg_kernel<4, kWave, false><<<groups(kWave), kBlock, 0, st>>>(x, y, p);
   } else if (nvec <= 8 * kWave && rows >= 2048) {
     norm_rows_reg_kernel<8, kWave, false><<<groups(kWave), kBlock, 0, st>>>(x, y, p);
-  } else if (nvec > 3 * kBlock && nvec <= 15 * kWave && rows >= 2048) {
-    // A wave a row where 256 lanes would leave a part of their last step idle, no barrier: rows of
-    // 3136 and 3600 (12.8 M elements) 17.5 and 18.1 us, with 256 lanes 19.4 and 21.1; of 4096 and
-    // 2500, which fill the 256 lanes or need three steps, 20.4 and 23.7 against 19.5 and 20.4.
+  } else if (nvec > 3 * kBlock && nvec <= 15 * kWave && rows >= 2048 && even_rows(rows, p.affine != kAffineNone)) {
+    // A wave a row where 256 lanes would leave a part of their last step idle, no barrier.
     norm_rows_reg_kernel<16, kWave, false><<<groups(kWave), kBlock, 0, st>>>(x, y, p);
   } else if (nvec <= 2 * kBlock) {
     norm_rows_reg_kernel<2, kBlock, false><<<rows, kBlock, 0, st>>>(x, y, p);

@@ -80,7 +80,8 @@ def test_subnormal_zero_and_special_quotients(gpu, shape):
 # one to eight vectors on eight lanes, rows in whole lines and not; a wave a row beside 256 lanes
 ROWS = [(1027, n) for n in (4, 8, 12, 16, 20, 32, 36, 48, 64, 96, 128, 160, 196, 224, 252, 256)] + \
        [(2049, n) for n in (3072, 3076, 3136, 3840, 3844)] + \
-       [(rows, n) for rows in (1023, 1024, 1300) for n in (4100, 5120, 6004, 8188, 8192)]
+       [(rows, n) for rows in (1023, 1024, 1300) for n in (4100, 5120, 6004, 8188, 8192)] + \
+       [(rows, n) for rows in (2048, 2559, 2560, 3277, 4095, 4097) for n in (3076, 3136, 3840)]
 
 
 @pytest.mark.gpu
