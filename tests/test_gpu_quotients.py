@@ -1,32 +1,45 @@
 """Quotients by a divisor that many dividends share (quotients, device_common.h): dividends whose
 quotient lies as near to the middle between two floats as any, subnormal and zero quotients and
 special values, bit for bit against a division; and the rows of the norms that take new forms."""
+from fractions import Fraction
+
 import numpy as np
 import pytest
 
-import oracle
 from tests import gpuops
-from tests.helpers import assert_rel_close, normal, uniform
+from tests.helpers import normal, uniform
 from tests.test_gpu_gate import Case
 
 F = np.float32
 
 
-def near_midpoints(d, rng, n):
-    """n dividends x with x / d as near as possible to a midpoint: |x 2^24 - M B| = 1 for the 24-bit
-    integer B of d, a midpoint M of 25 bits, which is the inverse of +-B modulo 2^24."""
+def odd_mantissa(d):
     b = int(np.frexp(np.float64(d))[0] * (1 << 24))
     while b % 2 == 0:
         b //= 2
-    out = []
-    for sign in (1, -1):
-        m = (sign * pow(b, -1, 1 << 24)) % (1 << 24) + (1 << 24)
-        a = (m * b - sign) >> 24
-        if a < (1 << 24):
-            out.append(a)
-    near = [F(a) for a in out]
+    return b
+
+
+def nearest_dividends(d):
+    """Whole numbers a below 2^24 with |a 2^k - M B| = 1 for the mantissa B of d as an odd number and a midpoint M of
+    25 bits: a / d is then 1 / 2 B of a last place off the middle between two floats, and no quotient by d that
+    is off at all is nearer.  M is the inverse of B or of -B modulo 2^k; of those two modulo 2^25 one has 25 bits."""
+    b, near = odd_mantissa(d), []
+    for k in (24, 25):
+        for sign in (1, -1):
+            m = sign * pow(b, -1, 1 << k) % (1 << k)
+            m += (1 << 24) if k == 24 else 0
+            a = (m * b - sign) >> k
+            if m >= 1 << 24 and 0 < a < 1 << 24:
+                near.append(a)
+    return near
+
+
+def near_midpoints(d, rng, n):
+    """n dividends, the nearest ones and up to three last places beside them, over many powers of two."""
+    near = [F(a) for a in nearest_dividends(d)]
     steps = rng.integers(-3, 4, n).astype(np.int32)
-    got = np.array([near[k % len(near)] if near else F(1) for k in range(n)], F)
+    got = np.array([near[k % len(near)] for k in range(n)], F)
     got = np.where(steps == 0, got, (got.view(np.int32) + steps).astype(np.int32).view(F))
     return np.ldexp(got, rng.integers(-20, 3, n) - 24).astype(F)
 
@@ -44,15 +57,23 @@ def gate_case(shape, fill):
     return case
 
 
+def off_the_middle(x, d):
+    """How far x / d is from the nearest middle between two floats, in last places of the quotient, exactly."""
+    q = abs(Fraction(float(x)) / Fraction(float(d)))
+    ulp = Fraction(float(np.spacing(F(float(q)))))
+    return abs(q / ulp - q // ulp - Fraction(1, 2))
+
+
 def test_near_midpoints_are_that_near():
-    """The oracle's side: what the dividends are said to be."""
+    """The oracle's side: every divisor has such dividends, they are as near as said, and they are among those used."""
     rng = np.random.default_rng(1)
-    for d in uniform(3, 50, 0.3, 3.0):
-        x = near_midpoints(d, rng, 64).astype(np.float64)
-        q = x / np.float64(d)
-        ulp = np.abs(np.spacing(q.astype(F)).astype(np.float64))
-        off = np.abs(np.abs(q - q.astype(F)) / ulp - 0.5)
-        assert off.min() < 2.0 ** -20 or (x > 0).all()
+    for d in np.concatenate([uniform(3, 200, 0.3, 3.0), np.array([3, 5, 1.5, 0.75, 16777215], F)]):
+        near = nearest_dividends(d)
+        assert near
+        for a in near:
+            assert off_the_middle(F(a), d) == Fraction(1, 2 * odd_mantissa(d))
+        x = near_midpoints(d, rng, 64)
+        assert np.all(np.isfinite(x)) and min(off_the_middle(v, d) for v in x) == Fraction(1, 2 * odd_mantissa(d))
 
 
 @pytest.mark.gpu
