@@ -5,7 +5,8 @@
 // Each routine is written with IEEE-754 fp32/fp64 operations and integer bit
 // manipulation only, so gfx950 and the host evaluate it identically as long as
 // the compiler neither contracts a*b+c nor reassociates.  fma() appears only
-// where the host library's selected variant fuses.  The same text is compiled
+// where the host library's selected variant fuses, and in expf_main, where a fused
+// addition and Horner's form round to the same float.  The same text is compiled
 // by the host C++ compiler for exhaustive comparison against the host's libm.
 //
 //   exact_expf  : ARM optimized-routines expf as shipped in glibc

@@ -31,6 +31,9 @@ float ref_erf(float x) { return std::erf(x); }
 float ref_softplus(float x) { return std::log1p(std::exp(x)); }
 float ref_gelu(float x) { return 0.5f * x * (1 + std::erf(0.707107f * x)); }
 
+// exact_expf_nonpositive over the inputs it is meant for
+float exp_nonpositive(float x) { return x > 0 ? ref_exp(x) : shdw::libm::exact_expf_nonpositive(x, shdw::libm::kExp2fTab); }
+
 struct Pair {
   fn1 mine, ref;
 };
@@ -53,6 +56,7 @@ Pair pick(int id) {
     case 12: return {exact_softplusf, ref_softplus};
     case 13: return {exact_geluf, ref_gelu};
     case 14: return {exact_tanf, ref_tan};
+    case 15: return {exp_nonpositive, ref_exp};
     default: return {nullptr, nullptr};
   }
 }

@@ -13,7 +13,8 @@ import pytest
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 FUNCS = {"exp": 0, "tanh": 1, "sigmoid": 2, "expm1": 3, "log": 4, "sin": 5, "cos": 6, "atan": 7,
-         "asin": 8, "acos": 9, "log1p": 10, "erf": 11, "softplus": 12, "gelu": 13, "tan": 14}
+         "asin": 8, "acos": 9, "log1p": 10, "erf": 11, "softplus": 12, "gelu": 13, "tan": 14,
+         "exp_nonpositive": 15}
 # float bit patterns where the restated algorithms switch paths
 EDGES = [0x00000000, 0x00800000, 0x04000000, 0x24000000, 0x24800000, 0x31000000, 0x31800000,
          0x32000000, 0x32800000, 0x33000000, 0x39000000, 0x39800000, 0x3eb17218, 0x3ed413d7,
