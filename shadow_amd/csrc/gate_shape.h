@@ -16,8 +16,8 @@ struct GateShape {
   int slots;
 };
 
-// Five workgroups on a CU: the tile and 2.5 KB of parameters, table and partial sums each
-// (28.5 KB of 160), as many as the registers of eight vectors a lane leave room for
+// Five workgroups on a CU: the tile and 3.5 KB of parameters, table and partial sums each
+// (28.9 KB of 160), as many as the registers of eight vectors a lane leave room for
 // (gate_waves).  Rows that do not fit whole go through LDS in chunks (four of the
 // 112x112 planes' rows per CU instead of three, [16,64,112,112] 124 -> 81 us; with 18 KB
 // eight 28x28 planes would be cut too, [32,512,28,28] 26.0 -> 28.1), unless there are no

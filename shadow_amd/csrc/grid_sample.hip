@@ -62,8 +62,10 @@ __global__ __launch_bounds__(kBlock) void grid_sample_kernel(const float* x, con
   const float* src = x + (static_cast<size_t>(b) * channel + c0) * in_plane;
   float* dst = y + (static_cast<size_t>(b) * channel + c0) * out_plane + s;
   // Stores carry the streams' hint, and the reads of a whole share of channels are under way before
-  // the first of them is used: bilinear [64,256,56,56] 119 -> 68.5 us, [8,64,112,112] 12.6 -> 11.0,
-  // of which the reads' part is 119 -> 107 and 12.6 -> 12.0.
+  // the first of them is used.  Along a flow, neither / the hint / both, operands new in every call: bilinear
+  // [64,256,56,56] 118 / 113 / 106 us, [8,64,112,112] 18.1 / 16.4 / 14.7, [16,64,80,80] 16.4 / 15.0 / 13.5.  A grid that
+  // points anywhere gains as long as the input is large ([64,256,56,56] 252 / 247 / 225) and loses by the
+  // reads where it is small ([8,20,57,57] 5.2 / 5.1 / 6.0, [8,9,112,112] 12.3 / 11.8 / 12.8).
   const auto store = [&](int c, float v) { __builtin_nontemporal_store(v, dst + static_cast<size_t>(c) * out_plane); };
   const float src_h_f = (gy + 1) / 2.f * static_cast<float>(in_h - 1);
   const float src_w_f = (gx + 1) / 2.f * static_cast<float>(in_w - 1);

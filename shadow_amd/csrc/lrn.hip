@@ -144,7 +144,7 @@ SHDW_DEVICE float lrn_walk(const float (&own)[kLrnRound], const float (&prev)[SI
 //
 // STREAM: the stores carry the streams' hint; not where rows of positions start inside a vector, whose
 // pieces of lines would leave one by one ([44,96,55,55] 32.6 us plain, 34.0 with it, [68,256,27,27] 35.0
-// and 40.5; [64,256,56,56] 93.2 and 82.1, [256,64,14,14] 11.8 and 10.5).
+// and 40.5; [64,256,56,56] 93.2 and 82.1, [256,64,14,14] 11.8 and 10.5, all with four waves a position).
 template <int SIZE, int WAVES, bool STREAM>
 __global__ __launch_bounds__(kBlock, 5) void lrn_window_kernel(const float* x, float* y, uint32_t positions, uint32_t step,
                                                                uint32_t channels, float alpha_over_size, float neg_beta,
@@ -353,10 +353,11 @@ extern "C" int shdw_hip_lrn(const int* in_shape, int size, float alpha, float be
     return launch_status();
   }
   // A tensor with few positions has few waves, and each walks all the channels one round after
-  // the other (82 us for 256 channels, however few the waves).  Up to eight workgroups then share
-  // the rounds of a position, about 4096 waves in all and four rounds each at the least; measured
-  // on 12.8 M elements, with windows in registers: [16,256,56,56] (784 waves) 82 -> 65, 56, 60, 77 us with 2, 4, 8, 16 shares,
-  // [44,96,55,55] (2080 waves) 49 -> 42, 47, 55; [64,256,56,56] (3136 waves) 141 -> 139, 149.
+  // the other (72 us for 256 channels, however few the waves).  Up to eight workgroups then share
+  // the rounds of a position, about 4096 waves in all and four rounds each at the least.  A window of nine
+  // with 1 / 2 / 4 / 8 / 16 shares: [1,256,56,56] (49 waves) 72 / 56 / 49 / 45 / 43 us, [4,256,56,56] 72 / 57 / 50 / 48 / 49,
+  // [16,256,56,56] (784) 82 / 71 / 67 / 78 / 105, [44,96,55,55] (2080) 44 / 42 / 49 / 64 / 95, [64,256,56,56] (3136)
+  // 126 / 137 / 162; of 31 [44,96,55,55] 47 / 51 / 56, [16,256,56,56] 83 / 72 / 68.
   // In place a workgroup would overwrite what another still has to read: one share.
   const uint32_t waves = (positions + kWave - 1) / kWave;
   const uint32_t rounds = (chan + static_cast<uint32_t>(post) + kLrnRound - 1) / kLrnRound;

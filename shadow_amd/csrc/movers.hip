@@ -289,7 +289,7 @@ static bool shared_rows(const float* x, uint32_t cols, uint32_t tile_cols, uint3
 // whole thin side and `span` elements of the long one; the side that is
 // contiguous in memory moves with 128-bit accesses as it lies, the element
 // shuffle happens in LDS.
-constexpr uint32_t kThinMax = 127;         // thin side up to this many elements: the tile keeps 64 and more of the long side
+constexpr uint32_t kThinMax = 127;         // thin side up to this many elements: a tile has room for 64 and more of the long side
 constexpr uint32_t kThinNarrow = 16;       // ... and sides of 17 to 64 stay with the 64 x 64 tiles
 constexpr uint32_t kThinTileFloats = 8192;  // 32 KB
 
@@ -1223,8 +1223,9 @@ int shdw_hip_permute(int num_axes, const int* in_shape, const int* order, const 
       if (span && groups <= INT32_MAX) {
         const FastDiv ft = make_fastdiv(tiles), fthin = make_fastdiv(thin);
         const uint32_t g = static_cast<uint32_t>(groups);
-        // tiles of a side of up to 15 rows keep 512 and more of the other, little of it shared:
-        // [64,3,50625] 18.6 us plain and 18.4 with the hint, [64,8,12321] 11.0 both
+        // tiles of a side of up to 15 rows hold 512 and more of the other, little of it shared: [64,3,50625]
+        // 18.6 us plain and 18.4 with the hint, [64,8,12321] 11.0 both; where they are made shorter the
+        // call takes four microseconds either way ([1,8,4225] 4.0 / 3.9, [16,5,4225] 4.3 / 4.1, [64,8,729] 4.3 / 4.2)
         const bool shared = thin >= 16 && shared_rows(x, big, span, 32);
         if (cols_thin && pad)
           transpose_thin_kernel<true, true, false><<<g, kBlock, 0, st>>>(x, y, big, fthin, span, ft);

@@ -2,9 +2,11 @@
 // over `dim` for every (outer, inner) column and then applied to the column.
 //
 // Shadow folds each column front to back (an fp32 running sum for Softmax, an
-// fp64 one for Normalize); both are order-dependent, so a column is always
-// folded by ONE lane in that order and the results match bit for bit.  Two
-// layouts keep the global accesses coalesced around that constraint:
+// fp64 one for Normalize); both are order-dependent.  A column is folded by one lane
+// in that order, or by lanes that hold consecutive pieces of it and take turns (Softmax
+// over the last axis), or in any order where the result provably cannot depend on it
+// (maxima; Normalize's tiles, norm_settled), so the results match bit for bit.
+// The first two of the layouts that keep the global accesses coalesced around that:
 //   * columns : inner >= 64 (or a slab too large for LDS).  Lane = column,
 //               neighbouring lanes read neighbouring addresses.
 //   * slab    : inner < 64.  One workgroup per outer index copies its
@@ -1259,9 +1261,11 @@ static void launch_normalize_tile(int outer_num, int dim, int inner_num, float p
                                   const float* scale, float* y, hipStream_t st) {
   // 64 positions per tile row while a lane has at most eight vectors of them (up to 128 rows; the kernel
   // holds no more of these, so that eight waves fit a SIMD: [32,96,3025] 18.9 -> 13.7 us, [16,128,5625]
-  // 22.2 -> 17.2 with a factor a row), else 32, up to 16 vectors, else 16.  Measured when the columns were walked out of a tile in
-  // LDS: [64,256,56,56] 85 us with 64 positions, 80 us with 32; [64,512,38,38] 105 us with 32, 115
-  // with 16.  Softmax takes the widest tile that fits.
+  // 22.2 -> 17.2 with a factor a row), else 32, up to 16 vectors, else 16.  With 64 / 32 / 16 positions, factors:
+  // [32,100,3136] 14.4 / 20.4 / -, [16,128,5625] 17.1 / 23.8 / -, [1,100,3136] 4.6 / 4.6 / -; sixteen vectors of 64:
+  // [16,200,3136] 15.4 / 18.9 / 25.0, [16,256,3136] 19.4 / 22.0 / 30.2, but [64,256,3136] 75.4 / 75.6 / 104.2,
+  // [64,256,361] 14.3 / 12.0 / 14.9, [16,256,1444] 12.1 / 11.0 / 14.4, [1,256,3136] 6.7 / 5.4 / 5.0; [16,512,38,38] - / 17.0 /
+  // 26.7, [1,512,1444] - / 7.7 / 6.3.  Softmax takes the widest tile that fits.
   const int shift = normalize_tile_shift(dim);
   if (shift == 6)
     launch_normalize_tile_ts<PMODE, SM, 6>(outer_num, dim, inner_num, p, eps, x, scale, y, st);
