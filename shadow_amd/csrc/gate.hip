@@ -13,8 +13,8 @@
 //
 // What bounds it: five workgroups on a CU (LDS and registers), whose loads, ordered
 // sums (784 dependent additions: 3 us; without them [32,512,28,28] takes 22.9 us instead of
-// 27) and stores overlap each other's, and 20 vector instructions an element.  One block
-// with its tail takes, per call: [32,512,28,28]
+// 27) and stores overlap each other's, and 47 vector instructions an element (7x7 planes 61, 112x112
+// in chunks 100).  One block with its tail takes, per call: [32,512,28,28]
 // (103 MB) 26.5 us (28.7 with the quotients in fp32 and the row's parameters read for every
 // vector), where its five launches took 78; [64,64,56,56] 44; [64,512,14,14]
 // 12.1; [64,1024,7,7] 8.8; [16,64,112,112] 72 and [16,64,96,96] 54, both in chunks (their sums
