@@ -1281,12 +1281,11 @@ static void launch_normalize_tile(int outer_num, int dim, int inner_num, float p
 //
 // The maxima are taken in any order: from the lanes' own rows, then over the lanes and the
 // waves (a NaN anywhere in a column makes all of it NaN whatever the maximum was).  The sum of
-// the exponentials is an fp32 running sum and is always walked in index order, by one wave; which
-// of the four changes from one group of 256 workgroups to the next, since wave i of every
-// workgroup of a CU is on the same SIMD and walks that share one take turns.
+// the exponentials is an fp32 running sum and is always walked in index order, by wave 0 (the four waves
+// taking turns from workgroup to workgroup or from 256 to 256: level, 24.9 / 24.6 / 24.6 us here).
 //
-// [16,150,72,72], 99.5 MB: 23.6 us.  Its vector instructions bound it together with the rounds of
-// load, walk and store (the exponential 17 an element, the quotient 4); 28.4 us with the maxima by
+// [16,150,72,72], 99.5 MB: 24.6 us.  Its vector instructions bound it together with the rounds of
+// load, walk and store (29 an element by the counters); 28.8 us with the maxima by
 // compare and select, a division and the longer exponential, and five barriers.
 template <int TS_SHIFT, int ROWS>
 __global__ __launch_bounds__(kBlock) void softmax_tile_kernel(const float* x, float* y, uint32_t dim,
@@ -1340,8 +1339,8 @@ __global__ __launch_bounds__(kBlock) void softmax_tile_kernel(const float* x, fl
     }
   }
   __syncthreads();  // also: every lane has its maxima before the sums replace them
-  if (wave == blockIdx.x / kBlock % kWaves) {
-    const uint32_t pos = threadIdx.x % kWave;
+  if (wave == 0) {
+    const uint32_t pos = threadIdx.x;
     if (pos < width) {
       __builtin_amdgcn_s_setprio(3);
       const float sum = fold_tile_column<TS_SHIFT>(lds + pos, dim, 0.f, [](float a, float v) { return a + v; });
