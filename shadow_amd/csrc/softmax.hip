@@ -931,6 +931,7 @@ __global__ __launch_bounds__(kBlock) void normalize_packed_kernel(const float* x
 // lane, which run at the address-unit rate: 185 us against 84 us on
 // [64,150,73,73] / [64,150,72,72]).  Neighbouring tiles share the straddled
 // lines, hence the XCD-contiguous workgroup order.
+constexpr uint32_t kTileMaxRows = 1024;
 constexpr int kTilePerLane = 16;  // 64 KB / (256 lanes x 16 bytes)
 
 // ROWS says how the tile rows lie in memory:
@@ -1090,7 +1091,7 @@ SHDW_DEVICE float strided_lane_max(float m) {
 // each column, and only if that does not settle all of them adds up in order.  18-bit numbers, p = 1, on
 // [16,512,38,38] 17.8 us (always in order 23.4), one column that needs the order on [2,512,400] 14.8 (others 7.5),
 // every column on [16,512,38,38] 25.5.
-template <int PMODE, int SM, int TS_SHIFT, int ROWS>
+template <int PMODE, int SM, int TS_SHIFT, int ROWS, bool FEW>
 __global__ __launch_bounds__(kBlock, TS_SHIFT == 6 ? 7 : SM == kSsdChannelScale ? 4 : 5) void normalize_tile_kernel(const float* x, float* y, uint32_t dim,
                                                                  uint32_t inner, const float* scale, float p,
                                                                  float eps, FastDiv f_tiles) {
@@ -1103,6 +1104,7 @@ __global__ __launch_bounds__(kBlock, TS_SHIFT == 6 ? 7 : SM == kSsdChannelScale 
   __shared__ __align__(16) float handed[TS];
   __shared__ __align__(16) float chunk[Lane::STEP * TS];
   __shared__ uint64_t unsettled;  // a bit a position
+  __shared__ float factors[FEW ? kTileMaxRows : 1];
   uint32_t n, tile;
   fd_divmod(xcd_contiguous(blockIdx.x, gridDim.x), f_tiles, n, tile);
   const uint32_t p0 = tile << TS_SHIFT;
@@ -1121,15 +1123,24 @@ __global__ __launch_bounds__(kBlock, TS_SHIFT == 6 ? 7 : SM == kSsdChannelScale 
       for (int k = 0; k < 4; ++k) acc[k] += static_cast<double>(lane.has(u) ? term(r[u][k]) : 0.f);
     }
   }
-  // the rows' factors are asked for when the rows are through: [16,512,38,38] 18.6 -> 17.2 us, [1,512,1444] 9.5 -> 7.8
-  float factor[kPerLane];
-  if (SM == kSsdChannelScale) {
+  // The rows' factors are asked for when the rows are through: [16,512,38,38] 18.6 -> 17.2 us, [1,512,1444] 9.5 -> 7.8.
+  // FEW (launch_normalize_tile_ts): one load a lane and the rest through LDS, in place of one for every row.
+  constexpr int kFactors = kTileMaxRows / kBlock;
+  float factor[kPerLane], few_factors[kFactors];
+  if (FEW) {
+#pragma unroll
+    for (int k = 0; k < kFactors; ++k) few_factors[k] = scale[min(k * kBlock + threadIdx.x, dim - 1)];
+  } else if (SM == kSsdChannelScale) {
 #pragma unroll
     for (int u = 0; u < kPerLane; ++u)
       if (lane.step(u)) factor[u] = scale[lane.row(u)];
   }
 #pragma unroll
   for (int k = 0; k < 4; ++k) acc[k] = strided_lane_sum<Lane::LANES_PER_ROW>(acc[k]);
+  if (FEW) {
+#pragma unroll
+    for (int k = 0; k < kFactors; ++k) factors[k * kBlock + threadIdx.x] = few_factors[k];
+  }
   if (threadIdx.x % kWave < Lane::LANES_PER_ROW) {
 #pragma unroll
     for (int k = 0; k < 4; ++k) partial[threadIdx.x / kWave][lane.j + k] = acc[k];
@@ -1212,7 +1223,7 @@ __global__ __launch_bounds__(kBlock, TS_SHIFT == 6 ? 7 : SM == kSsdChannelScale 
     const uint32_t c = lane.c0 + u * Lane::STEP;
     v4f v = q(r[u]);
 #pragma unroll
-    for (int k = 0; k < 4; ++k) v[k] = SM == kSsdChannelScale ? v[k] * factor[u] : ssd_scaled<SM>(v[k], scale, c);
+    for (int k = 0; k < 4; ++k) v[k] = SM == kSsdChannelScale ? v[k] * (FEW ? factors[c] : factor[u]) : ssd_scaled<SM>(v[k], scale, c);
     lane.store(y + base, u, v);
   }
 }
@@ -1236,23 +1247,39 @@ static bool tile_fits(int dim, int inner_num, bool softmax) {
   return inner_num >= (softmax ? kTileMinInnerTallSoftmax : kTileMinInnerTallNormalize);
 }
 
+template <int PMODE, int SM, int TS_SHIFT, bool FEW>
+static void launch_normalize_tile_rows(uint32_t grid, uint32_t tiles, int dim, int inner_num, float p, float eps, const float* x,
+                                       const float* scale, float* y, hipStream_t st) {
+  const uint32_t d = static_cast<uint32_t>(dim), in = static_cast<uint32_t>(inner_num);
+  const FastDiv ft = make_fastdiv(tiles);
+  switch (tile_rows(inner_num, y)) {
+    case kRowsSector:
+      normalize_tile_kernel<PMODE, SM, TS_SHIFT, kRowsSector, FEW><<<grid, kBlock, 0, st>>>(x, y, d, in, scale, p, eps, ft);
+      break;
+    case kRowsQuad:
+      normalize_tile_kernel<PMODE, SM, TS_SHIFT, kRowsQuad, FEW><<<grid, kBlock, 0, st>>>(x, y, d, in, scale, p, eps, ft);
+      break;
+    default:
+      normalize_tile_kernel<PMODE, SM, TS_SHIFT, kRowsAny, FEW><<<grid, kBlock, 0, st>>>(x, y, d, in, scale, p, eps, ft);
+  }
+}
+
+// Tall tiles (513 rows and more, sixteen vectors a lane) with a factor a row, up to two a CU: the loads of a lane's
+// sixteen factors are what such a tile waits for.  A load a row / through LDS: [1,951,1681] 11.4 / 9.5 us,
+// [1,600,1681] 8.4 / 7.1, [8,1024,361] 12.4 / 10.6, [4,700,1000] 9.1 / 8.7, [3,800,77] 8.5 / 6.7, [2,1024,4096] (512 tiles) 20.6 /
+// 20.1; beyond, where the chip is full, [1,800,10000] 15.6 / 17.3, [16,1000,729] 22.1 / 27.2, [16,600,1600] 36.6 / 37.5.
+constexpr uint32_t kFewTiles = 512;
+
 template <int PMODE, int SM, int TS_SHIFT>
 static void launch_normalize_tile_ts(int outer_num, int dim, int inner_num, float p, float eps, const float* x,
                                      const float* scale, float* y, hipStream_t st) {
   const uint32_t tiles = (static_cast<uint32_t>(inner_num) + (1u << TS_SHIFT) - 1) >> TS_SHIFT;
   const uint32_t grid = static_cast<uint32_t>(outer_num) * tiles;
-  const uint32_t d = static_cast<uint32_t>(dim), in = static_cast<uint32_t>(inner_num);
-  const FastDiv ft = make_fastdiv(tiles);
-  switch (tile_rows(inner_num, y)) {
-    case kRowsSector:
-      normalize_tile_kernel<PMODE, SM, TS_SHIFT, kRowsSector><<<grid, kBlock, 0, st>>>(x, y, d, in, scale, p, eps, ft);
-      break;
-    case kRowsQuad:
-      normalize_tile_kernel<PMODE, SM, TS_SHIFT, kRowsQuad><<<grid, kBlock, 0, st>>>(x, y, d, in, scale, p, eps, ft);
-      break;
-    default:
-      normalize_tile_kernel<PMODE, SM, TS_SHIFT, kRowsAny><<<grid, kBlock, 0, st>>>(x, y, d, in, scale, p, eps, ft);
-  }
+  constexpr bool kMayBeFew = TS_SHIFT == 4 && SM == kSsdChannelScale;
+  if (kMayBeFew && grid <= kFewTiles)
+    launch_normalize_tile_rows<PMODE, SM, TS_SHIFT, kMayBeFew>(grid, tiles, dim, inner_num, p, eps, x, scale, y, st);
+  else
+    launch_normalize_tile_rows<PMODE, SM, TS_SHIFT, false>(grid, tiles, dim, inner_num, p, eps, x, scale, y, st);
 }
 
 static int normalize_tile_shift(int dim);

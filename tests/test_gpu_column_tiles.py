@@ -113,3 +113,14 @@ def test_negative_eps_next_to_the_sum(gpu, outer, dim, inner):
         for e in (-1.0, -eps, -eps * (1 + 2.0 ** -20), -eps * (1 - 2.0 ** -20), -1e9):
             want = oracle.ssd_normalize(x, outer, dim, inner, False, True, e, None)
             assert_bit_exact(gpuops.ssd_normalize(x, outer, dim, inner, False, True, e, None), want, "eps %g" % e)
+
+
+# a factor a row on tall tiles: up to 512 of them take the factors through LDS
+@pytest.mark.gpu
+@pytest.mark.parametrize("outer,dim,inner", [(1, 513, 8192), (1, 513, 8193), (2, 700, 4094), (3, 1024, 77), (1, 951, 1681), (2, 1023, 64), (2, 601, 4112)])
+def test_factors_of_tall_tiles(gpu, outer, dim, inner):
+    x = normal(8, outer * dim * inner, 2.0)
+    scale = uniform(9, dim, 0.5, 2.0)
+    want = oracle.ssd_normalize(x, outer, dim, inner, False, False, 1e-10, scale)
+    assert_bit_exact(gpuops.ssd_normalize(x, outer, dim, inner, False, False, 1e-10, scale), want, "ssd")
+    assert_bit_exact(gpuops.ssd_normalize(x, outer, dim, inner, False, False, 1e-10, scale, inplace=True, offset=1), want, "ssd in place")
