@@ -1,0 +1,129 @@
+// The fp32 running sum of a row, front to back, by a whole wave: the bits of
+//   for (i = 0; i < n; ++i) sum += v[i];
+// for terms that are not negative, without n additions that wait for one another.
+//
+// While a running sum stays between two powers of two, 2^e <= sum < 2^(e+1), it is a multiple
+// of one unit u (its last place), and rounding sum + v to such a multiple depends on sum in one
+// respect only: a tie goes to the even multiple.  A run of terms therefore adds one of two
+// numbers of units to any such sum, one where its last bit is 0 and one where it is 1, and these
+// two can be had by adding the terms to 2^e and to 2^e + u.  Read as an integer, a float's bits
+// count units: the run takes the bits b to b + (b & 1 ? odd : even).  Two runs of the same e
+// make one (the second's number is chosen by the first's last bit), so 64 lanes' runs make
+// one in six steps.
+//
+// Each lane has a guess of the sum that reaches it, from the lanes' sums in any order: of that only
+// e is used.  The true sum then goes through the lanes: over lanes of one e at once, from the
+// guessed power of two on (checked: the sum in front of them and the sum behind them must both lie
+// there, and as no term is negative every sum between them does), and by adding a lane's terms
+// one after the other where the sum passes a power of two inside it, or where a guess was wrong.
+// A row of n equal terms passes log2(n) powers of two, half of them in its first lane's terms.
+#ifndef SHADOW_AMD_CSRC_ORDERED_SUM_H_
+#define SHADOW_AMD_CSRC_ORDERED_SUM_H_
+
+#include "device_common.h"
+
+namespace shdw {
+
+constexpr uint32_t kBinade = 1u << 23, kExponentBits = 0x7f800000u;
+
+// What a lane's terms add to bits below a power of two, for even and odd ones; `first`: nothing in front of this
+// lane is included (`even` and `odd` are of its own terms alone).
+struct UnitRun {
+  uint32_t even, odd, first;
+};
+
+// The lanes named by the DPP control in front of this lane's own; lanes without such a lane keep theirs.
+template <int CTRL, int ROWS>
+SHDW_DEVICE void join_run(UnitRun& r) {
+  const auto moved = [](uint32_t v) {
+    return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), CTRL, ROWS, 0xf, false));
+  };
+  const uint32_t even = moved(r.even), odd = moved(r.odd), first = moved(r.first);
+  const uint32_t joined_even = even + (even & 1u ? r.odd : r.even);
+  const uint32_t joined_odd = odd + (odd & 1u ? r.even : r.odd);
+  r.even = r.first ? r.even : joined_even;
+  r.odd = r.first ? r.odd : joined_odd;
+  r.first |= first;
+}
+
+template <int CTRL, int ROWS>
+SHDW_DEVICE float add_lane(float v) {
+  return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, ROWS, 0xf, false));
+}
+
+constexpr int kDppShr1 = 0x111, kDppShr2 = 0x112, kDppShr4 = 0x114, kDppShr8 = 0x118;  // inside 16 lanes
+constexpr int kDppBcast15 = 0x142, kDppBcast31 = 0x143;  // the last lane of 16, of 32, to the 16, 32 behind them
+
+// sum + v[0] + v[1] + ... of lane 0, then of lane 1, ...: the same sum in all lanes.  All 64 lanes call it, with
+// the same sum; neither it nor any term is negative or NaN (infinities are fine).
+template <int K>
+SHDW_DEVICE float wave_sum_in_order(const float (&v)[K], float sum) {
+  float own[4] = {v[0], v[1], v[2], v[3]};
+  static_assert(K % 4 == 0 && K >= 4, "");
+#pragma unroll
+  for (int k = 4; k < K; ++k) own[k % 4] += v[k];
+  const float mine = (own[0] + own[1]) + (own[2] + own[3]);
+  float upto = mine;
+  upto = add_lane<kDppShr1, 0xf>(upto);
+  upto = add_lane<kDppShr2, 0xf>(upto);
+  upto = add_lane<kDppShr4, 0xf>(upto);
+  upto = add_lane<kDppShr8, 0xf>(upto);
+  upto = add_lane<kDppBcast15, 0xa>(upto);
+  upto = add_lane<kDppBcast31, 0xc>(upto);
+  const float before = sum + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(upto), kDppWaveShr1, 0xf, 0xf, false));
+  const uint32_t power = __float_as_uint(before) & kExponentBits;
+  const uint32_t guess = __float_as_uint(before) & ~1u;  // lane 0's is the sum's own, so its terms are added to the sum itself
+  float from_even = __uint_as_float(guess), from_odd = __uint_as_float(guess | 1u);
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    from_even += v[k];
+    from_odd += v[k];
+  }
+  UnitRun run{__float_as_uint(from_even) - guess, __float_as_uint(from_odd) - (guess | 1u), 0};
+  // passes: this lane's terms are added one by one; first: at, and behind, such a lane, and where e changes
+  const uint32_t lane_id = threadIdx.x % kWave;
+  const bool passes = lane_id == 0 || power == kExponentBits ||
+                      max(__float_as_uint(from_even), __float_as_uint(from_odd)) - power >= kBinade;
+  const uint32_t tag = passes ? 1u : power;  // of the powers none is 1
+  const uint32_t tag_before = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(1, static_cast<int>(tag), kDppWaveShr1, 0xf, 0xf, false));
+  const bool starts = passes || tag != tag_before;
+  run.first = starts ? 1u : 0u;
+  join_run<kDppShr1, 0xf>(run);
+  join_run<kDppShr2, 0xf>(run);
+  join_run<kDppShr4, 0xf>(run);
+  join_run<kDppShr8, 0xf>(run);
+  join_run<kDppBcast15, 0xa>(run);
+  join_run<kDppBcast31, 0xc>(run);
+
+  const uint64_t all_starts = __builtin_amdgcn_ballot_w64(starts), all_passes = __builtin_amdgcn_ballot_w64(passes);
+  uint32_t bits = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(__float_as_int(sum)));
+  const auto of_lane = [](uint32_t value, uint32_t lane) {
+    return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(value), static_cast<int>(lane)));
+  };
+  bits = bits & 1u ? of_lane(__float_as_uint(from_odd), 0) : of_lane(__float_as_uint(from_even), 0);
+  uint32_t lane = 1;
+  while (lane < kWave) {  // the same for all lanes; every turn is of one lane at least
+    const uint64_t later = lane + 1 < kWave ? all_starts >> (lane + 1) : 0;
+    const uint32_t end = later ? lane + 1 + static_cast<uint32_t>(__builtin_ctzll(later)) : kWave;
+    if ((all_passes >> lane & 1u) == 0) {
+      const uint32_t low = of_lane(power, lane);
+      const uint32_t next = bits + (bits & 1u ? of_lane(run.odd, end - 1) : of_lane(run.even, end - 1));
+      if (bits - low < kBinade && next - low < kBinade) {
+        bits = next;
+        lane = end;
+        continue;
+      }
+    }
+    for (; lane < end; ++lane) {
+      float s = __uint_as_float(bits);
+#pragma unroll
+      for (int k = 0; k < K; ++k) s += v[k];
+      bits = of_lane(__float_as_uint(s), lane);
+    }
+  }
+  return __uint_as_float(bits);
+}
+
+}  // namespace shdw
+
+#endif  // SHADOW_AMD_CSRC_ORDERED_SUM_H_

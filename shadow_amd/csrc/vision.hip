@@ -15,6 +15,7 @@
 #include "../../include/shadow_hip.h"
 #include "device_common.h"
 #include "launch.h"
+#include "ordered_sum.h"
 
 #pragma clang fp contract(off)
 
@@ -1221,20 +1222,19 @@ constexpr int kSpanPitch = kSpan + 4;  // in LDS: 128-bit accesses of 16 neighbo
 constexpr int kStreamVectors = kSpan / 4;  // per lane and chunk
 constexpr int kStreamWaves = kBlock / kWave;
 
+// A wave's G rows from row0 on, a chunk of W columns at a time: requested, then through LDS into `mine`,
+// kSpan consecutive columns of a row a lane.
 template <int G>
-__global__ __launch_bounds__(kBlock) void pool_rows_stream_kernel(const float* x, float* y, uint32_t rows,
-                                                                   uint32_t len, float pool_size) {
-  constexpr uint32_t L = kWave / G, W = kSpan * L, VW = W / 4;
-  __shared__ __align__(16) float tiles[kStreamWaves][kWave * kSpanPitch];
-  const uint32_t lane = threadIdx.x % kWave;
-  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  float* tile = tiles[wave];
-  const uint32_t row0 = (blockIdx.x * kStreamWaves + wave) * G;
-  if (row0 >= rows) return;  // the whole wave
+struct PlaneRows {
+  static constexpr uint32_t L = kWave / G, W = kSpan * L, VW = W / 4;
+  const float* x;
+  float* tile;
+  uint32_t row0, rows, len, lane;
   v4f reg[kStreamVectors];
+
   // No branch around a load: vectors past the end of a row take its last four elements (rows
   // have 256 and more), rows past the end take the last row.
-  auto request = [&](uint32_t c0) {
+  SHDW_DEVICE void request(uint32_t c0) {
     const float* at = x + static_cast<uint64_t>(row0) * len;
     const uint32_t last_row = rows - 1 - row0;
 #pragma unroll
@@ -1242,15 +1242,13 @@ __global__ __launch_bounds__(kBlock) void pool_rows_stream_kernel(const float* x
       const uint32_t v = lane + kWave * i;
       reg[i] = load4_stream_any(at + (min(v / VW, last_row) * len + min(c0 + 4 * (v % VW), len - 4)));
     }
-  };
-  float sum = 0.f;
-  uint32_t turns = 0;
-  request(0);
-  for (uint32_t c0 = 0; c0 < len; c0 += W) {
-    auto slot = [&](int i) {
-      const uint32_t v = lane + kWave * i, c = 4 * (v % VW);
-      return tile + (v / VW * L + c / kSpan) * kSpanPitch + c % kSpan;
-    };
+  }
+  SHDW_DEVICE float* slot(int i) const {
+    const uint32_t v = lane + kWave * i, c = 4 * (v % VW);
+    return tile + (v / VW * L + c / kSpan) * kSpanPitch + c % kSpan;
+  }
+  // The requested chunk c0 into `mine`, and the next one requested.
+  SHDW_DEVICE void take(uint32_t c0, float (&mine)[kSpan]) {
     if (c0 + W <= len) {
 #pragma unroll
       for (int i = 0; i < kStreamVectors; ++i) *reinterpret_cast<v4f*>(slot(i)) = reg[i];
@@ -1269,22 +1267,84 @@ __global__ __launch_bounds__(kBlock) void pool_rows_stream_kernel(const float* x
     }
     __builtin_amdgcn_wave_barrier();
     if (c0 + W < len) request(c0 + W);
-    v4f mine[kStreamVectors];
 #pragma unroll
-    for (int i = 0; i < kStreamVectors; ++i) mine[i] = *reinterpret_cast<const v4f*>(tile + lane * kSpanPitch + 4 * i);
-    if (c0 != 0) sum = __shfl(sum, lane | (L - 1));  // from the last lane of the row to its first
-    turns = min(L, (len - c0 + kSpan - 1) / kSpan);
+    for (int i = 0; i < kStreamVectors; ++i) {
+      const v4f q = *reinterpret_cast<const v4f*>(tile + lane * kSpanPitch + 4 * i);
 #pragma unroll
-    for (int k = 0; k < kSpan; ++k) sum += mine[k / 4][k % 4];
-    for (uint32_t t = 1; t < turns; ++t) {
-      sum = dpp_f32<kDppWaveShr1>(sum);
-#pragma unroll
-      for (int k = 0; k < kSpan; ++k) sum += mine[k / 4][k % 4];
+      for (int j = 0; j < 4; ++j) mine[4 * i + j] = q[j];
     }
     __builtin_amdgcn_wave_barrier();
   }
-  const uint32_t row = row0 + lane / L;
-  if (lane % L == turns - 1 && row < rows) y[row] = sum / pool_size;
+};
+
+template <int G>
+__global__ __launch_bounds__(kBlock) void pool_rows_stream_kernel(const float* x, float* y, uint32_t rows,
+                                                                   uint32_t len, float pool_size) {
+  __shared__ __align__(16) float tiles[kStreamWaves][kWave * kSpanPitch];
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const uint32_t row0 = (blockIdx.x * kStreamWaves + wave) * G;
+  if (row0 >= rows) return;  // the whole wave
+  using Rows = PlaneRows<G>;
+  Rows r{x, tiles[wave], row0, rows, len, threadIdx.x % kWave, {}};
+  float mine[kSpan], sum = 0.f;
+  uint32_t turns = 0;
+  r.request(0);
+  for (uint32_t c0 = 0; c0 < len; c0 += Rows::W) {
+    r.take(c0, mine);
+    if (c0 != 0) sum = __shfl(sum, r.lane | (Rows::L - 1));  // from the last lane of the row to its first
+    turns = min(Rows::L, (len - c0 + kSpan - 1) / kSpan);
+#pragma unroll
+    for (int k = 0; k < kSpan; ++k) sum += mine[k];
+    for (uint32_t t = 1; t < turns; ++t) {
+      sum = dpp_f32<kDppWaveShr1>(sum);
+#pragma unroll
+      for (int k = 0; k < kSpan; ++k) sum += mine[k];
+    }
+  }
+  const uint32_t row = row0 + r.lane / Rows::L;
+  if (r.lane % Rows::L == turns - 1 && row < rows) y[row] = sum / pool_size;
+}
+
+// Whether some element is negative, -0 or NaN.
+SHDW_DEVICE bool any_sign(const float (&v)[kSpan]) {
+  uint32_t most = __float_as_uint(v[0]);
+#pragma unroll
+  for (int k = 1; k < kSpan; ++k) most = max(most, __float_as_uint(v[k]));
+  return most > kExponentBits;
+}
+
+// Few long rows, a wave each: where no element of a chunk is negative (what ReLU and the poolings behind
+// it leave) the chunk's additions are taken side by side (ordered_sum.h), otherwise lane by lane as
+// above.  Bound by latencies: the first loads, 64 dependent additions of a guess per chunk,
+// the joining of the lanes' runs (0.3 us) and the lanes where the sum passes a power of two (0.1 us
+// each, six in the first chunk).  Against the additions in turn (rows x columns): 3 x 50176 125 -> 29 us,
+// 512 x 12544 36.2 -> 12.0, 1024 x 3136 12.2 -> 6.9, 2048 x 3136 12.5 -> 8.8, 2048 x 12544 40.7 -> 19.1.
+// Rows of N(0, 1) take as long as before or less, up to 3 % more at 2048 rows of 3136.
+__global__ __launch_bounds__(kBlock, 4) void pool_rows_runs_kernel(const float* x, float* y, uint32_t rows,
+                                                                    uint32_t len, float pool_size) {
+  using Rows = PlaneRows<1>;
+  __shared__ __align__(16) float tiles[kStreamWaves][kWave * kSpanPitch];
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const uint32_t row = blockIdx.x * kStreamWaves + wave;
+  if (row >= rows) return;  // the whole wave
+  Rows r{x, tiles[wave], row, rows, len, threadIdx.x % kWave, {}};
+  float mine[kSpan], sum = 0.f;
+  r.request(0);
+  for (uint32_t c0 = 0; c0 < len; c0 += Rows::W) {
+    r.take(c0, mine);
+    if (__builtin_amdgcn_ballot_w64(any_sign(mine)) == 0 && sum >= 0.f) {
+      sum = wave_sum_in_order(mine, sum);
+      continue;
+    }
+    const uint32_t turns = min(static_cast<uint32_t>(kWave), (len - c0 + kSpan - 1) / kSpan);
+    for (uint32_t t = 0; t < turns; ++t) {
+      if (t != 0) sum = dpp_f32<kDppWaveShr1>(sum);
+#pragma unroll
+      for (int k = 0; k < kSpan; ++k) sum += mine[k];
+    }
+    sum = __shfl(sum, turns - 1);
+  }
+  if (r.lane == 0) y[row] = sum / pool_size;
 }
 
 // From this row length on the whole-plane average takes the streaming kernel
@@ -1304,8 +1364,19 @@ static int stream_rows_per_wave(uint32_t rows) {
   return g;
 }
 
+// Up to here a wave a row fills no more than two waves of a SIMD, and rows with signs lose nothing by not
+// sharing a wave (2500 x 3136 of N(0, 1) 12.6 us as eight rows a wave, 20.1 as one; without signs 12.6 and
+// 10.7); below 1152 columns the additions in turn are over as soon (2048 x 1024 5.5 us in turn, 5.9 side by
+// side, 2048 x 1200 6.5 and 5.9).
+constexpr uint32_t kRunsMaxRows = 2048, kRunsMinLen = 1152;
+
 static void launch_pool_rows_stream(const float* x, float* y, uint32_t rows, uint32_t len, hipStream_t st) {
   const float size = static_cast<float>(static_cast<int>(len));
+  if (rows <= kRunsMaxRows && len >= kRunsMinLen) {
+    const uint32_t grid = (rows + kStreamWaves - 1) / kStreamWaves;
+    pool_rows_runs_kernel<<<grid, kBlock, 0, st>>>(x, y, rows, len, size);
+    return;
+  }
   const int g = stream_rows_per_wave(rows);
   const uint32_t per_wg = static_cast<uint32_t>(g) * kStreamWaves;
   const uint32_t grid = (rows + per_wg - 1) / per_wg;

@@ -34,3 +34,37 @@ def test_whole_plane_average_of_special_values(gpu, length):
     args = ((5, 7, 1, length), 1, (1, length), (1, 1), (0, 0), (5, 7, 1, 1))
     with np.errstate(all="ignore"):
         assert_bit_exact(gpuops.pooling(x, *args), oracle.pooling(x, *args), "average")
+
+
+def rows_without_signs(seed, planes, length):
+    """Rows whose running sums pass powers of two in every way: sums that grow evenly, ties in
+    every addition, terms of all sizes, subnormal sums, sums that overflow, and a sign somewhere."""
+    rng = np.random.default_rng(seed)
+    x = np.maximum(rng.standard_normal((planes, length)), 0).astype(np.float32)
+    kinds = [lambda: np.full(length, 1.0),
+             lambda: np.ldexp(1.0, rng.integers(-24, 1, length)),                  # ties
+             lambda: np.ldexp(rng.random(length), rng.integers(-40, 41, length)),
+             lambda: np.ldexp(rng.integers(0, 9, length).astype(float), -149),     # subnormal all the way
+             lambda: rng.random(length) * 3e38,                                    # overflows
+             lambda: np.where(np.arange(length) < length // 2, 0.0, rng.random(length)),
+             lambda: np.where(np.arange(length) == 3 * length // 4, -50.0, rng.random(length)),
+             lambda: np.where(np.arange(length) == length - 1, np.inf, 0.1),
+             lambda: np.where(np.arange(length) == 40, -0.0, rng.random(length)),
+             lambda: np.where(np.arange(length) == 1, np.nan, 1.0),
+             lambda: np.where(np.arange(length) % 64 == 0, 2.0 ** 24, 1.0),
+             lambda: np.where(np.arange(length) == 0, 2.0 ** 24 - 1, 0.5)]
+    for r in range(min(planes, 5 * len(kinds))):
+        x[r] = kinds[r % len(kinds)]()
+    return x
+
+
+# lengths either side of where the additions are taken side by side, of a chunk, of a lane's span
+# and of whole vectors; planes either side of the most that a wave each is taken for
+@pytest.mark.parametrize("length", [1151, 1152, 1155, 2016, 2047, 2048, 2049, 4098, 6211])
+@pytest.mark.parametrize("planes", [60, 2048, 2049])
+def test_whole_plane_average_without_signs(gpu, planes, length):
+    x = rows_without_signs(planes + length, planes, length)
+    args = ((1, planes, 1, length), 1, (1, length), (1, 1), (0, 0), (1, planes, 1, 1))
+    with np.errstate(all="ignore"):
+        want = oracle.pooling(x, *args)
+        assert_bit_exact(gpuops.pooling(x, *args, offset=length % 4), want, "average")
