@@ -1312,17 +1312,22 @@ static void launch_normalize_tile(int outer_num, int dim, int inner_num, float p
 // the exponentials is an fp32 running sum and is always walked in index order, by wave 0 (the four waves
 // taking turns from workgroup to workgroup or from 256 to 256: level, 24.9 / 24.6 / 24.6 us here).
 //
-// [16,150,72,72], 99.5 MB: 24.6 us.  Its vector instructions bound it together with the rounds of
-// load, walk and store (29 an element by the counters); 28.8 us with the maxima by
-// compare and select, a division and the longer exponential, and five barriers.
-template <int TS_SHIFT, int ROWS>
-__global__ __launch_bounds__(kBlock) void softmax_tile_kernel(const float* x, float* y, uint32_t dim,
-                                                               uint32_t inner, FastDiv f_tiles) {
+// LDS holds the rows of `pass_steps` steps (two at least, an even number), pass after pass; the sum goes on from
+// pass to pass in wave 0's lanes.
+//
+// [16,150,72,72], 99.5 MB: 20.0 us, all tiles on the chip at once; with whole columns in LDS and four tiles a CU,
+// so that a fifth of them came in a second round, 24.6.  29 vector instructions an element bound it
+// together with the rounds of load, walk and store; 28.8 us with the maxima by compare and select, a division and the
+// longer exponential, and five barriers.
+template <int TS_SHIFT, int ROWS, int N, int WAVES>
+__global__ __launch_bounds__(kBlock, WAVES) void softmax_tile_kernel(const float* x, float* y, uint32_t dim,
+                                                               uint32_t inner, uint32_t pass_steps, FastDiv f_tiles) {
   extern __shared__ __align__(16) float lds[];
   constexpr uint32_t TS = 1u << TS_SHIFT;
   constexpr uint32_t kWaves = kBlock / kWave;
   using Lane = TileLane<TS_SHIFT, ROWS>;
-  uint64_t* tab = reinterpret_cast<uint64_t*>(lds + (dim << TS_SHIFT));  // after the tile, 16-byte aligned
+  const uint32_t pass_rows = min(pass_steps * Lane::STEP, dim);
+  uint64_t* tab = reinterpret_cast<uint64_t*>(lds + (pass_rows << TS_SHIFT));  // after the tile, 16-byte aligned
   float* maxima = reinterpret_cast<float*>(tab + 32);                    // [wave][TS]
   double* recip = reinterpret_cast<double*>(tab + 32);                   // [TS], when the maxima have been read
   float* handed = reinterpret_cast<float*>(recip + TS);                  // [TS]
@@ -1334,12 +1339,12 @@ __global__ __launch_bounds__(kBlock) void softmax_tile_kernel(const float* x, fl
   const uint64_t base = static_cast<uint64_t>(n) * dim * inner + p0;
   const Lane lane(width, dim, inner);
   const uint32_t wave = threadIdx.x / kWave;
-  v4f r[kTilePerLane];
+  v4f r[N];
   lane.load(x + base, r);
   v4f m = {-FLT_MAX, -FLT_MAX, -FLT_MAX, -FLT_MAX};
   if (lane.valid != 0) {
 #pragma unroll
-    for (int u = 0; u < kTilePerLane; u += 2) {
+    for (int u = 0; u < N; u += 2) {
       if (!lane.step(u)) continue;
 #pragma unroll
       for (int k = 0; k < 4; ++k) m[k] = max3_any_order(m[k], r[u][k], r[u + 1][k]);
@@ -1356,32 +1361,37 @@ __global__ __launch_bounds__(kBlock) void softmax_tile_kernel(const float* x, fl
 #pragma unroll
       for (int k = 0; k < 4; ++k) m[k] = max3_any_order(m[k], m[k], other[k]);
     }
-#pragma unroll
-    for (int u = 0; u < kTilePerLane; u += 2) {  // eight exponentials, each a chain, side by side
-      if (!lane.step(u)) continue;
-#pragma unroll
-      for (int k = 0; k < 8; ++k) r[u + k / 4][k % 4] = libm::exact_expf_nonpositive(r[u + k / 4][k % 4] - m[k % 4], tab);
-#pragma unroll
-      for (int k = 0; k < 2; ++k)
-        if (lane.has(u + k)) *reinterpret_cast<v4f*>(lds + ((lane.c0 + (u + k) * Lane::STEP) << TS_SHIFT) + lane.j) = r[u + k];
-    }
   }
-  __syncthreads();  // also: every lane has its maxima before the sums replace them
-  if (wave == 0) {
-    const uint32_t pos = threadIdx.x;
-    if (pos < width) {
+  float sum = 0.f;
+  for (uint32_t first = 0; first * Lane::STEP < dim; first += pass_steps) {
+    if (first) __syncthreads();  // wave 0 has read the rows of the pass before
+    if (lane.valid != 0) {
+#pragma unroll
+      for (int u = 0; u < N; u += 2) {  // eight exponentials, each a chain, side by side
+        if (!lane.step(u) || static_cast<uint32_t>(u) - first >= pass_steps) continue;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) r[u + k / 4][k % 4] = libm::exact_expf_nonpositive(r[u + k / 4][k % 4] - m[k % 4], tab);
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+          if (lane.has(u + k)) *reinterpret_cast<v4f*>(lds + ((lane.c0 + (u + k - first) * Lane::STEP) << TS_SHIFT) + lane.j) = r[u + k];
+      }
+    }
+    __syncthreads();  // also: every lane has its maxima before the sums replace them
+    if (threadIdx.x < width && wave == 0) {
       __builtin_amdgcn_s_setprio(3);
-      const float sum = fold_tile_column<TS_SHIFT>(lds + pos, dim, 0.f, [](float a, float v) { return a + v; });
-      handed[pos] = sum;
-      recip[pos] = reciprocal(sum);
+      sum = fold_tile_column<TS_SHIFT>(lds + threadIdx.x, min(pass_rows, dim - first * Lane::STEP), sum, [](float a, float v) { return a + v; });
       __builtin_amdgcn_s_setprio(0);
     }
+  }
+  if (threadIdx.x < width && wave == 0) {
+    handed[threadIdx.x] = sum;
+    recip[threadIdx.x] = reciprocal(sum);
   }
   __syncthreads();
   if (lane.valid == 0) return;
   const TileQuotients q(handed + lane.j, recip + lane.j);
 #pragma unroll
-  for (int u = 0; u < kTilePerLane; ++u)
+  for (int u = 0; u < N; ++u)
     if (lane.has(u)) lane.store(y + base, u, q(r[u]));
 }
 
@@ -1390,18 +1400,68 @@ constexpr size_t kExpTabBytes = 32 * sizeof(uint64_t);
 // (32 positions of 512 channels, or 16 of 1024, with it: 66 KB at most, two workgroups per CU all the same)
 static size_t softmax_tile_extra_bytes(int ts) { return kExpTabBytes + static_cast<size_t>(kBlock / kWave) * ts * sizeof(float); }
 
-template <int TS_SHIFT>
-static void launch_softmax_tile_ts(int outer_num, int dim, int inner_num, const float* x, float* y,
-                                   hipStream_t st) {
-  const uint32_t tiles = (static_cast<uint32_t>(inner_num) + (1u << TS_SHIFT) - 1) >> TS_SHIFT;
-  const uint32_t grid = static_cast<uint32_t>(outer_num) * tiles;
-  const size_t bytes = (static_cast<size_t>(dim) << TS_SHIFT) * sizeof(float) + softmax_tile_extra_bytes(1 << TS_SHIFT);
+// How a shape is cut into tiles: positions, vectors a lane has room for (what fixes how many waves a SIMD
+// holds), steps of rows that LDS holds at a time.
+struct SoftmaxTiles {
+  int shift, slots;
+  uint32_t grid, pass_steps, lds_bytes;
+};
+
+// Tiles that all fit the chip at once finish together; a second round of a few of them costs as much as the
+// first.  So: as many positions as a lane's sixteen vectors hold (64, 32 or 16), or half of them where that
+// gives no more than three tiles a CU ([1,150,5184] 7.1 us with 64 positions, 5.7 with 32; [4,150,5184] 9.5, 8.7;
+// [8,150,5184], 1296 tiles of 32, 12.0 and 12.5; [4,500,3025] 19.2 with 32, 16.1 with 16; [16,300,1444] 16.2, 16.8), and
+// where a lane of 64 positions had more than ten vectors, as long as the chip holds seven a CU ([16,250,1444]
+// 16.1 and 13.7, [16,250,3136] 22.5 in two passes, 19.8; [64,250,1444] 41.7 and 45.7).  One pass through LDS where
+// the tiles fit beside each other so, otherwise two passes of half the rows ([16,150,5184] 24.8 and 20.0 us,
+// [16,180,3136] 21.6 and 16.6, [16,500,1600] 31.3 and 22.7, [16,1000,784] 38.7 and 26.8; where they fit the second pass
+// costs: [1,150,5184] 7.1 and 7.4).
+static SoftmaxTiles softmax_tiles(int outer_num, int dim, int inner_num) {
+  constexpr uint32_t kCus = 256, kCuLds = 160 * 1024, kFewTiles = 3 * kCus, kNarrowTiles = 7 * kCus;
+  const auto tiles = [&](int shift) {
+    return static_cast<uint32_t>(outer_num) * ((static_cast<uint32_t>(inner_num) + (1u << shift) - 1) >> shift);
+  };
+  const uint32_t d = static_cast<uint32_t>(dim);
+  SoftmaxTiles t{};
+  t.shift = d <= 256 ? 6 : d <= 512 ? 5 : 4;
+  if (t.shift > 4 && tiles(t.shift - 1) <= (t.shift == 6 && d > 160 ? kNarrowTiles : kFewTiles)) --t.shift;
+  t.grid = tiles(t.shift);
+  const uint32_t step = kBlock / ((1u << t.shift) / 4), steps = (d + step - 1) / step;
+  t.slots = steps <= 8 && t.shift < 6 ? 8 : steps <= 10 ? 10 : 16;
+  const uint32_t waves = t.slots == 8 ? 7 : t.slots == 10 ? 6 : 4;
+  const auto bytes = [&](uint32_t pass_steps) {
+    const uint32_t rows = pass_steps * step < d ? pass_steps * step : d;
+    return static_cast<uint32_t>((rows << t.shift) * sizeof(float) + softmax_tile_extra_bytes(1 << t.shift));
+  };
+  t.pass_steps = (steps + 1) & ~1u;
+  const uint32_t fit = kCuLds / bytes(t.pass_steps);
+  if (t.grid > kCus * (fit < waves ? fit : waves)) t.pass_steps = 2 * ((steps + 3) / 4);
+  t.lds_bytes = bytes(t.pass_steps);
+  return t;
+}
+
+template <int TS_SHIFT, int N, int WAVES>
+static void launch_softmax_tile(const SoftmaxTiles& t, int dim, int inner_num, const float* x, float* y, hipStream_t st) {
   const uint32_t d = static_cast<uint32_t>(dim), in = static_cast<uint32_t>(inner_num);
-  const FastDiv ft = make_fastdiv(tiles);
+  const FastDiv ft = make_fastdiv((in + (1u << TS_SHIFT) - 1) >> TS_SHIFT);
+  const auto launch = [&](auto kernel) { kernel<<<t.grid, kBlock, t.lds_bytes, st>>>(x, y, d, in, t.pass_steps, ft); };
   switch (tile_rows(inner_num, y)) {
-    case kRowsSector: softmax_tile_kernel<TS_SHIFT, kRowsSector><<<grid, kBlock, bytes, st>>>(x, y, d, in, ft); break;
-    case kRowsQuad: softmax_tile_kernel<TS_SHIFT, kRowsQuad><<<grid, kBlock, bytes, st>>>(x, y, d, in, ft); break;
-    default: softmax_tile_kernel<TS_SHIFT, kRowsAny><<<grid, kBlock, bytes, st>>>(x, y, d, in, ft);
+    case kRowsSector: launch(softmax_tile_kernel<TS_SHIFT, kRowsSector, N, WAVES>); break;
+    case kRowsQuad: launch(softmax_tile_kernel<TS_SHIFT, kRowsQuad, N, WAVES>); break;
+    default: launch(softmax_tile_kernel<TS_SHIFT, kRowsAny, N, WAVES>);
+  }
+}
+
+static void launch_softmax_tile(const SoftmaxTiles& t, int dim, int inner_num, const float* x, float* y, hipStream_t st) {
+  switch (t.shift * 100 + t.slots) {
+    case 610: launch_softmax_tile<6, 10, 6>(t, dim, inner_num, x, y, st); break;
+    case 616: launch_softmax_tile<6, 16, 4>(t, dim, inner_num, x, y, st); break;
+    case 508: launch_softmax_tile<5, 8, 7>(t, dim, inner_num, x, y, st); break;
+    case 510: launch_softmax_tile<5, 10, 6>(t, dim, inner_num, x, y, st); break;
+    case 516: launch_softmax_tile<5, 16, 4>(t, dim, inner_num, x, y, st); break;
+    case 408: launch_softmax_tile<4, 8, 7>(t, dim, inner_num, x, y, st); break;
+    case 410: launch_softmax_tile<4, 10, 6>(t, dim, inner_num, x, y, st); break;
+    default: launch_softmax_tile<4, 16, 4>(t, dim, inner_num, x, y, st);
   }
 }
 
@@ -2554,13 +2614,9 @@ static int run_softmax(int outer_num, int dim, int inner_num, const float* x, fl
     else
       softmax_columns_reg_kernel<64, 48><<<grid, kBlock, 0, st>>>(x, y, g.columns, d, fi);
   } else if (tile_fits(dim, inner_num, true)) {
-    // the widest tile (64, 32 or 16 positions) that fits 64 KB beside the table and the hand-over row
-    const int shift = dim * 64 * sizeof(float) <= kTileLdsBytes - 1024 ? 6 : (dim * 32 * sizeof(float) <= kTileLdsBytes ? 5 : 4);
-    const uint32_t tiles = (static_cast<uint32_t>(inner_num) + (1u << shift) - 1) >> shift;
-    if (pl->chosen(SHDW_PATH_TILE, shift, static_cast<uint32_t>(outer_num) * tiles)) return SHDW_OK;
-    if (shift == 6) launch_softmax_tile_ts<6>(outer_num, dim, inner_num, x, y, st);
-    else if (shift == 5) launch_softmax_tile_ts<5>(outer_num, dim, inner_num, x, y, st);
-    else launch_softmax_tile_ts<4>(outer_num, dim, inner_num, x, y, st);
+    const SoftmaxTiles t = softmax_tiles(outer_num, dim, inner_num);
+    if (pl->chosen(SHDW_PATH_TILE, t.shift, t.grid)) return SHDW_OK;
+    launch_softmax_tile(t, dim, inner_num, x, y, st);
   } else if (TallLaunch t; tall_launch(outer_num, dim, inner_num, &t)) {
     if (pl->chosen(SHDW_PATH_TALL, static_cast<int>(t.width_log2), t.grid)) return SHDW_OK;
     softmax_tall_kernel<<<t.grid, kBlock, 0, st>>>(x, y, static_cast<uint32_t>(dim), static_cast<uint32_t>(inner_num),
