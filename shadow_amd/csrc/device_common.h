@@ -198,6 +198,12 @@ SHDW_DEVICE double dpp_f64(double v) {
   const int hi = dpp_i32<CTRL>(static_cast<int>(b >> 32));
   return __longlong_as_double((static_cast<long long>(hi) << 32) | static_cast<unsigned int>(lo));
 }
+// The lane in front's, 0 in lane 0: with a constant there the shift is an operand of the addition that
+// follows, where dpp_f32 takes an instruction of its own, which the chain of a sum waits for (whole-plane
+// averages of 512 x 12544 with signs 39.3 -> 29.4 us).
+SHDW_DEVICE float lane_in_front(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138, 0xf, 0xf, true));
+}
 template <int CTRL>
 SHDW_DEVICE uint32_t dpp_u32(uint32_t v) {
   return static_cast<uint32_t>(dpp_i32<CTRL>(static_cast<int>(v)));
@@ -205,7 +211,7 @@ SHDW_DEVICE uint32_t dpp_u32(uint32_t v) {
 
 constexpr int kDppXor1 = 0xB1;        // quad_perm [1,0,3,2]
 constexpr int kDppXor2 = 0x4E;        // quad_perm [2,3,0,1]
-constexpr int kDppWaveShr1 = 0x138;    // lane i takes lane i - 1, lane 0 keeps its own
+constexpr int kDppWaveShr1 = 0x138;    // lane i takes lane i - 1
 constexpr int kDppRor4 = 0x124;        // lane i takes lane i - 4 (modulo 16) inside 16
 constexpr int kDppRor8 = 0x128;        // lane i <-> i + 8 (modulo 16) inside 16
 constexpr int kDppHalfMirror = 0x141;  // lane i <-> 7-i inside 8

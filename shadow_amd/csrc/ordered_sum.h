@@ -54,6 +54,15 @@ SHDW_DEVICE float add_lane(float v) {
 constexpr int kDppShr1 = 0x111, kDppShr2 = 0x112, kDppShr4 = 0x114, kDppShr8 = 0x118;  // inside 16 lanes
 constexpr int kDppBcast15 = 0x142, kDppBcast31 = 0x143;  // the last lane of 16, of 32, to the 16, 32 behind them
 
+// Whether some element is negative, -0 or NaN.
+template <int K>
+SHDW_DEVICE bool any_sign(const float (&v)[K]) {
+  uint32_t most = __float_as_uint(v[0]);
+#pragma unroll
+  for (int k = 1; k < K; ++k) most = max(most, __float_as_uint(v[k]));
+  return most > kExponentBits;
+}
+
 // sum + v[0] + v[1] + ... of lane 0, then of lane 1, ...: the same sum in all lanes.  All 64 lanes call it, with
 // the same sum; neither it nor any term is negative or NaN (infinities are fine).
 template <int K>
@@ -70,7 +79,7 @@ SHDW_DEVICE float wave_sum_in_order(const float (&v)[K], float sum) {
   upto = add_lane<kDppShr8, 0xf>(upto);
   upto = add_lane<kDppBcast15, 0xa>(upto);
   upto = add_lane<kDppBcast31, 0xc>(upto);
-  const float before = sum + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(upto), kDppWaveShr1, 0xf, 0xf, false));
+  const float before = sum + lane_in_front(upto);
   const uint32_t power = __float_as_uint(before) & kExponentBits;
   const uint32_t guess = __float_as_uint(before) & ~1u;  // lane 0's is the sum's own, so its terms are added to the sum itself
   float from_even = __uint_as_float(guess), from_odd = __uint_as_float(guess | 1u);
@@ -95,32 +104,30 @@ SHDW_DEVICE float wave_sum_in_order(const float (&v)[K], float sum) {
   join_run<kDppBcast15, 0xa>(run);
   join_run<kDppBcast31, 0xc>(run);
 
-  const uint64_t all_starts = __builtin_amdgcn_ballot_w64(starts), all_passes = __builtin_amdgcn_ballot_w64(passes);
+  const uint64_t all_starts = __builtin_amdgcn_ballot_w64(starts), whole_runs = all_starts & ~__builtin_amdgcn_ballot_w64(passes);
   uint32_t bits = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(__float_as_int(sum)));
   const auto of_lane = [](uint32_t value, uint32_t lane) {
     return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(value), static_cast<int>(lane)));
   };
-  bits = bits & 1u ? of_lane(__float_as_uint(from_odd), 0) : of_lane(__float_as_uint(from_even), 0);
+  bits = of_lane(bits & 1u ? __float_as_uint(from_odd) : __float_as_uint(from_even), 0);
+  // The lanes from `lane` on that make one run, if they do, at once; then the lane behind them, one by one.
+  const uint64_t ends = all_starts >> 1 | 1ull << 63;  // lanes in front of a start, and the last
   uint32_t lane = 1;
-  while (lane < kWave) {  // the same for all lanes; every turn is of one lane at least
-    const uint64_t later = lane + 1 < kWave ? all_starts >> (lane + 1) : 0;
-    const uint32_t end = later ? lane + 1 + static_cast<uint32_t>(__builtin_ctzll(later)) : kWave;
-    if ((all_passes >> lane & 1u) == 0) {
-      const uint32_t low = of_lane(power, lane);
-      const uint32_t next = bits + (bits & 1u ? of_lane(run.odd, end - 1) : of_lane(run.even, end - 1));
-      if (bits - low < kBinade && next - low < kBinade) {
-        bits = next;
-        lane = end;
-        continue;
-      }
+  do {  // the same for all lanes; every turn is of one lane at least
+    const uint32_t last = static_cast<uint32_t>(__builtin_ctzll(ends >> lane)) + lane;
+    const uint32_t low = of_lane(power, lane), even = of_lane(run.even, last), odd = of_lane(run.odd, last);
+    const uint32_t next = bits + (bits & 1u ? odd : even);
+    // a run is known from its first lane on: not behind a lane whose guess was wrong
+    if ((whole_runs >> lane & 1u) != 0 && bits - low < kBinade && next - low < kBinade) {
+      bits = next;
+      lane = last + 1;
+      if (lane == kWave) break;
     }
-    for (; lane < end; ++lane) {
-      float s = __uint_as_float(bits);
+    float s = __uint_as_float(bits);
 #pragma unroll
-      for (int k = 0; k < K; ++k) s += v[k];
-      bits = of_lane(__float_as_uint(s), lane);
-    }
-  }
+    for (int k = 0; k < K; ++k) s += v[k];
+    bits = of_lane(__float_as_uint(s), lane);
+  } while (++lane < kWave);
   return __uint_as_float(bits);
 }
 

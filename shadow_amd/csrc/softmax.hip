@@ -21,6 +21,7 @@
 #include "../../include/shadow_hip.h"
 #include "device_common.h"
 #include "launch.h"
+#include "ordered_sum.h"
 #include "libm_exact.h"
 
 #pragma clang fp contract(off)
@@ -294,9 +295,11 @@ SHDW_DEVICE float block_max_any_order(float m, float* scratch4) {
 // Front-to-back fp32 sum of lds[0..n) by a whole wave, the result in all its lanes: a lane holds 16
 // consecutive elements of a chunk of 1024 and the sum goes from lane to lane, as in
 // pool_rows_stream_kernel (by one lane out of LDS, eight 128-bit reads at a time, softmax of [16,1000]
-// takes 7.2 us, so 5.6; [8192,4096] 120 and 99).  lds is 16-byte aligned and readable up to the next multiple of four.
+// takes 7.2 us, so 5.6; [8192,4096] 120 and 99).  From 42 lanes' worth on, the additions are taken side by side
+// (ordered_sum.h; no exponential is negative): [16,1000] 5.6 -> 5.0 us, [4,4096] 15.8 -> 10.4, [512,8192] 33.9 -> 22.6;
+// [16,700] 4.8 and 4.7, [32,512] 4.1 and 4.5.  lds is 16-byte aligned and readable up to the next multiple of four.
 SHDW_DEVICE float wave_ordered_sum(const float* lds, uint32_t n) {
-  constexpr uint32_t kSpan = 16, kChunk = kWave * kSpan;
+  constexpr uint32_t kSpan = 16, kChunk = kWave * kSpan, kSideBySide = 42;
   const uint32_t lane = threadIdx.x % kWave;
   float sum = 0.f;
   for (uint32_t c0 = 0; c0 < n; c0 += kChunk) {
@@ -309,23 +312,22 @@ SHDW_DEVICE float wave_ordered_sum(const float* lds, uint32_t n) {
       for (uint32_t j = 0; j < 4; ++j) v[k + j] = first + k + j < n ? q[j] : 0.f;  // a sum that starts at +0 stays as it is
     }
     const uint32_t turns = min(static_cast<uint32_t>(kWave), (n - c0 + kSpan - 1) / kSpan);
-    auto turn = [&]() {
+    if (turns >= kSideBySide && __builtin_amdgcn_ballot_w64(any_sign(v)) == 0) {
+      sum = wave_sum_in_order(v, sum);
+      continue;
+    }
+    const auto turn = [&](float from) {
+      sum = from;
 #pragma unroll
       for (uint32_t k = 0; k < kSpan; ++k) sum += v[k];
     };
-    turn();
+    turn(sum);
     uint32_t t = 1;
     for (; t + 4 <= turns; t += 4) {
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        sum = dpp_f32<kDppWaveShr1>(sum);
-        turn();
-      }
+      for (int u = 0; u < 4; ++u) turn(lane_in_front(sum));
     }
-    for (; t < turns; ++t) {
-      sum = dpp_f32<kDppWaveShr1>(sum);
-      turn();
-    }
+    for (; t < turns; ++t) turn(lane_in_front(sum));
     sum = __shfl(sum, turns - 1);
   }
   return sum;
@@ -1706,7 +1708,7 @@ __global__ __launch_bounds__(kBlock, 4) void softmax_rows_kernel(const float* x,
   float sum = 0.f;
   const uint32_t turns = (w.dim + span - 1) / span;
   for (uint32_t t = 0; t < turns; ++t) {
-    if (t > 0) sum = dpp_f32<kDppWaveShr1>(sum);
+    if (t > 0) sum = lane_in_front(sum);
 #pragma unroll
     for (int k = 0; k < kRowsSpan; k += 4) {
       if (k >= span) continue;

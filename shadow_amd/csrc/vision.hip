@@ -1204,7 +1204,7 @@ static void launch_pool_plane(const float* x, float* y, uint32_t rows, uint32_t 
 // Whole-plane average over rows of any length, without a barrier: every wave of a
 // workgroup works by itself on G consecutive rows, in chunks of W = 32 * 64 / G
 // columns.  An fp32 running sum has no order but the index order, so a row costs a
-// chain of as many dependent additions, 2.8 ns each (9 us for 3136), and a wave alone
+// chain of as many dependent additions, 2 ns each (6.5 us for 3136), and a wave alone
 // on its SIMD issues nothing faster than that whatever it issues: what counts is to
 // issue little besides the additions.  A chunk passes through the wave's LDS once, so
 // that every one of the 64 / G lanes of a row holds 32 consecutive columns of it in
@@ -1293,33 +1293,29 @@ __global__ __launch_bounds__(kBlock) void pool_rows_stream_kernel(const float* x
     r.take(c0, mine);
     if (c0 != 0) sum = __shfl(sum, r.lane | (Rows::L - 1));  // from the last lane of the row to its first
     turns = min(Rows::L, (len - c0 + kSpan - 1) / kSpan);
-#pragma unroll
-    for (int k = 0; k < kSpan; ++k) sum += mine[k];
-    for (uint32_t t = 1; t < turns; ++t) {
-      sum = dpp_f32<kDppWaveShr1>(sum);
+    const auto add = [&](float from) {
+      sum = from;
 #pragma unroll
       for (int k = 0; k < kSpan; ++k) sum += mine[k];
+    };
+    add(sum);
+    uint32_t t = 1;
+    for (; t + 4 <= turns; t += 4) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) add(lane_in_front(sum));
     }
+    for (; t < turns; ++t) add(lane_in_front(sum));
   }
   const uint32_t row = row0 + r.lane / Rows::L;
   if (r.lane % Rows::L == turns - 1 && row < rows) y[row] = sum / pool_size;
-}
-
-// Whether some element is negative, -0 or NaN.
-SHDW_DEVICE bool any_sign(const float (&v)[kSpan]) {
-  uint32_t most = __float_as_uint(v[0]);
-#pragma unroll
-  for (int k = 1; k < kSpan; ++k) most = max(most, __float_as_uint(v[k]));
-  return most > kExponentBits;
 }
 
 // Few long rows, a wave each: where no element of a chunk is negative (what ReLU and the poolings behind
 // it leave) the chunk's additions are taken side by side (ordered_sum.h), otherwise lane by lane as
 // above.  Bound by latencies: the first loads, 64 dependent additions of a guess per chunk,
 // the joining of the lanes' runs (0.3 us) and the lanes where the sum passes a power of two (0.1 us
-// each, six in the first chunk).  Against the additions in turn (rows x columns): 3 x 50176 125 -> 29 us,
-// 512 x 12544 36.2 -> 12.0, 1024 x 3136 12.2 -> 6.9, 2048 x 3136 12.5 -> 8.8, 2048 x 12544 40.7 -> 19.1.
-// Rows of N(0, 1) take as long as before or less, up to 3 % more at 2048 rows of 3136.
+// each, six in the first chunk).  Against the additions in turn with a wave a row (rows x columns): 3 x 50176
+// 105 -> 27 us, 512 x 12544 29.4 -> 11.1, 1024 x 3136 9.9 -> 6.3, 2048 x 3136 12.0 -> 8.2, 2048 x 12544 38.2 -> 19.1.
 __global__ __launch_bounds__(kBlock, 4) void pool_rows_runs_kernel(const float* x, float* y, uint32_t rows,
                                                                     uint32_t len, float pool_size) {
   using Rows = PlaneRows<1>;
@@ -1337,11 +1333,18 @@ __global__ __launch_bounds__(kBlock, 4) void pool_rows_runs_kernel(const float* 
       continue;
     }
     const uint32_t turns = min(static_cast<uint32_t>(kWave), (len - c0 + kSpan - 1) / kSpan);
-    for (uint32_t t = 0; t < turns; ++t) {
-      if (t != 0) sum = dpp_f32<kDppWaveShr1>(sum);
+    const auto add = [&](float from) {
+      sum = from;
 #pragma unroll
       for (int k = 0; k < kSpan; ++k) sum += mine[k];
+    };
+    add(sum);
+    uint32_t t = 1;
+    for (; t + 4 <= turns; t += 4) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) add(lane_in_front(sum));
     }
+    for (; t < turns; ++t) add(lane_in_front(sum));
     sum = __shfl(sum, turns - 1);
   }
   if (r.lane == 0) y[row] = sum / pool_size;
@@ -1350,7 +1353,7 @@ __global__ __launch_bounds__(kBlock, 4) void pool_rows_runs_kernel(const float* 
 // From this row length on the whole-plane average takes the streaming kernel
 // (per 51 MB, against pool_plane_kernel: 28x28 planes 10.7 / 23.5 us, 56x56 planes
 // 14.5 / 59 us; 14x14 planes, before the sum went from lane to lane, 13.2 / 14.2 us but
-// 45.8 / 42.0 us per 205 MB).  Few rows as well: [1,3,224,224] 126 us against 630.
+// 45.8 / 42.0 us per 205 MB).  Few rows as well: [1,3,224,224] 105 us against 630 (27 without signs, see below).
 constexpr int kPlaneStreamMinLen = 256;
 // Rows per wave: up to eight while there are 512 waves (two a CU) and more.  Every wave issues all
 // the additions of a row whatever the number of its rows, so few rows go one to a wave and many
@@ -1365,9 +1368,9 @@ static int stream_rows_per_wave(uint32_t rows) {
 }
 
 // Up to here a wave a row fills no more than two waves of a SIMD, and rows with signs lose nothing by not
-// sharing a wave (2500 x 3136 of N(0, 1) 12.6 us as eight rows a wave, 20.1 as one; without signs 12.6 and
-// 10.7); below 1152 columns the additions in turn are over as soon (2048 x 1024 5.5 us in turn, 5.9 side by
-// side, 2048 x 1200 6.5 and 5.9).
+// sharing a wave (2500 x 3136 of N(0, 1) 11.0 us as four rows a wave, 20.1 as one; without signs 11.1 and
+// 10.7); below 1152 columns the additions in turn are over as soon (2048 x 1024 5.1 us in turn, 5.9 side by
+// side, 2048 x 1200 6.0 and 5.5).
 constexpr uint32_t kRunsMaxRows = 2048, kRunsMinLen = 1152;
 
 static void launch_pool_rows_stream(const float* x, float* y, uint32_t rows, uint32_t len, hipStream_t st) {
