@@ -11,17 +11,14 @@
 // x + (-0)).  The plane sum is fp32, front to back, by one lane, as Vision::Pooling
 // adds; the mean at the end is fp64, rounded once after the divide.
 //
-// What bounds it: five workgroups on a CU (LDS and registers), whose loads, ordered
-// sums (784 dependent additions: 3 us; without them [32,512,28,28] takes 22.9 us instead of
-// 27) and stores overlap each other's, and 47 vector instructions an element (7x7 planes 61, 112x112
-// in chunks 100).  One block with its tail takes, per call: [32,512,28,28]
-// (103 MB) 26.5 us (28.7 with the quotients in fp32 and the row's parameters read for every
-// vector), where its five launches took 78; [64,64,56,56] 44; [64,512,14,14]
-// 12.1; [64,1024,7,7] 8.8; [16,64,112,112] 72 and [16,64,96,96] 54, both in chunks (their sums
-// are 12 544 and 9216 long).  With loads in
-// branches of their own, a division per element, LDS reads next to the additions that
-// use them and rows whole in LDS whatever their length: 29, 43, 13.9, 11.3 and 112; with the residual
-// another tensor than x 35 -> 27.5, 49 -> 44, 15.1 -> 12.0, 12.3 -> 8.2, 116 -> 80.
+// Rows of whole vectors behind BatchNorm and ReLU take gate_whole_kernel, all others squeeze_gate_kernel.
+//
+// What bounds it: rows held in LDS and registers leave four to six workgroups on a CU, whose loads, ordered sums and
+// stores overlap each other's; the sums, dependent additions, take 2 ns each (long rows without signs
+// less); and 30 to 60 vector instructions an element.  One block with its tail takes, per call: [32,512,28,28]
+// (103 MB) 21.8 us (its five launches 78), [64,64,56,56] 24.6, [16,64,112,112] 32.3, [8,128,64,64] 10.9,
+// [64,512,14,14] 11.5, [64,1024,7,7] 7.8, [16,64,55,55] 10.1, [16,64,111,113] 29.3.  With a lane for each row's sum that
+// reads it from LDS, and one kernel for all: 25.3, 41.4, 70.1, 30.2, 11.4, 7.8, 24.2 and 70.1.
 #include <hip/hip_runtime.h>
 
 #include "../../include/shadow_hip.h"
@@ -29,6 +26,7 @@
 #include "gate_shape.h"
 #include "launch.h"
 #include "libm_exact.h"
+#include "ordered_sum.h"
 
 #pragma clang fp contract(off)
 
@@ -48,13 +46,15 @@ struct GateParams {
   FastDiv channel;
 };
 
+constexpr uint32_t kGateWalkRows = 16;  // rows that a wave walks as one (gate_walk), a lane each beyond
 enum { kNoResidual = 0, kOtherResidual = 1, kSameResidual = 2 };
 
 // Waves per SIMD that the registers are held to: what a lane's vectors leave room for.
 constexpr int gate_waves(int slots) { return slots == 16 ? 4 : slots == 8 ? 5 : 6; }
 
-// sum + row[0] + row[1] + ..., in that order.  Two sets of six vectors take turns: one is
-// read while the other is added.  A last part of a vector reads the whole of it.
+// sum + row[0] + row[1] + ..., in that order, by a lane; for groups of more than sixteen rows, which are short.
+// Two sets of six vectors take turns: one is read while the other is added.  A last part of a vector reads the
+// whole of it.
 SHDW_DEVICE float add_in_order(float sum, const v4f* row, uint32_t cols) {
   constexpr uint32_t kSet = 6;
   const uint32_t n = cols / 4;
@@ -95,6 +95,58 @@ SHDW_DEVICE float add_in_order(float sum, const v4f* row, uint32_t cols) {
       if (k >= left) break;
       sum += a[k / 4][k % 4];
     }
+  }
+  return sum;
+}
+
+// sum + row[0] + row[1] + ... of 2^log2_rows rows of `cols` numbers, front to back, by a whole wave: as many lanes a
+// row, a lane with 28 consecutive numbers of a chunk in registers, and the sum from lane to lane (4.8 cycles an
+// addition; a lane a row that reads it from LDS takes 8, and 16 where four workgroups a CU are all there is).
+// One long row without signs: side by side (ordered_sum.h).  The rows lie pitch vectors apart; of those past the last one
+// the last is read.  All lanes of a row give and get its sum.
+template <bool VEC>
+SHDW_DEVICE float gate_walk(float sum, const v4f* tile, uint32_t pitch, uint32_t cols, uint32_t log2_rows, uint32_t nrows) {
+  constexpr uint32_t kVectors = 7, kSpan = 4 * kVectors, kSideBySide = 36;  // lanes' worth (of 28): 1008 numbers
+  const uint32_t lane = threadIdx.x % kWave, shift = 6 - log2_rows, per_row = 1u << shift, at = lane & (per_row - 1);
+  const uint32_t nv = (cols + 3) / 4;
+  const v4f* row = tile + min(lane >> shift, nrows - 1) * pitch;
+  for (uint32_t v0 = 0; v0 < nv; v0 += kVectors * per_row) {
+    float v[kSpan];
+    const uint32_t first = v0 + at * kVectors;
+    if (4 * (v0 + kVectors * per_row) <= cols) {
+#pragma unroll
+      for (uint32_t i = 0; i < kVectors; ++i) {
+        const v4f q = row[first + i];
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j) v[4 * i + j] = q[j];
+      }
+    } else {
+#pragma unroll
+      for (uint32_t i = 0; i < kVectors; ++i) {
+        const v4f q = row[min(first + i, nv - 1)];
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j)  // a sum that starts at +0 stays as it is
+          v[4 * i + j] = (VEC ? first + i < nv : 4 * (first + i) + j < cols) ? q[j] : 0.f;
+      }
+    }
+    const uint32_t turns = min(per_row, (nv - v0 + kVectors - 1) / kVectors);
+    if (log2_rows == 0 && turns >= kSideBySide && __builtin_amdgcn_ballot_w64(any_sign(v) || !(sum >= 0.f)) == 0) {
+      sum = wave_sum_in_order(v, sum);
+      continue;
+    }
+    const auto turn = [&](float from) {
+      sum = from;
+#pragma unroll
+      for (uint32_t k = 0; k < kSpan; ++k) sum += v[k];
+    };
+    turn(sum);
+    uint32_t t = 1;
+    for (; t + 4 <= turns; t += 4) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) turn(lane_in_front(sum));
+    }
+    for (; t < turns; ++t) turn(lane_in_front(sum));
+    sum = __shfl(sum, (lane & ~(per_row - 1)) + turns - 1);
   }
   return sum;
 }
@@ -197,11 +249,12 @@ __global__ __launch_bounds__(kBlock, gate_waves(SLOTS)) void squeeze_gate_kernel
     return t;
   };
 
-  // The ordered sums, a lane per row: all in one wave, which issues one addition for
-  // all rows; a different wave in neighbouring workgroups, so that the walks of a CU
-  // do not meet on one SIMD.
-  const uint32_t walked = threadIdx.x & (kWave - 1);
-  const bool walks = threadIdx.x / kWave == ((blockIdx.x / kXcds) & 3u) && walked < nrows;
+  // The ordered sums: all in one wave, which issues one addition for all rows; a different
+  // wave in neighbouring workgroups, so that the walks of a CU do not meet on one SIMD.
+  const bool together = group <= kGateWalkRows;  // the wave walks all rows as one
+  const uint32_t log2_rows = group > 1 ? 32 - __builtin_clz(group - 1) : 0;
+  const uint32_t walked = together ? (threadIdx.x & (kWave - 1)) >> (6 - log2_rows) : threadIdx.x & (kWave - 1);
+  const bool walks = threadIdx.x / kWave == ((blockIdx.x / kXcds) & 3u) && (together || walked < nrows);
   GateRow g;
   float sum = 0.f;
   for (uint32_t k0 = 0; k0 < pieces; k0 += chunk) {
@@ -228,15 +281,15 @@ __global__ __launch_bounds__(kBlock, gate_waves(SLOTS)) void squeeze_gate_kernel
     if (RESIDUAL == kOtherResidual && WHOLE) request(res, reg);
     __syncthreads();
     if (walks) {
-      const v4f* mine = tile + walked * pitch;
       const uint32_t cols = WHOLE ? len : min(len - 4 * k0 * lanes, 4 * chunk * lanes);
       __builtin_amdgcn_s_setprio(3);  // nothing else of the workgroup moves meanwhile: 26.9 -> 26.4 us on [32,512,28,28]
-      sum = add_in_order(sum, mine, cols);
+      if (together) sum = gate_walk<VEC>(sum, tile, pitch, cols, log2_rows, nrows);
+      else sum = add_in_order(sum, tile + walked * pitch, cols);
       __builtin_amdgcn_s_setprio(0);
     }
     if (WHOLE) break;
   }
-  if (walks) row_params[walked].gate = libm::exact_sigmoidf(sum / p.plane, tab);
+  if (walks && walked < nrows) row_params[walked].gate = libm::exact_sigmoidf(sum / p.plane, tab);
   __syncthreads();
 
   asm("" : "+v"(sub), "+v"(lead));  // the slots' offsets are taken again instead of kept
@@ -319,6 +372,124 @@ __global__ __launch_bounds__(kBlock, gate_waves(SLOTS)) void squeeze_gate_kernel
   }
 }
 
+// Rows of whole, aligned vectors that lie in LDS whole, with BatchNorm and ReLU in front and a residual behind:
+// PIECES vectors of one row a lane.  Where a vector lies is worked out once for a lane, or is uniform, so that an element
+// costs its arithmetic and little else, and the walk reads LDS ahead of its additions.  Against squeeze_gate_kernel, with
+// 47 vector instructions an element and a lane of a wave for each row's walk: [32,512,28,28] 25.4 -> 22.6 us, [64,64,56,56]
+// 41.4 -> 24.8, [8,128,64,64] 29.9 -> 10.8, [16,256,48,48] 32.6 -> 21.9, [16,64,40,40] 11.2 -> 8.8.
+constexpr int whole_waves(int pieces) { return pieces <= 4 ? 6 : pieces <= 8 ? 5 : 3; }
+
+template <int PIECES, int RESIDUAL>
+__global__ __launch_bounds__(kBlock, whole_waves(PIECES)) void gate_whole_kernel(
+    const float* x, const float* res, float* y, float* mean, uint32_t rows, uint32_t len, uint32_t log2_lanes, uint32_t pitch,
+    GateParams p) {
+  extern __shared__ v4f tile[];  // the group's rows, pitch vectors apart
+  __shared__ uint64_t tab[32];
+  __shared__ GateRow row_params[kBlock / 16];
+  __shared__ double part[kBlock / kWave];
+  const uint32_t lanes = 1u << log2_lanes, group = kBlock >> log2_lanes;
+  const uint32_t sub = threadIdx.x & (lanes - 1), lead = threadIdx.x >> log2_lanes;
+  const uint32_t row0 = xcd_runs(blockIdx.x, gridDim.x, 2) * group;
+  const uint32_t nrows = min(group, rows - row0), nv = len / 4, row = min(lead, nrows - 1);
+  const bool live = lead < nrows, whole = sub + (PIECES - 1) * lanes < nv;
+  const uint64_t start = static_cast<uint64_t>(row0) * len;
+  // Bytes from the group's first element: a lane's offset, which a piece's uniform part is added to, and the last
+  // piece's, where lanes past the row's end take its last vector.
+  const uint32_t at = (row * nv + sub) * static_cast<uint32_t>(sizeof(v4f));
+  const uint32_t at_last = (row * nv + min(sub + (PIECES - 1) * lanes, nv - 1)) * static_cast<uint32_t>(sizeof(v4f));
+  const auto place = [&](int k) { return k + 1 < PIECES ? static_cast<size_t>(k * lanes) * sizeof(v4f) + at : static_cast<size_t>(at_last); };
+  const auto request = [&](const float* src, v4f (&to)[PIECES]) {
+    const char* from = reinterpret_cast<const char*>(src + start);
+#pragma unroll
+    for (int k = 0; k < PIECES; ++k) to[k] = load4_stream(reinterpret_cast<const float*>(from + place(k)));
+  };
+  const uint32_t own = row0 + min(threadIdx.x, nrows - 1), ch = own - fd_div(own, p.channel) * p.channel.d;
+  const auto param = [&](const float* from) { return (from ? from : x)[ch]; };  // an absent one from an address that is there
+  const float stat_mean = p.stat_mean[ch], stat_variance = p.stat_variance[ch], scale = param(p.scale);
+  const float bias = param(p.bias), tail_scale = param(p.tail_scale), tail_bias = param(p.tail_bias);
+  const uint64_t entry = libm::kExp2fTab[threadIdx.x & 31u];
+  v4f reg[PIECES];
+  request(x, reg);
+  if (threadIdx.x < nrows) {
+    GateRow g{stat_mean * p.scale_factor, 1.f, 1.0, 1.f, -0.f, 1.f, -0.f, 0.f};
+    g.d = __builtin_sqrtf(__builtin_fabsf(stat_variance * p.scale_factor) + p.eps);
+    g.r = reciprocal(g.d);
+    if (p.scale) g.s = scale;
+    if (p.bias) g.b = bias;
+    if (p.tail_scale) g.tail_s = tail_scale;
+    if (p.tail_bias) g.tail_b = tail_bias;
+    row_params[threadIdx.x] = g;
+  }
+  if (threadIdx.x < 32) tab[threadIdx.x] = entry;
+  __syncthreads();
+
+  v4f* const mine = tile + lead * pitch + sub;
+  {
+    const GateRow g = row_params[row];
+#pragma unroll
+    for (int k = 0; k < PIECES; ++k) {
+      v4f t = reg[k];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) t[j] = t[j] - g.m;
+      t = quotients4(t, g.d, g.r);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        t[j] = t[j] * g.s;
+        t[j] = __builtin_fmaxf(t[j] + g.b, 0.f);  // as in squeeze_gate_kernel
+      }
+      if (live && (k + 1 < PIECES || whole)) mine[k * lanes] = t;
+    }
+  }
+  // the residual travels while the rows are summed
+  if (RESIDUAL == kOtherResidual) request(res, reg);
+  __syncthreads();
+  if (threadIdx.x / kWave == ((blockIdx.x / kXcds) & 3u)) {  // as in squeeze_gate_kernel
+    __builtin_amdgcn_s_setprio(3);
+    const uint32_t log2_rows = 8 - log2_lanes, walked = (threadIdx.x & (kWave - 1)) >> (6 - log2_rows);
+    const float sum = gate_walk<true>(0.f, tile, pitch, len, log2_rows, nrows);
+    if (walked < nrows) row_params[walked].gate = libm::exact_sigmoidf(sum / p.plane, tab);  // all lanes of a row the same
+    __builtin_amdgcn_s_setprio(0);
+  }
+  __syncthreads();
+
+  const float gate = row_params[row].gate, tail_s = row_params[row].tail_s, tail_b = row_params[row].tail_b;
+  char* const to = reinterpret_cast<char*>(y + start);
+  double total = 0.0;
+  const auto finish = [&](int k) {
+    v4f t = mine[k * lanes];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      t[j] = t[j] * gate;
+      t[j] = t[j] * tail_s;
+      t[j] = t[j] + tail_b;
+      t[j] = __builtin_fmaxf(t[j] + reg[k][j], 0.f);  // as in squeeze_gate_kernel
+    }
+    store4_stream(reinterpret_cast<float*>(to + place(k)), t);
+    if (mean) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) total += static_cast<double>(t[j]);
+    }
+  };
+  if (live) {
+#pragma unroll
+    for (int k = 0; k + 1 < PIECES; ++k) finish(k);
+    if (whole) finish(PIECES - 1);
+  }
+  if (!mean) return;
+  total += dpp_f64<kDppXor1>(total);
+  total += dpp_f64<kDppXor2>(total);
+  total += dpp_f64<kDppHalfMirror>(total);
+  total += dpp_f64<kDppMirror>(total);
+  if (log2_lanes > 4) total += __shfl_xor(total, 16, kWave);
+  if (log2_lanes > 5) total += __shfl_xor(total, 32, kWave);
+  if (log2_lanes > 6) {  // the workgroup's one row
+    if ((threadIdx.x & (kWave - 1)) == 0) part[threadIdx.x / kWave] = total;
+    __syncthreads();
+    total = ((part[0] + part[1]) + part[2]) + part[3];
+  }
+  if (sub == 0 && live) mean[row0 + lead] = static_cast<float>(total / static_cast<double>(static_cast<int>(len)));
+}
+
 }  // namespace shdw
 
 using namespace shdw;
@@ -378,6 +549,28 @@ void launch_gate(const GateShape& g, uint32_t rows, uint32_t len, const float* x
   }
 }
 
+template <int PIECES>
+void launch_gate_whole(const GateWhole& g, uint32_t rows, uint32_t len, const float* x, const float* res, float* y, float* mean,
+                       const GateParams& p, hipStream_t st) {
+  const uint32_t grid = (rows + g.group - 1) / g.group;
+  const size_t lds = static_cast<size_t>(g.group) * g.pitch * sizeof(v4f);
+  const auto launch = [&](auto kernel) { kernel<<<grid, kBlock, lds, st>>>(x, res, y, mean, rows, len, g.log2_lanes, g.pitch, p); };
+  if (res == x) launch(gate_whole_kernel<PIECES, kSameResidual>);
+  else launch(gate_whole_kernel<PIECES, kOtherResidual>);
+}
+
+static_assert(kGateWholePieces == 15, "the switch covers up to 15 vectors a lane");
+
+void launch_gate_whole(const GateWhole& g, uint32_t rows, uint32_t len, const float* x, const float* res, float* y, float* mean,
+                       const GateParams& p, hipStream_t st) {
+  switch (g.pieces) {
+#define SHDW_PIECES(P) case P: launch_gate_whole<P>(g, rows, len, x, res, y, mean, p, st); break;
+    SHDW_PIECES(1) SHDW_PIECES(2) SHDW_PIECES(3) SHDW_PIECES(4) SHDW_PIECES(5) SHDW_PIECES(6) SHDW_PIECES(7) SHDW_PIECES(8)
+    SHDW_PIECES(9) SHDW_PIECES(10) SHDW_PIECES(11) SHDW_PIECES(12) SHDW_PIECES(13) SHDW_PIECES(14) SHDW_PIECES(15)
+#undef SHDW_PIECES
+  }
+}
+
 }  // namespace
 
 extern "C" int shdw_hip_squeeze_gate(int n, int channel, int inner_num, const float* x, const float* stat_mean,
@@ -393,6 +586,10 @@ extern "C" int shdw_hip_squeeze_gate(int n, int channel, int inner_num, const fl
   const GateParams p{stat_mean, stat_variance, scale, bias, tail_scale, tail_bias, scale_factor, eps,
                      static_cast<float>(inner_num), relu, make_fastdiv(static_cast<uint32_t>(channel))};
   const bool vec = len % 4 == 0 && aligned16(x) && aligned16(y) && (!residual || aligned16(residual));
+  if (GateWhole w; vec && stat_mean && relu && residual && gate_whole(rows, len, &w)) {
+    launch_gate_whole(w, rows, len, x, residual, y, mean, p, static_cast<hipStream_t>(stream));
+    return launch_status();
+  }
   const GateShape g = gate_shape(rows, len);
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (vec) launch_gate<true>(g, rows, len, x, residual, y, mean, p, st);

@@ -52,6 +52,38 @@ inline GateShape gate_shape(uint32_t rows, uint32_t len) {
   return g;
 }
 
+// How gate_whole_kernel cuts rows of nv whole vectors: `pieces` vectors of one row a lane.
+struct GateWhole {
+  uint32_t log2_lanes, pieces, group, pitch;
+};
+
+constexpr uint32_t kGateWholePieces = 15, kGateWholeMinVectors = 96, kGateWholeFewRows = 1024;
+constexpr uint32_t kGateWholeTileBytes = 33000;  // four workgroups a CU; a row of the whole workgroup may take kGateMaxTileBytes
+
+// Of 16, 32, 64 and 256 lanes a row, the ones with the fewest vector instructions an element: about 16 an
+// element of a lane's share, whether it holds something or not, and the walk's additions, of which
+// one instruction serves all rows of a workgroup; but with less than 1024 workgroups as many lanes as gate_shape
+// takes ([32,512,28,28] 22.4 us with 32 lanes, 23.8 with 64; [8,512,28,28] 9.2 and 8.0; [64,64,40,40] 13.1 with 64, 14.3 with
+// 256; [2,256,28,28] 6.9 / 5.7 / 5.4 with 32 / 64 / 256).  false: no cut holds the rows, or many rows are so short
+// that squeeze_gate_kernel's several rows a lane are faster ([64,512,14,14] 11.5 and 12.8 at best, [64,256,20,20] 11.5 and 11.2).
+inline bool gate_whole(uint32_t rows, uint32_t len, GateWhole* out) {
+  const uint32_t nv = len / 4, usual = gate_shape(rows, len).log2_lanes;
+  if (nv < kGateWholeMinVectors && rows >= kGateWholeFewRows) return false;
+  float least = 0.f;
+  bool found = false;
+  for (uint32_t log2_lanes = 4; log2_lanes <= 8; log2_lanes += log2_lanes == 6 ? 2 : 1) {
+    const uint32_t lanes = 1u << log2_lanes, pieces = (nv + lanes - 1) / lanes, group = kGateLanes >> log2_lanes, pitch = nv | 1u;
+    const uint32_t bytes = group * pitch * kGateVectorBytes;
+    if (pieces > (log2_lanes == 8 ? kGateWholePieces : 8u) || bytes > (log2_lanes == 8 ? kGateMaxTileBytes : kGateWholeTileBytes)) continue;
+    if ((rows + group - 1) / group < 1024u && log2_lanes != usual) continue;
+    const float cost = 16.f * static_cast<float>(pieces * lanes) / static_cast<float>(nv) + 64.f / static_cast<float>(group);
+    if (found && cost >= least) continue;
+    found = true, least = cost;
+    *out = GateWhole{log2_lanes, pieces, group, pitch};
+  }
+  return found;
+}
+
 }  // namespace shdw
 
 #endif  // SHADOW_AMD_CSRC_GATE_SHAPE_H_

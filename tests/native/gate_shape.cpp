@@ -25,3 +25,24 @@ extern "C" unsigned gate_shape_scan(unsigned rows, unsigned last) {
   }
   return 0;
 }
+
+extern "C" int gate_whole(unsigned rows, unsigned len, unsigned* out) {
+  shdw::GateWhole g{};
+  if (!shdw::gate_whole(rows, len, &g)) return 0;
+  out[0] = 1u << g.log2_lanes, out[1] = g.pieces, out[2] = g.group;
+  return 1;
+}
+
+// The same for gate_whole, lengths of whole vectors.
+extern "C" unsigned gate_whole_scan(unsigned rows, unsigned last) {
+  for (unsigned len = 4; len <= last; len += 4) {
+    shdw::GateWhole g{};
+    if (!shdw::gate_whole(rows, len, &g)) continue;
+    const unsigned nv = len / 4, lanes = 1u << g.log2_lanes;
+    const bool ok = g.log2_lanes >= 4 && g.log2_lanes <= 8 && g.log2_lanes != 7 && g.group * lanes == 256 && g.group <= 16 &&
+                    g.pieces >= 1 && g.pieces <= shdw::kGateWholePieces && (g.pieces - 1) * lanes < nv && nv <= g.pieces * lanes &&
+                    g.pitch >= nv && g.pitch % 2 == 1 && g.group * g.pitch * 16u + 1280u <= 65536u;
+    if (!ok) return len;
+  }
+  return 0;
+}

@@ -38,3 +38,21 @@ def test_forms_of_the_gpu_shapes(native):
         got = cut(native, n * c, h * w)
         assert {k: got[k] for k in form} == form, (n, c, h, w, got)
     assert {f["slots"] for f in FORMS.values()} == {1, 4, 8, 16}
+
+
+@pytest.mark.parametrize("rows", [1, 2, 255, 1023, 1024, 1025, 4095, 4096, 8192, 16384, 65536])
+def test_every_cut_of_whole_rows_fits_its_kernel(native, rows):
+    assert native.gate_whole_scan(rows, 15360) == 0
+
+
+def test_whole_rows_of_the_gpu_shapes(native):
+    """The shapes of test_gpu_gate.py take every number of vectors a lane and every number of lanes a row."""
+    from tests.test_gpu_gate import WHOLE
+    out = (ctypes.c_uint * 3)()
+    got = []
+    for n, c, h, w in WHOLE:
+        assert native.gate_whole(n * c, h * w, out) == 1, (n, c, h, w)
+        got.append((out[0], out[1], n * c % out[2] != 0))
+    assert {p for _, p, _ in got} == set(range(1, 16))
+    assert {lanes for lanes, _, _ in got} == {16, 32, 64, 256}
+    assert {lanes for lanes, _, cut in got if cut} == {16, 32, 64}

@@ -39,6 +39,13 @@ FORMS = {
 }
 
 
+# rows of whole vectors behind BatchNorm and ReLU: one to fifteen vectors of 256 lanes a row, the last one whole and
+# cut, and 16, 32 and 64 lanes with last groups cut short
+WHOLE = [(5, 3, 8, 8), (2, 3, 32, 32), (3, 2, 28, 44), (2, 2, 50, 50), (2, 2, 64, 64), (1, 3, 68, 72), (1, 2, 78, 78), (1, 2, 88, 88),
+         (2, 1, 94, 96), (1, 2, 96, 100), (1, 2, 104, 104), (1, 2, 108, 108), (1, 2, 112, 112), (1, 2, 120, 112), (1, 2, 120, 120),
+         (1, 2, 120, 128), (32001, 1, 20, 20), (17003, 1, 18, 28), (8201, 1, 28, 28), (4101, 1, 32, 32), (4101, 1, 40, 40), (1025, 1, 56, 56)]
+
+
 class Case:
     """Inputs of one shape; parts that are left out are None."""
 
@@ -114,6 +121,21 @@ class Case:
 @pytest.mark.parametrize("shape", sorted(FORMS))
 def test_every_form(gpu, shape, residual):
     Case(shape, residual).check(gpu, "%s %s" % (shape, residual))
+
+
+@pytest.mark.parametrize("residual", ["x", "other"])
+@pytest.mark.parametrize("shape", WHOLE)
+def test_whole_rows(gpu, shape, residual):
+    """Special values among the elements of small shapes; in place of the residual as well."""
+    case = Case(shape, residual, special=shape[0] * shape[1] < 32)
+    case.check(gpu, "%s %s" % (shape, residual))
+    case.check(gpu, "%s %s in place" % (shape, residual), alias="x" if residual == "x" else "residual", mean=False)
+
+
+# long rows without ReLU, whose sums have signs, whole and chunked
+@pytest.mark.parametrize("shape", [(3, 2, 40, 40), (2, 2, 63, 65), (600, 1, 64, 64), (516, 1, 84, 84), (516, 1, 81, 81)])
+def test_long_rows_with_signs(gpu, shape):
+    Case(shape, "other", relu=False, special=shape[0] < 9).check(gpu, "%s signs" % (shape,))
 
 
 # whole and chunked, whole vectors and not
