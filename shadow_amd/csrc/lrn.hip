@@ -160,7 +160,10 @@ __global__ __launch_bounds__(kBlock, 5) void lrn_window_kernel(const float* x, f
   // in_group is below 4, which the compiler does not know: spelt out, [2,56,28,28] takes 6.1 us instead of 6.4
   const uint32_t share = WAVES == kLrnWaves ? 0u : in_group / WAVES, wave = WAVES == kLrnWaves ? in_group : in_group % WAVES;
   LrnHand<SIZE>& hand = hands[share];
-  const uint32_t p = (blockIdx.x * (kLrnWaves / WAVES) + share) * kWave + lane, at = min(p, positions - 1);
+  // Runs of positions that start inside a line share it with the run before: the XCD's own neighbours then
+  // ([44,96,55,55] 32.3 -> 30.4 us, [64,256,27,27] 34.1 -> 30.2; no gain where rows are whole vectors).
+  const uint32_t block = STREAM ? blockIdx.x : xcd_contiguous(blockIdx.x, gridDim.x);
+  const uint32_t p = (block * (kLrnWaves / WAVES) + share) * kWave + lane, at = min(p, positions - 1);
   const uint32_t b = fd_div(at, f_step);
   const size_t base = static_cast<size_t>(b) * channels * step + (at - b * step);
   const float* in = x + base;
