@@ -104,7 +104,7 @@ SHDW_DEVICE void lrn_powers(const float (&scale)[kLrnRound], float y, bool small
 // Bound by the vector ALUs: the powers, fp64 for the most part.  With one wave
 // walking all channels of its positions, and up to eight workgroups sharing the rounds of a
 // position where there are few (each walking from the first channel on): [44,96,55,55]
-// 36.9 -> 28.9 us, [16,256,56,56] 48.6 -> 31.5, [64,256,56,56] 122 -> 92, [64,256,27,27] 50.0 ->
+// 36.9 -> 28.9 us (27.6 with what launch_windows cuts), [16,256,56,56] 48.6 -> 31.5, [64,256,56,56] 122 -> 92, [64,256,27,27] 50.0 ->
 // 30.6, [1,96,55,55] 14.8 -> 8.8, [512,8,56,56] 48.0 -> 27.5, [100,40,56,56] 31.3 -> 24.0.  Rounds of 16
 // and 24 channels: 37.8 and 37.6 on the first.
 //
@@ -146,24 +146,18 @@ SHDW_DEVICE float lrn_walk(const float (&own)[kLrnRound], const float (&prev)[SI
 // pieces of lines would leave one by one ([44,96,55,55] 32.6 us plain, 34.0 with it, [68,256,27,27] 35.0
 // and 40.5; [64,256,56,56] 93.2 and 82.1, [256,64,14,14] 11.8 and 10.5, all with four waves a position).
 template <int SIZE, int WAVES, bool STREAM>
-__global__ __launch_bounds__(kBlock, 5) void lrn_window_kernel(const float* x, float* y, uint32_t positions, uint32_t step,
-                                                               uint32_t channels, float alpha_over_size, float neg_beta,
-                                                               float k, FastDiv f_step) {
+SHDW_DEVICE void lrn_window(LrnTables& tables, LrnHand<SIZE>* hands, uint32_t block, uint32_t first, const float* x, float* y,
+                            uint32_t positions, uint32_t step, uint32_t channels, float alpha_over_size, float neg_beta, float k,
+                            const FastDiv& f_step) {
   constexpr int SEG = kLrnRound;
   static_assert(SIZE % 2 == 1 && SIZE <= SEG, "the window must fit into a round");
   constexpr uint32_t post = (SIZE - 1) / 2;
-  __shared__ LrnTables tables;
-  __shared__ LrnHand<SIZE> hands[kLrnWaves / WAVES];
-  lrn_stage_tables(&tables);
   const uint32_t lane = threadIdx.x % kWave;
   const uint32_t in_group = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   // in_group is below 4, which the compiler does not know: spelt out, [2,56,28,28] takes 6.1 us instead of 6.4
   const uint32_t share = WAVES == kLrnWaves ? 0u : in_group / WAVES, wave = WAVES == kLrnWaves ? in_group : in_group % WAVES;
   LrnHand<SIZE>& hand = hands[share];
-  // Runs of positions that start inside a line share it with the run before: the XCD's own neighbours then
-  // ([44,96,55,55] 32.3 -> 30.4 us, [64,256,27,27] 34.1 -> 30.2; no gain where rows are whole vectors).
-  const uint32_t block = STREAM ? blockIdx.x : xcd_contiguous(blockIdx.x, gridDim.x);
-  const uint32_t p = (block * (kLrnWaves / WAVES) + share) * kWave + lane, at = min(p, positions - 1);
+  const uint32_t p = first + (block * (kLrnWaves / WAVES) + share) * kWave + lane, at = min(p, positions - 1);
   const uint32_t b = fd_div(at, f_step);
   const size_t base = static_cast<size_t>(b) * channels * step + (at - b * step);
   const float* in = x + base;
@@ -219,6 +213,26 @@ __global__ __launch_bounds__(kBlock, 5) void lrn_window_kernel(const float* x, f
       }
     }
   }
+}
+
+// `whole` workgroups of WAVES waves for 64 positions, and behind them, if there are more, workgroups of four waves
+// for what positions are left.
+template <int SIZE, int WAVES, bool STREAM>
+__global__ __launch_bounds__(kBlock, 5) void lrn_window_kernel(const float* x, float* y, uint32_t positions, uint32_t step,
+                                                               uint32_t channels, float alpha_over_size, float neg_beta,
+                                                               float k, uint32_t whole, FastDiv f_step) {
+  __shared__ LrnTables tables;
+  __shared__ LrnHand<SIZE> hands[kLrnWaves / WAVES];
+  lrn_stage_tables(&tables);
+  if (WAVES == 2 && blockIdx.x >= whole) {
+    lrn_window<SIZE, kLrnWaves, STREAM>(tables, hands, blockIdx.x - whole, whole * (kLrnWaves / WAVES * kWave), x, y, positions, step,
+                                        channels, alpha_over_size, neg_beta, k, f_step);
+    return;
+  }
+  // Runs of positions that start inside a line share it with the run before: the XCD's own neighbours then
+  // ([44,96,55,55] 32.3 -> 30.4 us, [64,256,27,27] 34.1 -> 30.2; no gain where rows are whole vectors).
+  const uint32_t block = STREAM ? blockIdx.x : xcd_contiguous(blockIdx.x, whole);
+  lrn_window<SIZE, WAVES, STREAM>(tables, hands, block, 0, x, y, positions, step, channels, alpha_over_size, neg_beta, k, f_step);
 }
 
 // The channels of the round that starts at head0 (zeros past the last one).
@@ -293,14 +307,21 @@ using namespace shdw;
 
 namespace {
 
+// Two waves for 64 positions: the vector ALUs bound this, so the CU with the most workgroups does. Workgroups beyond
+// the CUs' even share, if they are half a share or less, are cut in two, of four waves for 64 positions, so that no CU
+// gets more than half of one on top: [44,96,55,55], 1040 workgroups, 29.8 -> 27.6 us, [44,96,56,56] 26.2 -> 22.8,
+// [45,96,50,50] 24.8 -> 21.4, [33,64,64,64] 18.9 -> 17.1.
 template <int SIZE, int WAVES>
 void launch_windows(const float* x, float* y, uint32_t positions, uint32_t step, uint32_t channels, float alpha_over_size,
                     float neg_beta, float k, bool stream, hipStream_t st) {
-  constexpr uint32_t kOwned = kLrnWaves / WAVES * kWave;
-  const uint32_t grid = positions / kOwned + (positions % kOwned != 0);
+  constexpr uint32_t kOwned = kLrnWaves / WAVES * kWave, kCus = 256;
+  const uint32_t all = positions / kOwned + (positions % kOwned != 0), rest = all % kCus;
+  const bool cut = WAVES == 2 && all > kCus && rest != 0 && rest <= kCus / 2 && channels > 4 * kLrnRound;
+  const uint32_t whole = cut ? all - rest : all;
+  const uint32_t grid = cut ? whole + (positions - whole * kOwned + kWave - 1) / kWave : all;
   const FastDiv f_step = make_fastdiv(step);
-  if (stream) lrn_window_kernel<SIZE, WAVES, true><<<grid, kBlock, 0, st>>>(x, y, positions, step, channels, alpha_over_size, neg_beta, k, f_step);
-  else lrn_window_kernel<SIZE, WAVES, false><<<grid, kBlock, 0, st>>>(x, y, positions, step, channels, alpha_over_size, neg_beta, k, f_step);
+  if (stream) lrn_window_kernel<SIZE, WAVES, true><<<grid, kBlock, 0, st>>>(x, y, positions, step, channels, alpha_over_size, neg_beta, k, whole, f_step);
+  else lrn_window_kernel<SIZE, WAVES, false><<<grid, kBlock, 0, st>>>(x, y, positions, step, channels, alpha_over_size, neg_beta, k, whole, f_step);
 }
 
 // One wave for 64 positions works without barriers and leaves no wave without a round, four finish soonest and

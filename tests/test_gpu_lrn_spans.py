@@ -46,3 +46,15 @@ def test_lrn_spans_of_many_positions(gpu, channels, positions, size):
     want = oracle.lrn(x, shape, size, 1e-2, 0.75, 1.0)[0]
     assert_bit_exact(gpuops.lrn(x, shape, size, 1e-2, 0.75, 1.0), want, "lrn")
     assert_bit_exact(gpuops.lrn(x, shape, size, 1e-2, 0.75, 1.0, inplace=True), want, "lrn in place")
+
+
+# two waves for 64 positions, 769 to 897 workgroups of 128: the ones beyond 768 cut in two where they are up to 128; several
+# images, and a last run of one position
+@pytest.mark.parametrize("images,positions", [(1, 98305), (3, 32789), (1, 114688), (1, 114689), (7, 14337)])
+@pytest.mark.parametrize("channels,size", [(33, 5), (40, 3)])
+def test_lrn_spans_cut_in_two(gpu, images, positions, channels, size):
+    shape = (images, channels, 1, positions)
+    x = normal(channels + size, images * channels * positions, 4.0)
+    want = oracle.lrn(x, shape, size, 1e-2, 0.75, 1.0)[0]
+    assert_bit_exact(gpuops.lrn(x, shape, size, 1e-2, 0.75, 1.0), want, "lrn")
+    assert_bit_exact(gpuops.lrn(x, shape, size, 1e-2, 0.75, 1.0, inplace=True), want, "lrn in place")
