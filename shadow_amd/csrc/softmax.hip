@@ -1643,10 +1643,11 @@ __global__ __launch_bounds__(kBlock) void softmax_short_rows_kernel(const float*
 // (WHOLE: moved 128 bits at a time), others one element apart, and a span is odd too, so that
 // neighbouring lanes meet different banks.
 // [139712,21,1], 23.5 MB: 11.7 -> 8.5 us; [600000,21,1] 33.4 -> 24.7, [4096,1000,1] 20.9 -> 16.2,
-// [262144,49,1] 30.6 -> 25.6.
+// [262144,49,1] 30.6 -> 25.6.  A kernel for every number of fours a lane holds, without a test an element and with all
+// exponentials side by side: 8.5 -> 7.0, 16.2 -> 14.5, [5000,91,1] 5.8 -> 4.1, [1024,64,1] 5.1 -> 3.6, [60000,91,1] 11.9 -> 10.5.
 constexpr int kRowsSpan = 36;  // at most: 1023 elements over 32 lanes, made odd
 
-template <bool WHOLE>
+template <bool WHOLE, int QUADS>
 __global__ __launch_bounds__(kBlock, 4) void softmax_rows_kernel(const float* x, float* y, uint32_t rows, uint32_t span,
                                                               uint32_t tile_floats, WaveRows w) {
   extern __shared__ __align__(16) float lds[];
@@ -1669,7 +1670,7 @@ __global__ __launch_bounds__(kBlock, 4) void softmax_rows_kernel(const float* x,
       if (k * kWave < nvec) reg[k] = load4_stream_any(x + base + 4 * min(k * kWave + lane, nvec - 1));
 #pragma unroll
     for (int k = 0; k < kMost; ++k)
-      if (k * kWave + lane < nvec) *reinterpret_cast<v4f*>(tile + 4 * (k * kWave + lane)) = reg[k];
+      if (k * kWave < nvec && k * kWave + lane < nvec) *reinterpret_cast<v4f*>(tile + 4 * (k * kWave + lane)) = reg[k];
     if (rest < cells) tile[rest] = x[base + rest];
   } else {
     rows_stage_in(tile, x + base, cells, w, lane);
@@ -1677,20 +1678,29 @@ __global__ __launch_bounds__(kBlock, 4) void softmax_rows_kernel(const float* x,
   __builtin_amdgcn_wave_barrier();
   const uint32_t group = 1u << w.group_log2, r = lane >> w.group_log2, sub = lane & (group - 1);
   const uint32_t c0 = sub * span;
-  const uint32_t n = r < nrows && c0 < w.dim ? min(span, w.dim - c0) : 0u;  // elements of this lane
-  // lanes without any read row 0, which does not matter; a span is read in whole fours, past the row's end
-  float* mine = tile + (n ? r * w.pitch + c0 : 0u);
-  float v[kRowsSpan];
+  const uint32_t turns = (w.dim + span - 1) / span;
+  const bool used = r < nrows && c0 < w.dim;
+  // Elements of this lane, and of the last lane of a row, which has the fewest: what every lane has needs no
+  // test.  Lanes without any take what the row's first lane has, or a row's that is there, and keep it to themselves.
+  const uint32_t n = c0 < w.dim ? min(span, w.dim - c0) : min(span, w.dim), least = w.dim - (turns - 1) * span;
+  float* mine = tile + (used ? r * w.pitch + c0 : r < nrows ? r * w.pitch : 0u);
+  float v[4 * QUADS];
 #pragma unroll
-  for (int k = 0; k < kRowsSpan; k += 4) {
-    if (k >= span) continue;
+  for (int k = 0; k < 4 * QUADS; k += 4) {
+    if (k + 4 <= least) {
 #pragma unroll
-    for (int j = k; j < k + 4; ++j) v[j] = j < n ? mine[j] : -__builtin_inff();  // its exponential is 0, which adds nothing
+      for (int j = k; j < k + 4; ++j) v[j] = mine[j];
+    } else {
+#pragma unroll
+      for (int j = k; j < k + 4; ++j) {
+        const float e = mine[j];  // a span is read in whole fours, past the row's end
+        v[j] = j < n ? e : -__builtin_inff();  // its exponential is 0, which adds nothing
+      }
+    }
   }
   float m = -FLT_MAX;
 #pragma unroll
-  for (int k = 0; k < kRowsSpan; k += 4) {
-    if (k >= span) continue;
+  for (int k = 0; k < 4 * QUADS; k += 4) {
     m = max3_any_order(m, v[k], v[k + 1]);
     m = max3_any_order(m, v[k + 2], v[k + 3]);
   }
@@ -1700,37 +1710,39 @@ __global__ __launch_bounds__(kBlock, 4) void softmax_rows_kernel(const float* x,
   if (group >= 16) m = max3_any_order(m, m, dpp_f32<kDppMirror>(m));
   if (group >= 32) m = max3_any_order(m, m, __shfl_xor(m, 16));
 #pragma unroll
-  for (int k = 0; k < kRowsSpan; k += 4) {
-    if (k >= span) continue;
-#pragma unroll
-    for (int j = k; j < k + 4; ++j) v[j] = libm::exact_expf_nonpositive(v[j] - m, tab);
-  }
+  for (int k = 0; k < 4 * QUADS; ++k) v[k] = libm::exact_expf_nonpositive(v[k] - m, tab);
   float sum = 0.f;
-  const uint32_t turns = (w.dim + span - 1) / span;
   for (uint32_t t = 0; t < turns; ++t) {
     if (t > 0) sum = lane_in_front(sum);
 #pragma unroll
-    for (int k = 0; k < kRowsSpan; k += 4) {
-      if (k >= span) continue;
-#pragma unroll
-      for (int j = k; j < k + 4; ++j) sum += v[j];
-    }
+    for (int k = 0; k < 4 * QUADS; ++k) sum += v[k];
   }
   if (group > 1) sum = __shfl(sum, (lane & ~(group - 1)) + turns - 1);
   const double recip = reciprocal(sum);
 #pragma unroll
-  for (int k = 0; k < kRowsSpan; k += 4) {
-    if (k >= span) continue;
+  for (int k = 0; k < 4 * QUADS; k += 4) {
     const v4f q = quotients4(v4f{v[k], v[k + 1], v[k + 2], v[k + 3]}, sum, recip);
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (k + j < n) mine[k + j] = q[j];
+    for (int j = 0; j < 4; ++j) v[k + j] = q[j];
+  }
+  if (used) {
+#pragma unroll
+    for (int k = 0; k < 4 * QUADS; k += 4) {
+      if (k + 4 <= least) {
+#pragma unroll
+        for (int j = k; j < k + 4; ++j) mine[j] = v[j];
+      } else {
+#pragma unroll
+        for (int j = k; j < k + 4; ++j)
+          if (j < n) mine[j] = v[j];
+      }
+    }
   }
   __builtin_amdgcn_wave_barrier();
   if (WHOLE) {
 #pragma unroll
     for (int k = 0; k < kMost; ++k)
-      if (k * kWave + lane < nvec)
+      if (k * kWave < nvec && k * kWave + lane < nvec)
         store4_stream_any(y + base + 4 * (k * kWave + lane), *reinterpret_cast<const v4f*>(tile + 4 * (k * kWave + lane)));
     if (rest < cells) y[base + rest] = tile[rest];
   } else {
@@ -1797,8 +1809,17 @@ static void launch_softmax_rows(uint32_t rows, const WaveRows& w, uint32_t grid,
   const uint32_t span = group > 1 ? ((w.dim + group - 1) / group) | 1u : w.dim;
   const uint32_t tile = (w.rows_per_wave * w.pitch + kRowsSpan + 3) & ~3u;  // a lane's last four may lie behind the last row
   const size_t bytes = static_cast<size_t>(kBlock / kWave) * tile * sizeof(float);
-  if (w.pitch == w.dim) softmax_rows_kernel<true><<<grid, kBlock, bytes, st>>>(x, y, rows, span, tile, w);
-  else softmax_rows_kernel<false><<<grid, kBlock, bytes, st>>>(x, y, rows, span, tile, w);
+  const auto launch = [&](auto kernel) { kernel<<<grid, kBlock, bytes, st>>>(x, y, rows, span, tile, w); };
+  static_assert(kRowsSpan == 36, "the switch covers up to nine fours a lane");
+  switch ((span + 3) / 4) {
+#define SHDW_QUADS(Q)                                           \
+  case Q:                                                       \
+    if (w.pitch == w.dim) launch(softmax_rows_kernel<true, Q>); \
+    else launch(softmax_rows_kernel<false, Q>);                 \
+    break;
+    SHDW_QUADS(1) SHDW_QUADS(2) SHDW_QUADS(3) SHDW_QUADS(4) SHDW_QUADS(5) SHDW_QUADS(6) SHDW_QUADS(7) SHDW_QUADS(8) SHDW_QUADS(9)
+#undef SHDW_QUADS
+  }
 }
 
 // ---------------------------------------------------------------------------

@@ -52,3 +52,16 @@ def test_rows_of_special_values(gpu, rows, dim):
     with np.errstate(all="ignore"):
         want = oracle.softmax(x, rows, dim, 1)
         assert_bit_exact(gpuops.softmax(x, rows, dim, 1), want, "softmax")
+
+
+# one to nine fours a lane, the last lane of a row with one element, a few and as many as the others; odd and even rows
+@pytest.mark.parametrize("dim", [17, 20, 24, 25, 28, 33, 36, 37, 53, 56, 66, 79, 99, 131, 160, 201, 259, 272, 400, 515, 777, 992, 993, 1023])
+@pytest.mark.parametrize("rows", [1025, 33003])
+def test_last_lanes_of_rows(gpu, rows, dim):
+    rows = min(rows, 4000000 // dim)
+    x = normal(dim, rows * dim, 4.0)
+    x[:dim] = -np.inf
+    x[dim - 1] = 1.0
+    x[3 * dim] = np.nan
+    with np.errstate(all="ignore"):
+        assert_bit_exact(gpuops.softmax(x, rows, dim, 1, offset=dim % 4), oracle.softmax(x, rows, dim, 1), "softmax")
