@@ -11,7 +11,7 @@
 // x + (-0)).  The plane sum is fp32, front to back, by one lane, as Vision::Pooling
 // adds; the mean at the end is fp64, rounded once after the divide.
 //
-// Rows of whole vectors behind BatchNorm and ReLU take gate_whole_kernel, all others squeeze_gate_kernel.
+// Rows of whole vectors behind BatchNorm and ReLU take whole_squeeze_gate_kernel, all others squeeze_gate_kernel.
 //
 // What bounds it: rows held in LDS and registers leave four to six workgroups on a CU, whose loads, ordered sums and
 // stores overlap each other's; the sums, dependent additions, take 2 ns each (long rows without signs
@@ -106,7 +106,7 @@ SHDW_DEVICE float add_in_order(float sum, const v4f* row, uint32_t cols) {
 // the last is read.  All lanes of a row give and get its sum.
 template <bool VEC>
 SHDW_DEVICE float gate_walk(float sum, const v4f* tile, uint32_t pitch, uint32_t cols, uint32_t log2_rows, uint32_t nrows) {
-  constexpr uint32_t kVectors = 7, kSpan = 4 * kVectors, kSideBySide = 36;  // lanes' worth (of 28): 1008 numbers
+  constexpr uint32_t kVectors = 7, kSpan = 4 * kVectors, kSideBySide = 36;  // lanes' worth: 1008 numbers
   const uint32_t lane = threadIdx.x % kWave, shift = 6 - log2_rows, per_row = 1u << shift, at = lane & (per_row - 1);
   const uint32_t nv = (cols + 3) / 4;
   const v4f* row = tile + min(lane >> shift, nrows - 1) * pitch;
@@ -251,7 +251,7 @@ __global__ __launch_bounds__(kBlock, gate_waves(SLOTS)) void squeeze_gate_kernel
 
   // The ordered sums: all in one wave, which issues one addition for all rows; a different
   // wave in neighbouring workgroups, so that the walks of a CU do not meet on one SIMD.
-  const bool together = group <= kGateWalkRows;  // the wave walks all rows as one
+  const bool together = !WHOLE || group <= kGateWalkRows;  // the wave walks all rows as one (chunks: sixteen at most)
   const uint32_t log2_rows = group > 1 ? 32 - __builtin_clz(group - 1) : 0;
   const uint32_t walked = together ? (threadIdx.x & (kWave - 1)) >> (6 - log2_rows) : threadIdx.x & (kWave - 1);
   const bool walks = threadIdx.x / kWave == ((blockIdx.x / kXcds) & 3u) && (together || walked < nrows);
@@ -380,7 +380,7 @@ __global__ __launch_bounds__(kBlock, gate_waves(SLOTS)) void squeeze_gate_kernel
 constexpr int whole_waves(int pieces) { return pieces <= 4 ? 6 : pieces <= 8 ? 5 : 3; }
 
 template <int PIECES, int RESIDUAL>
-__global__ __launch_bounds__(kBlock, whole_waves(PIECES)) void gate_whole_kernel(
+__global__ __launch_bounds__(kBlock, whole_waves(PIECES)) void whole_squeeze_gate_kernel(
     const float* x, const float* res, float* y, float* mean, uint32_t rows, uint32_t len, uint32_t log2_lanes, uint32_t pitch,
     GateParams p) {
   extern __shared__ v4f tile[];  // the group's rows, pitch vectors apart
@@ -555,8 +555,8 @@ void launch_gate_whole(const GateWhole& g, uint32_t rows, uint32_t len, const fl
   const uint32_t grid = (rows + g.group - 1) / g.group;
   const size_t lds = static_cast<size_t>(g.group) * g.pitch * sizeof(v4f);
   const auto launch = [&](auto kernel) { kernel<<<grid, kBlock, lds, st>>>(x, res, y, mean, rows, len, g.log2_lanes, g.pitch, p); };
-  if (res == x) launch(gate_whole_kernel<PIECES, kSameResidual>);
-  else launch(gate_whole_kernel<PIECES, kOtherResidual>);
+  if (res == x) launch(whole_squeeze_gate_kernel<PIECES, kSameResidual>);
+  else launch(whole_squeeze_gate_kernel<PIECES, kOtherResidual>);
 }
 
 static_assert(kGateWholePieces == 15, "the switch covers up to 15 vectors a lane");

@@ -52,7 +52,7 @@ inline GateShape gate_shape(uint32_t rows, uint32_t len) {
   return g;
 }
 
-// How gate_whole_kernel cuts rows of nv whole vectors: `pieces` vectors of one row a lane.
+// How whole_squeeze_gate_kernel cuts rows of nv whole vectors: `pieces` vectors of one row a lane.
 struct GateWhole {
   uint32_t log2_lanes, pieces, group, pitch;
 };

@@ -36,6 +36,8 @@ extern "C" int gate_whole(unsigned rows, unsigned len, unsigned* out) {
 // The same for gate_whole, lengths of whole vectors.
 extern "C" unsigned gate_whole_scan(unsigned rows, unsigned last) {
   for (unsigned len = 4; len <= last; len += 4) {
+    const shdw::GateShape other = shdw::gate_shape(rows, len);
+    if (other.chunk != other.pieces && other.group > 16) return len;  // rows in chunks: one wave walks all of them together
     shdw::GateWhole g{};
     if (!shdw::gate_whole(rows, len, &g)) continue;
     const unsigned nv = len / 4, lanes = 1u << g.log2_lanes;
