@@ -350,6 +350,74 @@ SHDW_DEVICE double sequential_sum(const float* lds, uint32_t n) {
   return sum;
 }
 
+// A row of up to 1024 V floats by a workgroup, V vectors a lane in registers from the maximum to the quotients; the
+// exponentials alone go through LDS, to the wave that adds them up.  The maximum in any order, as below.
+// Bound by its chain: one load, three barriers, the ordered sum (2 us for 1000).  With the row staged in LDS and
+// four passes over it there: [16,1000] 5.0 -> 4.1 us, [500,1024] 6.5 -> 4.6, [4,4096] 10.6 -> 7.3,
+// [1000,4096] 22.0 -> 11.3.
+template <int V>
+__global__ __launch_bounds__(kBlock) void softmax_row_kernel(const float* x, float* y, uint32_t dim) {
+  extern __shared__ __align__(16) float lds[];
+  __shared__ uint64_t tab[32];
+  __shared__ float wave_max[kBlock / kWave];
+  const float* xs = x + static_cast<uint64_t>(blockIdx.x) * dim;
+  float* ys = y + static_cast<uint64_t>(blockIdx.x) * dim;
+  const uint64_t entry = libm::kExp2fTab[threadIdx.x & 31u];
+  v4f r[V];
+#pragma unroll
+  for (int u = 0; u < V; ++u) {
+    const uint32_t c = 4 * (threadIdx.x + u * kBlock);
+    r[u] = v4f{-__builtin_inff(), -__builtin_inff(), -__builtin_inff(), -__builtin_inff()};
+    if (c + 4 <= dim) {
+      r[u] = load4_stream_any(xs + c);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 3; ++j)
+        if (c + j < dim) r[u][j] = xs[c + j];
+    }
+  }
+  if (threadIdx.x < 32) tab[threadIdx.x] = entry;
+  float m = -FLT_MAX;
+#pragma unroll
+  for (int u = 0; u < V; ++u) m = max3_any_order(max3_any_order(m, r[u][0], r[u][1]), r[u][2], r[u][3]);
+  m = max3_any_order(m, m, dpp_f32<kDppXor1>(m));
+  m = max3_any_order(m, m, dpp_f32<kDppXor2>(m));
+  m = max3_any_order(m, m, dpp_f32<kDppHalfMirror>(m));
+  m = max3_any_order(m, m, dpp_f32<kDppMirror>(m));
+  m = max3_any_order(m, m, __shfl_xor(m, 16));
+  m = max3_any_order(m, m, __shfl_xor(m, 32));
+  if (threadIdx.x % kWave == 0) wave_max[threadIdx.x / kWave] = m;
+  __syncthreads();
+  m = max3_any_order(max3_any_order(m, wave_max[0], wave_max[1]), wave_max[2], wave_max[3]);
+#pragma unroll
+  for (int u = 0; u < V; ++u) {
+    const uint32_t c = 4 * (threadIdx.x + u * kBlock);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) r[u][j] = libm::exact_expf_nonpositive(r[u][j] - m, tab);
+    if (c < dim) *reinterpret_cast<v4f*>(lds + c) = r[u];
+  }
+  __syncthreads();
+  if (threadIdx.x < kWave) {
+    const float sum = wave_ordered_sum(lds, dim);
+    if (threadIdx.x == 0) wave_max[0] = sum;  // everyone has read the maxima
+  }
+  __syncthreads();
+  const float sum = wave_max[0];
+  const double recip = reciprocal(sum);
+#pragma unroll
+  for (int u = 0; u < V; ++u) {
+    const uint32_t c = 4 * (threadIdx.x + u * kBlock);
+    const v4f q = quotients4(r[u], sum, recip);
+    if (c + 4 <= dim) {
+      store4_stream_any(ys + c, q);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 3; ++j)
+        if (c + j < dim) ys[c + j] = q[j];
+    }
+  }
+}
+
 // inner == 1 takes the maximum with all lanes in any order.  That is exact:
 // the value of the maximum does not depend on the order unless the column
 // holds a NaN, and then every output is NaN whatever maximum was used (the
@@ -2622,7 +2690,12 @@ static int run_softmax(int outer_num, int dim, int inner_num, const float* x, fl
     softmax_long_slab_kernel<<<outer_num, kBlock, 0, st>>>(x, y, static_cast<uint32_t>(dim), fi);
   } else if (g.use_slab) {
     if (pl->chosen(SHDW_PATH_SLAB, 0, static_cast<uint32_t>(outer_num))) return SHDW_OK;
-    softmax_slab_kernel<<<outer_num, kBlock, g.slab_bytes, st>>>(x, y, static_cast<uint32_t>(dim), fi);
+    const uint32_t d = static_cast<uint32_t>(dim);
+    if (inner_num == 1 && d <= 1024) softmax_row_kernel<1><<<outer_num, kBlock, g.slab_bytes, st>>>(x, y, d);
+    else if (inner_num == 1 && d <= 2048) softmax_row_kernel<2><<<outer_num, kBlock, g.slab_bytes, st>>>(x, y, d);
+    else if (inner_num == 1 && d <= 4096) softmax_row_kernel<4><<<outer_num, kBlock, g.slab_bytes, st>>>(x, y, d);
+    else if (inner_num == 1 && d <= 8192) softmax_row_kernel<8><<<outer_num, kBlock, g.slab_bytes, st>>>(x, y, d);
+    else softmax_slab_kernel<<<outer_num, kBlock, g.slab_bytes, st>>>(x, y, static_cast<uint32_t>(dim), fi);
   } else if (dim <= 64) {
     // the tile kernel is slower here: [64,49,128,128] 115 us against 88
     const uint32_t grid = grid_for(g.columns), d = static_cast<uint32_t>(dim);

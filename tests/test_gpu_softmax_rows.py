@@ -65,3 +65,20 @@ def test_last_lanes_of_rows(gpu, rows, dim):
     x[3 * dim] = np.nan
     with np.errstate(all="ignore"):
         assert_bit_exact(gpuops.softmax(x, rows, dim, 1, offset=dim % 4), oracle.softmax(x, rows, dim, 1), "softmax")
+
+
+# a workgroup a row, in registers: one to eight vectors a lane, the last vector whole and cut, and the longest beyond
+@pytest.mark.parametrize("dim", [5, 1022, 1028, 2045, 2048, 2049, 4093, 4096, 4097, 8189, 8190, 8192, 8193, 12000])
+@pytest.mark.parametrize("rows", [1, 37])
+def test_long_rows_of_a_workgroup(gpu, rows, dim):
+    x = normal(dim, rows * dim, 4.0)
+    if rows > 1:
+        x[:dim] = -np.inf
+        x[dim:2 * dim] = 1.0
+        x[3 * dim - 1] = np.nan
+        x[3 * dim:4 * dim] = -100.0
+        x[4 * dim - 1] = 100.0
+    with np.errstate(all="ignore"):
+        want = oracle.softmax(x, rows, dim, 1)
+        assert_bit_exact(gpuops.softmax(x, rows, dim, 1, offset=dim % 4), want, "softmax")
+        assert_bit_exact(gpuops.softmax(x, rows, dim, 1, inplace=True), want, "softmax in place")
