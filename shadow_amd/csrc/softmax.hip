@@ -354,7 +354,7 @@ SHDW_DEVICE double sequential_sum(const float* lds, uint32_t n) {
 // exponentials alone go through LDS, to the wave that adds them up.  The maximum in any order, as below.
 // Bound by its chain: one load, three barriers, the ordered sum (2 us for 1000).  With the row staged in LDS and
 // four passes over it there: [16,1000] 5.0 -> 4.1 us, [500,1024] 6.5 -> 4.6, [4,4096] 10.6 -> 7.3,
-// [1000,4096] 22.0 -> 11.3.
+// [1000,4096] 22.0 -> 11.3; waves without a part of a short row skip the arithmetic ([1000,200] 4.5 -> 3.9, [550,44] 3.8 -> 3.4).
 template <int V>
 __global__ __launch_bounds__(kBlock) void softmax_row_kernel(const float* x, float* y, uint32_t dim) {
   extern __shared__ __align__(16) float lds[];
@@ -363,11 +363,15 @@ __global__ __launch_bounds__(kBlock) void softmax_row_kernel(const float* x, flo
   const float* xs = x + static_cast<uint64_t>(blockIdx.x) * dim;
   float* ys = y + static_cast<uint64_t>(blockIdx.x) * dim;
   const uint64_t entry = libm::kExp2fTab[threadIdx.x & 31u];
+  // whether some lane of the wave has something in its vector u: waves without skip it
+  const uint32_t wave_first = 4 * __builtin_amdgcn_readfirstlane(threadIdx.x & ~(kWave - 1u));
+  const auto busy = [&](int u) { return wave_first + 4 * u * kBlock < dim; };
   v4f r[V];
 #pragma unroll
   for (int u = 0; u < V; ++u) {
     const uint32_t c = 4 * (threadIdx.x + u * kBlock);
     r[u] = v4f{-__builtin_inff(), -__builtin_inff(), -__builtin_inff(), -__builtin_inff()};
+    if (!busy(u)) continue;
     if (c + 4 <= dim) {
       r[u] = load4_stream_any(xs + c);
     } else {
@@ -392,6 +396,7 @@ __global__ __launch_bounds__(kBlock) void softmax_row_kernel(const float* x, flo
 #pragma unroll
   for (int u = 0; u < V; ++u) {
     const uint32_t c = 4 * (threadIdx.x + u * kBlock);
+    if (!busy(u)) continue;
 #pragma unroll
     for (int j = 0; j < 4; ++j) r[u][j] = libm::exact_expf_nonpositive(r[u][j] - m, tab);
     if (c < dim) *reinterpret_cast<v4f*>(lds + c) = r[u];
@@ -402,11 +407,13 @@ __global__ __launch_bounds__(kBlock) void softmax_row_kernel(const float* x, flo
     if (threadIdx.x == 0) wave_max[0] = sum;  // everyone has read the maxima
   }
   __syncthreads();
+  if (!busy(0)) return;
   const float sum = wave_max[0];
   const double recip = reciprocal(sum);
 #pragma unroll
   for (int u = 0; u < V; ++u) {
     const uint32_t c = 4 * (threadIdx.x + u * kBlock);
+    if (!busy(u)) continue;
     const v4f q = quotients4(r[u], sum, recip);
     if (c + 4 <= dim) {
       store4_stream_any(ys + c, q);
