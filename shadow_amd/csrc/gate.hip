@@ -46,13 +46,14 @@ struct GateParams {
   FastDiv channel;
 };
 
-constexpr uint32_t kGateWalkRows = 16;  // rows that a wave walks as one (gate_walk), a lane each beyond
 enum { kNoResidual = 0, kOtherResidual = 1, kSameResidual = 2 };
 
-// Waves per SIMD that the registers are held to: what a lane's vectors leave room for.
-constexpr int gate_waves(int slots) { return slots == 16 ? 4 : slots == 8 ? 5 : 6; }
+// Waves per SIMD that the registers are held to: what a lane's vectors leave room for.  ONE as in squeeze_gate_kernel: seven
+// for four vectors of one row are 72 registers; with 74, and a workgroup a CU less, 6700 rows of 784 (1675
+// workgroups) take 13.5 us instead of 9.1, of 943 15.8 instead of 11.0.
+constexpr int gate_waves(int slots, bool one) { return slots == 16 ? 4 : slots == 8 ? 5 : slots == 4 && one ? 7 : 6; }
 
-// sum + row[0] + row[1] + ..., in that order, by a lane; for groups of more than sixteen rows, which are short.
+// sum + row[0] + row[1] + ..., in that order, by a lane (gate_shape.h: where).
 // Two sets of six vectors take turns: one is read while the other is added.  A last part of a vector reads the
 // whole of it.
 SHDW_DEVICE float add_in_order(float sum, const v4f* row, uint32_t cols) {
@@ -158,11 +159,12 @@ SHDW_DEVICE float gate_walk(float sum, const v4f* tile, uint32_t pitch, uint32_t
 // the compiler copy the registers of the loads before it, and wait for them): lanes with
 // nothing to load take the row's or the group's last vector again.  WHOLE: the front's
 // result stays in LDS; otherwise LDS holds `chunk` pieces of the rows at a time and the
-// front is taken again on the way out.  ONE: one turn, a lane's vectors are of one row.  FULL: every slot
+// front is taken again on the way out.  ONE: one turn, a lane's vectors are of one row.  TOGETHER: the walk (gate_shape.h; both
+// in one kernel, 30000 rows of 49 take 5.1 us instead of 5.0, and four vectors a lane 74 registers).  FULL: every slot
 // holds something ([64,1024,7,7] with x as the residual 9.8 us, 11.2 with a test a slot; without the test where
 // slots are empty [32,300,27,27] 14.8 instead of 13.9).
-template <int SLOTS, bool VEC, bool WHOLE, bool ONE, bool FULL, int RESIDUAL>
-__global__ __launch_bounds__(kBlock, gate_waves(SLOTS)) void squeeze_gate_kernel(const float* x, const float* res, float* y, float* mean,
+template <int SLOTS, bool VEC, bool WHOLE, bool ONE, bool TOGETHER, bool FULL, int RESIDUAL>
+__global__ __launch_bounds__(kBlock, gate_waves(SLOTS, ONE)) void squeeze_gate_kernel(const float* x, const float* res, float* y, float* mean,
                                                               uint32_t rows, uint32_t len, uint32_t group,
                                                               uint32_t log2_lanes, uint32_t pieces, uint32_t chunk,
                                                               uint32_t pitch, uint32_t used_slots, GateParams p) {
@@ -251,10 +253,9 @@ __global__ __launch_bounds__(kBlock, gate_waves(SLOTS)) void squeeze_gate_kernel
 
   // The ordered sums: all in one wave, which issues one addition for all rows; a different
   // wave in neighbouring workgroups, so that the walks of a CU do not meet on one SIMD.
-  const bool together = !WHOLE || group <= kGateWalkRows;  // the wave walks all rows as one (chunks: sixteen at most)
   const uint32_t log2_rows = group > 1 ? 32 - __builtin_clz(group - 1) : 0;
-  const uint32_t walked = together ? (threadIdx.x & (kWave - 1)) >> (6 - log2_rows) : threadIdx.x & (kWave - 1);
-  const bool walks = threadIdx.x / kWave == ((blockIdx.x / kXcds) & 3u) && (together || walked < nrows);
+  const uint32_t walked = TOGETHER ? (threadIdx.x & (kWave - 1)) >> (6 - log2_rows) : threadIdx.x & (kWave - 1);
+  const bool walks = threadIdx.x / kWave == ((blockIdx.x / kXcds) & 3u) && (TOGETHER || walked < nrows);
   GateRow g;
   float sum = 0.f;
   for (uint32_t k0 = 0; k0 < pieces; k0 += chunk) {
@@ -283,7 +284,7 @@ __global__ __launch_bounds__(kBlock, gate_waves(SLOTS)) void squeeze_gate_kernel
     if (walks) {
       const uint32_t cols = WHOLE ? len : min(len - 4 * k0 * lanes, 4 * chunk * lanes);
       __builtin_amdgcn_s_setprio(3);  // nothing else of the workgroup moves meanwhile: 26.9 -> 26.4 us on [32,512,28,28]
-      if (together) sum = gate_walk<VEC>(sum, tile, pitch, cols, log2_rows, nrows);
+      if (TOGETHER) sum = gate_walk<VEC>(sum, tile, pitch, cols, log2_rows, nrows);
       else sum = add_in_order(sum, tile + walked * pitch, cols);
       __builtin_amdgcn_s_setprio(0);
     }
@@ -498,18 +499,17 @@ namespace {
 
 uint32_t used_slots(const GateShape& g) { return (g.group << g.log2_lanes) / kBlock * g.pieces; }
 
-template <int SLOTS, bool VEC, bool WHOLE, bool ONE>
-void launch_gate(const GateShape& g, uint32_t rows, uint32_t len, const float* x, const float* res, float* y, float* mean,
-                 const GateParams& p, hipStream_t st) {
+template <int SLOTS, bool VEC, bool WHOLE, bool ONE, bool TOGETHER>
+void launch_gate_form(const GateShape& g, uint32_t rows, uint32_t len, const float* x, const float* res, float* y, float* mean,
+                      const GateParams& p, hipStream_t st) {
   const uint32_t grid = (rows + g.group - 1) / g.group, used = used_slots(g);
   const size_t lds = static_cast<size_t>(g.group) * g.pitch * sizeof(v4f);
-#define SHDW_LAUNCH(R)                                                                                                \
-  if (used == SLOTS)                                                                                                  \
-    squeeze_gate_kernel<SLOTS, VEC, WHOLE, ONE, true, R><<<grid, kBlock, lds, st>>>(x, res, y, mean, rows, len, g.group, \
-                                                                                    g.log2_lanes, g.pieces, g.chunk, g.pitch, used, p); \
-  else                                                                                                                \
-    squeeze_gate_kernel<SLOTS, VEC, WHOLE, ONE, SLOTS == 1, R><<<grid, kBlock, lds, st>>>(x, res, y, mean, rows, len, g.group, \
-                                                                                          g.log2_lanes, g.pieces, g.chunk, g.pitch, used, p)
+  const auto launch = [&](auto kernel) {
+    kernel<<<grid, kBlock, lds, st>>>(x, res, y, mean, rows, len, g.group, g.log2_lanes, g.pieces, g.chunk, g.pitch, used, p);
+  };
+#define SHDW_LAUNCH(R)                                                                        \
+  if (used == SLOTS) launch(squeeze_gate_kernel<SLOTS, VEC, WHOLE, ONE, TOGETHER, true, R>);  \
+  else launch(squeeze_gate_kernel<SLOTS, VEC, WHOLE, ONE, TOGETHER, SLOTS == 1, R>)
   if (!res) {
     SHDW_LAUNCH(kNoResidual);
   } else if (res == x) {
@@ -518,6 +518,18 @@ void launch_gate(const GateShape& g, uint32_t rows, uint32_t len, const float* x
     SHDW_LAUNCH(kOtherResidual);
   }
 #undef SHDW_LAUNCH
+}
+
+template <int SLOTS, bool VEC, bool WHOLE, bool ONE>
+void launch_gate(const GateShape& g, uint32_t rows, uint32_t len, const float* x, const float* res, float* y, float* mean,
+                 const GateParams& p, hipStream_t st) {
+  constexpr int kWalks = gate_walks(SLOTS, WHOLE, ONE);
+  if constexpr (kWalks == (kGateLaneARow | kGateTogether)) {
+    if (g.walk == kGateTogether) launch_gate_form<SLOTS, VEC, WHOLE, ONE, true>(g, rows, len, x, res, y, mean, p, st);
+    else launch_gate_form<SLOTS, VEC, WHOLE, ONE, false>(g, rows, len, x, res, y, mean, p, st);
+  } else {
+    launch_gate_form<SLOTS, VEC, WHOLE, ONE, kWalks == kGateTogether>(g, rows, len, x, res, y, mean, p, st);
+  }
 }
 
 // Four vectors a lane of every row and the rows' odd pitch stay below the tile: never cut.

@@ -10,10 +10,20 @@ namespace shdw {
 constexpr uint32_t kGateMaxRows = 64;  // per workgroup: a lane of one wave each in the ordered sum
 constexpr uint32_t kGateLanes = 256, kGateVectorBytes = 16;
 
+// How a group's rows are summed by the wave that does it: a lane a row, which reads LDS as it adds, or the lanes shared out
+// among the rows (gate_walk).
+enum : int { kGateLaneARow = 1, kGateTogether = 2 };
+
+// The walks that a form's shapes have (gate_shape below): several turns of four vectors are up to 512 numbers a row and eight
+// rows or more; rows in chunks, of five vectors a lane and more, and of sixteen are long.
+constexpr int gate_walks(int slots, bool whole, bool one) {
+  return !whole || slots == 16 || (slots == 8 && one) ? kGateTogether : slots == 4 && !one ? kGateLaneARow : kGateLaneARow | kGateTogether;
+}
+
 // How a shape is cut.
 struct GateShape {
   uint32_t log2_lanes, pieces, group, chunk, pitch;
-  int slots;
+  int slots, walk;
 };
 
 // Five workgroups on a CU: the tile and 3.5 KB of parameters, table and partial sums each
@@ -49,6 +59,14 @@ inline GateShape gate_shape(uint32_t rows, uint32_t len) {
     const uint32_t bytes = g.group * g.pitch * kGateVectorBytes;
     if (bytes <= (rows <= 2 * kGateCus * g.group ? kGateMaxTileBytes : kGateTileBytes) || g.chunk == 1) break;
   }
+  // Together, an addition takes 4.8 cycles instead of 8, but has its SIMD to itself meanwhile, and what a chunk's last
+  // lanes lack is added as zeros.  So where rows are long for their number, or their walks few enough to have a SIMD
+  // each.  A lane a row / together, us: groups of four, 6700 rows of 784 9.6 / 9.1, of 400 6.9 / 6.5, of 225 5.5 / 5.9, but
+  // 4000 (1000 workgroups) 5.0 / 4.9; of eight, 13000 of 784 21.3 / 20.7, 10000 of 289 7.9 / 8.2; of twelve, 13000 of 225
+  // 8.9 / 9.4; of sixteen, 30000 of 49 5.1 / 5.7, of 289 18.8 / 19.8.
+  const uint32_t grid = (rows + g.group - 1) / g.group;
+  const bool together = len >= 96 * g.group || (g.group <= 4 && grid <= 4 * kGateCus) || g.chunk != g.pieces;
+  g.walk = together ? kGateTogether : kGateLaneARow;
   return g;
 }
 

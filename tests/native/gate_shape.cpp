@@ -3,14 +3,17 @@
 
 extern "C" void gate_shape(unsigned rows, unsigned len, unsigned* out) {
   const shdw::GateShape g = shdw::gate_shape(rows, len);
-  const unsigned all[] = {g.log2_lanes, g.pieces, g.group, g.chunk, g.pitch, static_cast<unsigned>(g.slots)};
-  for (int k = 0; k < 6; ++k) out[k] = all[k];
+  const unsigned all[] = {g.log2_lanes, g.pieces, g.group, g.chunk, g.pitch, static_cast<unsigned>(g.slots),
+                          g.walk == shdw::kGateTogether};
+  for (int k = 0; k < 7; ++k) out[k] = all[k];
 }
 
 // The first length in [1, last] whose cut breaks what the kernel relies on, or 0.
 extern "C" unsigned gate_shape_scan(unsigned rows, unsigned last) {
   for (unsigned len = 1; len <= last; ++len) {
     const shdw::GateShape g = shdw::gate_shape(rows, len);
+    const int walks = shdw::gate_walks(g.slots, g.chunk == g.pieces, ((g.group << g.log2_lanes) / 256u) == 1u);
+    if ((g.walk & walks) == 0 || (g.walk == shdw::kGateTogether && g.group > 16)) return len;  // a wave walks sixteen rows at most
     const unsigned nv = (len + 3) / 4, lanes = 1u << g.log2_lanes, turn_rows = 256u >> g.log2_lanes;
     const unsigned turns = g.group / turn_rows, kept = g.chunk * lanes < nv ? g.chunk * lanes : nv;
     const bool ok = (g.slots == 1 || g.slots == 4 || g.slots == 8 || g.slots == 16) &&

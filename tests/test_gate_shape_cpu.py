@@ -24,11 +24,11 @@ def test_every_cut_fits_the_kernel(native, rows):
 
 
 def cut(native, rows, length):
-    out = (ctypes.c_uint * 6)()
+    out = (ctypes.c_uint * 7)()
     native.gate_shape(rows, length, out)
-    lanes, pieces, group, chunk, _, slots = out
+    lanes, pieces, group, chunk, _, slots, together = out
     return {"lanes": 1 << lanes, "turns": group * (1 << lanes) // 256, "slots": slots, "chunked": chunk != pieces,
-            "cut_group": rows % group != 0}
+            "cut_group": rows % group != 0, "together": bool(together)}
 
 
 def test_forms_of_the_gpu_shapes(native):
@@ -38,6 +38,15 @@ def test_forms_of_the_gpu_shapes(native):
         got = cut(native, n * c, h * w)
         assert {k: got[k] for k in form} == form, (n, c, h, w, got)
     assert {f["slots"] for f in FORMS.values()} == {1, 4, 8, 16}
+
+
+# groups of 4, 8, 12 and 16 rows, longer and shorter than the rule asks for, and few workgroups of four
+@pytest.mark.parametrize("rows,length,together", [
+    (6700, 784, True), (6700, 400, True), (6700, 384, True), (6700, 383, False), (6700, 225, False), (4096, 225, True), (4097, 225, False),
+    (13000, 784, True), (13000, 767, False), (10000, 289, False), (13000, 225, False), (30000, 49, False), (30000, 289, False),
+    (300, 49, False), (300, 81, True), (1000, 12543, True), (2000, 6561, True)])
+def test_which_rows_are_walked_together(native, rows, length, together):
+    assert cut(native, rows, length)["together"] is together
 
 
 @pytest.mark.parametrize("rows", [1, 2, 255, 1023, 1024, 1025, 4095, 4096, 8192, 16384, 65536])

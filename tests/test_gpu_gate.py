@@ -36,6 +36,15 @@ FORMS = {
     (5, 3, 9, 9): {"lanes": 256, "turns": 1, "slots": 1, "chunked": False},
     (4099, 1, 1, 3): {"lanes": 16, "turns": 1, "slots": 1, "chunked": False, "cut_group": True},
     (4099, 1, 1, 1): {"lanes": 16, "turns": 1, "slots": 1, "chunked": False, "cut_group": True},
+    # a lane a row in the walk, and all lanes together, where a form has both
+    (4101, 1, 16, 20): {"lanes": 64, "turns": 1, "slots": 4, "chunked": False, "cut_group": True, "together": False},
+    (4101, 1, 17, 17): {"lanes": 64, "turns": 1, "slots": 4, "chunked": False, "cut_group": True, "together": False},
+    (4101, 1, 16, 24): {"lanes": 64, "turns": 1, "slots": 4, "chunked": False, "cut_group": True, "together": True},
+    (2001, 1, 17, 17): {"lanes": 64, "turns": 1, "slots": 4, "chunked": False, "cut_group": True, "together": True},
+    (4101, 1, 13, 13): {"lanes": 64, "turns": 1, "slots": 1, "chunked": False, "cut_group": True, "together": False},
+    (2001, 1, 13, 13): {"lanes": 64, "turns": 1, "slots": 1, "chunked": False, "cut_group": True, "together": True},
+    (13003, 1, 20, 20): {"lanes": 64, "turns": 3, "slots": 8, "chunked": False, "cut_group": True, "together": False},
+    (13003, 1, 19, 19): {"lanes": 64, "turns": 3, "slots": 8, "chunked": False, "cut_group": True, "together": False},
 }
 
 
