@@ -598,7 +598,7 @@ extern "C" int shdw_hip_squeeze_gate(int n, int channel, int inner_num, const fl
   const GateParams p{stat_mean, stat_variance, scale, bias, tail_scale, tail_bias, scale_factor, eps,
                      static_cast<float>(inner_num), relu, make_fastdiv(static_cast<uint32_t>(channel))};
   const bool vec = len % 4 == 0 && aligned16(x) && aligned16(y) && (!residual || aligned16(residual));
-  if (GateWhole w; vec && stat_mean && relu && residual && gate_whole(rows, len, &w)) {
+  if (GateWhole w; gate_takes_whole(vec, stat_mean != nullptr, relu != 0, residual != nullptr, rows, len, &w)) {
     launch_gate_whole(w, rows, len, x, residual, y, mean, p, static_cast<hipStream_t>(stream));
     return launch_status();
   }

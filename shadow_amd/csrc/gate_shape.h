@@ -102,6 +102,11 @@ inline bool gate_whole(uint32_t rows, uint32_t len, GateWhole* out) {
   return found;
 }
 
+// Whether a call is whole_squeeze_gate_kernel's, and its cut.  vec: whole, aligned vectors in every row.
+inline bool gate_takes_whole(bool vec, bool stats, bool relu, bool residual, uint32_t rows, uint32_t len, GateWhole* out) {
+  return vec && stats && relu && residual && gate_whole(rows, len, out);
+}
+
 }  // namespace shdw
 
 #endif  // SHADOW_AMD_CSRC_GATE_SHAPE_H_

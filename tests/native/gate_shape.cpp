@@ -36,6 +36,12 @@ extern "C" int gate_whole(unsigned rows, unsigned len, unsigned* out) {
   return 1;
 }
 
+// Whether a call with these parts and aligned operands is whole_squeeze_gate_kernel's.
+extern "C" int gate_takes_whole(unsigned rows, unsigned len, int stats, int relu, int residual) {
+  shdw::GateWhole g{};
+  return shdw::gate_takes_whole(len % 4 == 0, stats != 0, relu != 0, residual != 0, rows, len, &g);
+}
+
 // The same for gate_whole, lengths of whole vectors.
 extern "C" unsigned gate_whole_scan(unsigned rows, unsigned last) {
   for (unsigned len = 4; len <= last; len += 4) {

@@ -49,6 +49,25 @@ def test_which_rows_are_walked_together(native, rows, length, together):
     assert cut(native, rows, length)["together"] is together
 
 
+def test_which_kernel_the_gpu_shapes_get(native):
+    """Forms of whole vectors reach both kernels: with all parts some are whole_squeeze_gate_kernel's, with one left out none."""
+    from tests.test_gpu_gate import FORMS, GENERIC, WHOLE
+
+    def whole(shape, stats=True, relu=True, residual=True):
+        return native.gate_takes_whole(shape[0] * shape[1], shape[2] * shape[3], stats, relu, residual) == 1
+    vectors = [s for s in FORMS if s[2] * s[3] % 4 == 0]
+    assert {s for s in FORMS if whole(s)} == {(516, 1, 84, 84), (2060, 1, 44, 44), (2061, 1, 60, 60), (600, 1, 112, 112), (3, 2, 112, 112),
+                                              (8201, 1, 28, 28), (4101, 1, 16, 24), (13003, 1, 20, 20)}
+    assert all(whole(s) for s in WHOLE)
+    for parts in GENERIC + [dict(residual=False)]:
+        assert not any(whole(s, **parts) for s in vectors + WHOLE)
+    # what is left to squeeze_gate_kernel: every number of vectors a lane and both walks
+    forms = [cut(native, s[0] * s[1], s[2] * s[3]) for s in vectors]
+    assert {(f["slots"], f["chunked"], f["turns"] > 1) for f in forms} >= {
+        (4, False, False), (4, False, True), (8, False, True), (8, True, False), (8, True, True), (16, False, False), (16, True, False)}
+    assert {(f["slots"], f["together"]) for f in forms} >= {(4, False), (4, True), (8, False), (8, True), (16, True)}
+
+
 @pytest.mark.parametrize("rows", [1, 2, 255, 1023, 1024, 1025, 4095, 4096, 8192, 16384, 65536])
 def test_every_cut_of_whole_rows_fits_its_kernel(native, rows):
     assert native.gate_whole_scan(rows, 15360) == 0

@@ -1,9 +1,9 @@
-"""shdw_hip_squeeze_gate through the C ABI, every form its kernel has: rows whole in LDS and in
+"""shdw_hip_squeeze_gate through the C ABI, every form its kernels have: rows whole in LDS and in
 chunks, one and several rows a lane, last groups cut short, one to sixteen vectors a lane,
 each with rows of whole vectors and not, and with x, another tensor or nothing as the
 residual.  Bit for bit against the operators of the oracle; the plane means, 64-bit sums
-in another order, to 1e-5.  tests/test_gate_shape_cpu.py checks that the shapes reach the
-forms named here."""
+in another order, to 1e-5.  tests/test_gate_shape_cpu.py checks that the shapes and parts reach the
+kernels and forms named here."""
 import numpy as np
 import pytest
 
@@ -132,6 +132,18 @@ def test_every_form(gpu, shape, residual):
     Case(shape, residual).check(gpu, "%s %s" % (shape, residual))
 
 
+# Whole vectors behind BatchNorm and ReLU, with a residual, may be whole_squeeze_gate_kernel's: with one of these two left out
+# they are squeeze_gate_kernel's, in the same forms.
+GENERIC = [dict(relu=False), dict(stats=False)]
+
+
+@pytest.mark.parametrize("residual", ["x", "other", "first"])
+@pytest.mark.parametrize("parts", GENERIC)
+@pytest.mark.parametrize("shape", sorted(s for s in FORMS if int(np.prod(s[2:])) % 4 == 0))
+def test_every_form_of_whole_vectors(gpu, shape, parts, residual):
+    Case(shape, residual, **parts).check(gpu, "%s %s %s" % (shape, parts, residual))
+
+
 @pytest.mark.parametrize("residual", ["x", "other"])
 @pytest.mark.parametrize("shape", WHOLE)
 def test_whole_rows(gpu, shape, residual):
@@ -154,7 +166,8 @@ ALIASED = [(8201, 1, 28, 28), (8201, 1, 27, 29), (2060, 1, 44, 44), (2060, 1, 45
 @pytest.mark.parametrize("alias,residual", [("x", "x"), ("x", "other"), ("residual", "other"), ("residual", "first"), ("x", None)])
 @pytest.mark.parametrize("shape", ALIASED)
 def test_result_in_place_of_an_operand(gpu, shape, alias, residual):
-    Case(shape, residual).check(gpu, "%s y is %s, residual %s" % (shape, alias, residual), alias=alias)
+    for parts in [{}] + (GENERIC[:1] if int(np.prod(shape[2:])) % 4 == 0 else []):
+        Case(shape, residual, **parts).check(gpu, "%s y is %s, residual %s %s" % (shape, alias, residual, parts), alias=alias)
 
 
 @pytest.mark.parametrize("off", [(1, 0, 0), (0, 2, 0), (0, 0, 3), (1, 1, 1)])
