@@ -23,6 +23,7 @@
 #include "launch.h"
 #include "ordered_sum.h"
 #include "libm_exact.h"
+#include "softmax_shape.h"
 
 #pragma clang fp contract(off)
 
@@ -1104,7 +1105,10 @@ struct TileQuotients {
 // then take 14 us per tile).  One set of registers: the folding waves of the
 // workgroups on a CU share one SIMD, and a second set that the next batch is
 // read into while this one is folded costs that SIMD a move per value.
-template <int TS_SHIFT, typename T, typename F>
+// HELD: the compiler keeps to that.  Otherwise it requests half of them ahead of the
+// first addition and half behind it: [4,231,304] softmax 6.9 us instead of 6.3, but with two passes
+// through LDS [97,119,927] 20.2 instead of 21.7.
+template <int TS_SHIFT, bool HELD = false, typename T, typename F>
 SHDW_DEVICE T fold_tile_column(const float* column, uint32_t dim, T acc, F f) {
   constexpr int kBatch = 16;
   uint32_t c = 0;
@@ -1112,6 +1116,7 @@ SHDW_DEVICE T fold_tile_column(const float* column, uint32_t dim, T acc, F f) {
     float v[kBatch];
 #pragma unroll
     for (int u = 0; u < kBatch; ++u) v[u] = column[(c + u) << TS_SHIFT];
+    if (HELD) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int u = 0; u < kBatch; ++u) acc = f(acc, v[u]);
   }
@@ -1389,21 +1394,22 @@ static void launch_normalize_tile(int outer_num, int dim, int inner_num, float p
 // the exponentials is an fp32 running sum and is always walked in index order, by wave 0 (the four waves
 // taking turns from workgroup to workgroup or from 256 to 256: level, 24.9 / 24.6 / 24.6 us here).
 //
-// LDS holds the rows of `pass_steps` steps (two at least, an even number), pass after pass; the sum goes on from
-// pass to pass in wave 0's lanes.
+// WHOLE: LDS holds all rows; otherwise those of `pass_steps` steps (two at least, an even number), pass after pass, and
+// the sum goes on from pass to pass in wave 0's lanes (a form of its own: with the passes' tests one pass takes 4 % more,
+// and spills two registers of eight and of ten vectors, as the passes do).
 //
 // [16,150,72,72], 99.5 MB: 20.0 us, all tiles on the chip at once; with whole columns in LDS and four tiles a CU,
 // so that a fifth of them came in a second round, 24.6.  29 vector instructions an element bound it
 // together with the rounds of load, walk and store; 28.8 us with the maxima by compare and select, a division and the
 // longer exponential, and five barriers.
-template <int TS_SHIFT, int ROWS, int N, int WAVES>
+template <int TS_SHIFT, int ROWS, int N, int WAVES, bool WHOLE>
 __global__ __launch_bounds__(kBlock, WAVES) void softmax_tile_kernel(const float* x, float* y, uint32_t dim,
                                                                uint32_t inner, uint32_t pass_steps, FastDiv f_tiles) {
   extern __shared__ __align__(16) float lds[];
   constexpr uint32_t TS = 1u << TS_SHIFT;
   constexpr uint32_t kWaves = kBlock / kWave;
   using Lane = TileLane<TS_SHIFT, ROWS>;
-  const uint32_t pass_rows = min(pass_steps * Lane::STEP, dim);
+  const uint32_t pass_rows = WHOLE ? dim : min(pass_steps * Lane::STEP, dim);
   uint64_t* tab = reinterpret_cast<uint64_t*>(lds + (pass_rows << TS_SHIFT));  // after the tile, 16-byte aligned
   float* maxima = reinterpret_cast<float*>(tab + 32);                    // [wave][TS]
   double* recip = reinterpret_cast<double*>(tab + 32);                   // [TS], when the maxima have been read
@@ -1440,12 +1446,12 @@ __global__ __launch_bounds__(kBlock, WAVES) void softmax_tile_kernel(const float
     }
   }
   float sum = 0.f;
-  for (uint32_t first = 0; first * Lane::STEP < dim; first += pass_steps) {
-    if (first) __syncthreads();  // wave 0 has read the rows of the pass before
+  for (uint32_t first = 0; WHOLE || first * Lane::STEP < dim; first += pass_steps) {
+    if (!WHOLE && first) __syncthreads();  // wave 0 has read the rows of the pass before
     if (lane.valid != 0) {
 #pragma unroll
       for (int u = 0; u < N; u += 2) {  // eight exponentials, each a chain, side by side
-        if (!lane.step(u) || static_cast<uint32_t>(u) - first >= pass_steps) continue;
+        if (!lane.step(u) || (!WHOLE && static_cast<uint32_t>(u) - first >= pass_steps)) continue;
 #pragma unroll
         for (int k = 0; k < 8; ++k) r[u + k / 4][k % 4] = libm::exact_expf_nonpositive(r[u + k / 4][k % 4] - m[k % 4], tab);
 #pragma unroll
@@ -1456,9 +1462,10 @@ __global__ __launch_bounds__(kBlock, WAVES) void softmax_tile_kernel(const float
     __syncthreads();  // also: every lane has its maxima before the sums replace them
     if (threadIdx.x < width && wave == 0) {
       __builtin_amdgcn_s_setprio(3);
-      sum = fold_tile_column<TS_SHIFT>(lds + threadIdx.x, min(pass_rows, dim - first * Lane::STEP), sum, [](float a, float v) { return a + v; });
+      sum = fold_tile_column<TS_SHIFT, WHOLE>(lds + threadIdx.x, min(pass_rows, dim - first * Lane::STEP), sum, [](float a, float v) { return a + v; });
       __builtin_amdgcn_s_setprio(0);
     }
+    if (WHOLE) break;
   }
   if (threadIdx.x < width && wave == 0) {
     handed[threadIdx.x] = sum;
@@ -1472,73 +1479,30 @@ __global__ __launch_bounds__(kBlock, WAVES) void softmax_tile_kernel(const float
     if (lane.has(u)) lane.store(y + base, u, q(r[u]));
 }
 
-constexpr size_t kExpTabBytes = 32 * sizeof(uint64_t);
-// the exp table and the maxima of four waves, whose place the sums (fp32) and their reciprocals (fp64) take
-// (32 positions of 512 channels, or 16 of 1024, with it: 66 KB at most, two workgroups per CU all the same)
-static size_t softmax_tile_extra_bytes(int ts) { return kExpTabBytes + static_cast<size_t>(kBlock / kWave) * ts * sizeof(float); }
+// behind the rows: the exp table and the maxima of four waves, whose place the sums (fp32) and their reciprocals (fp64) take
+static_assert(kSoftmaxTileLanes == kBlock && kSoftmaxTileTable == 32 * sizeof(uint64_t) && kBlock / kWave == 4, "softmax_shape.h counts in these");
 
-// How a shape is cut into tiles: positions, vectors a lane has room for (what fixes how many waves a SIMD
-// holds), steps of rows that LDS holds at a time.
-struct SoftmaxTiles {
-  int shift, slots;
-  uint32_t grid, pass_steps, lds_bytes;
-};
-
-// Tiles that all fit the chip at once finish together; a second round of a few of them costs as much as the
-// first.  So: as many positions as a lane's sixteen vectors hold (64, 32 or 16), or half of them where that
-// gives no more than three tiles a CU ([1,150,5184] 7.1 us with 64 positions, 5.7 with 32; [4,150,5184] 9.5, 8.7;
-// [8,150,5184], 1296 tiles of 32, 12.0 and 12.5; [4,500,3025] 19.2 with 32, 16.1 with 16; [16,300,1444] 16.2, 16.8), and
-// where a lane of 64 positions had more than ten vectors, as long as the chip holds seven a CU ([16,250,1444]
-// 16.1 and 13.7, [16,250,3136] 22.5 in two passes, 19.8; [64,250,1444] 41.7 and 45.7).  One pass through LDS where
-// the tiles fit beside each other so, otherwise two passes of half the rows ([16,150,5184] 24.8 and 20.0 us,
-// [16,180,3136] 21.6 and 16.6, [16,500,1600] 31.3 and 22.7, [16,1000,784] 38.7 and 26.8; where they fit the second pass
-// costs: [1,150,5184] 7.1 and 7.4).
-static SoftmaxTiles softmax_tiles(int outer_num, int dim, int inner_num) {
-  constexpr uint32_t kCus = 256, kCuLds = 160 * 1024, kFewTiles = 3 * kCus, kNarrowTiles = 7 * kCus;
-  const auto tiles = [&](int shift) {
-    return static_cast<uint32_t>(outer_num) * ((static_cast<uint32_t>(inner_num) + (1u << shift) - 1) >> shift);
-  };
-  const uint32_t d = static_cast<uint32_t>(dim);
-  SoftmaxTiles t{};
-  t.shift = d <= 256 ? 6 : d <= 512 ? 5 : 4;
-  if (t.shift > 4 && tiles(t.shift - 1) <= (t.shift == 6 && d > 160 ? kNarrowTiles : kFewTiles)) --t.shift;
-  t.grid = tiles(t.shift);
-  const uint32_t step = kBlock / ((1u << t.shift) / 4), steps = (d + step - 1) / step;
-  t.slots = steps <= 8 && t.shift < 6 ? 8 : steps <= 10 ? 10 : 16;
-  const uint32_t waves = t.slots == 8 ? 7 : t.slots == 10 ? 6 : 4;
-  const auto bytes = [&](uint32_t pass_steps) {
-    const uint32_t rows = pass_steps * step < d ? pass_steps * step : d;
-    return static_cast<uint32_t>((rows << t.shift) * sizeof(float) + softmax_tile_extra_bytes(1 << t.shift));
-  };
-  t.pass_steps = (steps + 1) & ~1u;
-  const uint32_t fit = kCuLds / bytes(t.pass_steps);
-  if (t.grid > kCus * (fit < waves ? fit : waves)) t.pass_steps = 2 * ((steps + 3) / 4);
-  t.lds_bytes = bytes(t.pass_steps);
-  return t;
-}
-
-template <int TS_SHIFT, int N, int WAVES>
+template <int TS_SHIFT, int N, bool WHOLE>
 static void launch_softmax_tile(const SoftmaxTiles& t, int dim, int inner_num, const float* x, float* y, hipStream_t st) {
+  constexpr int kWaves = softmax_tile_waves(N);
   const uint32_t d = static_cast<uint32_t>(dim), in = static_cast<uint32_t>(inner_num);
   const FastDiv ft = make_fastdiv((in + (1u << TS_SHIFT) - 1) >> TS_SHIFT);
   const auto launch = [&](auto kernel) { kernel<<<t.grid, kBlock, t.lds_bytes, st>>>(x, y, d, in, t.pass_steps, ft); };
   switch (tile_rows(inner_num, y)) {
-    case kRowsSector: launch(softmax_tile_kernel<TS_SHIFT, kRowsSector, N, WAVES>); break;
-    case kRowsQuad: launch(softmax_tile_kernel<TS_SHIFT, kRowsQuad, N, WAVES>); break;
-    default: launch(softmax_tile_kernel<TS_SHIFT, kRowsAny, N, WAVES>);
+    case kRowsSector: launch(softmax_tile_kernel<TS_SHIFT, kRowsSector, N, kWaves, WHOLE>); break;
+    case kRowsQuad: launch(softmax_tile_kernel<TS_SHIFT, kRowsQuad, N, kWaves, WHOLE>); break;
+    default: launch(softmax_tile_kernel<TS_SHIFT, kRowsAny, N, kWaves, WHOLE>);
   }
 }
 
+// Tiles of sixteen positions with eight vectors a lane are half tiles, three a CU at most: always whole.
 static void launch_softmax_tile(const SoftmaxTiles& t, int dim, int inner_num, const float* x, float* y, hipStream_t st) {
-  switch (t.shift * 100 + t.slots) {
-    case 610: launch_softmax_tile<6, 10, 6>(t, dim, inner_num, x, y, st); break;
-    case 616: launch_softmax_tile<6, 16, 4>(t, dim, inner_num, x, y, st); break;
-    case 508: launch_softmax_tile<5, 8, 7>(t, dim, inner_num, x, y, st); break;
-    case 510: launch_softmax_tile<5, 10, 6>(t, dim, inner_num, x, y, st); break;
-    case 516: launch_softmax_tile<5, 16, 4>(t, dim, inner_num, x, y, st); break;
-    case 408: launch_softmax_tile<4, 8, 7>(t, dim, inner_num, x, y, st); break;
-    case 410: launch_softmax_tile<4, 10, 6>(t, dim, inner_num, x, y, st); break;
-    default: launch_softmax_tile<4, 16, 4>(t, dim, inner_num, x, y, st);
+  switch (t.shift * 100 + t.slots + t.whole()) {
+#define SHDW_TILE(SHIFT, N, WHOLE) case SHIFT * 100 + N + WHOLE: launch_softmax_tile<SHIFT, N, WHOLE>(t, dim, inner_num, x, y, st); break;
+    SHDW_TILE(6, 8, true) SHDW_TILE(6, 8, false) SHDW_TILE(6, 10, true) SHDW_TILE(6, 10, false) SHDW_TILE(6, 16, true) SHDW_TILE(6, 16, false)
+    SHDW_TILE(5, 8, true) SHDW_TILE(5, 8, false) SHDW_TILE(5, 10, true) SHDW_TILE(5, 10, false) SHDW_TILE(5, 16, true) SHDW_TILE(5, 16, false)
+    SHDW_TILE(4, 8, true) SHDW_TILE(4, 10, true) SHDW_TILE(4, 10, false) SHDW_TILE(4, 16, true) SHDW_TILE(4, 16, false)
+#undef SHDW_TILE
   }
 }
 
@@ -2717,7 +2681,7 @@ static int run_softmax(int outer_num, int dim, int inner_num, const float* x, fl
     else
       softmax_columns_reg_kernel<64, 48><<<grid, kBlock, 0, st>>>(x, y, g.columns, d, fi);
   } else if (tile_fits(dim, inner_num, true)) {
-    const SoftmaxTiles t = softmax_tiles(outer_num, dim, inner_num);
+    const SoftmaxTiles t = softmax_tiles(outer_num, dim, inner_num, tile_rows(inner_num, y) == kRowsSector);
     if (pl->chosen(SHDW_PATH_TILE, t.shift, t.grid)) return SHDW_OK;
     launch_softmax_tile(t, dim, inner_num, x, y, st);
   } else if (TallLaunch t; tall_launch(outer_num, dim, inner_num, &t)) {

@@ -38,7 +38,9 @@ def build():
           "-Wl,--unresolved-symbols=ignore-all", "-o", readback])
     gate = os.path.join(HERE, "gate_shape.so")
     _run(["g++", "-std=c++17", "-O2", "-fPIC", "-shared", os.path.join(HERE, "gate_shape.cpp"), "-o", gate])
-    return [out, shapes, readback, gate]
+    softmax = os.path.join(HERE, "softmax_shape.so")
+    _run(["g++", "-std=c++17", "-O2", "-fPIC", "-shared", os.path.join(HERE, "softmax_shape.cpp"), "-o", softmax])
+    return [out, shapes, readback, gate, softmax]
 
 
 if __name__ == "__main__":
