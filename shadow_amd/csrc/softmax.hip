@@ -313,7 +313,7 @@ SHDW_DEVICE float wave_ordered_sum(const float* lds, uint32_t n) {
       for (uint32_t j = 0; j < 4; ++j) v[k + j] = first + k + j < n ? q[j] : 0.f;  // a sum that starts at +0 stays as it is
     }
     const uint32_t turns = min(static_cast<uint32_t>(kWave), (n - c0 + kSpan - 1) / kSpan);
-    if (turns >= kSideBySide && __builtin_amdgcn_ballot_w64(any_sign(v)) == 0) {
+    if (turns >= kSideBySide && __builtin_amdgcn_ballot_w64(any_sign(v) || !(sum >= 0.f)) == 0) {  // a NaN of an earlier chunk
       sum = wave_sum_in_order(v, sum);
       continue;
     }

@@ -67,6 +67,26 @@ def test_last_lanes_of_rows(gpu, rows, dim):
         assert_bit_exact(gpuops.softmax(x, rows, dim, 1, offset=dim % 4), oracle.softmax(x, rows, dim, 1), "softmax")
 
 
+# Rows longer than a chunk of 1024 of the ordered sum: a NaN in the first chunk and none behind it, sums that stay at a power of
+# two, ties in every addition, and exponentials of all sizes; a workgroup a row in registers, and the longest beyond.
+@pytest.mark.parametrize("dim", [1025, 2048, 3001, 4096, 8192, 9001])
+def test_long_rows_of_special_sums(gpu, dim):
+    rng = np.random.default_rng(dim)
+    ln2 = np.log(2.0)
+    kinds = [np.where(np.arange(dim) == 7, np.nan, rng.standard_normal(dim)),
+             np.where(np.arange(dim) < dim // 2, 0.0, -25 * ln2),
+             np.full(dim, -3.0),
+             -ln2 * rng.integers(0, 27, dim),
+             rng.uniform(-100.0, 0.0, dim),
+             np.where(np.arange(dim) < 1024, 0.0, -24 * ln2),
+             np.where(np.arange(dim) % 64 == 0, 0.0, -14 * ln2),
+             np.where(np.arange(dim) == dim - 1, 80.0, rng.uniform(-20.0, 0.0, dim))]
+    x = np.concatenate(kinds).astype(np.float32)
+    with np.errstate(all="ignore"):
+        want = oracle.softmax(x, len(kinds), dim, 1)
+        assert_bit_exact(gpuops.softmax(x, len(kinds), dim, 1, offset=dim % 4), want, "softmax")
+
+
 # a workgroup a row, in registers: one to eight vectors a lane, the last vector whole and cut, and the longest beyond
 @pytest.mark.parametrize("dim", [5, 1022, 1028, 2045, 2048, 2049, 4093, 4096, 4097, 8189, 8190, 8192, 8193, 12000])
 @pytest.mark.parametrize("rows", [1, 37])
