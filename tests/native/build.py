@@ -40,7 +40,9 @@ def build():
     _run(["g++", "-std=c++17", "-O2", "-fPIC", "-shared", os.path.join(HERE, "gate_shape.cpp"), "-o", gate])
     softmax = os.path.join(HERE, "softmax_shape.so")
     _run(["g++", "-std=c++17", "-O2", "-fPIC", "-shared", os.path.join(HERE, "softmax_shape.cpp"), "-o", softmax])
-    return [out, shapes, readback, gate, softmax]
+    ordered = os.path.join(HERE, "ordered_sum.so")
+    _run(["g++", "-std=c++17", "-O2", "-ffp-contract=off", "-fPIC", "-shared", os.path.join(HERE, "ordered_sum.cpp"), "-o", ordered])
+    return [out, shapes, readback, gate, softmax, ordered]
 
 
 if __name__ == "__main__":

@@ -11,6 +11,7 @@ import oracle
 import shadow_amd
 from shadow_amd import Buffer
 from tests.helpers import assert_bit_exact, assert_rel_close, normal, uniform, with_specials
+from tests.test_gpu_plane_average import rows_without_signs
 
 pytestmark = pytest.mark.gpu
 F = np.float32
@@ -157,6 +158,21 @@ def test_whole_rows(gpu, shape, residual):
 @pytest.mark.parametrize("shape", [(3, 2, 40, 40), (2, 2, 63, 65), (600, 1, 64, 64), (516, 1, 84, 84), (516, 1, 81, 81)])
 def test_long_rows_with_signs(gpu, shape):
     Case(shape, "other", relu=False, special=shape[0] < 9).check(gpu, "%s signs" % (shape,))
+
+
+# Rows whose sums are taken side by side and pass powers of two in every way: of whole_squeeze_gate_kernel and, without
+# BatchNorm or without ReLU, of the other kernel; whole, and in chunks that hand the sum on; whole vectors and not.  A
+# variance that makes the divisor 1, a mean of 0 and no scale or bias keep the elements as they are.
+@pytest.mark.parametrize("parts", [dict(), dict(stats=False), dict(relu=False)])
+@pytest.mark.parametrize("shape", [(39, 1, 32, 32), (39, 1, 31, 33), (39, 1, 45, 45), (39, 1, 84, 84), (516, 1, 84, 84), (516, 1, 81, 81)])
+def test_sums_side_by_side(gpu, shape, parts):
+    case = Case(shape, "other", scale=False, bias=False, **parts)
+    planes, length = shape[0], shape[2] * shape[3]
+    case.x = rows_without_signs(length, planes, length).reshape(shape)
+    if case.stats[0] is not None:
+        case.stats = (np.zeros(1, F), np.full(1, 1.998, F))
+        assert np.sqrt(F(1.998) * F(0.5) + F(1e-3)) == F(1)
+    case.check(gpu, "%s %s" % (shape, parts))
 
 
 # whole and chunked, whole vectors and not
