@@ -32,7 +32,7 @@ int source(int step, int lane) {
 }
 
 struct Counts {
-  long wrong = 0, one_by_one = 0;  // guesses that were off, lanes added one by one behind the first
+  long wrong = 0, one_by_one = 0, joins = 0;  // guesses that were off, lanes added one by one behind the first, runs joined anew
 };
 
 template <int K>
@@ -48,7 +48,7 @@ float wave_sum_in_order(const float (&v)[kLanes][K], float sum, Counts& n) {
     for (int l = 0; l < kLanes; ++l) moved[l] = source(step, l) < 0 ? 0.f : upto[source(step, l)];
     for (int l = 0; l < kLanes; ++l) upto[l] += moved[l];
   }
-  uint32_t power[kLanes], even[kLanes], odd[kLanes], first[kLanes], tag[kLanes];
+  uint32_t power[kLanes], own_even[kLanes], own_odd[kLanes], tag[kLanes];
   float from_even[kLanes], from_odd[kLanes];
   uint64_t all_starts = 0, all_passes = 0;
   for (int l = 0; l < kLanes; ++l) {
@@ -56,46 +56,77 @@ float wave_sum_in_order(const float (&v)[kLanes][K], float sum, Counts& n) {
     power[l] = before & kExponentBits;
     from_even[l] = float_of(guess), from_odd[l] = float_of(guess | 1u);
     for (int k = 0; k < K; ++k) from_even[l] += v[l][k], from_odd[l] += v[l][k];
-    even[l] = bits_of(from_even[l]) - guess, odd[l] = bits_of(from_odd[l]) - (guess | 1u);
+    own_even[l] = bits_of(from_even[l]) - guess, own_odd[l] = bits_of(from_odd[l]) - (guess | 1u);
     const uint32_t most = std::max(bits_of(from_even[l]), bits_of(from_odd[l]));
     const bool passes = l == 0 || power[l] == kExponentBits || most - power[l] >= kBinade;
     tag[l] = passes ? 1u : power[l];
     const bool starts = passes || tag[l] != (l ? tag[l - 1] : 1u);
-    first[l] = starts;
     all_starts |= static_cast<uint64_t>(starts) << l, all_passes |= static_cast<uint64_t>(passes) << l;
   }
-  for (int step = 0; step < 6; ++step) {
-    uint32_t e[kLanes], o[kLanes], f[kLanes];
-    for (int l = 0; l < kLanes; ++l) {
-      const int s = source(step, l);
-      e[l] = s < 0 ? 0 : even[s], o[l] = s < 0 ? 0 : odd[s], f[l] = s < 0 ? 0 : first[s];
+  uint32_t even[kLanes], odd[kLanes];
+  const auto join = [&](uint64_t starts) {
+    uint32_t first[kLanes];
+    for (int l = 0; l < kLanes; ++l) even[l] = own_even[l], odd[l] = own_odd[l], first[l] = starts >> l & 1u;
+    for (int step = 0; step < 6; ++step) {
+      uint32_t e[kLanes], o[kLanes], f[kLanes];
+      for (int l = 0; l < kLanes; ++l) {
+        const int s = source(step, l);
+        e[l] = s < 0 ? 0 : even[s], o[l] = s < 0 ? 0 : odd[s], f[l] = s < 0 ? 0 : first[s];
+      }
+      for (int l = 0; l < kLanes; ++l) {
+        const uint32_t joined_even = e[l] + (e[l] & 1u ? odd[l] : even[l]), joined_odd = o[l] + (o[l] & 1u ? even[l] : odd[l]);
+        if (!first[l]) even[l] = joined_even, odd[l] = joined_odd;
+        first[l] |= f[l];
+      }
     }
-    for (int l = 0; l < kLanes; ++l) {
-      const uint32_t joined_even = e[l] + (e[l] & 1u ? odd[l] : even[l]), joined_odd = o[l] + (o[l] & 1u ? even[l] : odd[l]);
-      if (!first[l]) even[l] = joined_even, odd[l] = joined_odd;
-      first[l] |= f[l];
-    }
-  }
-  const uint64_t whole_runs = all_starts & ~all_passes, ends = all_starts >> 1 | 1ull << 63;
+  };
+  join(all_starts);
   uint32_t bits = bits_of(bits_of(sum) & 1u ? from_odd[0] : from_even[0]);
+  const auto add_one = [&](int lane) {
+    float s = float_of(bits);
+    for (int k = 0; k < K; ++k) s += v[lane][k];
+    bits = bits_of(s);
+    ++n.one_by_one;
+  };
+  const uint64_t whole_runs = all_starts & ~all_passes, ends = all_starts >> 1 | 1ull << 63;
   int lane = 1;
   do {
     const int last = __builtin_ctzll(ends >> lane) + lane;
     const uint32_t low = power[lane], next = bits + (bits & 1u ? odd[last] : even[last]);
     if ((whole_runs >> lane & 1u) != 0) {
-      if (bits - low < kBinade && next - low < kBinade) {
+      if (bits - low >= kBinade || next - low >= kBinade) break;
+      bits = next;
+      lane = last + 1;
+      if (lane == kLanes) break;
+    }
+    add_one(lane);
+  } while (++lane < kLanes);
+  uint64_t new_starts = all_starts, new_whole = whole_runs;
+  int joins_left = 3;
+  while (lane < kLanes) {
+    const uint64_t new_ends = new_starts >> 1 | 1ull << 63;
+    const int last = __builtin_ctzll(new_ends >> lane) + lane;
+    const uint32_t low = power[lane], next = bits + (bits & 1u ? odd[last] : even[last]);
+    const bool inside = bits - low < kBinade;
+    if ((new_whole >> lane & 1u) != 0) {
+      if (inside && next - low < kBinade) {
         bits = next;
         lane = last + 1;
-        if (lane == kLanes) break;
-      } else {
-        ++n.wrong;
+        continue;
+      }
+      ++n.wrong;
+      if (joins_left != 0 && last > lane) {
+        --joins_left;
+        const uint64_t start = 1ull << (inside ? last : lane + 1);
+        new_starts |= start, new_whole |= start;
+        join(new_starts);
+        ++n.joins;
+        if (inside) continue;
       }
     }
-    float s = float_of(bits);
-    for (int k = 0; k < K; ++k) s += v[lane][k];
-    bits = bits_of(s);
-    ++n.one_by_one;
-  } while (++lane < kLanes);
+    add_one(lane);
+    ++lane;
+  }
   return float_of(bits);
 }
 
@@ -146,18 +177,47 @@ long scan(unsigned seed, long chunks, long* counts) {
     for (int i = 0; i < kLanes * K; ++i) want += v[i / K][i % K];
     if (bits_of(want) != bits_of(wave_sum_in_order(v, sum, n))) ++bad;
   }
-  counts[0] = n.wrong, counts[1] = n.one_by_one;
+  counts[0] = n.wrong, counts[1] = n.one_by_one, counts[2] = n.joins;
+  return bad;
+}
+
+// Uniform terms scaled so that their sum reaches a power of two just where a lane's terms end.
+template <int K>
+long near(unsigned seed, long chunks, long* counts) {
+  std::mt19937_64 gen(seed);
+  Counts n;
+  long bad = 0;
+  for (long c = 0; c < chunks; ++c) {
+    double t[kLanes * K], total = 0;
+    for (double& u : t) u = std::ldexp(static_cast<double>(gen() >> 11), -53);
+    const int end = K * (3 + static_cast<int>(gen() % 58));
+    for (int i = 0; i < end; ++i) total += t[i];
+    const double factor = std::ldexp(1.0, std::ilogb(total)) / total;
+    float v[kLanes][K], want = 0.f;
+    for (int i = 0; i < kLanes * K; ++i) want += v[i / K][i % K] = static_cast<float>(t[i] * factor);
+    if (bits_of(want) != bits_of(wave_sum_in_order(v, 0.f, n))) ++bad;
+  }
+  counts[0] = n.wrong, counts[1] = n.one_by_one, counts[2] = n.joins;
   return bad;
 }
 
 }  // namespace
 
-// Chunks whose sum is not the running sum's to the bit; counts: guesses that were off, lanes added one by one.
+// Chunks whose sum is not the running sum's to the bit; counts: guesses that were off, lanes added one by one, runs joined anew.
 extern "C" long ordered_sum_scan(int terms, unsigned seed, long chunks, long* counts) {
   switch (terms) {
     case 16: return scan<16>(seed, chunks, counts);
     case 28: return scan<28>(seed, chunks, counts);
     case 32: return scan<32>(seed, chunks, counts);
+  }
+  return -1;
+}
+
+extern "C" long ordered_sum_near(int terms, unsigned seed, long chunks, long* counts) {
+  switch (terms) {
+    case 16: return near<16>(seed, chunks, counts);
+    case 28: return near<28>(seed, chunks, counts);
+    case 32: return near<32>(seed, chunks, counts);
   }
   return -1;
 }

@@ -45,6 +45,14 @@ def settles_near_one(rng, length):
     return x
 
 
+def reaches_a_power_at_a_lanes_end(rng, length):
+    """The sum is a power of two, but for rounding, where a lane's 16, 28 or 32 terms end: guesses of it differ."""
+    x = rng.random(length)
+    end = int(rng.choice([16, 28, 32])) * int(rng.integers(3, 36))
+    total = x[:end].sum()
+    return x * (2.0 ** np.floor(np.log2(total)) / total)
+
+
 def rows_without_signs(seed, planes, length):
     """Rows whose running sums pass powers of two in every way: sums that grow evenly, ties in
     every addition, terms of all sizes, subnormal sums, sums that overflow, and a sign somewhere."""
@@ -62,7 +70,9 @@ def rows_without_signs(seed, planes, length):
              lambda: np.where(np.arange(length) == 1, np.nan, 1.0),
              lambda: np.where(np.arange(length) % 64 == 0, 2.0 ** 24, 1.0),
              lambda: np.where(np.arange(length) == 0, 2.0 ** 24 - 1, 0.5),
-             lambda: settles_near_one(rng, length)]
+             lambda: settles_near_one(rng, length),
+             lambda: reaches_a_power_at_a_lanes_end(rng, length),
+             lambda: reaches_a_power_at_a_lanes_end(rng, length)]
     for r in range(min(planes, 30 * len(kinds))):
         x[r] = kinds[r % len(kinds)]()
     return x

@@ -18,14 +18,26 @@ def native():
         build.build()
     lib = ctypes.CDLL(path)
     lib.ordered_sum_scan.restype = ctypes.c_long
-    lib.ordered_sum_scan.argtypes = [ctypes.c_int, ctypes.c_uint, ctypes.c_long, ctypes.POINTER(ctypes.c_long)]
+    lib.ordered_sum_near.restype = ctypes.c_long
+    for fn in (lib.ordered_sum_scan, lib.ordered_sum_near):
+        fn.argtypes = [ctypes.c_int, ctypes.c_uint, ctypes.c_long, ctypes.POINTER(ctypes.c_long)]
     return lib
 
 
 @pytest.mark.parametrize("seed", [1, 2, 3])
 @pytest.mark.parametrize("terms", [16, 28, 32])  # Softmax's rows, the gated block's, whole-plane averages
 def test_sums_of_a_wave_are_the_running_sums(native, terms, seed):
-    counts = (ctypes.c_long * 2)()
+    counts = (ctypes.c_long * 3)()
     assert native.ordered_sum_scan(terms, seed, 20000, counts) == 0
-    wrong, one_by_one = counts
-    assert wrong > 100 and one_by_one > 20000
+    wrong, one_by_one, joined_anew = counts
+    assert wrong > 1000 and one_by_one > 20000 and joined_anew > 1000
+
+
+@pytest.mark.parametrize("terms", [16, 28, 32])
+def test_a_wrong_guess_leaves_few_lanes_to_add_one_by_one(native, terms):
+    """Sums that pass a power of two within rounding of a lane's end, any lane: what is left of the run is joined anew."""
+    counts = (ctypes.c_long * 3)()
+    assert native.ordered_sum_near(terms, 7, 4000, counts) == 0
+    wrong, one_by_one, joined_anew = counts
+    assert wrong > 400 and joined_anew > 400
+    assert one_by_one < 9 * 4000  # the lanes that a sum passes powers of two in, about six
