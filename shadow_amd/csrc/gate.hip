@@ -378,7 +378,8 @@ __global__ __launch_bounds__(kBlock, gate_waves(SLOTS, ONE)) void squeeze_gate_k
 // costs its arithmetic and little else, and the walk reads LDS ahead of its additions.  Against squeeze_gate_kernel, with
 // 47 vector instructions an element and a lane of a wave for each row's walk: [32,512,28,28] 25.4 -> 22.6 us, [64,64,56,56]
 // 41.4 -> 24.8, [8,128,64,64] 29.9 -> 10.8, [16,256,48,48] 32.6 -> 21.9, [16,64,40,40] 11.2 -> 8.8.
-constexpr int whole_waves(int pieces) { return pieces <= 4 ? 6 : pieces <= 8 ? 5 : 3; }
+// Seven workgroups a CU with up to four vectors a lane: 14000 rows of 448 12.5 us as six, 8.5.
+constexpr int whole_waves(int pieces) { return pieces <= 4 ? 7 : pieces <= 8 ? 5 : 3; }
 
 template <int PIECES, int RESIDUAL>
 __global__ __launch_bounds__(kBlock, whole_waves(PIECES)) void whole_squeeze_gate_kernel(

@@ -94,7 +94,6 @@ SHDW_DEVICE float wave_sum_in_order(const float (&v)[K], float sum) {
     from_even += v[k];
     from_odd += v[k];
   }
-  const uint32_t own_even = __float_as_uint(from_even) - guess, own_odd = __float_as_uint(from_odd) - (guess | 1u);
   // passes: this lane's terms are added one by one; first: at, and behind, such a lane, and where e changes
   const uint32_t lane_id = threadIdx.x % kWave;
   const bool passes = lane_id == 0 || power == kExponentBits ||
@@ -102,18 +101,8 @@ SHDW_DEVICE float wave_sum_in_order(const float (&v)[K], float sum) {
   const uint32_t tag = passes ? 1u : power;  // of the powers none is 1
   const uint32_t tag_before = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(1, static_cast<int>(tag), kDppWaveShr1, 0xf, 0xf, false));
   const bool starts = passes || tag != tag_before;
-  const auto join = [&](uint64_t at) {
-    UnitRun run{own_even, own_odd, static_cast<uint32_t>(at >> lane_id) & 1u};
-    join_run<kDppShr1, 0xf>(run);
-    join_run<kDppShr2, 0xf>(run);
-    join_run<kDppShr4, 0xf>(run);
-    join_run<kDppShr8, 0xf>(run);
-    join_run<kDppBcast15, 0xa>(run);
-    join_run<kDppBcast31, 0xc>(run);
-    return run;
-  };
   const uint64_t all_starts = __builtin_amdgcn_ballot_w64(starts), whole_runs = all_starts & ~__builtin_amdgcn_ballot_w64(passes);
-  UnitRun run{own_even, own_odd, starts ? 1u : 0u};
+  UnitRun run{__float_as_uint(from_even) - guess, __float_as_uint(from_odd) - (guess | 1u), starts ? 1u : 0u};
   join_run<kDppShr1, 0xf>(run);
   join_run<kDppShr2, 0xf>(run);
   join_run<kDppShr4, 0xf>(run);
@@ -150,7 +139,26 @@ SHDW_DEVICE float wave_sum_in_order(const float (&v)[K], float sum) {
   if (__builtin_expect(lane == kWave, 1)) return __uint_as_float(bits);
 
   // The same from `lane` on, the first of a run whose guess was wrong, with new starts.  Every turn is of one lane at
-  // least, or is one of the joins.
+  // least, or is one of the joins.  What a lane adds is the same from any even, from any odd number of units that keeps it
+  // inside its power of two: taken again, from the lowest, so that the loop above need not hold it.  Two registers, with
+  // which the gated block's rows of four vectors a lane have 74 and a workgroup a CU less (gate.hip).
+  const auto join = [&](uint64_t at) {
+    const uint32_t id = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));  // lane_id
+    float low_even = __uint_as_float(power), low_odd = __uint_as_float(power | 1u);
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      low_even += v[k];
+      low_odd += v[k];
+    }
+    UnitRun joined{__float_as_uint(low_even) - power, __float_as_uint(low_odd) - (power | 1u), static_cast<uint32_t>(at >> id) & 1u};
+    join_run<kDppShr1, 0xf>(joined);
+    join_run<kDppShr2, 0xf>(joined);
+    join_run<kDppShr4, 0xf>(joined);
+    join_run<kDppShr8, 0xf>(joined);
+    join_run<kDppBcast15, 0xa>(joined);
+    join_run<kDppBcast31, 0xc>(joined);
+    return joined;
+  };
   uint64_t new_starts = all_starts, new_whole = whole_runs;
   uint32_t joins_left = 3;
   while (lane < kWave) {

@@ -356,8 +356,10 @@ SHDW_DEVICE double sequential_sum(const float* lds, uint32_t n) {
 // Bound by its chain: one load, three barriers, the ordered sum (2 us for 1000).  With the row staged in LDS and
 // four passes over it there: [16,1000] 5.0 -> 4.1 us, [500,1024] 6.5 -> 4.6, [4,4096] 10.6 -> 7.3,
 // [1000,4096] 22.0 -> 11.3; waves without a part of a short row skip the arithmetic ([1000,200] 4.5 -> 3.9, [550,44] 3.8 -> 3.4).
+// Seven workgroups of eight vectors a lane are 72 registers; with 73, and six, [1792,4100] takes 19.5 us instead of 15.7, and
+// [2000,4500] 24.6 instead of 22.
 template <int V>
-__global__ __launch_bounds__(kBlock) void softmax_row_kernel(const float* x, float* y, uint32_t dim) {
+__global__ __launch_bounds__(kBlock, V == 8 ? 7 : 8) void softmax_row_kernel(const float* x, float* y, uint32_t dim) {
   extern __shared__ __align__(16) float lds[];
   __shared__ uint64_t tab[32];
   __shared__ float wave_max[kBlock / kWave];

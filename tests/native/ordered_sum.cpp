@@ -117,6 +117,11 @@ float wave_sum_in_order(const float (&v)[kLanes][K], float sum, Counts& n) {
       ++n.wrong;
       if (joins_left != 0 && last > lane) {
         --joins_left;
+        for (int l = 0; l < kLanes; ++l) {  // again, from the lowest even and odd number of units of the lane's power of two
+          float low_even = float_of(power[l]), low_odd = float_of(power[l] | 1u);
+          for (int k = 0; k < K; ++k) low_even += v[l][k], low_odd += v[l][k];
+          own_even[l] = bits_of(low_even) - power[l], own_odd[l] = bits_of(low_odd) - (power[l] | 1u);
+        }
         const uint64_t start = 1ull << (inside ? last : lane + 1);
         new_starts |= start, new_whole |= start;
         join(new_starts);
