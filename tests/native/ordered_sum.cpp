@@ -88,7 +88,7 @@ float wave_sum_in_order(const float (&v)[kLanes][K], float sum, Counts& n) {
     bits = bits_of(s);
     ++n.one_by_one;
   };
-  const uint64_t whole_runs = all_starts & ~all_passes, ends = all_starts >> 1 | 1ull << 63;
+  const uint64_t whole_runs = (all_starts & ~all_passes) | 1u, ends = all_starts >> 1 | 1ull << 63;
   int lane = 1;
   do {
     const int last = __builtin_ctzll(ends >> lane) + lane;
@@ -97,7 +97,7 @@ float wave_sum_in_order(const float (&v)[kLanes][K], float sum, Counts& n) {
       if (bits - low >= kBinade || next - low >= kBinade) break;
       bits = next;
       lane = last + 1;
-      if (lane == kLanes) break;
+      if ((whole_runs >> lane % kLanes & 1u) != 0) break;
     }
     add_one(lane);
   } while (++lane < kLanes);
@@ -186,12 +186,13 @@ long scan(unsigned seed, long chunks, long* counts) {
   return bad;
 }
 
-// Uniform terms scaled so that their sum reaches a power of two just where a lane's terms end.
+// Uniform terms scaled so that their sum reaches a power of two just where a lane's terms end; counts[3]: the most lanes
+// of a chunk that were added one by one.
 template <int K>
 long near(unsigned seed, long chunks, long* counts) {
   std::mt19937_64 gen(seed);
   Counts n;
-  long bad = 0;
+  long bad = 0, most = 0;
   for (long c = 0; c < chunks; ++c) {
     double t[kLanes * K], total = 0;
     for (double& u : t) u = std::ldexp(static_cast<double>(gen() >> 11), -53);
@@ -200,9 +201,11 @@ long near(unsigned seed, long chunks, long* counts) {
     const double factor = std::ldexp(1.0, std::ilogb(total)) / total;
     float v[kLanes][K], want = 0.f;
     for (int i = 0; i < kLanes * K; ++i) want += v[i / K][i % K] = static_cast<float>(t[i] * factor);
+    const long before = n.one_by_one;
     if (bits_of(want) != bits_of(wave_sum_in_order(v, 0.f, n))) ++bad;
+    most = std::max(most, n.one_by_one - before);
   }
-  counts[0] = n.wrong, counts[1] = n.one_by_one, counts[2] = n.joins;
+  counts[0] = n.wrong, counts[1] = n.one_by_one, counts[2] = n.joins, counts[3] = most;
   return bad;
 }
 

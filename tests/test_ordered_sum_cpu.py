@@ -36,8 +36,9 @@ def test_sums_of_a_wave_are_the_running_sums(native, terms, seed):
 @pytest.mark.parametrize("terms", [16, 28, 32])
 def test_a_wrong_guess_leaves_few_lanes_to_add_one_by_one(native, terms):
     """Sums that pass a power of two within rounding of a lane's end, any lane: what is left of the run is joined anew."""
-    counts = (ctypes.c_long * 3)()
+    counts = (ctypes.c_long * 4)()
     assert native.ordered_sum_near(terms, 7, 4000, counts) == 0
-    wrong, one_by_one, joined_anew = counts
+    wrong, one_by_one, joined_anew, most = counts
     assert wrong > 400 and joined_anew > 400
     assert one_by_one < 9 * 4000  # the lanes that a sum passes powers of two in, about six
+    assert most <= 10  # of any chunk: those, and two or three more for a wrong guess
