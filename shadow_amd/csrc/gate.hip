@@ -8,16 +8,17 @@
 //
 // Arithmetic per element is exactly the operator sequence (parts that are absent
 // are skipped, or done with a neutral operand that keeps every bit: x - 0, x * 1,
-// x + (-0)).  The plane sum is fp32, front to back, by one lane, as Vision::Pooling
+// x + (-0)).  The plane sum is fp32, front to back, or has its bits (ordered_sum.h), as Vision::Pooling
 // adds; the mean at the end is fp64, rounded once after the divide.
 //
 // Rows of whole vectors behind BatchNorm and ReLU take whole_squeeze_gate_kernel, all others squeeze_gate_kernel.
 //
-// What bounds it: rows held in LDS and registers leave four to six workgroups on a CU, whose loads, ordered sums and
+// What bounds it: rows held in LDS and registers leave five to seven workgroups on a CU, with nine vectors a lane and more
+// three, and two where a row takes more than 52 KB of LDS, whose loads, ordered sums and
 // stores overlap each other's; the sums, dependent additions, take 2 ns each (long rows without signs
 // less); and 30 to 60 vector instructions an element.  One block with its tail takes, per call: [32,512,28,28]
 // (103 MB) 21.8 us (its five launches 78), [64,64,56,56] 24.6, [16,64,112,112] 32.3, [8,128,64,64] 10.9,
-// [64,512,14,14] 11.5, [64,1024,7,7] 7.8, [16,64,55,55] 10.1, [16,64,111,113] 29.3.  With a lane for each row's sum that
+// [64,512,14,14] 11.5, [64,1024,7,7] 7.8, [16,64,55,55] 10.1, [16,64,111,113] 28.3.  With a lane for each row's sum that
 // reads it from LDS, and one kernel for all: 25.3, 41.4, 70.1, 30.2, 11.4, 7.8, 24.2 and 70.1.
 #include <hip/hip_runtime.h>
 
@@ -263,7 +264,7 @@ __global__ __launch_bounds__(kBlock, gate_waves(SLOTS, ONE)) void squeeze_gate_k
     asm("" : "+v"(sub), "+v"(lead));
     // Read again for every chunk: of a row's parameters that stay the same the compiler takes the front of
     // all slots ahead of the chunks, and spills what does not fit (500 bytes a lane of sixteen
-    // vectors: [16,64,112,112] 92 us instead of 72, [16,64,96,96] 75 instead of 54).
+    // vectors: [16,64,112,112] 92 us instead of 72, [16,64,96,96] 75 instead of 54, when all blocks came here).
     if (ONE) g = row_params[min(lead, nrows - 1)];
     uint32_t k = 0, turn_row = 0;
 #pragma unroll

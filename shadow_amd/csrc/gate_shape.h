@@ -30,7 +30,8 @@ struct GateShape {
 // (28.9 KB of 160), as many as the registers of eight vectors a lane leave room for
 // (gate_waves).  Rows that do not fit whole go through LDS in chunks (four of the
 // 112x112 planes' rows per CU instead of three, [16,64,112,112] 124 -> 81 us; with 18 KB
-// eight 28x28 planes would be cut too, [32,512,28,28] 26.0 -> 28.1), unless there are no
+// eight 28x28 planes would be cut too, [32,512,28,28] 26.0 -> 28.1; both before gate_whole took them
+// where BatchNorm, ReLU and a residual are there), unless there are no
 // more than two workgroups per CU to hold.
 constexpr uint32_t kGateTileBytes = 26000, kGateMaxTileBytes = 62000, kGateCus = 256;
 

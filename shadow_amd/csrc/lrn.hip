@@ -230,7 +230,7 @@ __global__ __launch_bounds__(kBlock, 5) void lrn_window_kernel(const float* x, f
     return;
   }
   // Runs of positions that start inside a line share it with the run before: the XCD's own neighbours then
-  // ([44,96,55,55] 32.3 -> 30.4 us, [64,256,27,27] 34.1 -> 30.2; no gain where rows are whole vectors).
+  // ([44,96,55,55] 31.2 -> 29.8 us, [64,256,27,27] 34.1 -> 30.3; no gain where rows are whole vectors).
   const uint32_t block = STREAM ? blockIdx.x : xcd_contiguous(blockIdx.x, whole);
   lrn_window<SIZE, WAVES, STREAM>(tables, hands, block, 0, x, y, positions, step, channels, alpha_over_size, neg_beta, k, f_step);
 }

@@ -296,7 +296,7 @@ SHDW_DEVICE float block_max_any_order(float m, float* scratch4) {
 // Front-to-back fp32 sum of lds[0..n) by a whole wave, the result in all its lanes: a lane holds 16
 // consecutive elements of a chunk of 1024 and the sum goes from lane to lane, as in
 // pool_rows_stream_kernel (by one lane out of LDS, eight 128-bit reads at a time, softmax of [16,1000]
-// takes 7.2 us, so 5.6; [8192,4096] 120 and 99).  From 42 lanes' worth on, the additions are taken side by side
+// takes 7.2 us, so 5.6; [8192,4096] 120 and 99, in softmax_row_kernel 53).  From 42 lanes' worth on, the additions are taken side by side
 // (ordered_sum.h; no exponential is negative): [16,1000] 5.6 -> 5.0 us, [4,4096] 15.8 -> 10.4, [512,8192] 33.9 -> 22.6;
 // [16,700] 4.8 and 4.7, [32,512] 4.1 and 4.5.  lds is 16-byte aligned and readable up to the next multiple of four.
 SHDW_DEVICE float wave_ordered_sum(const float* lds, uint32_t n) {
@@ -2651,7 +2651,7 @@ static int run_softmax(int outer_num, int dim, int inner_num, const float* x, fl
   }
   // Fewer rows than the forms above take: a workgroup each, whose lanes share the row, where the packed
   // kernel walks a row with one lane for the maximum and one for the sum ([1,256,1] 3.3 us against 7.0, [256,64,1]
-  // 3.3 / 16.3, [1000,200,1] 4.1 / 19.8, [1000,18,1] 3.7 / 8.1).
+  // 3.3 / 16.3, [1000,200,1] 3.7 / 19.8, [1000,18,1] 3.5 / 8.1).
   const bool few_rows = inner_num == 1 && outer_num < kRowsMinRows && g.use_slab;
   if (const uint32_t group = few_rows ? 0u : packed_group(dim, inner_num)) {
     const uint32_t slabs = static_cast<uint32_t>(outer_num);

@@ -1358,19 +1358,19 @@ constexpr int kPlaneStreamMinLen = 256;
 // Rows per wave: up to eight while there are 512 waves (two a CU) and more.  Every wave issues all
 // the additions of a row whatever the number of its rows, so few rows go one to a wave and many
 // eight, from where on memory bounds the launch and shorter row pieces do not help it.  With 1 / 2
-// / 4 / 8 / 16 rows per wave: 512 rows of 12544 36.7 / 36.3 / 40.5 / 47.6 / 73.6 us, 2048 of 3136
-// 13.4 / 13.4 / 12.6 / 14.1 / 21.1, 4096 of 3136 23.8 / 15.2 / 14.5 / 14.8 / 21.8, 16384 of 784
-// 24.2 / 14.8 / 11.8 / 10.7 / 11.1, 50200 of 256 33.3 / 18.3 / 11.9 / 9.9 / 10.1.
+// / 4 / 8 rows per wave: 2500 rows of 3136 16.6 / 11.6 / 10.8 / 12.8 us, 4096 of 3136 21.0 / 14.1 / 12.2 / 13.6,
+// 16384 of 784 21.4 / 13.4 / 11.7 / 9.3, 50200 of 256 30.5 / 17.3 / 10.8 / 8.7.
 static int stream_rows_per_wave(uint32_t rows) {
   int g = 1;
   while (g < 8 && rows / static_cast<uint32_t>(2 * g) >= 512u) g <<= 1;
   return g;
 }
 
-// Up to here a wave a row fills no more than two waves of a SIMD, and rows with signs lose nothing by not
-// sharing a wave (2500 x 3136 of N(0, 1) 11.0 us as four rows a wave, 20.1 as one; without signs 11.1 and
-// 10.7); below 1152 columns the additions in turn are over as soon (2048 x 1024 5.1 us in turn, 5.9 side by
-// side, 2048 x 1200 6.0 and 5.5).
+// Up to here a wave a row fills no more than two waves of a SIMD, and rows with signs, which a look at the data alone
+// tells from the others, lose little by not sharing a wave.  Shared by as many as suits them / this kernel, us: with signs
+// 512 x 12544 28.3 / 28.9, 1024 x 3136 9.3 / 9.5, 2048 x 3136 10.2 / 10.9, 2048 x 12544, the most, 33.4 / 39.0 and 2500 x 3136
+// 10.8 / 17.1; without 28.7 / 11.1, 9.4 / 5.8, 10.4 / 7.0, 33.6 / 17.2 and 10.9 / 8.9.  Below 1152 columns the additions in turn
+// are over as soon (2048 x 1024 5.1 us in turn, 5.9 side by side, 2048 x 1200 5.3 and 4.7).
 constexpr uint32_t kRunsMaxRows = 2048, kRunsMinLen = 1152;
 
 static void launch_pool_rows_stream(const float* x, float* y, uint32_t rows, uint32_t len, hipStream_t st) {
