@@ -303,6 +303,7 @@ SHDW_DEVICE float wave_ordered_sum(const float* lds, uint32_t n) {
   constexpr uint32_t kSpan = 16, kChunk = kWave * kSpan, kSideBySide = 42;
   const uint32_t lane = threadIdx.x % kWave;
   float sum = 0.f;
+  uint64_t nan = 0;  // lanes that have seen one, which the sum then is: of the terms alone, so that it does not wait for the sum
   for (uint32_t c0 = 0; c0 < n; c0 += kChunk) {
     const uint32_t first = c0 + lane * kSpan, last = (n - 1) & ~3u;
     float v[kSpan];
@@ -313,7 +314,8 @@ SHDW_DEVICE float wave_ordered_sum(const float* lds, uint32_t n) {
       for (uint32_t j = 0; j < 4; ++j) v[k + j] = first + k + j < n ? q[j] : 0.f;  // a sum that starts at +0 stays as it is
     }
     const uint32_t turns = min(static_cast<uint32_t>(kWave), (n - c0 + kSpan - 1) / kSpan);
-    if (turns >= kSideBySide && __builtin_amdgcn_ballot_w64(any_sign(v) || !(sum >= 0.f)) == 0) {  // a NaN of an earlier chunk
+    nan |= __builtin_amdgcn_ballot_w64(any_sign(v));
+    if (turns >= kSideBySide && nan == 0) {
       sum = wave_sum_in_order(v, sum);
       continue;
     }
@@ -357,9 +359,9 @@ SHDW_DEVICE double sequential_sum(const float* lds, uint32_t n) {
 // four passes over it there: [16,1000] 5.0 -> 4.1 us, [500,1024] 6.5 -> 4.6, [4,4096] 10.6 -> 7.3,
 // [1000,4096] 22.0 -> 11.3; waves without a part of a short row skip the arithmetic ([1000,200] 4.5 -> 3.9, [550,44] 3.8 -> 3.4).
 // Seven workgroups of eight vectors a lane are 72 registers; with 73, and six, [1792,4100] takes 19.5 us instead of 15.7, and
-// [2000,4500] 24.6 instead of 22.
+// [2000,4500] 24.6 instead of 22; held to 72 by launch bounds the compiler orders all of it otherwise ([53,7773] 14.1, not 13.5).
 template <int V>
-__global__ __launch_bounds__(kBlock, V == 8 ? 7 : 8) void softmax_row_kernel(const float* x, float* y, uint32_t dim) {
+__global__ __launch_bounds__(kBlock) void softmax_row_kernel(const float* x, float* y, uint32_t dim) {
   extern __shared__ __align__(16) float lds[];
   __shared__ uint64_t tab[32];
   __shared__ float wave_max[kBlock / kWave];

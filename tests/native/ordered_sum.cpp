@@ -31,6 +31,18 @@ int source(int step, int lane) {
   return lane >= 32 ? 31 : -1;
 }
 
+// Lanes that have met a start behind a step, of those that had in front of it, in a mask as join_runs_masked has them; the last
+// step's are not asked for.
+uint64_t met(int step, uint64_t starts) {
+  switch (step) {
+    case 0: return starts | (starts << 1 & 0xfffefffefffefffeull);
+    case 1: return starts | (starts << 2 & 0xfffcfffcfffcfffcull);
+    case 2: return starts | (starts << 4 & 0xfff0fff0fff0fff0ull);
+    case 3: return starts | (starts << 8 & 0xff00ff00ff00ff00ull);
+    default: return starts | (starts >> 15 & 0x0000000100000001ull) * 0xffff0000ull;
+  }
+}
+
 struct Counts {
   long wrong = 0, one_by_one = 0, joins = 0;  // guesses that were off, lanes added one by one behind the first, runs joined anew
 };
@@ -65,19 +77,18 @@ float wave_sum_in_order(const float (&v)[kLanes][K], float sum, Counts& n) {
   }
   uint32_t even[kLanes], odd[kLanes];
   const auto join = [&](uint64_t starts) {
-    uint32_t first[kLanes];
-    for (int l = 0; l < kLanes; ++l) even[l] = own_even[l], odd[l] = own_odd[l], first[l] = starts >> l & 1u;
+    for (int l = 0; l < kLanes; ++l) even[l] = own_even[l], odd[l] = own_odd[l];
     for (int step = 0; step < 6; ++step) {
-      uint32_t e[kLanes], o[kLanes], f[kLanes];
+      uint32_t e[kLanes], o[kLanes];
       for (int l = 0; l < kLanes; ++l) {
         const int s = source(step, l);
-        e[l] = s < 0 ? 0 : even[s], o[l] = s < 0 ? 0 : odd[s], f[l] = s < 0 ? 0 : first[s];
+        e[l] = s < 0 ? 0 : even[s], o[l] = s < 0 ? 0 : odd[s];
       }
       for (int l = 0; l < kLanes; ++l) {
         const uint32_t joined_even = e[l] + (e[l] & 1u ? odd[l] : even[l]), joined_odd = o[l] + (o[l] & 1u ? even[l] : odd[l]);
-        if (!first[l]) even[l] = joined_even, odd[l] = joined_odd;
-        first[l] |= f[l];
+        if (!(starts >> l & 1u)) even[l] = joined_even, odd[l] = joined_odd;
       }
+      starts = met(step, starts);
     }
   };
   join(all_starts);
