@@ -71,7 +71,7 @@ constexpr int kDppShr1 = 0x111, kDppShr2 = 0x112, kDppShr4 = 0x114, kDppShr8 = 0
 constexpr int kDppBcast15 = 0x142, kDppBcast31 = 0x143;  // the last lane of 16, of 32, to the 16, 32 behind them
 
 // All lanes' runs joined with the lanes that have met a start in a mask: two registers fewer than six of join_run, but
-// 0.05 us more (with it everywhere 64 averages of 50176 take 29.0 us instead of 27.8).
+// 0.05 us more (with it everywhere 64 averages of 50176 take 29.0 us instead of 27.6).
 SHDW_DEVICE void join_runs_masked(UnitRun& r, uint64_t starts) {
   const auto first = [&] { return __builtin_amdgcn_inverse_ballot_w64(starts); };
   join_units<kDppShr1, 0xf>(r, first());
